@@ -11,8 +11,7 @@ constexpr int kBlock = 256;
 // What the finishing pass of a forward rhs has to do, as far as the host knows it:
 // far-field patches present; whether the patches are at most one Kolmogorov forcing
 // over the whole domain (`kolmogorov`: its strength array, null for none) -- then, with
-// no dissipation and no sources, the pass rides on the last derivative kernel of the
-// periodic 3-D path.
+// no dissipation and no sources, the marches of the periodic 3-D path do it themselves.
 struct FinishInfo {
   int has_farfield = 0;
   int simple = 0;
@@ -40,10 +39,9 @@ struct RkStage {
   bool stress_ready = false;
 };
 // What launch_rhs_forward did with `rk`.
-enum RkDone { RK_NOT_APPLIED = 0, RK_IN_PLACE = 1, RK_TO_YOUT = 2 };
-// RK_IN_PLACE / RK_TO_YOUT when it applied `rk` (then rhs is not written; with RK_TO_YOUT
-// the new stage state is in rk->yout and y is unchanged); RK_NOT_APPLIED when the caller
-// still has to (launch_rk_forward) -- always for rk == nullptr.
+enum RkDone { RK_NOT_APPLIED = 0, RK_TO_YOUT = 2 };
+// RK_TO_YOUT when it applied `rk` (then rhs is not written, the new stage state is in
+// rk->yout and y is unchanged); RK_NOT_APPLIED when the caller still has to (launch_rk_forward) -- always for rk == nullptr.
 int launch_rhs_forward(const Geo& g, const Patches* P, const double* q, double* rhs, double* w,
                        double* G, double* t, double* F, const double* control, long control_stride,
                        const Source* src, int nsrc, const double* src_amp, long src_inst_stride,
@@ -59,6 +57,10 @@ bool launch_rhs_adjoint(const Geo& g, const Patches* P, const double* q, const d
 // heat-flux kernel (9 slots of the 12-slot gradient buffer S); the march itself, which
 // writes rhs, or with rk (rk->yout set, not q) applies the RK4 stage out of place.
 bool fwd3d_march_path(const Geo& g, const FinishInfo& fin, int nsrc);
+// Rows of a march tile, and the work units of a march with tiles of mtile x kMarchRows points
+// and zc planes per unit (per instance).
+constexpr int kMarchRows = 16;
+int march_units(const Geo& g, int mtile, int zc);
 // Whether the forward and the adjoint rhs both run on the 3-D marches, each from the stress
 // / heat-flux slots of its state that launch_stress3d writes into G: then slots the forward
 // stage computed serve the adjoint stage about the same state.

@@ -12,6 +12,14 @@
 
 namespace mgd {
 
+// Accesses of values that no other block reads (stage outputs, RK operands): STREAM marks
+// them non-temporal, so that the caches keep the stencil operands, whose halo lines
+// neighbouring tiles share.
+template <bool STREAM>
+__device__ __forceinline__ double ld_own(const double* p) {
+  return STREAM ? __builtin_nontemporal_load(p) : *p;
+}
+
 __device__ __forceinline__ long gidx() { return (long)blockIdx.x * blockDim.x + threadIdx.x; }
 
 // ------------------------------------------------------------------ state helpers
@@ -59,13 +67,146 @@ __global__ void __launch_bounds__(kBlock) k_grad(Geo g, int d, const double* __r
   for (int c = 0; c <= ND; ++c) Gi[(c * ND + d) * g.N + p] = jm * out[c];
 }
 
+// One work unit of a 3-D march: a column tile of at most BX x BY points, from a balanced
+// partition of the x and y lines (the first n mod tiles of them hold one point more), over
+// the planes [z0, z1) of a z chunk.  XCD-aware order: blocks are dealt to the 8 XCDs
+// round-robin by index, so block b takes unit (b mod 8) * ceil(units / 8) + b / 8, tiles
+// x-fastest: each XCD marches one contiguous band, and the halo lines of neighbouring tiles
+// are fetched into its own L2 by blocks running beside it.  False for the padding blocks of
+// a grid rounded up to a multiple of 8 (uniform over the block).
+struct MarchUnit {
+  int x0, y0, sx, sy, z0, z1;
+};
+template <int BX, int BY>
+__device__ __forceinline__ bool march_unit(const Geo& g, int zc, MarchUnit& u) {
+  const int ntx = (g.n[0] + BX - 1) / BX, nty = (g.n[1] + BY - 1) / BY;
+  const int ntiles = ntx * nty, nunits = ntiles * ((g.n[2] + zc - 1) / zc);
+  const int per_xcd = (nunits + 7) / 8;
+  const int unit = (int)(blockIdx.x % 8) * per_xcd + (int)(blockIdx.x / 8);
+  if (unit >= nunits) return false;
+  const int tile = unit % ntiles, bx = tile % ntx, by = tile / ntx;
+  const int qx = g.n[0] / ntx, ex = g.n[0] % ntx, qy = g.n[1] / nty, ey = g.n[1] % nty;
+  u.x0 = bx * qx + min(bx, ex);
+  u.sx = qx + (bx < ex ? 1 : 0);
+  u.y0 = by * qy + min(by, ey);
+  u.sy = qy + (by < ey ? 1 : 0);
+  u.z0 = (unit / ntiles) * zc;
+  u.z1 = min(u.z0 + zc, g.n[2]);
+  return true;
+}
+
+// Thread t's point (tx, ty) of a unit's tile and its x / y halo point (at most one per
+// thread).  Threads beyond a partial tile double one of its last points (spare): they load
+// and stage what that point's own thread does, so that no access of the march sits in a
+// branch (a wait for a load would then have to wait for any store issued after it too), and
+// store at offsets past the array's end (st8_own), which the memory unit drops.  Halo points:
+// threads [0, 8 BY) the x-halo columns, [8 BY, 8 (BX + BY)) the y-halo rows; (hx, hy) is
+// the place in the haloed tile (the right and lower halo follow the tile's last point),
+// (hi, hj) the grid indices; hmask 1 for an x-halo point, 2 for a y-halo point, 0 for none
+// (then (hi, hj) is the thread's own point, loaded again and not used).
+struct MarchThread {
+  int tx, ty, i, j, hx, hy, hi, hj, hmask;
+  unsigned spare;   // 0, or the bits that put a byte offset past the end of every array
+};
+template <int BX, int BY>
+__device__ __forceinline__ MarchThread march_thread(const Geo& g, const MarchUnit& u) {
+  const int t = threadIdx.x;
+  MarchThread m;
+  m.tx = min(t % BX, u.sx - 1);
+  m.ty = min(t / BX, u.sy - 1);
+  m.spare = t % BX < u.sx && t / BX < u.sy ? 0u : 0xfffff000u;
+  m.i = u.x0 + m.tx;
+  m.j = u.y0 + m.ty;
+  m.hx = m.hy = m.hmask = 0;
+  m.hi = m.i;
+  m.hj = m.j;
+  if (t < 8 * BY) {
+    const int c = t % 8, r = t / 8;
+    if (r < u.sy) {
+      m.hy = r;
+      m.hx = c < 4 ? c : u.sx + c;
+      m.hi = wrap(u.x0 + m.hx - 4, g.dir[0]);
+      m.hj = u.y0 + r;
+      m.hmask = 1;
+    }
+  } else if (t < 8 * (BX + BY)) {
+    const int t2 = t - 8 * BY, r = t2 / BX, c = t2 % BX;
+    if (c < u.sx) {
+      m.hx = c;
+      m.hy = r < 4 ? r : u.sy + r;
+      m.hi = u.x0 + c;
+      m.hj = wrap(u.y0 + m.hy - 4, g.dir[1]);
+      m.hmask = 2;
+    }
+  }
+  return m;
+}
+
+// Element access at a 32-bit byte offset from a wave-uniform base pointer: the address
+// form of a global load / store with a scalar base and a 32-bit vector offset, so a
+// thread keeps one 32-bit offset per point instead of a 64-bit address per component.
+// Callers keep byte offsets below 2^32 - 4096 (fewer than 2^29 - 1024 points per component
+// array, so that the offsets of spare threads lie past its end).
+__device__ __forceinline__ double ld8(const double* base, unsigned off) {
+  return *reinterpret_cast<const double*>(reinterpret_cast<const char*>(base) + off);
+}
+__device__ __forceinline__ void st8(double* base, unsigned off, double v) {
+  *reinterpret_cast<double*>(reinterpret_cast<char*>(base) + off) = v;
+}
+template <bool STREAM>
+__device__ __forceinline__ double ld8_own(const double* base, unsigned off) {
+  return ld_own<STREAM>(reinterpret_cast<const double*>(reinterpret_cast<const char*>(base) + off));
+}
+// Store at byte offset `off` of an array of `bytes` bytes through a buffer descriptor, whose
+// range check drops a store at or beyond the end.
+template <bool STREAM>
+__device__ __forceinline__ void st8_own(double* base, unsigned bytes, unsigned off, double v) {
+  typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+  const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(base, 0, bytes, 0x00027000);
+  __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, v), r, off, 0, STREAM ? 2 : 0);
+}
+
+// The eight neighbours of a staged value along x (stride 1) and y (stride sy) that the
+// first-derivative stencil reads, fetched together: left to itself the compiler reads two
+// or four, waits and goes on, an LDS latency for each, with two waves a SIMD to hide it
+// (the barrier for the scheduler keeps the batch whole; it is not a barrier of the block).
+struct Cross {
+  double xp[4], xm[4], yp[4], ym[4];
+};
+__device__ __forceinline__ void cross_load(const double* x, const double* y, int sy, Cross& c) {
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    c.xp[k] = x[k + 1];
+    c.xm[k] = x[-(k + 1)];
+    c.yp[k] = y[(k + 1) * sy];
+    c.ym[k] = y[-(k + 1) * sy];
+  }
+}
+__device__ __forceinline__ double diff4(const double* p, const double* m, double c1, double c2,
+                                        double c3, double c4) {
+  double o = 0.0;
+  o += c1 * (p[0] - m[0]);
+  o += c2 * (p[1] - m[1]);
+  o += c3 * (p[2] - m[2]);
+  o += c4 * (p[3] - m[3]);
+  return o;
+}
+
+// Element i (wave-uniform) of an array that no kernel writes, through the scalar cache: a
+// vector load here would queue behind the planes in flight, and its wait for theirs.
+__device__ __forceinline__ double ld_const(const double* p, int i) {
+  typedef const double __attribute__((address_space(4))) cdouble;
+  return ((cdouble*)(unsigned long)p)[i];
+}
+
 // Gradients of w = (u_1..u_3, T) on a fully periodic 3-D grid in one pass: a BX x BY
-// column tile marches along z over a chunk of ZC planes.  Each thread keeps w of its
-// column for the 9 planes of the z stencil in registers; the plane being
-// differentiated is staged with a 4-point x / y halo in LDS, one halo point per thread
-// (threads below 8 (BX + BY)).  The halo point of the next plane (and, where the
-// registers allow, the column's next lead point) is loaded one iteration before it is
-// used, so its latency overlaps a plane's stencil work.
+// column tile marches along z over a chunk of zc planes.  Each thread keeps w of its
+// column for the 9 planes of the z stencil in registers; the plane being differentiated
+// is staged with its 4-point x / y halo in LDS.  The halo points (one per thread) are
+// loaded four planes ahead, with the column's lead point -- when the neighbouring tile,
+// marching beside this one, loads the same lines as its own lead plane, so that they are
+// fetched into the L2 once -- and wait in an LDS ring of four planes (each thread reads
+// back its own).  Both loads are issued one iteration before they are used.
 // Same sums as k_prim + k_grad (interior SBP rows, wrap-around indices), so the same
 // values.
 // STRESS: instead of the 12 gradient components, write what the fluxes need of them at
@@ -75,131 +216,115 @@ __global__ void __launch_bounds__(kBlock) k_grad(Geo g, int d, const double* __r
 // (visc_point's operations, so the same values); 72 instead of 96 bytes per point.
 // POWER: the viscosity follows a power law of the temperature (pow per point); without
 // it the transport coefficients are constants and the kernel needs far fewer registers.
-template <int BX, int BY, int ZC, bool STRESS = false, bool POWER = true>
-__global__ void __launch_bounds__(BX * BY, STRESS ? 2 : 4) k_grad3d_periodic(Geo g, const double* __restrict__ q,
+template <int BX, int BY, bool STRESS = false, bool POWER = true>
+__global__ void __launch_bounds__(BX * BY, STRESS ? 2 : 4) k_grad3d_periodic(Geo g, int zc,
+                                                              const double* __restrict__ q,
                                                               double* __restrict__ G) {
   constexpr int NT = BX * BY, EXW = BX + 8, EYW = BY + 8, NW = 4, NH = 8 * (BX + BY);
   static_assert(NH <= NT, "one halo point per thread");
-  __shared__ double sw[NW][EYW][EXW];
-  // XCD-aware block map (as in k_fwd3d_march): block b takes (tile, z chunk) unit
-  // (b mod 8) * ceil(units / 8) + b / 8, tiles x-fastest, so each XCD works on one
-  // contiguous band and neighbouring tiles' halo lines meet in its L2
-  const int ntx = g.n[0] / BX, ntiles = ntx * (g.n[1] / BY);
-  const int nunits = ntiles * ((g.n[2] + ZC - 1) / ZC);
-  const int per_xcd = (nunits + 7) / 8;
-  const int unit = (int)(blockIdx.x % 8) * per_xcd + (int)(blockIdx.x / 8);
-  if (unit >= nunits) return;   // padding of the grid to a multiple of 8 (whole block)
-  const int tile = unit % ntiles;
-  const int x0 = (tile % ntx) * BX, y0 = (tile / ntx) * BY;
-  const int z0 = (unit / ntiles) * ZC;
+  __shared__ double sw[2][NW][EYW][EXW];   // planes in turn: one barrier per plane
+  __shared__ double hring[4][NW][NH];
+  MarchUnit u;
+  if (!march_unit<BX, BY>(g, zc, u)) return;
   const long inst = blockIdx.z;
   const double* qi = q + inst * 5 * g.N;
   double* Gi = G + inst * 4 * 3 * g.N;
-  const int tx = threadIdx.x % BX, ty = threadIdx.x / BX;
-  const int i = x0 + tx, j = y0 + ty;
-  const Dir dx = g.dir[0], dy = g.dir[1], dz = g.dir[2];
-  const long n01 = (long)g.n[0] * g.n[1];
-  auto load_v = [&](int ii, int jj, int kk, double* v) {
-    const long p = ii + (long)g.n[0] * jj + n01 * kk;
+  const MarchThread m = march_thread<BX, BY>(g, u);
+  const int tx = m.tx, ty = m.ty, ht = min((int)threadIdx.x, NH - 1);
+  // place of the halo point in the one haloed tile
+  const int hx = m.hmask == 2 ? m.hx + 4 : m.hx, hy = m.hmask == 1 ? m.hy + 4 : m.hy;
+  const Dir dz = g.dir[2];
+  const unsigned n0 = (unsigned)g.n[0], plane8 = 8u * n0 * (unsigned)g.n[1];
+  const unsigned col8 = 8u * ((unsigned)m.i + n0 * (unsigned)m.j);
+  const unsigned hcol8 = 8u * ((unsigned)m.hi + n0 * (unsigned)m.hj);
+  const double h0 = g.h[0][m.i], h1 = g.h[1][m.j], h01 = h0 * h1;
+  auto load_v = [&](unsigned off, double* v) {
 #pragma unroll
-    for (int l = 0; l < 5; ++l) v[l] = qi[l * g.N + p];
+    for (int l = 0; l < 5; ++l) v[l] = ld8(qi + l * g.N, off);
   };
   auto to_w = [&](const double* v, double* w) {
     const Prim<3> s = prim<3>(v, g.gamma);
     w[0] = s.u[0]; w[1] = s.u[1]; w[2] = s.u[2]; w[3] = s.T;
   };
-  // this thread's halo point: y halo rows over the tile columns, then x halo columns over
-  // the tile rows (the corners are never read)
-  const int t = threadIdx.x;
-  const bool has_halo = t < NH;
-  int hx = 0, hy = 0;
-  if (t < 8 * BX) {
-    const int r = t / BX;
-    hy = r < 4 ? r : BY + r;
-    hx = 4 + t % BX;
-  } else if (has_halo) {
-    const int t2 = t - 8 * BX, c = t2 % 8;
-    hy = 4 + t2 / 8;
-    hx = c < 4 ? c : BX + c;
-  }
-  const int hi = wrap(x0 + hx - 4, dx), hj = wrap(y0 + hy - 4, dy);
-  double Q[9][NW];
-  double v[5];
+  // halo planes beyond the chunk are not used: the last one is loaded again
+  auto halo_plane = [&](int z) { return hcol8 + plane8 * (unsigned)min(z, u.z1 - 1); };
+  double Q[9][NW], v[5], hv[5];
 #pragma unroll
   for (int k = 0; k < 8; ++k) {
-    load_v(i, j, wrap(z0 - 4 + k, dz), v);
+    load_v(col8 + plane8 * (unsigned)wrap(u.z0 - 4 + k, dz), v);
     to_w(v, Q[k]);
   }
-  double hv[5];
-  if (has_halo) load_v(hi, hj, z0 % dz.len, hv);   // halo, plane z0
-  // with constant transport coefficients the registers allow the column's lead point to
-  // be loaded a plane ahead too
-  constexpr bool kAhead = STRESS && !POWER;
-  if (kAhead) load_v(i, j, wrap(z0 + 4, dz), v);   // the column's lead plane z0 + 4
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {              // halo planes z0 .. z0 + 3
+    double hw[NW];
+    load_v(halo_plane(u.z0 + k), hv);
+    to_w(hv, hw);
+    if (m.hmask) {
+#pragma unroll
+      for (int c = 0; c < NW; ++c) hring[k][c][ht] = hw[c];
+    }
+  }
+  load_v(col8 + plane8 * (unsigned)wrap(u.z0 + 4, dz), v);   // the lead plane z0 + 4
+  load_v(halo_plane(u.z0 + 4), hv);
   const Op& op = g.ops[SLOT_FIRST];
   const double c1 = op.c[kMaxHW + 1], c2 = op.c[kMaxHW + 2], c3 = op.c[kMaxHW + 3], c4 = op.c[kMaxHW + 4];
-  for (int s = 0; s < ZC; ++s) {
-    const int zc = z0 + s;
-    if (zc >= g.n[2]) break;   // uniform over the block
-    if (!kAhead) load_v(i, j, wrap(zc + 4, dz), v);
+  for (int zo = u.z0; zo < u.z1; ++zo) {     // uniform over the block
+    const int slot = (zo - u.z0) & 3, buf = (zo - u.z0) & 1;
     to_w(v, Q[8]);
     double hw[NW];
-    if (has_halo) to_w(hv, hw);
-    // the next plane's halo point (and lead point): the loads stay in flight through this
-    // plane's work
-    if (s + 1 < ZC && zc + 1 < g.n[2]) {
-      if (kAhead) load_v(i, j, wrap(zc + 5, dz), v);
-      if (has_halo) load_v(hi, hj, zc + 1, hv);
-    }
-    __syncthreads();            // readers of the previous plane are done
+    to_w(hv, hw);
+    // the next lead plane's points: the loads stay in flight through this plane's work
+    load_v(col8 + plane8 * (unsigned)wrap(min(zo + 5, u.z1 + 3), dz), v);
+    load_v(halo_plane(zo + 5), hv);
 #pragma unroll
-    for (int c = 0; c < NW; ++c) sw[c][ty + 4][tx + 4] = Q[4][c];
-    if (has_halo) {
+    for (int c = 0; c < NW; ++c) sw[buf][c][ty + 4][tx + 4] = Q[4][c];
+    if (m.hmask) {
+      // the halo values of this plane leave the ring, those of the lead plane take the slot
 #pragma unroll
-      for (int c = 0; c < NW; ++c) sw[c][hy][hx] = hw[c];
+      for (int c = 0; c < NW; ++c) {
+        sw[buf][c][hy][hx] = hring[slot][c][ht];
+        hring[slot][c][ht] = hw[c];
+      }
     }
     __syncthreads();
-    int ijk[3] = {i, j, zc};
-    const long p = i + (long)g.n[0] * j + n01 * zc;
-    const double jac = jacobian<3>(g, ijk);
+    const unsigned p8 = col8 + plane8 * (unsigned)zo;
+    const double h2 = ld_const(g.h[2], zo);
+    const double jac = 1.0 / (h01 * h2);                                  // jacobian<3>
+    const double jm[3] = {jac * (h1 * h2), jac * (h0 * h2), jac * h01};   // times metric<3>
     double gv[NW * 3];
+    Cross cr[2];
+    const double* row = &sw[buf][0][ty + 4][tx + 4];
+    cross_load(row, row, EXW, cr[0]);
 #pragma unroll
     for (int c = 0; c < NW; ++c) {
-      const double* row = &sw[c][ty + 4][tx + 4];
-      double ox = 0.0, oy = 0.0, oz = 0.0;
-      ox += c1 * (row[1] - row[-1]);
-      ox += c2 * (row[2] - row[-2]);
-      ox += c3 * (row[3] - row[-3]);
-      ox += c4 * (row[4] - row[-4]);
-      oy += c1 * (row[EXW] - row[-EXW]);
-      oy += c2 * (row[2 * EXW] - row[-2 * EXW]);
-      oy += c3 * (row[3 * EXW] - row[-3 * EXW]);
-      oy += c4 * (row[4 * EXW] - row[-4 * EXW]);
+      if (c + 1 < NW) cross_load(row + (c + 1) * EYW * EXW, row + (c + 1) * EYW * EXW, EXW, cr[(c + 1) & 1]);
+      __builtin_amdgcn_sched_barrier(0);
+      const Cross& k = cr[c & 1];
+      double oz = 0.0;
       oz += c1 * (Q[5][c] - Q[3][c]);
       oz += c2 * (Q[6][c] - Q[2][c]);
       oz += c3 * (Q[7][c] - Q[1][c]);
       oz += c4 * (Q[8][c] - Q[0][c]);
-      gv[c * 3 + 0] = (jac * metric<3>(g, 0, ijk)) * ox;
-      gv[c * 3 + 1] = (jac * metric<3>(g, 1, ijk)) * oy;
-      gv[c * 3 + 2] = (jac * metric<3>(g, 2, ijk)) * oz;
-      if constexpr (!STRESS) {
-#pragma unroll
-        for (int d = 0; d < 3; ++d) Gi[(c * 3 + d) * g.N + p] = gv[c * 3 + d];
-      }
+      gv[c * 3 + 0] = jm[0] * diff4(k.xp, k.xm, c1, c2, c3, c4);
+      gv[c * 3 + 1] = jm[1] * diff4(k.yp, k.ym, c1, c2, c3, c4);
+      gv[c * 3 + 2] = jm[2] * oz;
     }
-    if constexpr (STRESS) {
+    if constexpr (!STRESS) {
+#pragma unroll
+      for (int c = 0; c < NW * 3; ++c) st8(Gi + c * g.N, p8, gv[c]);
+    } else {
       double mu, la, ka;
       if constexpr (POWER) transport(g, Q[4][3], &mu, &la, &ka);
       else transport_const(g, &mu, &la, &ka);
       stress<3>(gv, mu, la);
-      Gi[0 * g.N + p] = gv[0];
-      Gi[1 * g.N + p] = gv[1];
-      Gi[2 * g.N + p] = gv[2];
-      Gi[3 * g.N + p] = gv[4];
-      Gi[4 * g.N + p] = gv[5];
-      Gi[5 * g.N + p] = gv[8];
+      st8(Gi + 0 * g.N, p8, gv[0]);
+      st8(Gi + 1 * g.N, p8, gv[1]);
+      st8(Gi + 2 * g.N, p8, gv[2]);
+      st8(Gi + 3 * g.N, p8, gv[4]);
+      st8(Gi + 4 * g.N, p8, gv[5]);
+      st8(Gi + 5 * g.N, p8, gv[8]);
 #pragma unroll
-      for (int d = 0; d < 3; ++d) Gi[(6 + d) * g.N + p] = -ka * gv[9 + d];
+      for (int d = 0; d < 3; ++d) st8(Gi + (6 + d) * g.N, p8, -ka * gv[9 + d]);
     }
 #pragma unroll
     for (int k = 0; k < 8; ++k)
@@ -486,13 +611,15 @@ __device__ __forceinline__ void adj_point_init(const Geo& g, const double* v, co
 
 // adj_point_init from the stress / heat-flux slots at the point (sv: xx xy xz yy yz zz,
 // then the heat flux x y z, as k_grad3d_periodic<.., true> writes them -- stress() and
-// -kappa grad T of the same gradient values, so the same tau and hf).
+// -kappa grad T of the same gradient values, so the same tau and hf).  The caller has set
+// P.h (metric<3>) and P.jac.
 template <bool POWER>
 __device__ __forceinline__ void adj_point_init_stress(const Geo& g, const double* v, const double* sv,
-                                                      const int* ijk, AdjPoint<3>& P) {
+                                                      AdjPoint<3>& P) {
   const double gm = g.gamma;
   P.s = prim<3>(v, gm);
-  transport(g, P.s.T, &P.mu, &P.la, &P.ka);
+  if (POWER) transport(g, P.s.T, &P.mu, &P.la, &P.ka);
+  else transport_const(g, &P.mu, &P.la, &P.ka);
   P.tau[0] = sv[0]; P.tau[1] = sv[1]; P.tau[2] = sv[2];
   P.tau[3] = sv[1]; P.tau[4] = sv[3]; P.tau[5] = sv[4];
   P.tau[6] = sv[2]; P.tau[7] = sv[4]; P.tau[8] = sv[5];
@@ -500,8 +627,6 @@ __device__ __forceinline__ void adj_point_init_stress(const Geo& g, const double
   double ke = 0.0;
   for (int i = 0; i < 3; ++i) ke += P.s.u[i] * P.s.u[i];
   P.phi2 = 0.5 * (gm - 1.0) * ke;
-  P.jac = jacobian<3>(g, ijk);
-  for (int d = 0; d < 3; ++d) P.h[d] = metric<3>(g, d, ijk);
   if (POWER) {
     const double pl = g.power_law, svol = P.s.sv, T = P.s.T;
     P.t2_0 = pl * gm * svol / T * (P.phi2 / (gm - 1.0) - T / gm);
@@ -1317,7 +1442,7 @@ __global__ void __launch_bounds__(kBlock) k_gradient(Geo g, const DPatch* __rest
 // per block row: each block stages the contravariant fluxes of its BX x BY points (x
 // rows and y columns, with the 4-point halo recomputed from q and G) in LDS and writes
 // D_x Fx + D_y Fy to rhs and Fz to its slot of F, for the z divergence (k_deriv_line,
-// k_fwd_finish_z or k_div) to finish.  The per-point flux and the derivative sums are
+// or k_div) to finish.  The per-point flux and the derivative sums are
 // those of k_flux_all and k_div (same operations in the same order, so the same
 // values).
 template <int BX, int BY>
@@ -1481,173 +1606,33 @@ __global__ void __launch_bounds__(kBlock) k_deriv_line(Geo g, int d, int slot,
   }
 }
 
-// The z divergence of a forward rhs fused with k_finish's forward operations, for 3-D
-// regions whose patches are at most one Kolmogorov forcing over the whole domain, with
-// no sources and no dissipation.  One thread per z-line as in k_deriv_line, the 9-point
-// windows of the five flux components in registers; at each point
-// rhs = 0 - (x/y divergence + D_z Fz) (k_deriv_line's add-negate), then the Jacobian
-// scaling and the forcing of the x momentum, in k_finish's order.  With rk_stage > 0 the
-// point's RK4 stage update follows (k_rk_forward's arithmetic, y = q updated in place,
-// copy optional), after all five components are formed since the forcing reads the
-// density at the point, and rhs is not written.
-__global__ void __launch_bounds__(kBlock) k_fwd_finish_z(Geo g, const double* __restrict__ Fz,
-                                                        long f_inst, const double* q,
-                                                        const double* __restrict__ kstr,
-                                                        double* __restrict__ rhs, int rk_stage,
-                                                        double dt, double* y, double* b1,
-                                                        double* b2, double* copy) {
-  constexpr int ND = 3, NV = 5;
-  const Dir dd = g.dir[2];
-  const long nlines = g.N / dd.len;
-  const long line = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (line >= nlines) return;
-  const long inst = blockIdx.z;
-  const long n0 = g.n[0];
-  const long i = line % n0, o = line / n0;
-  const long base = i + o * n0;
-  const long sd = dd.stride;
-  const double* x = Fz + inst * f_inst + base;
-  const double* qi = q + inst * NV * g.N;
-  double* ri = rhs + inst * NV * g.N;
-  const int z0 = blockIdx.y * kLineChunk;
-  const int z1 = min(z0 + kLineChunk, dd.len);
-  const Op& op = g.ops[SLOT_FIRST];
-  const double c1 = op.c[kMaxHW + 1], c2 = op.c[kMaxHW + 2], c3 = op.c[kMaxHW + 3],
-               c4 = op.c[kMaxHW + 4];
-  double Q[NV][9];
-#pragma unroll
-  for (int l = 0; l < NV; ++l)
-#pragma unroll
-    for (int k = 0; k < 8; ++k) Q[l][k] = x[l * g.N + wrap(z0 - 4 + k, dd) * sd];
-  for (int z = z0; z < z1; ++z) {
-    const long p = base + z * sd;
-    double r[NV];
-#pragma unroll
-    for (int l = 0; l < NV; ++l) {
-      Q[l][8] = x[l * g.N + wrap(z + 4, dd) * sd];
-      double out = 0.0;
-      out += c1 * (Q[l][5] - Q[l][3]);
-      out += c2 * (Q[l][6] - Q[l][2]);
-      out += c3 * (Q[l][7] - Q[l][1]);
-      out += c4 * (Q[l][8] - Q[l][0]);
-      double v = ri[l * g.N + p] + out;
-      r[l] = 0.0 - v;
-#pragma unroll
-      for (int k = 0; k < 8; ++k) Q[l][k] = Q[l][k + 1];
-    }
-    int ijk[3] = {(int)i, (int)o, z};
-    const double jac = jacobian<ND>(g, ijk);
-#pragma unroll
-    for (int l = 0; l < NV; ++l) r[l] = r[l] * jac;
-    if (kstr) r[1] = r[1] + qi[p] * kstr[p];
-    if (rk_stage == 0) {
-#pragma unroll
-      for (int l = 0; l < NV; ++l) ri[l * g.N + p] = r[l];
-      continue;
-    }
-#pragma unroll
-    for (int l = 0; l < NV; ++l) {
-      const long ii = inst * NV * g.N + l * g.N + p;
-      const double rl = r[l];
-      double qn;
-      switch (rk_stage) {
-        case 1: {
-          const double q0 = y[ii];
-          b1[ii] = q0;
-          b2[ii] = q0 + div6(dt * rl);
-          qn = q0 + dt * rl / 2.0;
-          break;
-        }
-        case 2:
-          b2[ii] = b2[ii] + div3(dt * rl);
-          qn = b1[ii] + dt * rl / 2.0;
-          break;
-        case 3:
-          b2[ii] = b2[ii] + div3(dt * rl);
-          qn = b1[ii] + dt * rl;
-          break;
-        default:
-          qn = b2[ii] + div6(dt * rl);
-          break;
-      }
-      y[ii] = qn;
-      if (copy) copy[ii] = qn;
-    }
-  }
-}
-
-// XCD-aware (tile, z chunk) work unit of block b of a 3-D march: units are dealt to the
-// 8 XCDs round-robin by block index, so block b takes unit (b mod 8) * ceil(units / 8) +
-// b / 8, tiles x-fastest: each XCD marches one contiguous band, and the halo lines of
-// neighbouring tiles are fetched into its own L2 by blocks running beside it.  False for
-// the padding blocks of a grid rounded up to a multiple of 8.
-template <int BX, int BY, int ZC>
-__device__ __forceinline__ bool march_unit(const Geo& g, int& x0, int& y0, int& z0) {
-  const int ntx = g.n[0] / BX, ntiles = ntx * (g.n[1] / BY);
-  const int nunits = ntiles * ((g.n[2] + ZC - 1) / ZC);
-  const int per_xcd = (nunits + 7) / 8;
-  const int unit = (int)(blockIdx.x % 8) * per_xcd + (int)(blockIdx.x / 8);
-  if (unit >= nunits) return false;
-  const int tile = unit % ntiles;
-  x0 = (tile % ntx) * BX;
-  y0 = (tile / ntx) * BY;
-  z0 = (unit / ntiles) * ZC;
-  return true;
-}
-
-// The x / y halo point of thread t of a BX x BY tile (at most one per thread, 8 (BX + BY)
-// of them): [0, 8 BY) the x-halo columns, [8 BY, 8 (BX + BY)) the y-halo rows, none for
-// the threads after them.  (hx, hy) is its place in the haloed tile, (hi, hj) its grid
-// indices; hmask 1 for an x-halo point, 2 for a y-halo point, 0 for none (then hi, hj are
-// the thread's own point, so that every index stays in the grid).
-template <int BX, int BY>
-__device__ __forceinline__ void march_halo(const Geo& g, int t, int x0, int y0, int& hx, int& hy,
-                                           int& hi, int& hj, int& hmask) {
-  if (t < 8 * BY) {
-    const int c = t % 8;
-    hy = t / 8;
-    hx = c < 4 ? c : BX + c;
-    hi = wrap(x0 + hx - 4, g.dir[0]);
-    hj = y0 + hy;
-    hmask = 1;
-  } else if (t < 8 * (BX + BY)) {
-    const int t2 = t - 8 * BY, r = t2 / BX;
-    hx = t2 % BX;
-    hy = r < 4 ? r : BY + r;
-    hi = x0 + hx;
-    hj = wrap(y0 + hy - 4, g.dir[1]);
-    hmask = 2;
-  } else {
-    hx = hy = 0;
-    hi = x0 + t % BX;
-    hj = y0 + t / BX;
-    hmask = 0;
-  }
-}
-
 // The whole forward rhs of a 3-D region periodic in every direction, in one z march
 // (computeRhsForward, src/RhsHelperImpl.f90:254-354, with k_finish's operations for at
 // most one whole-domain Kolmogorov forcing and no dissipation or sources): a BX x BY
-// column tile marches along z over a chunk of ZC planes.  At each lead plane zl every
+// column tile marches along z over a chunk of zc planes.  At each lead plane zl every
 // thread forms the contravariant fluxes of its tile point (from q and, viscous, the
 // stress / heat-flux slots S written by k_grad3d_periodic<.., true>) and of one x- or
 // y-halo point; the x and y fluxes go through LDS for D_x Fx + D_y Fy, which waits in a
 // 4-plane LDS ring, and Fz enters a 9-plane register window.  Four planes behind, at
 // zo = zl - 4, rhs = 0 - ((D_x Fx + D_y Fy) + D_z Fz) -- zo's ring slot is read before
-// zl's partial takes it over -- then the Jacobian scaling and the
-// forcing; with rk_stage > 0 the RK4 stage update follows and goes to yout, which must
-// not be q (other blocks still read q), and rhs is not written; at stage 1 b1 may be
-// null (the caller keeps q itself as the state at the start of the step), and at stages
-// 1-3 b2 may be null (a recompute that stops before stage 4 needs no accumulator).  The fluxes, sums and
-// finishing operations are those of k_fluxdiv3d_xy and k_fwd_finish_z, in the same
-// order, so the values are the same; no flux or partial rhs goes through HBM.
-// RK: the variant for RK stages (rk_stage > 0), which loads the RK operands of its output
-// plane early; the rhs-only variant leaves them out and keeps the registers for the rest.
-template <int BX, int BY, int ZC, bool RK>
-__global__ void __launch_bounds__(BX * BY, 512 / (BX * BY)) k_fwd3d_march(Geo g, const double* __restrict__ q,
+// zl's partial takes it over -- then the Jacobian scaling and the forcing, whose density
+// waits in the ring too and whose strength (kstr, a whole-domain patch array) depends on
+// the row alone and is read once; with STAGE > 0 the RK4 stage update follows and goes
+// to yout, which must not be q (other blocks still read q), and rhs is not written; at
+// stage 1 b1 may be null (the caller keeps q itself as the state at the start of the
+// step), and at stages 1-3 b2 may be null (a recompute that stops before stage 4 needs no
+// accumulator).  The sums and finishing operations are those of the separate kernels
+// (k_flux_all, k_div, k_finish), in the same order, so the values are the same; no flux or
+// partial rhs goes through HBM.
+// STAGE: 0 for the rhs alone, else the RK stage, a compile-time value: each variant loads
+// only the RK operands of its output plane that its update reads (early, so that their
+// latency overlaps the divergence).
+// STREAM (march_streams): RK operands and outputs non-temporal.
+template <int BX, int BY, int STAGE, bool STREAM>
+__global__ void __launch_bounds__(BX * BY, 512 / (BX * BY)) k_fwd3d_march(Geo g, int zc, const double* __restrict__ q,
                                                           const double* __restrict__ S,
                                                           const double* __restrict__ kstr,
-                                                          double* __restrict__ rhs, int rk_stage,
+                                                          double* __restrict__ rhs,
                                                           double dt, double* __restrict__ yout,
                                                           double* __restrict__ b1,
                                                           double* __restrict__ b2,
@@ -1656,112 +1641,141 @@ __global__ void __launch_bounds__(BX * BY, 512 / (BX * BY)) k_fwd3d_march(Geo g,
   static_assert(8 * (BX + BY) <= NT, "at most one halo point per thread");
   __shared__ double sfx[NV][BY][EXW];
   __shared__ double sfy[NV][EYW][BX];
-  __shared__ double ring[4][NV][NT];
-  int x0, y0, z0;
-  if (!march_unit<BX, BY, ZC>(g, x0, y0, z0)) return;
-  const int z1 = min(z0 + ZC, g.n[2]);
-  const long inst = blockIdx.z;
-  const double* qi = q + inst * NV * g.N;
-  const double* Si = g.viscous ? S + inst * 12 * g.N : nullptr;
-  const long n01 = (long)g.n[0] * g.n[1];
-  const int t = threadIdx.x, tx = t % BX, ty = t / BX;
-  const int i = x0 + tx, j = y0 + ty;
-  int hx, hy, hi, hj, hmask;
-  march_halo<BX, BY>(g, t, x0, y0, hx, hy, hi, hj, hmask);
-  // operands of one point: q and, viscous, the stress / heat-flux slots the fluxes of the
-  // directions in dmask read (tau is symmetric: slot order xx xy xz yy yz zz, then the
-  // heat flux x y z); slots not needed are not loaded
+  __shared__ double ring[4][NV + 1][NT];   // D_x Fx + D_y Fy of the waiting planes, density
+  MarchUnit u;
+  if (!march_unit<BX, BY>(g, zc, u)) return;
+  const int z0 = u.z0, z1 = u.z1;
+  const long io = (long)blockIdx.z * NV * g.N;
+  const double* qi = q + io;
+  const double* Si = g.viscous ? S + (long)blockIdx.z * 12 * g.N : nullptr;
+  const MarchThread m = march_thread<BX, BY>(g, u);
+  const int t = threadIdx.x, tx = m.tx, ty = m.ty, hmask = m.hmask;
+  const Dir dz = g.dir[2];
+  const unsigned n0 = (unsigned)g.n[0], plane8 = 8u * n0 * (unsigned)g.n[1];
+  const unsigned bytes = 8u * (unsigned)g.N;
+  const unsigned col8 = 8u * ((unsigned)m.i + n0 * (unsigned)m.j);
+  const unsigned hcol8 = 8u * ((unsigned)m.hi + n0 * (unsigned)m.hj);
+  const double kk = kstr ? kstr[n0 * (unsigned)m.j] : 0.0;
+  // the grid values of the metrics: metric<3> of d = 0, 1, 2 is h1 h2, h0 h2, h0 h1
+  const double h0 = g.h[0][m.i], h1 = g.h[1][m.j], h01 = h0 * h1;
+  const double hh = hmask == 2 ? g.h[0][m.hi] : g.h[1][m.hj];   // of the halo point's direction
+  // operands of a column point: q and, viscous, the stress / heat-flux slots its fluxes read
+  // (tau is symmetric: slot order xx xy xz yy yz zz, then the heat flux x y z); outside the
+  // chunk only those of the z flux
   struct Pt {
     double v[NV];
     double sv[9];
   };
-  auto load_pt = [&](int ii, int jj, int kk, int dmask, Pt& P) {
-    const long pp = ii + (long)g.n[0] * jj + n01 * kk;
-    load_q<3>(qi, g.N, pp, P.v);
-    if (g.viscous) {
-      const int need[9] = {dmask & 1, dmask & 3, dmask & 5, dmask & 2, dmask & 6, dmask & 4,
-                           dmask & 1, dmask & 2, dmask & 4};
+  auto load_pt = [&](unsigned off, auto xy, Pt& P) {
 #pragma unroll
-      for (int k = 0; k < 9; ++k) P.sv[k] = need[k] ? Si[k * g.N + pp] : 0.0;
+    for (int l = 0; l < NV; ++l) P.v[l] = ld8(qi + l * g.N, off);
+    if (g.viscous) {
+#pragma unroll
+      for (int k = 0; k < 9; ++k)
+        P.sv[k] = xy || k == 2 || k == 4 || k == 5 || k == 8 ? ld8(Si + k * g.N, off) : 0.0;
     }
   };
-  // contravariant fluxes of the directions in dmask at grid point (ii, jj, kk)
-  auto fluxes = [&](int ii, int jj, int kk, int dmask, const Pt& P, double (*out)[NV]) {
-    const Prim<3> s = prim<3>(P.v, g.gamma);
-    double tau[9], hf[3];
+  // operands of the halo point: q and the stress column and heat flux of its one direction
+  struct HaloPt {
+    double v[NV];
+    double td[4];
+  };
+  const double* hs[4] = {};
+  if (g.viscous) {
+    const bool y = hmask == 2;
+    hs[0] = Si + (y ? g.N : 0);
+    hs[1] = Si + (y ? 3 : 1) * g.N;
+    hs[2] = Si + (y ? 4 : 2) * g.N;
+    hs[3] = Si + (y ? 7 : 6) * g.N;
+  }
+  auto load_halo = [&](unsigned off, HaloPt& P) {
+#pragma unroll
+    for (int l = 0; l < NV; ++l) P.v[l] = ld8(qi + l * g.N, off);
     if (g.viscous) {
-      tau[0] = P.sv[0]; tau[1] = P.sv[1]; tau[2] = P.sv[2];
-      tau[3] = P.sv[1]; tau[4] = P.sv[3]; tau[5] = P.sv[4];
-      tau[6] = P.sv[2]; tau[7] = P.sv[4]; tau[8] = P.sv[5];
-      hf[0] = P.sv[6]; hf[1] = P.sv[7]; hf[2] = P.sv[8];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) P.td[k] = ld8(hs[k], off);
     }
-    const int ijk[3] = {ii, jj, kk};
+  };
+  // contravariant flux of direction d with metric md: inviscid minus viscous (td: the stress
+  // components tau_0d, tau_1d, tau_2d and the heat flux of the direction)
+  auto flux_dir = [&](double md, int d, const double* v, const Prim<3>& s, const double* td,
+                      double* out) {
+    double f[NV];
+    inviscid_flux<3>(v, s, d, f);
+    if (g.viscous) {
+      double e = 0.0;
 #pragma unroll
-    for (int d = 0; d < 3; ++d) {
-      if (!(dmask >> d & 1)) continue;
-      double f[NV];
-      inviscid_flux<3>(P.v, s, d, f);
-      if (g.viscous) {
-        double fv[NV];
-        viscous_flux<3>(s.u, tau, hf, d, fv);
-#pragma unroll
-        for (int l = 0; l < NV; ++l) f[l] = f[l] - fv[l];
+      for (int k = 0; k < 3; ++k) {
+        f[k + 1] = f[k + 1] - td[k];
+        e += s.u[k] * td[k];
       }
-      const double m = metric<3>(g, d, ijk);
-#pragma unroll
-      for (int l = 0; l < NV; ++l) out[d][l] = m * f[l];
+      f[4] = f[4] - (e - td[3]);
     }
+#pragma unroll
+    for (int l = 0; l < NV; ++l) out[l] = md * f[l];
+  };
+  auto flux_z = [&](const Pt& P, const Prim<3>& s, double* out) {
+    const double td[4] = {P.sv[2], P.sv[4], P.sv[5], P.sv[8]};
+    flux_dir(h01, 2, P.v, s, td, out);
   };
   const Op& op = g.ops[SLOT_FIRST];
   const double c1 = op.c[kMaxHW + 1], c2 = op.c[kMaxHW + 2], c3 = op.c[kMaxHW + 3], c4 = op.c[kMaxHW + 4];
-  const Dir dz = g.dir[2];
+  constexpr std::true_type yes{};
+  constexpr std::false_type no{};
   double W[9][NV];
+  Pt ct;
+  HaloPt ch;
+  // the four planes before the chunk enter the window (slots 4 .. 7) with their z fluxes
 #pragma unroll
-  for (int k = 0; k < 8; ++k)
-#pragma unroll
-    for (int l = 0; l < NV; ++l) W[k][l] = 0.0;
-  // the operands of the next plane are loaded once this plane's fluxes are formed, so
-  // their latency overlaps the divergence and the stage update
-  Pt ct, ch, nt, nh;
-  load_pt(i, j, wrap(z0 - 4, dz), z0 - 4 >= z0 ? 7 : 4, ct);
-  for (int zl = z0 - 4; zl < z1 + 4; ++zl) {      // uniform over the block
-    const int kz = wrap(zl, dz);
-    const bool xy = zl >= z0 && zl < z1;
-    double f[3][NV], fh[3][NV];
-    fluxes(i, j, kz, xy ? 7 : 4, ct, f);
-#pragma unroll
-    for (int l = 0; l < NV; ++l) W[8][l] = f[2][l];
-    if (xy && hmask) fluxes(hi, hj, kz, hmask, ch, fh);
-    // the operands of the output plane zl - 4 that the finish reads (RK buffers, the
-    // Kolmogorov term's density and strength) are loaded with the next plane's, once this
-    // plane's fluxes are formed, so their latency overlaps the divergence
-    const bool outp = zl >= z0 + 4;
-    double ra[NV], rb[NV], rho_k = 0.0, kk_k = 0.0;
-    if (outp) {
-      const long p = i + (long)g.n[0] * j + n01 * (zl - 4);
-      if (kstr) {
-        rho_k = qi[p];
-        kk_k = kstr[p];
+  for (int k = 0; k < 4; ++k) {
+    load_pt(col8 + plane8 * (unsigned)wrap(z0 - 4 + k, dz), no, ct);
+    flux_z(ct, prim<3>(ct.v, g.gamma), W[k + 4]);
+  }
+  load_pt(col8 + plane8 * (unsigned)z0, yes, ct);
+  load_halo(hcol8 + plane8 * (unsigned)z0, ch);
+  // One lead plane zl: XY: inside the chunk, its x / y fluxes are formed; OUT: the plane
+  // zl - 4 is finished.  Compile-time cases, so that the loads of each are unconditional
+  // and their waits exact; a plane inside the chunk loads the next one with its halo, also
+  // where that lies just beyond the chunk.
+  auto plane = [&](int zl, auto XY, auto OUT) {
+    const unsigned p8 = col8 + plane8 * (unsigned)(zl - 4);   // output plane (OUT only)
+    const unsigned w8 = p8 | m.spare;
+    const double h2 = ld_const(g.h[2], wrap(zl, dz));
+    double f[2][NV], fh[NV];
+    {
+      const Prim<3> sp = prim<3>(ct.v, g.gamma);
+      if constexpr (XY) {
+        const double tdx[4] = {ct.sv[0], ct.sv[1], ct.sv[2], ct.sv[6]};
+        const double tdy[4] = {ct.sv[1], ct.sv[3], ct.sv[4], ct.sv[7]};
+        flux_dir(h1 * h2, 0, ct.v, sp, tdx, f[0]);
+        flux_dir(h0 * h2, 1, ct.v, sp, tdy, f[1]);
       }
-      if constexpr (RK) {
+      flux_z(ct, sp, W[8]);
+    }
+    const double rho = ct.v[0];
+    if constexpr (XY) {
+      const Prim<3> sp = prim<3>(ch.v, g.gamma);
+      if (hmask == 1) flux_dir(hh * h2, 0, ch.v, sp, ch.td, fh);
+      else if (hmask == 2) flux_dir(hh * h2, 1, ch.v, sp, ch.td, fh);
+    }
+    // the RK operands of the output plane are loaded with the next plane's, once this
+    // plane's fluxes are formed, so their latency overlaps the divergence
+    double ra[NV] = {}, rb[NV] = {};
+    if (OUT && STAGE > 0) {
 #pragma unroll
-        for (int l = 0; l < NV; ++l) {
-          const long ii = inst * NV * g.N + l * g.N + p;
-          ra[l] = rk_stage == 1 ? q[ii] : (rk_stage == 2 || rk_stage == 3) ? b1[ii] : 0.0;
-          rb[l] = rk_stage >= 2 && b2 ? b2[ii] : 0.0;
-        }
+      for (int l = 0; l < NV; ++l) {
+        const long c = io + l * g.N;
+        if (STAGE == 1) ra[l] = ld8_own<STREAM>(q + c, p8);
+        if (STAGE == 2 || STAGE == 3) ra[l] = ld8_own<STREAM>(b1 + c, p8);
+        if (STAGE == 4 || (STAGE >= 2 && b2)) rb[l] = ld8_own<STREAM>(b2 + c, p8);
       }
     }
     // this plane's operands are spent: load the next plane's now
-    const int zn = zl + 1;
-    const bool nxy = zn >= z0 && zn < z1;
-    if (zn < z1 + 4) {
-      load_pt(i, j, wrap(zn, dz), nxy ? 7 : 4, nt);
-      if (nxy && hmask) load_pt(hi, hj, wrap(zn, dz), hmask, nh);
-    }
-    if (zl >= z0 + 4) {
+    const unsigned n8 = plane8 * (unsigned)wrap(min(zl + 1, z1 + 3), dz);
+    load_pt(col8 + n8, XY, ct);
+    if constexpr (XY) load_halo(hcol8 + n8, ch);
+    if constexpr (OUT) {
       const int zo = zl - 4;
-      const long p = i + (long)g.n[0] * j + n01 * zo;
       double r[NV];
 #pragma unroll
       for (int l = 0; l < NV; ++l) {
@@ -1773,46 +1787,35 @@ __global__ void __launch_bounds__(BX * BY, 512 / (BX * BY)) k_fwd3d_march(Geo g,
         const double v = ring[zo & 3][l][t] + out;
         r[l] = 0.0 - v;
       }
-      int ijk[3] = {i, j, zo};
-      const double jac = jacobian<3>(g, ijk);
+      const double jac = 1.0 / (h01 * ld_const(g.h[2], zo));   // jacobian<3>
 #pragma unroll
       for (int l = 0; l < NV; ++l) r[l] = r[l] * jac;
-      if (kstr) r[1] = r[1] + rho_k * kk_k;
-      if (!RK) {
+      if (kstr) r[1] = r[1] + ring[zo & 3][NV][t] * kk;
 #pragma unroll
-        for (int l = 0; l < NV; ++l) rhs[inst * NV * g.N + l * g.N + p] = r[l];
-      } else {
-#pragma unroll
-        for (int l = 0; l < NV; ++l) {
-          const long ii = inst * NV * g.N + l * g.N + p;
-          const double rl = r[l];
-          double qn;
-          switch (rk_stage) {
-            case 1: {
-              const double q0 = ra[l];
-              if (b1) b1[ii] = q0;
-              if (b2) b2[ii] = q0 + div6(dt * rl);
-              qn = q0 + dt * rl / 2.0;
-              break;
-            }
-            case 2:
-              if (b2) b2[ii] = rb[l] + div3(dt * rl);
-              qn = ra[l] + dt * rl / 2.0;
-              break;
-            case 3:
-              if (b2) b2[ii] = rb[l] + div3(dt * rl);
-              qn = ra[l] + dt * rl;
-              break;
-            default:
-              qn = rb[l] + div6(dt * rl);
-              break;
-          }
-          yout[ii] = qn;
-          if (copy) copy[ii] = qn;
+      for (int l = 0; l < NV; ++l) {
+        const long c = io + l * g.N;
+        const double rl = r[l];
+        if (STAGE == 0) {
+          st8_own<STREAM>(rhs + c, bytes, w8, rl);
+          continue;
         }
+        double qn;
+        if (STAGE == 1) {
+          const double q0 = ra[l];
+          if (b1) st8_own<STREAM>(b1 + c, bytes, w8, q0);
+          if (b2) st8_own<STREAM>(b2 + c, bytes, w8, q0 + div6(dt * rl));
+          qn = q0 + dt * rl / 2.0;
+        } else if (STAGE == 2 || STAGE == 3) {
+          if (b2) st8_own<STREAM>(b2 + c, bytes, w8, rb[l] + div3(dt * rl));
+          qn = STAGE == 2 ? ra[l] + dt * rl / 2.0 : ra[l] + dt * rl;
+        } else {
+          qn = rb[l] + div6(dt * rl);
+        }
+        st8_own<STREAM>(yout + c, bytes, w8, qn);
+        if (copy) st8_own<STREAM>(copy + c, bytes, w8, qn);
       }
     }
-    if (xy) {
+    if constexpr (XY) {
       __syncthreads();          // readers of the previous plane's fluxes are done
 #pragma unroll
       for (int l = 0; l < NV; ++l) {
@@ -1821,152 +1824,36 @@ __global__ void __launch_bounds__(BX * BY, 512 / (BX * BY)) k_fwd3d_march(Geo g,
       }
       if (hmask == 1) {
 #pragma unroll
-        for (int l = 0; l < NV; ++l) sfx[l][hy][hx] = fh[0][l];
+        for (int l = 0; l < NV; ++l) sfx[l][m.hy][m.hx] = fh[l];
       } else if (hmask == 2) {
 #pragma unroll
-        for (int l = 0; l < NV; ++l) sfy[l][hy][hx] = fh[1][l];
+        for (int l = 0; l < NV; ++l) sfy[l][m.hy][m.hx] = fh[l];
       }
       __syncthreads();
 #pragma unroll
       for (int l = 0; l < NV; ++l) {
-        const double* rx = &sfx[l][ty][tx + 4];
-        const double* cy = &sfy[l][ty + 4][tx];
-        double ox = 0.0, oy = 0.0;
-        ox += c1 * (rx[1] - rx[-1]);
-        ox += c2 * (rx[2] - rx[-2]);
-        ox += c3 * (rx[3] - rx[-3]);
-        ox += c4 * (rx[4] - rx[-4]);
-        oy += c1 * (cy[BX] - cy[-BX]);
-        oy += c2 * (cy[2 * BX] - cy[-2 * BX]);
-        oy += c3 * (cy[3 * BX] - cy[-3 * BX]);
-        oy += c4 * (cy[4 * BX] - cy[-4 * BX]);
-        ring[zl & 3][l][t] = ox + oy;   // each thread reads back only its own slots
+        Cross k;
+        cross_load(&sfx[l][ty][tx + 4], &sfy[l][ty + 4][tx], BX, k);
+        __builtin_amdgcn_sched_barrier(0);
+        // each thread reads back only its own slots
+        ring[zl & 3][l][t] = diff4(k.xp, k.xm, c1, c2, c3, c4) + diff4(k.yp, k.ym, c1, c2, c3, c4);
       }
+      ring[zl & 3][NV][t] = rho;
     }
 #pragma unroll
     for (int k = 0; k < 8; ++k)
 #pragma unroll
       for (int l = 0; l < NV; ++l) W[k][l] = W[k + 1][l];
-    ct = nt;
-    if (nxy && hmask) ch = nh;
-  }
-}
-
-// The z pass of the adjoint's second derivative pass (D-dagger of the viscous block
-// T1[z] components 1..4) fused with k_finish's adjoint operations, for 3-D regions whose
-// patches are at most one Kolmogorov forcing over the whole domain, with no dissipation
-// and no far field (the chain rule then sits in the finishing pass).  One thread per
-// z-line as in k_deriv_line, the 9-point windows of the four components in registers.
-// At each point t2_a = A_a + (D-dagger_z T1)_a, where A = S_x + S_y was accumulated by
-// the x and y passes in S slot 0 (the sum k_finish forms, in its order); then the chain
-// rule, the Jacobian scaling and the Kolmogorov term, as k_finish applies them.  With
-// rk_stage > 0 the point's RK4 adjoint update follows at once (k_rk_adjoint's
-// arithmetic; lam is then y, read at the point before it is written) and rhs is not
-// written.
-__global__ void __launch_bounds__(kBlock) k_adj_finish_z(Geo g, const double* __restrict__ T1z,
-                                                        const double* __restrict__ A, long t_inst,
-                                                        const double* __restrict__ q,
-                                                        const double* lam,
-                                                        const double* __restrict__ kstr,
-                                                        double* __restrict__ rhs, int rk_stage,
-                                                        double dt, double* y, double* b1,
-                                                        double* b2) {
-  constexpr int ND = 3, NV = 5, NW = 4;
-  const Dir dd = g.dir[2];
-  const long nlines = g.N / dd.len;
-  const long line = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (line >= nlines) return;
-  const long inst = blockIdx.z;
-  const long n0 = g.n[0];
-  const long i = line % n0, o = line / n0;
-  const long base = i + o * n0;
-  const long sd = dd.stride;
-  const double* x = T1z + inst * t_inst + base;
-  const double* ai = A + inst * t_inst + base;
-  const double* qi = q + inst * NV * g.N;
-  const double* li = lam + inst * NV * g.N;
-  double* ri = rhs + inst * NV * g.N;
-  const int z0 = blockIdx.y * kLineChunk;
-  const int z1 = min(z0 + kLineChunk, dd.len);
-  const Op& op = g.ops[SLOT_ADJ];
-  const double c1 = op.c[kMaxHW + 1], c2 = op.c[kMaxHW + 2], c3 = op.c[kMaxHW + 3],
-               c4 = op.c[kMaxHW + 4];
-  double Q[NW][9];
-#pragma unroll
-  for (int a = 0; a < NW; ++a)
-#pragma unroll
-    for (int k = 0; k < 8; ++k) Q[a][k] = x[a * g.N + wrap(z0 - 4 + k, dd) * sd];
-  for (int z = z0; z < z1; ++z) {
-    const long p = base + z * sd;
-    double t2[NW];
-#pragma unroll
-    for (int a = 0; a < NW; ++a) {
-      Q[a][8] = x[a * g.N + wrap(z + 4, dd) * sd];
-      double out = 0.0;
-      out += c1 * (Q[a][5] - Q[a][3]);
-      out += c2 * (Q[a][6] - Q[a][2]);
-      out += c3 * (Q[a][7] - Q[a][1]);
-      out += c4 * (Q[a][8] - Q[a][0]);
-      t2[a] = ai[a * g.N + z * sd] + out;
-#pragma unroll
-      for (int k = 0; k < 8; ++k) Q[a][k] = Q[a][k + 1];
-    }
-    double v[NV], r[NV];
-    load_q<ND>(qi, g.N, p, v);
-#pragma unroll
-    for (int l = 0; l < NV; ++l) r[l] = ri[l * g.N + p];
-    adj_chain_t2<ND>(g, v, t2, -1.0, r);
-    int ijk[3] = {(int)i, (int)o, z};
-    const double jac = jacobian<ND>(g, ijk);
-#pragma unroll
-    for (int l = 0; l < NV; ++l) r[l] = r[l] * jac;
-    if (kstr) r[0] = r[0] - li[g.N + p] * kstr[p];
-    if (rk_stage == 0) {
-#pragma unroll
-      for (int l = 0; l < NV; ++l) ri[l * g.N + p] = r[l];
-    } else {
-#pragma unroll
-      for (int l = 0; l < NV; ++l) {
-        const long ii = inst * NV * g.N + l * g.N + p;
-        const double rl = r[l];
-        switch (rk_stage) {
-          case 4: {
-            const double l0 = y[ii];
-            b1[ii] = l0;
-            b2[ii] = l0 - div6(dt * rl);
-            y[ii] = l0 - dt * rl / 2.0;
-            break;
-          }
-          case 3:
-            b2[ii] = b2[ii] - div3(dt * rl);
-            y[ii] = b1[ii] - dt * rl / 2.0;
-            break;
-          case 2:
-            b2[ii] = b2[ii] - div3(dt * rl);
-            y[ii] = b1[ii] - dt * rl;
-            break;
-          default:
-            y[ii] = b2[ii] - div6(dt * rl);
-            break;
-        }
-      }
-    }
-  }
-}
-
-// Element access at a 32-bit byte offset from a wave-uniform base pointer: the address
-// form of a global load / store with a scalar base and a 32-bit vector offset, so a
-// thread keeps one 32-bit offset per point instead of a 64-bit address per component.
-// Callers keep byte offsets below 2^32 (fewer than 2^29 points per component array).
-__device__ __forceinline__ double ld8(const double* base, unsigned off) {
-  return *reinterpret_cast<const double*>(reinterpret_cast<const char*>(base) + off);
-}
-__device__ __forceinline__ void st8(double* base, unsigned off, double v) {
-  *reinterpret_cast<double*>(reinterpret_cast<char*>(base) + off) = v;
+  };
+  int zl = z0;                                             // all bounds uniform over the block
+  for (; zl < min(z0 + 4, z1); ++zl) plane(zl, yes, no);
+  for (; zl < z0 + 4; ++zl) plane(zl, no, no);             // chunks of fewer than 4 planes
+  for (; zl < z1; ++zl) plane(zl, yes, yes);
+  for (; zl < z1 + 4; ++zl) plane(zl, no, yes);
 }
 
 // The first half of the adjoint rhs of a viscous 3-D region periodic in every direction,
-// in one z march: a BX x BY column tile marches along z over a chunk of ZC planes, each
+// in one z march: a BX x BY column tile marches along z over a chunk of zc planes, each
 // thread keeping lambda of its column for the 9 planes of the z stencil in registers; the
 // plane being worked on is staged in LDS with its 4-point x / y halo (one halo point per
 // thread), so T1_d = D-dagger_d lambda of all three directions is formed at the point
@@ -1979,8 +1866,8 @@ __device__ __forceinline__ void st8(double* base, unsigned off, double v) {
 // same.  The halo point of the next plane and the lambda entering the window are loaded
 // one plane ahead.  The window of the last NZL components lives in an LDS ring of 9
 // planes (each thread reads back only its own column), the others in registers.
-template <int BX, int BY, int ZC, bool POWER>
-__global__ void __launch_bounds__(BX * BY, 512 / (BX * BY)) k_adj3d_jac_march(Geo g, const double* __restrict__ q,
+template <int BX, int BY, bool POWER, bool STREAM>
+__global__ void __launch_bounds__(BX * BY, 512 / (BX * BY)) k_adj3d_jac_march(Geo g, int zc, const double* __restrict__ q,
                                                               const double* __restrict__ lam,
                                                               const double* __restrict__ S,
                                                               double* __restrict__ rhs,
@@ -1990,26 +1877,33 @@ __global__ void __launch_bounds__(BX * BY, 512 / (BX * BY)) k_adj3d_jac_march(Ge
   __shared__ double slx[NV][BY][EXW];
   __shared__ double sly[NV][BY + 8][BX];
   __shared__ double zring[9][NZL][NT];
-  int x0, y0, z0;
-  if (!march_unit<BX, BY, ZC>(g, x0, y0, z0)) return;
-  const int z1 = min(z0 + ZC, g.n[2]);
+  MarchUnit u;
+  if (!march_unit<BX, BY>(g, zc, u)) return;
+  const int z0 = u.z0, z1 = u.z1;
   const long inst = blockIdx.z;
   const double* qi = q + inst * NV * g.N;
   const double* li = lam + inst * NV * g.N;
   const double* Si = S + inst * 12 * g.N;
   double* ri = rhs + inst * NV * g.N;
   double* Ti = T1 + inst * 3 * NV * g.N;
-  const int t = threadIdx.x, tx = t % BX, ty = t / BX;
-  const int i = x0 + tx, j = y0 + ty;
-  int hx, hy, hi, hj, hmask;
-  march_halo<BX, BY>(g, t, x0, y0, hx, hy, hi, hj, hmask);
+  const MarchThread m = march_thread<BX, BY>(g, u);
+  const int t = threadIdx.x, tx = m.tx, ty = m.ty;
   // byte offsets of the thread's column and halo column, and of one plane
   const unsigned n0 = (unsigned)g.n[0], plane8 = 8u * n0 * (unsigned)g.n[1];
-  const unsigned col8 = 8u * ((unsigned)i + n0 * (unsigned)j);
-  const unsigned hcol8 = 8u * ((unsigned)hi + n0 * (unsigned)hj);
+  const unsigned bytes = 8u * (unsigned)g.N;
+  const unsigned col8 = 8u * ((unsigned)m.i + n0 * (unsigned)m.j);
+  const unsigned hcol8 = 8u * ((unsigned)m.hi + n0 * (unsigned)m.hj);
+  const double h0 = g.h[0][m.i], h1 = g.h[1][m.j], h01 = h0 * h1;
   auto load_l = [&](unsigned off, double* v) {
 #pragma unroll
     for (int l = 0; l < NV; ++l) v[l] = ld8(li + l * g.N, off);
+  };
+  double v[NV], sv[9];
+  auto load_pt = [&](unsigned off) {
+#pragma unroll
+    for (int l = 0; l < NV; ++l) v[l] = ld8_own<STREAM>(qi + l * g.N, off);
+#pragma unroll
+    for (int k = 0; k < 9; ++k) sv[k] = ld8_own<STREAM>(Si + k * g.N, off);
   };
   const Op& op = g.ops[SLOT_ADJ];
   const double c1 = op.c[kMaxHW + 1], c2 = op.c[kMaxHW + 2], c3 = op.c[kMaxHW + 3], c4 = op.c[kMaxHW + 4];
@@ -2018,56 +1912,49 @@ __global__ void __launch_bounds__(BX * BY, 512 / (BX * BY)) k_adj3d_jac_march(Ge
   double W[9][NZR];
 #pragma unroll
   for (int k = 0; k < 8; ++k) {
-    double v[NV];
-    load_l(col8 + plane8 * (unsigned)wrap(z0 - 4 + k, dz), v);
+    double w[NV];
+    load_l(col8 + plane8 * (unsigned)wrap(z0 - 4 + k, dz), w);
 #pragma unroll
-    for (int l = 0; l < NZR; ++l) W[k][l] = v[l];
+    for (int l = 0; l < NZR; ++l) W[k][l] = w[l];
 #pragma unroll
-    for (int l = NZR; l < NV; ++l) zring[k][l - NZR][t] = v[l];
+    for (int l = NZR; l < NV; ++l) zring[k][l - NZR][t] = w[l];
   }
-  double nl[NV], nh[NV] = {};
+  double nl[NV], nh[NV];
   load_l(col8 + plane8 * (unsigned)wrap(z0 + 4, dz), nl);
-  if (hmask) load_l(hcol8 + plane8 * (unsigned)z0, nh);
+  load_l(hcol8 + plane8 * (unsigned)z0, nh);
+  load_pt(col8 + plane8 * (unsigned)z0);
   int rb = 0;                            // ring slot of plane zo - 4
   for (int zo = z0; zo < z1; ++zo) {     // uniform over the block
-    double hv[NV], wc[NV];
     const int r8 = rb + 8 < 9 ? rb + 8 : rb - 1;
+    const int r4 = rb + 4 < 9 ? rb + 4 : rb - 5;
+    __syncthreads();            // readers of the previous plane are done
 #pragma unroll
     for (int l = 0; l < NV; ++l) {
       if (l < NZR) W[8][l] = nl[l];
       else zring[r8][l - NZR][t] = nl[l];
-      hv[l] = nh[l];
+      const double wc = l < NZR ? W[4][l] : zring[r4][l - NZR][t];
+      slx[l][ty][tx + 4] = wc;
+      sly[l][ty + 4][tx] = wc;
     }
-    const int r4 = rb + 4 < 9 ? rb + 4 : rb - 5;
+    if (m.hmask == 1) {
 #pragma unroll
-    for (int l = 0; l < NV; ++l) wc[l] = l < NZR ? W[4][l] : zring[r4][l - NZR][t];
-    if (zo + 1 < z1) {
-      load_l(col8 + plane8 * (unsigned)wrap(zo + 5, dz), nl);
-      if (hmask) load_l(hcol8 + plane8 * (unsigned)(zo + 1), nh);
+      for (int l = 0; l < NV; ++l) slx[l][m.hy][m.hx] = nh[l];
+    } else if (m.hmask == 2) {
+#pragma unroll
+      for (int l = 0; l < NV; ++l) sly[l][m.hy][m.hx] = nh[l];
     }
-    const unsigned p8 = col8 + plane8 * (unsigned)zo;
-    double v[NV], sv[9];
-#pragma unroll
-    for (int l = 0; l < NV; ++l) v[l] = ld8(qi + l * g.N, p8);
-#pragma unroll
-    for (int k = 0; k < 9; ++k) sv[k] = ld8(Si + k * g.N, p8);
-    __syncthreads();            // readers of the previous plane are done
-#pragma unroll
-    for (int l = 0; l < NV; ++l) {
-      slx[l][ty][tx + 4] = wc[l];
-      sly[l][ty + 4][tx] = wc[l];
-    }
-    if (hmask == 1) {
-#pragma unroll
-      for (int l = 0; l < NV; ++l) slx[l][hy][hx] = hv[l];
-    } else if (hmask == 2) {
-#pragma unroll
-      for (int l = 0; l < NV; ++l) sly[l][hy][hx] = hv[l];
-    }
+    // the next lead and halo points (the last plane's loads are not used)
+    load_l(col8 + plane8 * (unsigned)wrap(min(zo + 5, z1 + 3), dz), nl);
+    load_l(hcol8 + plane8 * (unsigned)min(zo + 1, z1 - 1), nh);
     __syncthreads();
-    const int ijk[3] = {i, j, zo};
+    const unsigned p8 = col8 + plane8 * (unsigned)zo, w8 = p8 | m.spare;
+    const double h2 = ld_const(g.h[2], zo);
     AdjPoint<3> P;
-    adj_point_init_stress<POWER>(g, v, sv, ijk, P);
+    P.h[0] = h1 * h2;             // metric<3>
+    P.h[1] = h0 * h2;
+    P.h[2] = h01;
+    P.jac = 1.0 / (h01 * h2);     // jacobian<3>
+    adj_point_init_stress<POWER>(g, v, sv, P);
     double r[NV], diff[3][NW];
 #pragma unroll
     for (int l = 0; l < NV; ++l) r[l] = 0.0;
@@ -2112,12 +1999,15 @@ __global__ void __launch_bounds__(BX * BY, 512 / (BX * BY)) k_adj3d_jac_march(Ge
       }
       adj_visc_dir<3, POWER>(P, g.gamma, d, t1, r, diff);
     }
+    // the point's q and slots are spent: the next plane's, before this one's stores (a wait
+    // for a load waits for the accesses issued before it)
+    load_pt(col8 + plane8 * (unsigned)min(zo + 1, z1 - 1));
 #pragma unroll
-    for (int l = 0; l < NV; ++l) st8(ri + l * g.N, p8, r[l]);
+    for (int l = 0; l < NV; ++l) st8_own<STREAM>(ri + l * g.N, bytes, w8, r[l]);
 #pragma unroll
     for (int d = 0; d < 3; ++d)
 #pragma unroll
-      for (int a = 0; a < NW; ++a) st8(Ti + (d * NV + 1 + a) * g.N, p8, diff[d][a]);
+      for (int a = 0; a < NW; ++a) st8_own<STREAM>(Ti + (d * NV + 1 + a) * g.N, bytes, w8, diff[d][a]);
 #pragma unroll
     for (int k = 0; k < 8; ++k)
 #pragma unroll
@@ -2129,23 +2019,23 @@ __global__ void __launch_bounds__(BX * BY, 512 / (BX * BY)) k_adj3d_jac_march(Ge
 // The second half, after k_adj3d_jac_march: t2 = (D-dagger_x T1_x + D-dagger_y T1_y) +
 // D-dagger_z T1_z over components 1..4 (the x / y operands of the plane staged in LDS with
 // their halo, one halo point per thread, the z operand in a 9-plane register window),
-// then, on the Jacobian part read back from rhs, k_adj_finish_z's operations: the chain
-// rule, the Jacobian scaling and the Kolmogorov term, and with rk_stage > 0 the RK4
-// adjoint update in place (y = lambda; only the point's own lambda is read), rhs not
-// written.  The sums and their order are those of k_deriv_row, k_deriv_line (x store, y
-// add) and k_adj_finish_z, so the values are the same.
-template <int BX, int BY, int ZC>
+// then, on the Jacobian part read back from rhs, k_finish's operations: the chain rule,
+// the Jacobian scaling and the Kolmogorov term, and with STAGE > 0 (the RK stage, a
+// compile-time value) the RK4 adjoint update in place (y = lambda; only the point's own
+// lambda is read), rhs not written.  The sums and their order are those of k_deriv_row, k_deriv_line (x store, y
+// add) and k_finish, so the values are the same.
+template <int BX, int BY, int STAGE, bool STREAM>
 __global__ void __launch_bounds__(BX * BY, 512 / (BX * BY)) k_adj3d_finish_march(
-    Geo g, const double* __restrict__ T1, const double* __restrict__ q, const double* lam,
-    const double* __restrict__ kstr, double* __restrict__ rhs, int rk_stage, double dt, double* y,
-    double* b1, double* b2) {
+    Geo g, int zc, const double* __restrict__ T1, const double* __restrict__ q, const double* lam,
+    const double* __restrict__ kstr, double* __restrict__ rhs, double dt, double* y, double* b1,
+    double* b2) {
   constexpr int NV = 5, NW = 4, EXW = BX + 8;
   static_assert(8 * (BX + BY) <= BX * BY, "at most one halo point per thread");
   __shared__ double snx[NW][BY][EXW];
   __shared__ double sny[NW][BY + 8][BX];
-  int x0, y0, z0;
-  if (!march_unit<BX, BY, ZC>(g, x0, y0, z0)) return;
-  const int z1 = min(z0 + ZC, g.n[2]);
+  MarchUnit u;
+  if (!march_unit<BX, BY>(g, zc, u)) return;
+  const int z0 = u.z0, z1 = u.z1;
   const long inst = blockIdx.z;
   const long io = inst * NV * g.N;
   const double* qi = q + io;
@@ -2154,14 +2044,16 @@ __global__ void __launch_bounds__(BX * BY, 512 / (BX * BY)) k_adj3d_finish_march
   const double* Ty = Tx + (long)NV * g.N;
   const double* Tz = Ty + (long)NV * g.N;
   double* ri = rhs + io;
-  const int t = threadIdx.x, tx = t % BX, ty = t / BX;
-  const int i = x0 + tx, j = y0 + ty;
-  int hx, hy, hi, hj, hmask;
-  march_halo<BX, BY>(g, t, x0, y0, hx, hy, hi, hj, hmask);
+  const MarchThread m = march_thread<BX, BY>(g, u);
+  const int tx = m.tx, ty = m.ty;
   const unsigned n0 = (unsigned)g.n[0], plane8 = 8u * n0 * (unsigned)g.n[1];
-  const unsigned col8 = 8u * ((unsigned)i + n0 * (unsigned)j);
-  const unsigned hcol8 = 8u * ((unsigned)hi + n0 * (unsigned)hj);
-  const double* Th = hmask == 1 ? Tx : Ty;
+  const unsigned bytes = 8u * (unsigned)g.N;
+  const unsigned col8 = 8u * ((unsigned)m.i + n0 * (unsigned)m.j);
+  const unsigned hcol8 = 8u * ((unsigned)m.hi + n0 * (unsigned)m.hj);
+  // the Kolmogorov strength depends on the row alone
+  const double kk = kstr ? kstr[n0 * (unsigned)m.j] : 0.0;
+  const double h01 = g.h[0][m.i] * g.h[1][m.j];
+  const double* Th = m.hmask == 1 ? Tx : Ty;
   auto load4 = [&](const double* src, unsigned off, double* v) {
 #pragma unroll
     for (int a = 0; a < NW; ++a) v[a] = ld8(src + a * g.N, off);
@@ -2172,118 +2064,79 @@ __global__ void __launch_bounds__(BX * BY, 512 / (BX * BY)) k_adj3d_finish_march
   double Z[9][NW];
 #pragma unroll
   for (int k = 0; k < 8; ++k) load4(Tz, col8 + plane8 * (unsigned)wrap(z0 - 4 + k, dz), Z[k]);
-  double nz[NW], nx[NW], ny[NW], nh[NW] = {};
+  double nz[NW], nx[NW], ny[NW], nh[NW];
   load4(Tz, col8 + plane8 * (unsigned)wrap(z0 + 4, dz), nz);
   load4(Tx, col8 + plane8 * (unsigned)z0, nx);
   load4(Ty, col8 + plane8 * (unsigned)z0, ny);
-  if (hmask) load4(Th, hcol8 + plane8 * (unsigned)z0, nh);
+  load4(Th, hcol8 + plane8 * (unsigned)z0, nh);
   for (int zo = z0; zo < z1; ++zo) {     // uniform over the block
-    double xv[NW], yv[NW], hv[NW];
-#pragma unroll
-    for (int a = 0; a < NW; ++a) {
-      Z[8][a] = nz[a];
-      xv[a] = nx[a];
-      yv[a] = ny[a];
-      hv[a] = nh[a];
-    }
-    if (zo + 1 < z1) {
-      const unsigned n8 = col8 + plane8 * (unsigned)(zo + 1);
-      load4(Tz, col8 + plane8 * (unsigned)wrap(zo + 5, dz), nz);
-      load4(Tx, n8, nx);
-      load4(Ty, n8, ny);
-      if (hmask) load4(Th, hcol8 + plane8 * (unsigned)(zo + 1), nh);
-    }
-    const unsigned p8 = col8 + plane8 * (unsigned)zo;
-    double v[NV], r[NV];
-#pragma unroll
-    for (int l = 0; l < NV; ++l) {
-      v[l] = ld8(qi + l * g.N, p8);
-      r[l] = ld8(ri + l * g.N, p8);
-    }
-    // the point's RK operands and Kolmogorov-term values, loaded here so that their
-    // latency overlaps the derivative work (stage 4 reads lambda before it writes it)
-    double ra[NV], rb[NV], lk = 0.0, kk = 0.0;
-    if (kstr) {
-      lk = ld8(li + g.N, p8);
-      kk = ld8(kstr, p8);
-    }
-#pragma unroll
-    for (int l = 0; l < NV; ++l) {
-      const long c = io + l * g.N;
-      ra[l] = rk_stage == 4 ? ld8(y + c, p8) : (rk_stage == 2 || rk_stage == 3) ? ld8(b1 + c, p8) : 0.0;
-      rb[l] = rk_stage >= 1 && rk_stage <= 3 ? ld8(b2 + c, p8) : 0.0;
-    }
     __syncthreads();            // readers of the previous plane are done
 #pragma unroll
     for (int a = 0; a < NW; ++a) {
-      snx[a][ty][tx + 4] = xv[a];
-      sny[a][ty + 4][tx] = yv[a];
+      snx[a][ty][tx + 4] = nx[a];
+      sny[a][ty + 4][tx] = ny[a];
+      Z[8][a] = nz[a];
     }
-    if (hmask == 1) {
+    if (m.hmask == 1) {
 #pragma unroll
-      for (int a = 0; a < NW; ++a) snx[a][hy][hx] = hv[a];
-    } else if (hmask == 2) {
+      for (int a = 0; a < NW; ++a) snx[a][m.hy][m.hx] = nh[a];
+    } else if (m.hmask == 2) {
 #pragma unroll
-      for (int a = 0; a < NW; ++a) sny[a][hy][hx] = hv[a];
+      for (int a = 0; a < NW; ++a) sny[a][m.hy][m.hx] = nh[a];
     }
+    // the point's state, rhs part, RK operands and Kolmogorov operand, used after the
+    // derivative work (stage 4 reads lambda before it writes it), then the next plane's
+    // stencil operands (the last plane's are not used)
+    const unsigned p8 = col8 + plane8 * (unsigned)zo, w8 = p8 | m.spare;
+    double v[NV], r[NV], ra[NV] = {}, rb[NV] = {}, lk = 0.0;
+#pragma unroll
+    for (int l = 0; l < NV; ++l) {
+      const long c = io + l * g.N;
+      v[l] = ld8_own<STREAM>(qi + l * g.N, p8);
+      r[l] = ld8_own<STREAM>(ri + l * g.N, p8);
+      if (STAGE == 4) ra[l] = ld8_own<STREAM>(y + c, p8);
+      if (STAGE == 2 || STAGE == 3) ra[l] = ld8_own<STREAM>(b1 + c, p8);
+      if (STAGE >= 1 && STAGE <= 3) rb[l] = ld8_own<STREAM>(b2 + c, p8);
+    }
+    if (kstr) lk = ld8(li + g.N, p8);
+    const int zn = min(zo + 1, z1 - 1);
+    const unsigned n8 = col8 + plane8 * (unsigned)zn;
+    load4(Tz, col8 + plane8 * (unsigned)wrap(min(zo + 5, z1 + 3), dz), nz);
+    load4(Tx, n8, nx);
+    load4(Ty, n8, ny);
+    load4(Th, hcol8 + plane8 * (unsigned)zn, nh);
     __syncthreads();
     double t2[NW];
 #pragma unroll
     for (int a = 0; a < NW; ++a) {
-      const double* rx = &snx[a][ty][tx + 4];
-      const double* cy = &sny[a][ty + 4][tx];
-      double ox = 0.0, oy = 0.0, oz = 0.0;
-      ox += c1 * (rx[1] - rx[-1]);
-      ox += c2 * (rx[2] - rx[-2]);
-      ox += c3 * (rx[3] - rx[-3]);
-      ox += c4 * (rx[4] - rx[-4]);
-      oy += c1 * (cy[BX] - cy[-BX]);
-      oy += c2 * (cy[2 * BX] - cy[-2 * BX]);
-      oy += c3 * (cy[3 * BX] - cy[-3 * BX]);
-      oy += c4 * (cy[4 * BX] - cy[-4 * BX]);
+      Cross k;
+      cross_load(&snx[a][ty][tx + 4], &sny[a][ty + 4][tx], BX, k);
+      __builtin_amdgcn_sched_barrier(0);
+      double oz = 0.0;
       oz += c1 * (Z[5][a] - Z[3][a]);
       oz += c2 * (Z[6][a] - Z[2][a]);
       oz += c3 * (Z[7][a] - Z[1][a]);
       oz += c4 * (Z[8][a] - Z[0][a]);
-      t2[a] = (ox + oy) + oz;
+      t2[a] = (diff4(k.xp, k.xm, c1, c2, c3, c4) + diff4(k.yp, k.ym, c1, c2, c3, c4)) + oz;
     }
     adj_chain_t2<3>(g, v, t2, -1.0, r);
-    const int ijk[3] = {i, j, zo};
-    const double jac = jacobian<3>(g, ijk);
+    const double jac = 1.0 / (h01 * ld_const(g.h[2], zo));   // jacobian<3>
 #pragma unroll
-    for (int l = 0; l < NV; ++l) r[l] = r[l] * jac;
-    if (kstr) r[0] = r[0] - lk * kk;
-    if (rk_stage == 0) {
-#pragma unroll
-      for (int l = 0; l < NV; ++l) st8(ri + l * g.N, p8, r[l]);
-    } else {
-#pragma unroll
-      for (int l = 0; l < NV; ++l) {
-        const long c = io + l * g.N;
-        double* yc = y + c;
-        double* b1c = b1 + c;
-        double* b2c = b2 + c;
-        const double rl = r[l];
-        switch (rk_stage) {
-          case 4: {
-            const double l0 = ra[l];
-            st8(b1c, p8, l0);
-            st8(b2c, p8, l0 - div6(dt * rl));
-            st8(yc, p8, l0 - dt * rl / 2.0);
-            break;
-          }
-          case 3:
-            st8(b2c, p8, rb[l] - div3(dt * rl));
-            st8(yc, p8, ra[l] - dt * rl / 2.0);
-            break;
-          case 2:
-            st8(b2c, p8, rb[l] - div3(dt * rl));
-            st8(yc, p8, ra[l] - dt * rl);
-            break;
-          default:
-            st8(yc, p8, rb[l] - div6(dt * rl));
-            break;
-        }
+    for (int l = 0; l < NV; ++l) {
+      const long c = io + l * g.N;
+      double rl = r[l] * jac;
+      if (l == 0 && kstr) rl = rl - lk * kk;
+      if (STAGE == 0) {
+        st8_own<STREAM>(rhs + c, bytes, w8, rl);
+      } else if (STAGE == 4) {
+        st8_own<STREAM>(b1 + c, bytes, w8, ra[l]);
+        st8_own<STREAM>(b2 + c, bytes, w8, ra[l] - div6(dt * rl));
+        st8_own<STREAM>(y + c, bytes, w8, ra[l] - dt * rl / 2.0);
+      } else if (STAGE >= 2) {
+        st8_own<STREAM>(b2 + c, bytes, w8, rb[l] - div3(dt * rl));
+        st8_own<STREAM>(y + c, bytes, w8, STAGE == 3 ? ra[l] - dt * rl / 2.0 : ra[l] - dt * rl);
+      } else {
+        st8_own<STREAM>(y + c, bytes, w8, rb[l] - div6(dt * rl));
       }
     }
 #pragma unroll
@@ -2390,12 +2243,12 @@ static dim3 grid_pts(const Geo& g) {
   return dim3((unsigned)((g.N + kBlock - 1) / kBlock), (unsigned)g.ninst);
 }
 
-// k_prim + k_grad, or the one-pass periodic 3-D gradient kernel where it applies
-// (3-D, every direction periodic, x / y sizes multiples of its 32 x 16 tile).
-constexpr int kG3X = 32, kG3Y = 16;
+// Where the one-pass gradient kernel and the marches apply: 3-D, periodic in every direction,
+// any size (their tiles may be partial; regions hold at least 9 points along a periodic
+// direction), and component arrays that 32-bit byte offsets reach.
 static bool grad3d_applies(const Geo& g) {
-  return g.nd == 3 && g.dir[0].periodic && g.dir[1].periodic && g.dir[2].periodic &&
-         g.n[0] % kG3X == 0 && g.n[1] % kG3Y == 0 && g.nv == 5;
+  return g.nd == 3 && g.nv == 5 && g.dir[0].periodic && g.dir[1].periodic && g.dir[2].periodic &&
+         g.N < (1L << 29) - 1024;
 }
 
 // x / y flux divergence kernel of 3-D grids periodic in x and y with sizes that are
@@ -2406,72 +2259,73 @@ static bool fluxdiv3d_applies(const Geo& g) {
          g.n[0] % kFD3X == 0 && g.n[1] % kFD3Y == 0;
 }
 
-// grid of the periodic gradient kernel: (tile, z chunk) units padded to a multiple of 8
-// The z chunk (planes per work unit) of the 3-D marches, g.zchunk: 32, 64 or 128, and the
-// x extent of their tiles, g.mtile: 16 (16 x 16 tiles of 256 threads, two work-groups
-// per CU) or 32 (32 x 16 tiles of 512 threads, one per CU: fewer halo points per point) --
-// the autotuner's choices; no value depends on them.  f is called with them as
-// compile-time values.
-// The forward march and the stress pass use (g.zchunk, g.mtile), the adjoint marches
-// (g.zchunk_adj, g.mtile_adj).
-static int zchunk_of(const Geo& g, bool adj = false) {
-  const int z = adj ? g.zchunk_adj : g.zchunk;
-  return z == 32 || z == 128 ? z : 64;
-}
+// The planes per work unit of the 3-D marches, g.zchunk, and the x extent of their tiles,
+// g.mtile: 16 (16 x 16 tiles of 256 threads, two work-groups per CU) or 32 (32 x 16 tiles of
+// 512 threads, one per CU: fewer halo points per point) -- the autotuner's choices; no value
+// depends on them.  The forward march and the stress pass use (g.zchunk, g.mtile), the
+// adjoint marches (g.zchunk_adj, g.mtile_adj).
+static int zchunk_of(const Geo& g, bool adj = false) { return adj ? g.zchunk_adj : g.zchunk; }
 static int mtile_of(const Geo& g, bool adj = false) {
-  return (adj ? g.mtile_adj : g.mtile) == 32 && g.n[0] % 32 == 0 ? 32 : 16;
+  return (adj ? g.mtile_adj : g.mtile) == 32 ? 32 : 16;
 }
-template <class F>
-static void with_zchunk(const Geo& g, bool adj, F&& f) {
-  switch (zchunk_of(g, adj)) {
-    case 32: f(std::integral_constant<int, 32>{}); break;
-    case 128: f(std::integral_constant<int, 128>{}); break;
-    default: f(std::integral_constant<int, 64>{}); break;
-  }
-}
+// f is called with the tile width as a compile-time value
 template <class F>
 static void with_march(const Geo& g, bool adj, F&& f) {
-  with_zchunk(g, adj, [&](auto Z) {
-    if (mtile_of(g, adj) == 32) f(std::integral_constant<int, 32>{}, Z);
-    else f(std::integral_constant<int, 16>{}, Z);
-  });
+  if (mtile_of(g, adj) == 32) f(std::integral_constant<int, 32>{});
+  else f(std::integral_constant<int, 16>{});
 }
-
-static dim3 grad3d_grid(const Geo& g) {
-  const int zc = zchunk_of(g);
-  const int units = (g.n[0] / kG3X) * (g.n[1] / kG3Y) * ((g.n[2] + zc - 1) / zc);
-  return dim3(8 * ((units + 7) / 8), 1, g.ninst);
+// Whether the marches stream (non-temporal) what no other block reads: where a stage's
+// arrays, some 200 bytes a point, do not fit the 256 MB Infinity Cache and none of it is
+// found there again (forward stages 256^3: 935 us, 887 streamed; 160^3: 256 and 247), not
+// where they do, and the next kernel reads them from it (100^3: 112 us, 136 streamed).
+static bool march_streams(const Geo& g) { return g.N * g.ninst > 1500000; }
+// f is called with the RK stage (0: none) and march_streams as compile-time values
+template <class F>
+static void with_stage(const Geo& g, int stage, F&& f) {
+  const auto go = [&](auto ST) {
+    if (march_streams(g)) f(ST, std::true_type{});
+    else f(ST, std::false_type{});
+  };
+  switch (stage) {
+    case 0: go(std::integral_constant<int, 0>{}); break;
+    case 1: go(std::integral_constant<int, 1>{}); break;
+    case 2: go(std::integral_constant<int, 2>{}); break;
+    case 3: go(std::integral_constant<int, 3>{}); break;
+    default: go(std::integral_constant<int, 4>{}); break;
+  }
 }
+int march_units(const Geo& g, int mtile, int zc) {
+  return ((g.n[0] + mtile - 1) / mtile) * ((g.n[1] + kMarchRows - 1) / kMarchRows) *
+         ((g.n[2] + zc - 1) / zc);
+}
+// grid of a march: its work units padded to a multiple of 8
+static dim3 units_grid(const Geo& g, int mtile, int zc) {
+  return dim3(8 * ((march_units(g, mtile, zc) + 7) / 8), 1, g.ninst);
+}
+// The gradient / stress pass runs on 16 x 16 tiles, two work-groups a CU (256^3: 464 us, 480
+// on 32 x 16 with one; 64^3: 54 and 80), over chunks of at most 64 planes (500 us at 128).
+constexpr int kG3X = 16, kG3Y = kMarchRows;
+static int grad3d_chunk(const Geo& g) { return min(zchunk_of(g), 64); }
+static dim3 grad3d_grid(const Geo& g) { return units_grid(g, kG3X, grad3d_chunk(g)); }
 
 template <int ND>
 static void launch_gradients(const Geo& g, const double* q, double* w, double* G, const dim3& grid,
                              hipStream_t st) {
   if (ND == 3 && grad3d_applies(g)) {
-    with_zchunk(g, false, [&](auto Z) {
-      k_grad3d_periodic<kG3X, kG3Y, decltype(Z)::value><<<grad3d_grid(g), kG3X * kG3Y, 0, st>>>(g, q, G);
-    });
+    k_grad3d_periodic<kG3X, kG3Y><<<grad3d_grid(g), kG3X * kG3Y, 0, st>>>(g, grad3d_chunk(g), q, G);
     return;
   }
   k_prim<ND><<<grid, kBlock, 0, st>>>(g, q, w);
   for (int d = 0; d < ND; ++d) k_grad<ND><<<grid, kBlock, 0, st>>>(g, d, w, G);
 }
 
-// The one-march forward kernel: 3-D, periodic in every direction, x / y sizes multiples
-// of its 16 x 16 tile; viscous regions also need the stress kernel (grad3d_applies).
-constexpr int kFMX = 16, kFMY = 16;
-// grid of the 3-D march kernels: (tile, z chunk) units padded to a multiple of 8
+// grid of the forward march (or the adjoint marches)
 static dim3 march_grid(const Geo& g, bool adj) {
-  const int zc = zchunk_of(g, adj);
-  const int units = (g.n[0] / mtile_of(g, adj)) * (g.n[1] / kFMY) * ((g.n[2] + zc - 1) / zc);
-  return dim3(8 * ((units + 7) / 8), 1, g.ninst);
-}
-static bool fwd3d_march_applies(const Geo& g) {
-  return g.nd == 3 && g.nv == 5 && g.dir[0].periodic && g.dir[1].periodic && g.dir[2].periodic &&
-         g.n[0] % kFMX == 0 && g.n[1] % kFMY == 0 && (!g.viscous || grad3d_applies(g));
+  return units_grid(g, mtile_of(g, adj), zchunk_of(g, adj));
 }
 
 bool fwd3d_march_path(const Geo& g, const FinishInfo& fin, int nsrc) {
-  return fin.simple && !g.dissipation && nsrc == 0 && fwd3d_march_applies(g);
+  return fin.simple && !g.dissipation && nsrc == 0 && grad3d_applies(g);
 }
 
 // The two-march adjoint path: viscous, periodic in every direction with the march tile
@@ -2479,7 +2333,7 @@ bool fwd3d_march_path(const Geo& g, const FinishInfo& fin, int nsrc) {
 // chain rule and the forcing then sit in the finishing march).
 static bool adj3d_march_path(const Geo& g, const FinishInfo& fin) {
   return g.viscous && !g.dissipation && !fin.has_farfield && fin.simple &&
-         fwd3d_march_applies(g) && g.N < (1L << 29);   // 32-bit byte offsets
+         grad3d_applies(g);
 }
 
 bool stress_reuse_path(const Geo& g, const FinishInfo& fin, int nsrc) {
@@ -2488,26 +2342,25 @@ bool stress_reuse_path(const Geo& g, const FinishInfo& fin, int nsrc) {
 
 void launch_stress3d(const Geo& g, const double* q, double* S, hipStream_t st) {
   const dim3 gg = grad3d_grid(g);
-  with_zchunk(g, false, [&](auto Z) {
-    if (g.power_law > 0.0)
-      k_grad3d_periodic<kG3X, kG3Y, decltype(Z)::value, true, true><<<gg, kG3X * kG3Y, 0, st>>>(g, q, S);
-    else
-      k_grad3d_periodic<kG3X, kG3Y, decltype(Z)::value, true, false><<<gg, kG3X * kG3Y, 0, st>>>(g, q, S);
-  });
+  const int zc = grad3d_chunk(g);
+  if (g.power_law > 0.0)
+    k_grad3d_periodic<kG3X, kG3Y, true, true><<<gg, kG3X * kG3Y, 0, st>>>(g, zc, q, S);
+  else
+    k_grad3d_periodic<kG3X, kG3Y, true, false><<<gg, kG3X * kG3Y, 0, st>>>(g, zc, q, S);
 }
 
 void launch_fwd3d_march(const Geo& g, const double* q, const double* S, const double* kstr,
                         double* rhs, const RkStage* rk, hipStream_t st) {
   const dim3 gm = march_grid(g, false);
   if (rk && rk->ev_begin) (void)hipEventRecord(rk->ev_begin, st);
-  with_march(g, false, [&](auto X, auto Z) {
-    constexpr int BX = decltype(X)::value;
-    if (rk)
-      k_fwd3d_march<BX, kFMY, decltype(Z)::value, true><<<gm, BX * kFMY, 0, st>>>(
-          g, q, S, kstr, rhs, rk->stage, rk->dt, rk->yout, rk->b1, rk->b2, rk->copy);
-    else
-      k_fwd3d_march<BX, kFMY, decltype(Z)::value, false><<<gm, BX * kFMY, 0, st>>>(
-          g, q, S, kstr, rhs, 0, 0.0, nullptr, nullptr, nullptr, nullptr);
+  const int zc = zchunk_of(g);
+  with_march(g, false, [&](auto X) {
+    constexpr int BX = decltype(X)::value, BY = kMarchRows;
+    with_stage(g, rk ? rk->stage : 0, [&](auto ST, auto NT) {
+      k_fwd3d_march<BX, BY, decltype(ST)::value, decltype(NT)::value><<<gm, BX * BY, 0, st>>>(
+          g, zc, q, S, kstr, rhs, rk ? rk->dt : 0.0, rk ? rk->yout : nullptr, rk ? rk->b1 : nullptr,
+          rk ? rk->b2 : nullptr, rk ? rk->copy : nullptr);
+    });
   });
   if (rk && rk->ev_end) (void)hipEventRecord(rk->ev_end, st);
 }
@@ -2518,35 +2371,22 @@ int launch_rhs_forward(const Geo& g, const Patches* P, const double* q, double* 
                        const FinishInfo& fin, hipStream_t st, const RkStage* rk) {
   const dim3 grid = grid_pts(g);
   const int has_farfield = fin.has_farfield;
-  if (F && fin.simple && !g.dissipation && nsrc == 0 && fwd3d_march_applies(g)) {
+  if (F && fwd3d_march_path(g, fin, nsrc)) {
     // the whole rhs in one z march; with an RK stage only out of place (rk->yout)
     if (g.viscous) launch_stress3d(g, q, G, st);
     const bool rk_out = rk && rk->yout;
     launch_fwd3d_march(g, q, G, fin.kolmogorov, rhs, rk_out ? rk : nullptr, st);
     return rk_out ? RK_TO_YOUT : RK_NOT_APPLIED;
   }
-  bool finished = false;
   MGD_DISPATCH(g.nd, {
     if (g.viscous) launch_gradients<ND>(g, q, w, G, grid, st);
     if (F && ND == 3 && fluxdiv3d_applies(g)) {
       const dim3 gg((g.n[0] / kFD3X) * (g.n[1] / kFD3Y), g.n[2], g.ninst);
       k_fluxdiv3d_xy<kFD3X, kFD3Y><<<gg, kFD3X * kFD3Y, 0, st>>>(g, q, g.viscous ? G : nullptr, F, rhs);
-      // the z divergence also finishes the rhs where nothing else follows it
-      const bool fuse = fin.simple && !g.dissipation && nsrc == 0 && deriv_line_applies(g, ND - 1);
       const double* fz = F + (long)(ND - 1) * g.nv * g.N;
-      if (fuse) {
-        const long nlines = g.N / g.dir[ND - 1].len;
-        const dim3 gz((unsigned)((nlines + kBlock - 1) / kBlock),
-                      (unsigned)((g.dir[ND - 1].len + kLineChunk - 1) / kLineChunk), (unsigned)g.ninst);
-        k_fwd_finish_z<<<gz, kBlock, 0, st>>>(g, fz, (long)ND * g.nv * g.N, q, fin.kolmogorov, rhs,
-                                              rk ? rk->stage : 0, rk ? rk->dt : 0.0,
-                                              rk ? rk->y : nullptr, rk ? rk->b1 : nullptr,
-                                              rk ? rk->b2 : nullptr, rk ? rk->copy : nullptr);
-        finished = true;
-      } else if (!launch_deriv_line(g, ND - 1, SLOT_FIRST, fz, (long)ND * g.nv * g.N, rhs,
-                                    (long)g.nv * g.N, g.nv, 2, st)) {
+      if (!launch_deriv_line(g, ND - 1, SLOT_FIRST, fz, (long)ND * g.nv * g.N, rhs,
+                             (long)g.nv * g.N, g.nv, 2, st))
         k_div<ND><<<grid, kBlock, 0, st>>>(g, ND - 1, F, rhs);
-      }
     } else if (F) {
       k_flux_all<ND><<<grid, kBlock, 0, st>>>(g, q, g.viscous ? G : nullptr, F);
       for (int d = 0; d < ND; ++d) {
@@ -2568,12 +2408,11 @@ int launch_rhs_forward(const Geo& g, const Patches* P, const double* q, double* 
     }
     if (g.viscous && has_farfield)
       k_ff_visc_terms<ND><<<grid, kBlock, 0, st>>>(g, MGD_FORWARD, P, q, nullptr, G);
-    if (!finished)
-      k_finish<ND><<<grid, kBlock, 0, st>>>(g, MGD_FORWARD, P, q, nullptr, G, rhs, control,
-                                            control_stride, nullptr, 0, 0.0, src, nsrc, src_amp,
-                                            src_inst_stride, nullptr);
+    k_finish<ND><<<grid, kBlock, 0, st>>>(g, MGD_FORWARD, P, q, nullptr, G, rhs, control,
+                                          control_stride, nullptr, 0, 0.0, src, nsrc, src_amp,
+                                          src_inst_stride, nullptr);
   });
-  return finished && rk != nullptr ? RK_IN_PLACE : RK_NOT_APPLIED;
+  return RK_NOT_APPLIED;
 }
 
 bool launch_rhs_adjoint(const Geo& g, const Patches* P, const double* q, const double* lam,
@@ -2589,19 +2428,23 @@ bool launch_rhs_adjoint(const Geo& g, const Patches* P, const double* q, const d
     (void)grid;
     if (!(rk && rk->stress_ready)) launch_stress3d(g, q, G, st);
     const dim3 gm = march_grid(g, true);
-    with_march(g, true, [&](auto X, auto Z) {
-      constexpr int BX = decltype(X)::value, ZC = decltype(Z)::value;
-      if (g.power_law != 0.0)
-        k_adj3d_jac_march<BX, kFMY, ZC, true><<<gm, BX * kFMY, 0, st>>>(g, q, lam, G, rhs, T1);
-      else
-        k_adj3d_jac_march<BX, kFMY, ZC, false><<<gm, BX * kFMY, 0, st>>>(g, q, lam, G, rhs, T1);
-      k_adj3d_finish_march<BX, kFMY, ZC><<<gm, BX * kFMY, 0, st>>>(
-          g, T1, q, lam, fin.kolmogorov, rhs, rk ? rk->stage : 0, rk ? rk->dt : 0.0,
-          rk ? rk->y : nullptr, rk ? rk->b1 : nullptr, rk ? rk->b2 : nullptr);
+    const int zc = zchunk_of(g, true);
+    with_march(g, true, [&](auto X) {
+      constexpr int BX = decltype(X)::value, BY = kMarchRows;
+      with_stage(g, rk ? rk->stage : 0, [&](auto ST, auto NT) {
+        constexpr int STAGE = decltype(ST)::value;
+        constexpr bool STREAM = decltype(NT)::value;
+        if (g.power_law != 0.0)
+          k_adj3d_jac_march<BX, BY, true, STREAM><<<gm, BX * BY, 0, st>>>(g, zc, q, lam, G, rhs, T1);
+        else
+          k_adj3d_jac_march<BX, BY, false, STREAM><<<gm, BX * BY, 0, st>>>(g, zc, q, lam, G, rhs, T1);
+        k_adj3d_finish_march<BX, BY, STAGE, STREAM><<<gm, BX * BY, 0, st>>>(
+            g, zc, T1, q, lam, fin.kolmogorov, rhs, rk ? rk->dt : 0.0, rk ? rk->y : nullptr,
+            rk ? rk->b1 : nullptr, rk ? rk->b2 : nullptr);
+      });
     });
     return rk != nullptr;
   }
-  bool finished = false;
   MGD_DISPATCH(g.nd, {
     constexpr int NV = ND + 2;
     if (g.viscous) launch_gradients<ND>(g, q, w, G, grid, st);
@@ -2614,25 +2457,7 @@ bool launch_rhs_adjoint(const Geo& g, const Patches* P, const double* q, const d
       k_adj_jac_visc2<ND><<<grid, kBlock, 0, st>>>(g, q, G, T1, rhs);
     else
       k_adj_jac<ND><<<grid, kBlock, 0, st>>>(g, q, G, T1, rhs);
-    // the z pass of the second derivative pass also finishes the rhs where nothing but a
-    // whole-domain Kolmogorov forcing follows (the x and y passes accumulate in S slot 0)
-    const bool fuse = ND == 3 && g.viscous && chain_in_finish && fin.simple &&
-                      deriv_line_applies(g, 0) && deriv_line_applies(g, 1) &&
-                      deriv_line_applies(g, 2);
-    if (fuse) {
-      const long ts = (long)ND * NV * g.N;
-      launch_deriv_line(g, 0, SLOT_ADJ, T1 + (long)1 * g.N, ts, S + (long)1 * g.N, ts, NV - 1, 0, st);
-      launch_deriv_line(g, 1, SLOT_ADJ, T1 + (long)(NV + 1) * g.N, ts, S + (long)1 * g.N, ts, NV - 1,
-                        1, st);
-      const long nlines = g.N / g.dir[ND - 1].len;
-      const dim3 gz((unsigned)((nlines + kBlock - 1) / kBlock),
-                    (unsigned)((g.dir[ND - 1].len + kLineChunk - 1) / kLineChunk), (unsigned)g.ninst);
-      k_adj_finish_z<<<gz, kBlock, 0, st>>>(g, T1 + (long)((ND - 1) * NV + 1) * g.N, S + (long)1 * g.N,
-                                            ts, q, lam, fin.kolmogorov, rhs, rk ? rk->stage : 0,
-                                            rk ? rk->dt : 0.0, rk ? rk->y : nullptr,
-                                            rk ? rk->b1 : nullptr, rk ? rk->b2 : nullptr);
-      finished = true;
-    } else if (g.viscous) {
+    if (g.viscous) {
       for (int d = 0; d < ND; ++d)
         if (!launch_deriv_line(g, d, SLOT_ADJ, T1 + (long)(d * NV + 1) * g.N, (long)ND * NV * g.N,
                                S + (long)(d * NV + 1) * g.N, (long)ND * NV * g.N, NV - 1, 0, st))
@@ -2658,12 +2483,11 @@ bool launch_rhs_adjoint(const Geo& g, const Patches* P, const double* q, const d
     }
     if (g.viscous && has_farfield)
       k_ff_visc_terms<ND><<<grid, kBlock, 0, st>>>(g, MGD_ADJOINT, P, q, lam, G);
-    if (!finished)
-      k_finish<ND><<<grid, kBlock, 0, st>>>(g, MGD_ADJOINT, P, q, lam, G, rhs, nullptr, 0, aforce,
-                                            aforce_stride, forcing_factor, nullptr, 0, nullptr, 0,
-                                            chain_in_finish ? S : nullptr);
+    k_finish<ND><<<grid, kBlock, 0, st>>>(g, MGD_ADJOINT, P, q, lam, G, rhs, nullptr, 0, aforce,
+                                          aforce_stride, forcing_factor, nullptr, 0, nullptr, 0,
+                                          chain_in_finish ? S : nullptr);
   });
-  return finished && rk != nullptr;
+  return false;
 }
 
 void launch_rk_forward(long M, int stage, double dt, double* q, double* b1, double* b2,

@@ -65,7 +65,7 @@ struct Geo {
   double gamma, re_inv, pr_inv, power_law, bulk_ratio, diss_amount;
   int viscous, dissipation, composite;
   int zchunk;               // z planes per work unit of the forward 3-D march and the
-                            // stress pass (32, 64 or 128)
+                            // stress pass
   int mtile;                // x extent of the forward march tiles (16 or 32; 16 rows)
   int zchunk_adj, mtile_adj;  // the same for the adjoint marches
 };

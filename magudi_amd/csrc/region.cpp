@@ -867,11 +867,12 @@ int tune_tiling(mgd_region* r) {
   return install_tiling(r, best);
 }
 
-// The shape of the 3-D marches' work units -- the z chunk (32, 64 or 128 planes) and the
-// tile width (16 or 32 points, 16 rows) -- unless fixed by option: one forward RK4 step
+// The shape of the 3-D marches' work units -- the z chunk (8 to 128 planes) and the tile
+// width (16 or 32 points, 16 rows) -- unless fixed by option: one forward RK4 step
 // (stress pass and march per stage, out of place) and one adjoint rhs (stress pass and
-// the two marches, where they serve the region) timed with HIP events for each shape,
-// three interleaved rounds, the fastest round of each compared; the forward march (with
+// the two marches, where they serve the region) timed with HIP events for each shape, in
+// two interleaved rounds (the second among the shapes within a tenth of the fastest), the
+// fastest round of each compared; the forward march (with
 // the stress pass) and the adjoint marches each keep their own.  No value depends on the
 // shape.
 int tune_march(mgd_region* r) {
@@ -901,9 +902,15 @@ int tune_march(mgd_region* r) {
   std::vector<std::pair<int, int>> shapes;   // (tile width, z chunk)
   for (int mt : {16, 32}) {
     if (r->opt_mtile != 0 && mt != r->opt_mtile) continue;
-    if (mt == 32 && r->geo.n[0] % 32 != 0) continue;
-    for (int zc : {32, 64, 128})
-      if (r->opt_zchunk == 0 || zc == r->opt_zchunk) shapes.emplace_back(mt, zc);
+    // a fixed chunk as it is; else every chunk but those that leave most of the GPU idle
+    // (fewer units than half its 256 CUs, unless the next smaller chunk is no better off),
+    // the chunks below 32 only where one of 32 does not fill it: their units spend most of
+    // their planes on the z windows' lead-in
+    for (int zc : {8, 16, 32, 64, 128}) {
+      const auto units = [&](int z) { return (long)r->ninst * march_units(r->geo, mt, z); };
+      const bool want = zc < 32 ? units(32) < 512 : zc == 32 || units(zc) >= 128;
+      if (r->opt_zchunk == 0 ? want : zc == r->opt_zchunk) shapes.emplace_back(mt, zc);
+    }
   }
   if (shapes.empty()) shapes.emplace_back(16, 64);
   // the forward step and the adjoint rhs are timed apart and each keeps its own shape
@@ -911,11 +918,18 @@ int tune_march(mgd_region* r) {
   MGD_HIP(hipEventCreate(&evm));
   std::vector<float> best_f(shapes.size(), 0.f), best_a(shapes.size(), 0.f);
   int rc = MGD_OK;
-  for (int round = 0; round < 3 && rc == MGD_OK; ++round)
+  for (int round = 0; round < 2 && rc == MGD_OK; ++round) {
+    float lead_f = 0.f, lead_a = 0.f;
     for (size_t k = 0; k < shapes.size(); ++k) {
+      lead_f = k == 0 ? best_f[k] : std::min(lead_f, best_f[k]);
+      lead_a = k == 0 ? best_a[k] : std::min(lead_a, best_a[k]);
+    }
+    for (size_t k = 0; k < shapes.size(); ++k) {
+      // the second round is among the shapes that came near the first one's fastest
+      if (round > 0 && best_f[k] > 1.1f * lead_f && best_a[k] > 1.1f * lead_a) continue;
       r->geo.mtile = r->geo.mtile_adj = shapes[k].first;
       r->geo.zchunk = r->geo.zchunk_adj = shapes[k].second;
-      round_trip();   // warm-up
+      if (round == 0) round_trip();   // warm-up
       float ms_f = 0.f, ms_a = 0.f;
       if (hipEventRecord(r->ev0, r->stream) != hipSuccess) { rc = MGD_ERR_HIP; break; }
       round_trip(evm);
@@ -929,6 +943,7 @@ int tune_march(mgd_region* r) {
       if (round == 0 || ms_f < best_f[k]) best_f[k] = ms_f;
       if (round == 0 || ms_a < best_a[k]) best_a[k] = ms_a;
     }
+  }
   (void)hipEventDestroy(evm);
   if (rc != MGD_OK) { set_error("HIP error in the march autotuner"); return rc; }
   size_t kf = 0, ka = 0;
@@ -2442,9 +2457,9 @@ int mgd_region_set_time_offsets(mgd_region* r, const double* offsets) {
 int mgd_region_get_march_shape(mgd_region* r, int* shape) {
   if (!r || !shape) { set_error("null argument"); return MGD_ERR_ARG; }
   shape[0] = r->geo.mtile;
-  shape[1] = r->geo.zchunk;
+  shape[1] = std::max(r->geo.zchunk, 32);   // reported as 32 below it
   shape[2] = r->geo.mtile_adj;
-  shape[3] = r->geo.zchunk_adj;
+  shape[3] = std::max(r->geo.zchunk_adj, 32);
   return MGD_OK;
 }
 
