@@ -7,8 +7,7 @@
 namespace mgd {
 
 // Tile shapes of the fused kernels (points along x, y): 0: 32 x 16, 1: 16 x 32,
-// 2: 16 x 16, 3: 24 x 16, one thread per point; 4: 16 x 16 and 5: 16 x 12 with two
-// threads per point (each forming two of the four components).
+// 2: 16 x 16, 3: 24 x 16, 4: 16 x 24, 5: 16 x 12; one thread per point.
 constexpr int kNumTileShapes = 6;
 constexpr int kNumXcd = 8;   // XCDs of an MI355X; work-groups are dealt to them round-robin
 

@@ -27,44 +27,55 @@ constexpr int HX = 4, HY = 4;     // halo of the staged operand
 constexpr int NV2 = 4;
 constexpr int kMinEdgeTile = 12;    // closure depth of the adjoint 4-8 operator
 constexpr int kRedThreads = 256;    // block size of the reduction kernels
+constexpr int kFarPoints = 32;      // far-field points of one patch that a tile forms ahead
 
-// Tile shape: TX x TY points and CS threads per point.  Every thread stages operand
-// points; in the stencil and point-wise phases each of the CS threads of a point forms
-// NC = 4 / CS of its components (thread group h = threadIdx / NP owns components
-// h NC .. h NC + NC - 1; a group is a whole number of waves), so CS = 2 gives a tile
-// twice the waves, each with half the stencil work.  LDS (doubles): operand [4][EY][EX];
-// scratch for the fluxes, reused for the dissipation intermediates.
-template <int TX_, int TY_, int CS_ = 1>
+// Tile shape: TX x TY points, one thread per point.  A thread beyond a partial tile loads and
+// stages clamped points and stores nothing.  LDS (doubles): the staged operand q[4][EY][EX];
+// forward, the contravariant fluxes of the tile rows (x) and columns (y); the boundary closure
+// rows of an edge tile; the far-field terms.
+template <int TX_, int TY_>
 struct Shape {
-  static constexpr int TX = TX_, TY = TY_, CS = CS_;
-  static constexpr int NP = TX * TY, NT = NP * CS, NC = NV2 / CS;
-  static_assert(NP % 64 == 0 && NV2 % CS == 0, "component groups are whole waves");
+  static constexpr int TX = TX_, TY = TY_, NT = TX * TY;
+  static_assert(NT % 64 == 0, "whole waves");
   static constexpr int EX = TX + 2 * HX, EY = TY + 2 * HY;
-  // staged points: the tile rows over the extended width, plus the halo rows over the tile
-  // columns (the halo corners are never read)
-  static constexpr int kStaged = TY * EX + 2 * HY * TX;
-  static constexpr int kStageIters = (kStaged + NT - 1) / NT;   // staged points per thread
-  static constexpr int SQ = NV2 * EY * EX;
-  static constexpr int SFX = NV2 * TY * EX, SFY = NV2 * EY * TX;
-  static constexpr int STX = NV2 * TY * (TX + 4), STY = NV2 * (TY + 4) * TX;
-  static constexpr int SSCR = (SFX + SFY) > (STX + STY) ? (SFX + SFY) : (STX + STY);
-  static_assert(CS == 1 || SSCR >= 2 * NV2 * NP, "the scratch space holds the adjoint exchange");
-  // waves per SIMD that the LDS use allows (160 KiB per CU); the register budget is
-  // sized to it
-  static constexpr int kLdsBytes = 8 * (SQ + SSCR + 3 * (TX + TY));
-  static constexpr int kBlocksPerCu = (160 * 1024) / kLdsBytes;
-  static constexpr int kWaves = kBlocksPerCu * NT / 64 / 4;
-  static constexpr int kWavesPerEU = kWaves < 1 ? 1 : kWaves > 8 ? 8 : kWaves;
-  // forward stage: form the dissipation intermediates in registers alongside the flux
-  // derivatives (where the register budget has room for them)
-  static constexpr bool kDissRegs = kWavesPerEU <= 3 || CS > 1;
-  // the tile splits into 8 x 8 blocks of points, one wave each (see point_of_lane)
+  // halo points (the corners are never read): x-halo columns, then y-halo rows
+  static constexpr int kHalo = 2 * HX * TY + 2 * HY * TX;
+  static constexpr int kHaloIters = (kHalo + NT - 1) / NT;
+  static constexpr int SQ = NV2 * EY * EX, SFX = NV2 * TY * EX, SFY = NV2 * EY * TX;
+  static constexpr int kFar = 2 * 4 * kFarPoints;
+  // closure rows of both ends: first derivative 8 x 12 and composite 8 x 12 (or dissipation
+  // transpose 5 x 7); adjoint derivative 12 x 16 and dissipation 8 x 12
+  static constexpr int kTabF = 2 * 96 + 2 * 96, kTabA = 2 * 192 + 2 * 96;
+  static constexpr int kFwdLds = SQ + SFX + SFY + kTabF + kFar;
+  static constexpr int kAdjLds = SQ + kTabA + kFar;
+  static constexpr int kDualLds = kFwdLds > kAdjLds ? kFwdLds : kAdjLds;
+  // waves per SIMD that the LDS use allows (160 KiB per CU), the register budget: at most 4
+  static constexpr int waves(int lds) {
+    const int w = (160 * 1024) / (8 * lds) * NT / 64 / 4;
+    return w < 1 ? 1 : w > 4 ? 4 : w;
+  }
+  // the tile splits into blocks of 8 x 8 points, one wave each (thread_point)
   static constexpr bool kQuads = TX % 8 == 0 && TY % 8 == 0;
 };
 
+// A pointer that comes out of a descriptor in memory (group kernels) is generic to the
+// compiler: flat accesses, which count as LDS and as global ones at once.  This says that it
+// points to global memory.
+template <class T>
+using global_ptr = __attribute__((address_space(1))) T*;
+template <class T>
+__device__ __forceinline__ global_ptr<T> glob(T* p) {
+  return (global_ptr<T>)p;
+}
+
+// The patch tables: no kernel writes them, so they are read through scalar loads, also behind
+// a barrier or a store.
+using ConstPatches = const __attribute__((address_space(4))) Patches;
+using ConstPatch = const __attribute__((address_space(4))) DPatch;
+
 struct TileGeo {
   int x0, y0, sx, sy;   // origin and size of the tile
-  int ex0, ey0;         // global index of LDS column / row 0 (origin - halo)
+  bool bx, by;          // at a non-periodic x / y boundary (closure rows in the tile)
 };
 
 // Tile of this launch block (XCD band map), or -1; its geometry from the balanced
@@ -74,103 +85,37 @@ __device__ __forceinline__ int block_tile(const Tiling& T, int b) {
   return tile < T.nbx * T.nby ? tile : -1;
 }
 
-// Point (tx, ty) of a thread of the forward stage (lane = index within its component
-// group).  Row-major in general: a wave covers 64 / TX whole rows.  In a tile on a
-// non-periodic x boundary the boundary-closure columns (the first / last 8 points) would
-// split every such wave into closure and interior lanes, and a wave runs both paths;
-// there each wave covers an 8 x 8 block of points instead, so the closure columns of the
-// first-derivative operator fill whole waves.  Which thread forms a point changes no
-// value.
-template <class S>
-__device__ __forceinline__ void point_of_lane(const Geo& g, const Tiling& T, int tile, int lane,
-                                              int* tx, int* ty) {
-  const int bx = tile % T.nbx;
-  if (S::kQuads && !g.dir[0].periodic && (bx == 0 || bx == T.nbx - 1)) {
-    const int l = lane & 63, w = lane >> 6;
-    constexpr int QX = S::TX / 8;
-    *tx = (l & 7) + 8 * (w % QX);
-    *ty = (l >> 3) + 8 * (w / QX);
-  } else {
-    *tx = lane % S::TX;
-    *ty = lane / S::TX;
-  }
-}
-
-__device__ __forceinline__ TileGeo tile_geo(const Tiling& T, int tile) {
+__device__ __forceinline__ TileGeo tile_geo(const Geo& g, const Tiling& T, int tile) {
   const int bx = tile % T.nbx, by = tile / T.nbx;
   TileGeo t;
   t.x0 = bx * T.qx + min(bx, T.lx) + max(0, bx - (T.nbx - T.rx));
   t.sx = T.qx + (bx < T.lx || bx >= T.nbx - T.rx ? 1 : 0);
   t.y0 = by * T.qy + min(by, T.ly) + max(0, by - (T.nby - T.ry));
   t.sy = T.qy + (by < T.ly || by >= T.nby - T.ry ? 1 : 0);
-  t.ex0 = t.x0 - HX;
-  t.ey0 = t.y0 - HY;
+  t.bx = !g.dir[0].periodic && (bx == 0 || bx == T.nbx - 1);
+  t.by = !g.dir[1].periodic && (by == 0 || by == T.nby - 1);
   return t;
 }
 
-// Interior stencil coefficients of the operators a stage kernel applies, read once at
-// kernel entry: d1[k] = c_k of the first-derivative-type operator (k = 1..4), dd / dt:
-// c_0..c_2 of the dissipation operator and of its transpose.
-struct Coefs {
-  double d1[5], dd[3], dt[3];
-};
-
-__device__ __forceinline__ Coefs load_coefs(const Geo& g, int first_slot) {
-  Coefs c;
-  const Op& o1 = g.ops[first_slot];
-  const Op& od = g.ops[SLOT_DISS];
-  const Op& ot = g.ops[SLOT_DISS_T];
-  c.d1[0] = 0.0;
-#pragma unroll
-  for (int k = 1; k <= 4; ++k) c.d1[k] = o1.c[kMaxHW + k];
-#pragma unroll
-  for (int k = 0; k < 3; ++k) {
-    c.dd[k] = od.c[kMaxHW + k];
-    c.dt[k] = ot.c[kMaxHW + k];
-  }
-  return c;
-}
-
-// The 1-D grid values of a tile's columns (x) and rows (y) -- h, the norm weight and the
-// coordinate -- held in LDS for the whole block: one thread loads each value at kernel
-// entry, so the later phases read them from LDS instead of each lane fetching its own
-// copy from memory.  Layout: [h | norm weight | coordinate], each TX column values
-// then TY row values.
+// Tile column tx and row ty of this thread.  Row-major in general; in a tile on a non-periodic
+// x boundary each wave covers 8 x 8 points, so that the 8 closure columns of the first
+// derivative fill whole waves (a wave with both kinds of columns runs both paths): the last
+// block of columns ends with the tile (its closure columns on the right boundary), the others
+// start from its left.  False: the thread has no point of its own.
 template <class S>
-struct TileGrid {
-  static constexpr int kRow = S::TX + S::TY;
-  static constexpr int kSize = 3 * kRow;
-  static_assert(kSize <= S::NT, "one grid value per thread");
-  const double* s;
-  __device__ double h0(int tx) const { return s[tx]; }
-  __device__ double h1(int ty) const { return s[S::TX + ty]; }
-  __device__ double hw0(int tx) const { return s[kRow + tx]; }
-  __device__ double hw1(int ty) const { return s[kRow + S::TX + ty]; }
-  __device__ double x0(int tx) const { return s[2 * kRow + tx]; }
-  __device__ double x1(int ty) const { return s[2 * kRow + S::TX + ty]; }
-};
-
-// This thread's grid value (threads below TileGrid::kSize), to be stored at its index.
-template <class S>
-__device__ __forceinline__ double load_tile_grid(const Geo& g, const TileGeo& t) {
-  constexpr int kRow = TileGrid<S>::kRow;
+__device__ __forceinline__ bool thread_point(const TileGeo& t, int* tx, int* ty) {
   const int e = threadIdx.x;
-  if (e >= TileGrid<S>::kSize) return 0.0;
-  const int what = e / kRow, i = e % kRow;
-  const int d = i < S::TX ? 0 : 1;
-  const int k = d == 0 ? i : i - S::TX;
-  if (k >= (d == 0 ? t.sx : t.sy)) return 0.0;
-  const int idx = (d == 0 ? t.x0 : t.y0) + k;
-  // constant indices into the kernel-argument arrays (a run-time index would copy the
-  // argument block to scratch memory)
-  const double* src = what == 0 ? (d == 0 ? g.h[0] : g.h[1])
-                    : what == 1 ? (d == 0 ? g.hw[0] : g.hw[1])
-                                : (d == 0 ? g.x[0] : g.x[1]);
-  return src[idx];
-}
-
-__device__ __forceinline__ bool closure(const Dir& dd, int i, int w) {
-  return !dd.periodic && (i < w || i >= dd.len - w);
+  if (S::kQuads && t.bx) {
+    const int l = e & 63, w = e >> 6;
+    constexpr int QX = S::TX / 8;
+    const int cb = w % QX, c = l & 7;
+    *ty = (l >> 3) + 8 * (w / QX);
+    *tx = cb == QX - 1 ? t.sx - 8 + c : 8 * cb + c;
+    return *ty < t.sy && (cb == QX - 1 || *tx < t.sx - 8);
+  }
+  *tx = e % S::TX;
+  *ty = e / S::TX;
+  return *tx < t.sx && *ty < t.sy;
 }
 
 // global index of an extended (halo) index, or -1 outside a non-periodic domain
@@ -180,350 +125,809 @@ __device__ __forceinline__ int ext_index(const Dir& dd, int gi) {
   return gi < 0 ? gi + dd.len - dd.off : gi - dd.len + dd.off;
 }
 
-// Staged operand of this tile (all four components) in registers: stage_load issues
-// every load of this thread before any is consumed; stage_store writes them to sq and,
-// for the forward stage, the contravariant fluxes of the tile rows (x) and tile columns
-// (y) to sfx / sfy.
-template <class S>
-struct StageRegs {
-  double v[S::kStageIters][NV2];
+// One halo point of this thread: its place (ex, ey) in the staged tile, grid indices and
+// which halo it is (1 x, 2 y, 0 none: then (gi, gj) is a point of the tile).
+struct HaloSlot {
+  int ex, ey, gi, gj, kind;
 };
-
-// Staging slot `it` of this thread: extended-layout indices (ex, ey), the grid point
-// (gi, gj) and whether the slot holds a staged point.  Slots enumerate the tile rows
-// over the extended width first, then the halo rows over the tile columns (the halo
-// rows below a partial tile follow its last row); slots beyond a partial tile, and
-// halo points outside a non-periodic domain, hold none.
 template <class S>
-__device__ __forceinline__ bool stage_slot(const Geo& g, const TileGeo& t, int it, int* ex,
-                                           int* ey, int* gi, int* gj) {
-  constexpr int TX = S::TX, TY = S::TY, EX = S::EX;
+__device__ __forceinline__ HaloSlot halo_slot(const Geo& g, const TileGeo& t, int it) {
   const int e = threadIdx.x + it * S::NT;
+  HaloSlot h;
   bool in;
-  if (e < TY * EX) {
-    const int r = e / EX;
-    *ex = e % EX;
-    *ey = HY + r;
-    in = r < t.sy && *ex < t.sx + 2 * HX;
+  if (e < 2 * HX * S::TY) {
+    const int c = e % 8, r = e / 8;
+    h.ex = c < 4 ? c : t.sx + c;
+    h.ey = HY + r;
+    in = r < t.sy;
+    h.kind = 1;
   } else {
-    const int e2 = e - TY * EX;
-    const int hr = e2 / TX, c = e2 % TX;
-    *ex = HX + c;
-    *ey = hr < HY ? hr : HY + t.sy + (hr - HY);
-    in = e2 < 2 * HY * TX && c < t.sx;
+    const int e2 = e - 2 * HX * S::TY, r = e2 / S::TX, c = e2 % S::TX;
+    h.ex = HX + c;
+    h.ey = r < 4 ? r : t.sy + r;
+    in = r < 8 && c < t.sx;
+    h.kind = 2;
   }
-  *gi = ext_index(g.dir[0], t.ex0 + *ex);
-  *gj = ext_index(g.dir[1], t.ey0 + *ey);
-  return in && *gi >= 0 && *gj >= 0;
+  h.gi = ext_index(g.dir[0], t.x0 - HX + h.ex);
+  h.gj = ext_index(g.dir[1], t.y0 - HY + h.ey);
+  if (!in || h.gi < 0 || h.gj < 0) {
+    h.kind = 0;
+    h.gi = t.x0;
+    h.gj = t.y0;
+  }
+  return h;
 }
 
-template <class S>
-__device__ __forceinline__ void stage_load(const Geo& g, const TileGeo& t, const double* xi,
-                                           StageRegs<S>& r) {
-#pragma unroll
-  for (int it = 0; it < S::kStageIters; ++it) {
-    int ex, ey, gi, gj;
-    if (stage_slot<S>(g, t, it, &ex, &ey, &gi, &gj)) {
-      const long pp = gi + (long)g.n[0] * gj;
-#pragma unroll
-      for (int l = 0; l < NV2; ++l) r.v[it][l] = xi[l * g.N + pp];
-    }
-  }
-}
-
-template <class S, bool FLUX>
-__device__ __forceinline__ void stage_store(const Geo& g, const TileGeo& t, const StageRegs<S>& r,
-                                            const TileGrid<S>& tg, double* sq, double* sfx,
-                                            double* sfy) {
-  constexpr int TX = S::TX, TY = S::TY, EX = S::EX, EY = S::EY;
-#pragma unroll
-  for (int it = 0; it < S::kStageIters; ++it) {
-    int ex, ey, gi, gj;
-    if (!stage_slot<S>(g, t, it, &ex, &ey, &gi, &gj)) continue;
-#pragma unroll
-    for (int l = 0; l < NV2; ++l) sq[(l * EY + ey) * EX + ex] = r.v[it][l];
-    if (FLUX) {
-      const Prim<2> s = prim<2>(r.v[it], g.gamma);
-      if (ey >= HY && ey < HY + t.sy) {
-        double f[NV2];
-        inviscid_flux<2>(r.v[it], s, 0, f);
-        const double m = tg.h1(ey - HY);   // metric<2>(g, 0, .) of the row
-#pragma unroll
-        for (int l = 0; l < NV2; ++l) sfx[(l * TY + (ey - HY)) * EX + ex] = m * f[l];
-      }
-      if (ex >= HX && ex < HX + t.sx) {
-        double f[NV2];
-        inviscid_flux<2>(r.v[it], s, 1, f);
-        const double m = tg.h0(ex - HX);   // metric<2>(g, 1, .) of the column
-#pragma unroll
-        for (int l = 0; l < NV2; ++l) sfy[(l * EY + ey) * TX + (ex - HX)] = m * f[l];
-      }
-    }
+// The dense closure rows (BD x BW) of operator `slot` into LDS, one value per thread and
+// turn: the left end's, then the right end's (row m: the m-th point from that end).
+template <class S, int BD, int BW>
+__device__ __forceinline__ void stage_rows(const Geo& g, int slot, double* tab) {
+  const Op& op = g.ops[slot];
+  for (int e = threadIdx.x; e < 2 * BD * BW; e += S::NT) {
+    const int m = e / BW % BD, c = e % BW;
+    tab[e] = e < BD * BW ? op.b1[m][c] : op.b2[m][c];
   }
 }
 
-// Boundary-closure row of an operator with compile-time block size BW x BD (SBP 4-8:
-// first derivative 12 x 8, adjoint 16 x 12, dissipation transpose 7 x 5, composite
-// 12 x 8) for NC components.  Unrolled so the coefficient loads issue together.  f(c, v)
-// writes the NC operand values at closure column c (0-based from the boundary,
-// mirrored on the right).
-template <int BW, int BD, int NC, class F>
-__device__ __forceinline__ void closure_row(const Op& op, int i, int len, F&& f, double* out) {
-  const bool left = i < BD;
-  const int m = left ? i : len - 1 - i;
-  const double* b = left ? op.b1[m] : op.b2[m];
-  const int base = left ? 0 : len - BW;
+// A closure row on the BW operands f(j, k) of the components j, in the order of the grid
+// index; four columns of LDS reads at a time (more would spill registers).
+template <int BW, class F>
+__device__ __forceinline__ void closure_row(const double* row, F&& f, double* out) {
 #pragma unroll
-  for (int j = 0; j < NC; ++j) out[j] = 0.0;
+  for (int j = 0; j < NV2; ++j) out[j] = 0.0;
 #pragma unroll
-  for (int c = 0; c < BW; ++c) {
-    double v[NC];
-    f(base + c, v);
-    const double bc = b[c];
+  for (int k = 0; k < BW; ++k) {
+    const double b = row[k];
 #pragma unroll
-    for (int j = 0; j < NC; ++j) out[j] += bc * v[j];
+    for (int j = 0; j < NV2; ++j) out[j] += b * f(j, k);
+    if (k % 4 == 3) __builtin_amdgcn_sched_barrier(0);
   }
 }
 
-// First-derivative-type operator (BW x BD closure) along x or y at a point of the tile
-// for components c0 .. c0 + NC - 1, operand in LDS; row(l, e) returns component l at
-// extended index e.
-template <int BW, int BD, int NC, class Row>
-__device__ __forceinline__ void deriv_lds(const Op& op, const double* ck, const Dir& dd, int i,
-                                          int e0, int c0, Row&& row, double* out) {
-  if (!dd.periodic && (i < BD || i >= dd.len - BD)) {
-    closure_row<BW, BD, NC>(op, i, dd.len,
-                            [&](int idx, double* v) {
-#pragma unroll
-                              for (int j = 0; j < NC; ++j) v[j] = row(c0 + j, idx - e0);
-                            },
-                            out);
-    return;
-  }
-  const int e = i - e0;
-#pragma unroll
-  for (int j = 0; j < NC; ++j) {
-    double s = 0.0;
-#pragma unroll
-    for (int k = 1; k <= 4; ++k) s += ck[k] * (row(c0 + j, e + k) - row(c0 + j, e - k));
-    out[j] = s;
-  }
-}
-
-// D4 x at index i along a direction, with magudi's boundary rows: on a non-periodic
-// direction rows 0,1 (and the last two) repeat the stencil centred two points inside
-// (src/StencilOperatorImpl.f90:1928-1940), summed in the closure-row order.
-template <class Row>
-__device__ __forceinline__ double d4_at(const Dir& dd, int i, double c0, double c1, double c2,
-                                        Row&& x) {
-  if (!dd.periodic && (i < 2 || i >= dd.len - 2)) {
-    const int ctr = i < 2 ? 2 : dd.len - 3;
-    double s = 0.0;
-    s += c2 * x(ctr - 2);
-    s += c1 * x(ctr - 1);
-    s += c0 * x(ctr);
-    s += c1 * x(ctr + 1);
-    s += c2 * x(ctr + 2);
-    return s;
-  }
-  double s = 0.0;
-  s += c1 * (x(i + 1) + x(i - 1));
-  s += c2 * (x(i + 2) + x(i - 2));
-  return s + c0 * x(i);
-}
-
-// Slots of diss_intermediates_to per thread, and the intermediates of one thread held in
-// registers (so that they can be formed before the flux space they are stored over is
-// free).  With one thread per point the x positions (plane PX) and then the y positions
-// (plane PY) are dealt to the threads together, slot it of lane holding position
-// lane + it NP: every thread forms at most NS of them (3 for 16 x 16 tiles, where
-// dealing the planes one after the other gives the first wave 4 and the others 2).  With
-// component groups (CS > 1) the planes are dealt one after the other (slots 0 .. IX - 1
-// for x, IX .. for y), which keeps their register budget.
-template <class S>
-struct DissSlots {
-  static constexpr int PX = S::TY * (S::TX + 4), PY = (S::TY + 4) * S::TX;   // planes
-  static constexpr bool kJoint = S::CS == 1;
-  static constexpr int IX = (PX + S::NP - 1) / S::NP, IY = (PY + S::NP - 1) / S::NP;
-  static constexpr int NS = kJoint ? (PX + PY + S::NP - 1) / S::NP : IX + IY;
-  double v[NS][S::NC];
-  int base[NS];   // LDS index in its plane, or -1
-  bool y[NS];     // position of the y plane
+// Place of index i on a non-periodic direction: m the distance from the nearer end, right
+// which end that is; m is large on a periodic direction.
+struct EdgePlace {
+  int m;
+  bool right;
 };
+__device__ __forceinline__ EdgePlace edge_place(const Dir& dd, int i) {
+  const int r = dd.len - 1 - i;
+  return {dd.periodic ? 1 << 30 : min(i, r), r < i};
+}
 
-// t = -arc D4 x on the tile rows (x direction, columns x0-2 .. x0+sx+1) and tile columns
-// (y direction, rows y0-2 .. y0+sy+1), for staged points inside the domain, components
-// c0 .. c0 + NC - 1; the positions are dealt to the NP threads of the component group
-// (lane = index within the group) as DissSlots describes.  Each value goes to
-// sink_x / sink_y (it, j, base, v): slot `it` of this thread, component c0 + j, LDS
-// index base + (c0 + j) * plane of the x or y plane.
-template <class S, class SinkX, class SinkY>
-__device__ __forceinline__ void diss_intermediates_to(const Geo& g, const TileGeo& t,
-                                                      const Coefs& cf, const TileGrid<S>& tg,
-                                                      const double* sq, int lane, int c0,
-                                                      SinkX&& sink_x, SinkY&& sink_y) {
-  constexpr int TX = S::TX, EX = S::EX, EY = S::EY, NP = S::NP, NC = S::NC;
-  constexpr int PX = DissSlots<S>::PX, PY = DissSlots<S>::PY;
-  const double k0 = cf.dd[0], k1 = cf.dd[1], k2 = cf.dd[2];
-  const Dir dx = g.dir[0], dy = g.dir[1];
-  const int wx = t.sx + 4, hy = t.sy + 4;
-  constexpr bool kJoint = DissSlots<S>::kJoint;
-  constexpr int IX = DissSlots<S>::IX;
+__device__ __forceinline__ double skew_sum(const double* p, const double* m, const double* c) {
+  double s = c[1] * (p[0] - m[0]);
 #pragma unroll
-  for (int it = 0; it < DissSlots<S>::NS; ++it) {
-    // joint: position lane + it NP of the concatenated planes; else x slots, then y
-    const int e = kJoint ? lane + it * NP : it < IX ? lane + it * NP : PX + lane + (it - IX) * NP;
-    if (e >= PX + PY || (!kJoint && it < IX && e >= PX)) continue;
-    // slot it holds positions it NP .. it NP + NP - 1: only a slot that straddles the
-    // end of the x plane needs both branches (it is a constant once unrolled)
-    if (kJoint ? ((it + 1) * NP <= PX || (it * NP < PX && e < PX)) : it < IX) {
-      const int ex = e % (TX + 4) + 2, ey = e / (TX + 4) + HY;
-      if (ex - 2 >= wx || ey - HY >= t.sy) continue;
-      const int gi = t.ex0 + ex;
-      if (!dx.periodic && (gi < 0 || gi >= dx.len)) continue;
-      const double arc = fabs(tg.h1(ey - HY));
+  for (int k = 2; k <= 4; ++k) s += c[k] * (p[k - 1] - m[k - 1]);
+  return s;
+}
+
+// Interior row of D4 (and of D4^T) on the window w[0..4].  The products with 1 and -4 are
+// exact, so the fused form rounds as the plain sum does.
+__device__ __forceinline__ double d4_row(const double* w) {
+  return __fma_rn(kD4[1], w[3] + w[1], w[4] + w[0]) + kD4[0] * w[2];
+}
+
+// Row of the 9-point symmetric operator c_0..c_4 about x, whose coefficients sum to zero:
+// sum_k c_k (x_k - x).
+__device__ __forceinline__ double sym9(double x, const double* p, const double* m, const double* c) {
+  double s = c[1] * ((p[0] - x) + (m[0] - x));
 #pragma unroll
-      for (int j = 0; j < NC; ++j) {
-        const int l = c0 + j;
-        const double* r = sq + (l * EY + ey) * EX;
-        const double v = d4_at(dx, gi, k0, k1, k2, [&](int k) { return r[k - t.ex0]; });
-        sink_x(it, j, (ey - HY) * (TX + 4) + (ex - 2), -arc * v);
+  for (int k = 2; k <= 4; ++k) s = __fma_rn(c[k], (p[k - 1] - x) + (m[k - 1] - x), s);
+  return s;
+}
+
+// D4^T (-arc D4 x) of the two-level dissipation at one point from the nine operands about it
+// (the metric is constant along a line of a rectilinear grid): the five intermediates that
+// the point's row needs are formed again by each thread, 35 operations instead of a pass of
+// the intermediates through LDS with two more barriers.
+__device__ __forceinline__ double two_level(const double* w, double marc) {
+  double z[5];
+#pragma unroll
+  for (int k = 0; k < 5; ++k) z[k] = marc * d4_row(w + k);
+  return d4_row(z);
+}
+
+// The same in a tile at a non-periodic end: w holds the nine operands of the window that
+// starts at index clamp(i - 4, 0, len - 9).  The first two rows of D4 repeat the stencil of
+// the third one, summed in the order of the index; D4^T has 5 closure rows of 7 columns.
+__device__ __forceinline__ double two_level_edge(const double* w, double marc, EdgePlace e,
+                                                 const double* rows) {
+  if (e.m >= 5) return two_level(w, marc);
+  double z[5], first = 0.0;
+#pragma unroll
+  for (int k = 0; k < 5; ++k) z[k] = marc * d4_row(w + k);
+#pragma unroll
+  for (int k = 0; k < 5; ++k) first += kD4[k < 2 ? 2 - k : k - 2] * (e.right ? w[k + 4] : w[k]);
+  first = marc * first;
+  const double* b = rows + (e.right ? 35 : 0) + 7 * e.m;
+  double s = 0.0;
+#pragma unroll
+  for (int c = 0; c < 7; ++c) {
+    const double l = c < 2 ? first : z[c < 2 ? 0 : c - 2];
+    const double r = c < 5 ? z[c < 5 ? c : 0] : first;
+    s += b[c] * (e.right ? r : l);
+  }
+  return s;
+}
+
+// Scale of the one-level (9-point) dissipation sum of the adjoint stage along a direction:
+// amount H^-1 (-arc) of the two-level operator, amount of the composite one.
+__device__ __forceinline__ double diss_scale(const Geo& g, double amount, double arc, double hw) {
+  if (g.composite) return amount;
+  double s = amount * -arc;
+  if (hw != 1.0) s = s / hw;    // 1 away from the first / last boundary rows
+  return s;
+}
+
+// The Jacobian part of the adjoint rhs for 2-D Euler (computeRhsAdjoint): r = sum_d A_d^T t_d
+// with the flux Jacobians A_d of the Cartesian directions and t_d = metric_d T1[d].  The
+// products are formed through the enthalpy, not through the entries of A_d (most of which
+// are multiples of one another): 46 operations instead of some 170.
+__device__ __forceinline__ void adj_jacobian_rows(const double* mx, const Prim<2>& s, double gamma,
+                                                  const double (*T1)[NV2], double* r) {
+  double t[NV2], w[NV2];
+#pragma unroll
+  for (int c = 0; c < NV2; ++c) {
+    t[c] = mx[0] * T1[0][c];
+    w[c] = mx[1] * T1[1][c];
+  }
+  const double u = s.u[0], v = s.u[1], ke = 0.5 * (u * u + v * v), H = s.T + ke;
+  const double a = u * t[1] + v * t[2], b = u * w[1] + v * w[2];
+  const double e = u * t[3] + v * w[3];
+  const double z = (gamma - 1.0) * ((t[1] + w[2]) + e);
+  r[0] = (ke * z - H * e) - (u * a + v * b);
+  r[1] = ((t[0] + a) + H * t[3]) + ((u * t[1] + v * w[1]) - u * z);
+  r[2] = ((w[0] + b) + H * w[3]) + ((u * t[2] + v * w[2]) - v * z);
+  r[3] = z + e;
+}
+
+__device__ __forceinline__ bool in_patch(ConstPatch& pt, int i, int j) {
+  return i >= pt.lo[0] && i <= pt.hi[0] && j >= pt.lo[1] && j <= pt.hi[1];
+}
+
+// The far-field terms of a tile formed ahead of the stencil work, while its operand loads are
+// in flight: of the first two far-field patches in the tile with at most kFarPoints of its
+// points, thread 4 k + i forms component i of point k -- sum_c A+[c][i] (q_c - qt_c)
+// forward, sum_c A+[i][c] lambda_c adjoint -- into LDS, where the point's thread finds it
+// (a chain of loads per patch at the end of the kernel otherwise, on the slowest tiles).
+struct FarAhead {
+  int ip[2];       // patch, or -1
+  int i0[2], j0[2], w[2];
+};
+template <class S, bool ADJ>
+__device__ __forceinline__ FarAhead far_ahead(const Geo& g, ConstPatches* P,
+                                              const TileGeo& t, unsigned m, global_ptr<const double> x,
+                                              double* ff) {
+  FarAhead f;
+#pragma unroll
+  for (int s = 0; s < 2; ++s) {
+    f.ip[s] = -1;
+    f.i0[s] = f.j0[s] = f.w[s] = 0;
+    if (!m) continue;
+    const int ip = __ffs(m) - 1;
+    m &= m - 1;
+    ConstPatch& pt = P->p[ip];
+    const int i0 = max(pt.lo[0], t.x0), i1 = min(pt.hi[0], t.x0 + t.sx - 1);
+    const int j0 = max(pt.lo[1], t.y0), j1 = min(pt.hi[1], t.y0 + t.sy - 1);
+    const int w = i1 - i0 + 1, n = w * (j1 - j0 + 1);
+    if (n <= 0 || n > kFarPoints) continue;
+    f.ip[s] = ip;
+    f.i0[s] = i0;
+    f.j0[s] = j0;
+    f.w[s] = w;
+    for (int e = threadIdx.x; e < 4 * n; e += S::NT) {
+      const int k = e >> 2, i = e & 3;
+      const int gi = i0 + k % w, gj = j0 + k / w;
+      const long p = gi + (long)g.n[0] * gj;
+      const int kp = (gi - pt.lo[0]) + pt.ls[0] * (gj - pt.lo[1]);
+      const global_ptr<const double> A = glob(pt.aplus) + (long)kp * 16;
+      double v = 0.0;
+      if (ADJ) {
+#pragma unroll
+        for (int c = 0; c < NV2; ++c) v += A[i * 4 + c] * x[c * g.N + p];
+      } else {
+        const global_ptr<const double> qt = glob(pt.aplus) + (long)pt.np * 16 + (long)kp * 4;
+#pragma unroll
+        for (int c = 0; c < NV2; ++c) v += A[c * 4 + i] * (x[c * g.N + p] - qt[c]);
       }
-    } else {
-      const int e2 = e - PX;
-      const int ex = e2 % TX + HX, ey = e2 / TX + 2;
-      if (ex - HX >= t.sx || ey - 2 >= hy) continue;
-      const int gj = t.ey0 + ey;
-      if (!dy.periodic && (gj < 0 || gj >= dy.len)) continue;
-      const double arc = fabs(tg.h0(ex - HX));
-#pragma unroll
-      for (int j = 0; j < NC; ++j) {
-        const int l = c0 + j;
-        const double* c = sq + l * EY * EX + ex;
-        const double v = d4_at(dy, gj, k0, k1, k2, [&](int k) { return c[(k - t.ey0) * EX]; });
-        sink_y(it, j, (ey - 2) * TX + (ex - HX), -arc * v);
-      }
+      ff[s * 4 * kFarPoints + e] = v;
     }
   }
+  return f;
 }
 
-// The intermediates straight into LDS.
-template <class S>
-__device__ __forceinline__ void diss_intermediates(const Geo& g, const TileGeo& t, const Coefs& cf,
-                                                   const TileGrid<S>& tg, const double* sq,
-                                                   double* stx, double* sty, int lane, int c0) {
-  diss_intermediates_to<S>(
-      g, t, cf, tg, sq, lane, c0,
-      [&](int, int j, int base, double v) { stx[(c0 + j) * DissSlots<S>::PX + base] = v; },
-      [&](int, int j, int base, double v) { sty[(c0 + j) * DissSlots<S>::PY + base] = v; });
-}
-
-// The intermediates into registers, then (diss_store) into LDS.
-template <class S>
-__device__ __forceinline__ void diss_compute(const Geo& g, const TileGeo& t, const Coefs& cf,
-                                             const TileGrid<S>& tg, const double* sq, int lane,
-                                             int c0, DissSlots<S>& d) {
+// The terms of patch ip (one of those formed ahead) at grid point (gi, gj).
+__device__ __forceinline__ void far_formed(const FarAhead& f, int ip, const double* ff, int gi,
+                                           int gj, double* out) {
+  const int s = ip == f.ip[0] ? 0 : 1;
+  const double* x = ff + s * 4 * kFarPoints + 4 * ((gi - f.i0[s]) + f.w[s] * (gj - f.j0[s]));
 #pragma unroll
-  for (int it = 0; it < DissSlots<S>::NS; ++it) {
-    d.base[it] = -1;
-    d.y[it] = false;
+  for (int l = 0; l < NV2; ++l) out[l] = x[l];
+}
+
+// -------------------------------------------------------------------------- forward
+// What bounds the stage: on small grids (a few blocks per CU) the chain load - LDS - stencils -
+// store of one block, so there is one barrier, and every operand is asked for before it; on
+// batches the 160 bytes per point and stage (0.09 ms for 20 instances of 401 x 401 at the rate
+// of a copy) beside 0.07 ms of FP64 issue and 0.06 ms of LDS reads, which overlap in part.
+// Plain stores: the rows of a tile end inside cache lines that the neighbour completes, and
+// non-temporal stores sent them to memory in pieces (8 x 273^2: 39.3 against 36.9 us).
+// Against the stage with the dissipation's intermediates in LDS (three barriers, every patch
+// read at the end): 401^2 15.2 -> 13.3 us, 201^2 10.8 -> 10.1, 20 x 401^2 191 -> 173.
+// One forward stage on tile block `blk` of instance `inst` (uniform per work-group).
+template <class S>
+__device__ __forceinline__ void fwd_stage_body(const Geo& g, const Patches* patches,
+                                               const Tiling& T, const FwdStage& a, int blk,
+                                               long inst, double* lds) {
+  constexpr int TX = S::TX, TY = S::TY, EX = S::EX, EY = S::EY, HS = S::kHaloIters;
+  double* sq = lds;
+  double* sfx = sq + S::SQ;
+  double* sfy = sfx + S::SFX;
+  double* tab = sfy + S::SFY;
+  double* ff = tab + S::kTabF;
+  const int tile = block_tile(T, blk);
+  ConstPatches* P = (ConstPatches*)patches;
+  if (tile < 0) return;   // block beyond the tiles of its XCD (uniform per block)
+  const TileGeo t = tile_geo(g, T, tile);
+  const long NVN = (long)NV2 * g.N;
+  const global_ptr<const double> qi = glob(a.qin) + inst * NVN;
+  const unsigned pmask = glob(T.pmask)[tile];
+  int tx, ty;
+  const bool mine = thread_point<S>(t, &tx, &ty);
+  const int gi = t.x0 + (mine ? tx : 0), gj = t.y0 + (mine ? ty : 0);
+  const long p = gi + (long)g.n[0] * gj;
+  // the operand: own point and halo points, then everything else the thread will need, in
+  // the order of use (a wait for a load waits for those issued before it)
+  double v[NV2], hv[HS][NV2], hm[HS];
+#pragma unroll
+  for (int l = 0; l < NV2; ++l) v[l] = qi[l * g.N + p];
+#pragma unroll
+  for (int it = 0; it < HS; ++it) {
+    const HaloSlot h = halo_slot<S>(g, t, it);
+    const long pp = h.gi + (long)g.n[0] * h.gj;
+#pragma unroll
+    for (int l = 0; l < NV2; ++l) hv[it][l] = qi[l * g.N + pp];
+    hm[it] = h.kind == 2 ? glob(g.h[0])[h.gi] : glob(g.h[1])[h.gj];   // metric<2> of the halo's direction
   }
-  diss_intermediates_to<S>(
-      g, t, cf, tg, sq, lane, c0,
-      [&](int it, int j, int base, double v) { d.base[it] = base; d.y[it] = false; d.v[it][j] = v; },
-      [&](int it, int j, int base, double v) { d.base[it] = base; d.y[it] = true; d.v[it][j] = v; });
-}
-
-template <class S>
-__device__ __forceinline__ void diss_store(const DissSlots<S>& d, int c0, double* stx, double* sty) {
+  const double h0 = glob(g.h[0])[gi], hw0 = glob(g.hw[0])[gi], h1 = glob(g.h[1])[gj], hw1 = glob(g.hw[1])[gj];
+  double d1[5];                     // interior coefficients
 #pragma unroll
-  for (int it = 0; it < DissSlots<S>::NS; ++it) {
-    if (d.base[it] < 0) continue;
-    if (d.y[it]) {
-#pragma unroll
-      for (int j = 0; j < S::NC; ++j) sty[(c0 + j) * DissSlots<S>::PY + d.base[it]] = d.v[it][j];
-    } else {
-#pragma unroll
-      for (int j = 0; j < S::NC; ++j) stx[(c0 + j) * DissSlots<S>::PX + d.base[it]] = d.v[it][j];
+  for (int k = 1; k <= 4; ++k) d1[k] = g.ops[SLOT_FIRST].c[kMaxHW + k];
+  const FarAhead far = far_ahead<S, false>(g, P, t, pmask & P->far_mask, qi, ff);
+  if (t.bx || t.by) {
+    stage_rows<S, 8, 12>(g, SLOT_FIRST, tab);
+    if (g.dissipation) {
+      if (g.composite) stage_rows<S, 8, 12>(g, SLOT_DISS, tab + 192);
+      else stage_rows<S, 5, 7>(g, SLOT_DISS_T, tab + 192);
     }
   }
-}
-
-// Dissipation terms at one point for components c0 .. c0 + NC - 1: w[d][j] = amount *
-// (H^-1 D4^T t) along direction d (closure rows of D4^T near non-periodic boundaries),
-// or amount * (composite operator on the staged operand).  The caller adds w[0] then
-// w[1].
-template <class S>
-__device__ __forceinline__ void diss_terms(const Geo& g, const TileGeo& t, const Coefs& cf,
-                                           const TileGrid<S>& tg, const double* sq,
-                                           const double* stx, const double* sty, int tx, int ty,
-                                           int gi, int gj, int c0, double amount,
-                                           double (*w)[S::NC]) {
-  constexpr int TX = S::TX, TY = S::TY, EX = S::EX, EY = S::EY, NC = S::NC;
-  const Op& od = g.ops[SLOT_DISS];
-  const Op& ot = g.ops[SLOT_DISS_T];
+  // stage the operand and the fluxes
+  if (mine) {
+    const Prim<2> s = prim<2>(v, g.gamma);
+    double f0[NV2], f1[NV2];
+    inviscid_flux<2>(v, s, 0, f0);
+    inviscid_flux<2>(v, s, 1, f1);
 #pragma unroll
-  for (int d = 0; d < 2; ++d) {
-    double dv[NC];
-    const Dir& dr = g.dir[d];
-    const int i = d == 0 ? gi : gj;
+    for (int l = 0; l < NV2; ++l) {
+      sq[(l * EY + ty + HY) * EX + tx + HX] = v[l];
+      sfx[(l * TY + ty) * EX + tx + HX] = h1 * f0[l];
+      sfy[(l * EY + ty + HY) * TX + tx] = h0 * f1[l];
+    }
+  }
+#pragma unroll
+  for (int it = 0; it < HS; ++it) {
+    const HaloSlot h = halo_slot<S>(g, t, it);
+    if (h.kind == 0) continue;
+    const Prim<2> s = prim<2>(hv[it], g.gamma);
+    double f[NV2];
+    if (h.kind == 1) {
+      inviscid_flux<2>(hv[it], s, 0, f);
+#pragma unroll
+      for (int l = 0; l < NV2; ++l) sfx[(l * TY + h.ey - HY) * EX + h.ex] = hm[it] * f[l];
+    } else {
+      inviscid_flux<2>(hv[it], s, 1, f);
+#pragma unroll
+      for (int l = 0; l < NV2; ++l) sfy[(l * EY + h.ey) * TX + h.ex - HX] = hm[it] * f[l];
+    }
+#pragma unroll
+    for (int l = 0; l < NV2; ++l) sq[(l * EY + h.ey) * EX + h.ex] = hv[it][l];
+  }
+  // RK operands, sponge, source and cost-target values, fetched while the stencils run
+  const bool sponge = (pmask & P->sponge_mask) != 0;            // uniform per block
+  const bool cost = a.jpartial && a.ip_cost >= 0 && ((pmask >> a.ip_cost) & 1u);
+  double q0[NV2], b2[NV2], qt[NV2], damp = 0.0, sx0 = 0.0, sy0 = 0.0, pb = 0.0, mo = 0.0;
+#pragma unroll
+  for (int l = 0; l < NV2; ++l) {
+    const long o = inst * NVN + l * g.N + p;
+    q0[l] = a.stage == 2 || a.stage == 3 ? glob(a.q0)[o] : 0.0;
+    b2[l] = a.stage >= 2 ? glob(a.b2)[o] : 0.0;
+    qt[l] = 0.0;
+  }
+  if (sponge) {
+    damp = glob(P->damp)[p];
+#pragma unroll
+    for (int l = 0; l < NV2; ++l) qt[l] = glob(P->qtarget)[l * g.N + p];
+  }
+  if (a.nsrc > 0) {
+    sx0 = glob(P->srcx)[gi];
+    sy0 = glob(P->srcy)[gj];
+  }
+  bool jin = false;
+  int kj = 0;
+  if (cost) {
+    ConstPatch& pt = P->p[a.ip_cost];
+    jin = mine && in_patch(pt, gi, gj);
+    kj = jin ? (gi - pt.lo[0]) + pt.ls[0] * (gj - pt.lo[1]) : 0;
+    pb = glob(pt.aplus)[kj];
+    mo = glob(pt.strength)[kj];
+  }
+  __syncthreads();
+  // r = 0 - (D_x F_x + D_y F_y) and the dissipation in x and y
+  double r[NV2];
+  const double ax = -fabs(h1), ay = -fabs(h0);          // -arc length along x, y
+  const double* fx = sfx + ty * EX + tx + HX;           // the point in the staged arrays
+  const double* fy = sfy + (ty + HY) * TX + tx;
+  const double* qc = sq + (ty + HY) * EX + tx + HX;
+  if (!mine) {
+    // nothing: no point of its own
+  } else if (!t.bx && !t.by) {
+#pragma unroll
+    for (int l = 0; l < NV2; ++l) {
+      double xp[4], xm[4], yp[4], ym[4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        xp[k] = fx[l * TY * EX + k + 1];
+        xm[k] = fx[l * TY * EX - (k + 1)];
+        yp[k] = fy[(l * EY + k + 1) * TX];
+        ym[k] = fy[(l * EY - (k + 1)) * TX];
+      }
+      __builtin_amdgcn_sched_barrier(0);   // one batch of LDS reads, one wait
+      r[l] = 0.0 - (skew_sum(xp, xm, d1) + skew_sum(yp, ym, d1));
+    }
+  } else {
+    const EdgePlace ex = edge_place(g.dir[0], gi), ey = edge_place(g.dir[1], gj);
+    double dx[NV2], dy[NV2];
+    if (t.bx && ex.m < 8) {
+      const double* b = sfx + ty * EX + HX + (ex.right ? t.sx - 12 : 0);
+      closure_row<12>(tab + 12 * ex.m + (ex.right ? 96 : 0),
+                      [&](int j, int k) { return b[j * TY * EX + k]; }, dx);
+    } else {
+#pragma unroll
+      for (int l = 0; l < NV2; ++l) {
+        const double* x = fx + l * TY * EX;
+        const double xp[4] = {x[1], x[2], x[3], x[4]}, xm[4] = {x[-1], x[-2], x[-3], x[-4]};
+        dx[l] = skew_sum(xp, xm, d1);
+      }
+    }
+    if (t.by && ey.m < 8) {
+      const double* b = sfy + (HY + (ey.right ? t.sy - 12 : 0)) * TX + tx;
+      closure_row<12>(tab + 12 * ey.m + (ey.right ? 96 : 0),
+                      [&](int j, int k) { return b[(j * EY + k) * TX]; }, dy);
+    } else {
+#pragma unroll
+      for (int l = 0; l < NV2; ++l) {
+        const double* c = fy + l * EY * TX;
+        const double yp[4] = {c[TX], c[2 * TX], c[3 * TX], c[4 * TX]};
+        const double ym[4] = {c[-TX], c[-2 * TX], c[-3 * TX], c[-4 * TX]};
+        dy[l] = skew_sum(yp, ym, d1);
+      }
+    }
+#pragma unroll
+    for (int l = 0; l < NV2; ++l) r[l] = 0.0 - (dx[l] + dy[l]);
+  }
+  if (g.dissipation && mine) {
     if (g.composite) {
-      auto row = [&](int l, int e) {
-        return d == 0 ? sq[(l * EY + ty + HY) * EX + e] : sq[(l * EY + e) * EX + tx + HX];
-      };
-      const int e0 = d == 0 ? t.ex0 : t.ey0;
-      if (!dr.periodic && (i < 8 || i >= dr.len - 8)) {
-        closure_row<12, 8, NC>(od, i, dr.len,
-                               [&](int idx, double* v) {
+      const EdgePlace ex = edge_place(g.dir[0], gi), ey = edge_place(g.dir[1], gj);
+#pragma unroll 1
+      for (int d = 0; d < 2; ++d) {
+        const EdgePlace e = d == 0 ? ex : ey;
+        const int step = d == 0 ? 1 : EX;
+        double dv[NV2];
+        if (e.m < 8) {
+          const double* b = d == 0 ? sq + (ty + HY) * EX + HX + (e.right ? t.sx - 12 : 0)
+                                   : sq + (HY + (e.right ? t.sy - 12 : 0)) * EX + tx + HX;
+          closure_row<12>(tab + 192 + 12 * e.m + (e.right ? 96 : 0),
+                          [&](int j, int k) { return b[j * EY * EX + k * step]; }, dv);
+        } else {
 #pragma unroll
-                                 for (int j = 0; j < NC; ++j) v[j] = row(c0 + j, idx - e0);
-                               },
-                               dv);
-      } else {
-        const int e = i - e0;
+          for (int l = 0; l < NV2; ++l) {
+            const double* x = qc + l * EY * EX;
+            double s = 0.0;
 #pragma unroll
-        for (int j = 0; j < NC; ++j) {
-          double v = 0.0;
-#pragma unroll
-          for (int k = 1; k <= 4; ++k)
-            v += od.c[kMaxHW + k] * (row(c0 + j, e + k) + row(c0 + j, e - k));
-          dv[j] = v + od.c[kMaxHW] * row(c0 + j, e);
+            for (int k = 1; k <= 4; ++k)
+              s += g.ops[SLOT_DISS].c[kMaxHW + k] * (x[k * step] + x[-k * step]);
+            dv[l] = s + g.ops[SLOT_DISS].c[kMaxHW] * x[0];
+          }
         }
+#pragma unroll
+        for (int l = 0; l < NV2; ++l) r[l] = r[l] + g.diss_amount * dv[l];
+      }
+    } else if (!t.bx && !t.by) {
+#pragma unroll
+      for (int l = 0; l < NV2; ++l) {
+        double w[9];
+#pragma unroll
+        for (int k = 0; k < 9; ++k) w[k] = k == 4 ? v[l] : qc[l * EY * EX + k - 4];
+        __builtin_amdgcn_sched_barrier(0);
+        r[l] = r[l] + g.diss_amount * two_level(w, ax);
+#pragma unroll
+        for (int k = 0; k < 9; ++k) w[k] = k == 4 ? v[l] : qc[(l * EY + k - 4) * EX];
+        __builtin_amdgcn_sched_barrier(0);
+        r[l] = r[l] + g.diss_amount * two_level(w, ay);
       }
     } else {
-      // t index: x uses columns from x0-2, y uses rows from y0-2
-      auto tv = [&](int l, int idx) {
-        return d == 0 ? stx[(l * TY + ty) * (TX + 4) + (idx - (t.x0 - 2))]
-                      : sty[(l * (TY + 4) + (idx - (t.y0 - 2))) * TX + tx];
-      };
-      if (!dr.periodic && (i < 5 || i >= dr.len - 5)) {
-        closure_row<7, 5, NC>(ot, i, dr.len,
-                              [&](int idx, double* v) {
+      const EdgePlace ex = edge_place(g.dir[0], gi), ey = edge_place(g.dir[1], gj);
+      // the windows of nine operands, moved inside the domain at its ends
+      const double* bx = qc - 4 + (ex.m < 4 ? (ex.right ? ex.m - 4 : 4 - ex.m) : 0);
+      const double* by = qc + (-4 + (ey.m < 4 ? (ey.right ? ey.m - 4 : 4 - ey.m) : 0)) * EX;
 #pragma unroll
-                                for (int j = 0; j < NC; ++j) v[j] = tv(c0 + j, idx);
-                              },
-                              dv);
-      } else {
-        const double k0 = cf.dt[0], k1 = cf.dt[1], k2 = cf.dt[2];
+      for (int l = 0; l < NV2; ++l) {
+        double w[9];
 #pragma unroll
-        for (int j = 0; j < NC; ++j) {
-          double v = 0.0;
-          v += k1 * (tv(c0 + j, i + 1) + tv(c0 + j, i - 1));
-          v += k2 * (tv(c0 + j, i + 2) + tv(c0 + j, i - 2));
-          dv[j] = v + k0 * tv(c0 + j, i);
-        }
+        for (int k = 0; k < 9; ++k) w[k] = bx[l * EY * EX + k];
+        double dv = two_level_edge(w, ax, ex, tab + 192);
+        if (hw0 != 1.0) dv = dv / hw0;   // 1 away from the first / last boundary rows
+        r[l] = r[l] + g.diss_amount * dv;
+#pragma unroll
+        for (int k = 0; k < 9; ++k) w[k] = by[(l * EY + k) * EX];
+        dv = two_level_edge(w, ay, ey, tab + 192);
+        if (hw1 != 1.0) dv = dv / hw1;
+        r[l] = r[l] + g.diss_amount * dv;
       }
-      // H^-1: the norm weight is exactly 1 away from the first / last boundary rows, where
-      // the division is the identity and is skipped
-      const double h = d == 0 ? tg.hw0(tx) : tg.hw1(ty);
-      if (h != 1.0) {
+    }
+  }
+  if (!mine) return;
+  // point terms, RK4 stage update (substepForwardRK4, src/RK4IntegratorImpl.f90:115-156) and
+  // the functional term of the new stage state
+  const double dt = a.dt;
+  const double jac = 1.0 / (h0 * h1);   // jacobian<2>
 #pragma unroll
-        for (int j = 0; j < NC; ++j) dv[j] = dv[j] / h;
+  for (int l = 0; l < NV2; ++l) r[l] = r[l] * jac;
+  // far fields, then sponges, then the other patches, each in the order of the patches
+  for (unsigned m = pmask & P->far_mask; m; m &= m - 1) {
+    const int ip = __ffs(m) - 1;
+    ConstPatch& pt = P->p[ip];
+    if (!in_patch(pt, gi, gj)) continue;
+    const double sj = pt.sigma_inv * jac;
+    double f[NV2];
+    if (ip == far.ip[0] || ip == far.ip[1]) {
+      far_formed(far, ip, ff, gi, gj, f);
+    } else {
+      const int kp = (gi - pt.lo[0]) + pt.ls[0] * (gj - pt.lo[1]);
+      const global_ptr<const double> A = glob(pt.aplus) + (long)kp * 16;
+      const global_ptr<const double> qf = glob(pt.aplus) + (long)pt.np * 16 + (long)kp * 4;
+#pragma unroll
+      for (int i = 0; i < NV2; ++i) {
+        f[i] = 0.0;
+#pragma unroll
+        for (int c = 0; c < NV2; ++c) f[i] += A[c * 4 + i] * (v[c] - qf[c]);
       }
     }
 #pragma unroll
-    for (int j = 0; j < NC; ++j) w[d][j] = amount * dv[j];
+    for (int l = 0; l < NV2; ++l) r[l] = r[l] - sj * f[l];
   }
+  if (damp != 0.0) {      // 0 outside the sponges, whatever the target holds there
+#pragma unroll
+    for (int l = 0; l < NV2; ++l) r[l] = r[l] - damp * (v[l] - qt[l]);
+  }
+  unsigned rest = pmask & ~(P->sponge_mask | P->far_mask);
+  if (a.ip_cost >= 0) rest &= ~(1u << a.ip_cost);
+  while (rest) {
+    const int ip = __ffs(rest) - 1;
+    rest &= rest - 1;
+    ConstPatch& pt = P->p[ip];
+    if (!in_patch(pt, gi, gj)) continue;
+    const int kp = (gi - pt.lo[0]) + pt.ls[0] * (gj - pt.lo[1]);
+    switch (pt.type) {
+      case MGD_PATCH_ACTUATOR:
+        if (a.control) r[3] = r[3] + glob(pt.strength)[kp] * glob(a.control)[inst * a.control_stride + kp];
+        break;
+      case MGD_PATCH_KOLMOGOROV:
+        r[1] = r[1] + v[0] * glob(pt.strength)[kp];
+        break;
+      default:
+        break;
+    }
+  }
+  // Gaussian sources: exp(-g (dx^2 + dy^2)) as the product of its 1-D factors
+  if (a.nsrc > 0) r[3] = r[3] + glob(a.src_amp)[inst * a.src_inst_stride] * (sx0 * sy0);
+  for (int s = 1; s < a.nsrc; ++s)
+    r[3] = r[3] + glob(a.src_amp)[inst * a.src_inst_stride + s] *
+                      (glob(P->srcx)[(long)s * g.n[0] + gi] * glob(P->srcy)[(long)s * g.n[1] + gj]);
+  double qn[NV2];
+#pragma unroll
+  for (int l = 0; l < NV2; ++l) {
+    const long o = inst * NVN + l * g.N + p;
+    const double rl = r[l];
+    if (a.stage == 1) {
+      glob(a.b2)[o] = v[l] + div6(dt * rl);
+      qn[l] = v[l] + dt * rl / 2.0;
+    } else if (a.stage == 2) {
+      glob(a.b2)[o] = b2[l] + div3(dt * rl);
+      qn[l] = q0[l] + dt * rl / 2.0;
+    } else if (a.stage == 3) {
+      glob(a.b2)[o] = b2[l] + div3(dt * rl);
+      qn[l] = q0[l] + dt * rl;
+    } else {
+      qn[l] = b2[l] + div6(dt * rl);
+    }
+    glob(a.qout)[o] = qn[l];
+    if (a.rhs_out) glob(a.rhs_out)[o] = rl;
+  }
+  if (cost && jin) {
+    const Prim<2> s = prim<2>(qn, g.gamma);
+    const double F = s.p - pb;
+    const double gn = (hw1 * (hw0 * 1.0)) * (h0 * h1);   // gnorm<2>
+    glob(a.jpartial)[(inst * a.nslots + a.slot) * a.npts + kj] = 1.0 * gn * (F * F * mo);
+  }
+}
+
+// -------------------------------------------------------------------------- adjoint
+// Bounded as the forward stage is (192 bytes per point and stage: 0.11 ms for 20 x 401^2).
+// Both directions' dissipation is one 9-point operator (SLOT_DISS2) on the staged values that
+// D+ reads anyway, and the Jacobian products go through the enthalpy.  The RK operands are
+// loaded behind the stencils: held across them, they cost 100 bytes of scratch per thread and
+// 0.1 ms (20 x 401^2: 252 against 162 us; with the edge tiles' closures kept from spilling the
+// last 20 bytes, 141).  Before: 401^2 15.1 -> 12.1 us, 201^2 10.8 -> 9.4, 20 x 401^2 170 -> 142.
+// One adjoint stage on tile block `blk` of instance `inst` (uniform per work-group).
+template <class S>
+__device__ __forceinline__ void adj_stage_body(const Geo& g, const Patches* patches,
+                                               const Tiling& T, const AdjStage& a, int blk,
+                                               long inst, double* lds) {
+  constexpr int EX = S::EX, EY = S::EY, HS = S::kHaloIters;
+  double* sq = lds;
+  double* tab = sq + S::SQ;
+  double* ff = tab + S::kTabA;
+  const int tile = block_tile(T, blk);
+  ConstPatches* P = (ConstPatches*)patches;
+  if (tile < 0) return;   // block beyond the tiles of its XCD (uniform per block)
+  const TileGeo t = tile_geo(g, T, tile);
+  const long NVN = (long)NV2 * g.N;
+  const global_ptr<const double> li = glob(a.lam) + inst * NVN;
+  const global_ptr<const double> qi = glob(a.q) + inst * NVN;
+  const unsigned pmask = glob(T.pmask)[tile];
+  int tx, ty;
+  const bool mine = thread_point<S>(t, &tx, &ty);
+  const int gi = t.x0 + (mine ? tx : 0), gj = t.y0 + (mine ? ty : 0);
+  const long p = gi + (long)g.n[0] * gj;
+  double v[NV2], hv[HS][NV2], q[NV2];
+#pragma unroll
+  for (int l = 0; l < NV2; ++l) v[l] = li[l * g.N + p];
+#pragma unroll
+  for (int it = 0; it < HS; ++it) {
+    const HaloSlot h = halo_slot<S>(g, t, it);
+    const long pp = h.gi + (long)g.n[0] * h.gj;
+#pragma unroll
+    for (int l = 0; l < NV2; ++l) hv[it][l] = li[l * g.N + pp];
+  }
+  double d1[5], ds[5];              // interior coefficients
+#pragma unroll
+  for (int k = 0; k <= 4; ++k) {
+    d1[k] = g.ops[SLOT_ADJ].c[kMaxHW + k];
+    ds[k] = g.ops[SLOT_DISS2].c[kMaxHW + k];
+  }
+  const FarAhead far = far_ahead<S, true>(g, P, t, pmask & P->far_mask, li, ff);
+  if (t.bx || t.by) {
+    stage_rows<S, 12, 16>(g, SLOT_ADJ, tab);
+    if (g.dissipation) stage_rows<S, 8, 12>(g, SLOT_DISS2, tab + 384);
+  }
+  if (mine) {
+#pragma unroll
+    for (int l = 0; l < NV2; ++l) sq[(l * EY + ty + HY) * EX + tx + HX] = v[l];
+  }
+#pragma unroll
+  for (int it = 0; it < HS; ++it) {
+    const HaloSlot h = halo_slot<S>(g, t, it);
+    if (h.kind == 0) continue;
+#pragma unroll
+    for (int l = 0; l < NV2; ++l) sq[(l * EY + h.ey) * EX + h.ex] = hv[it][l];
+  }
+  // the forward stage state at the point and the grid values, fetched while the stencils run
+#pragma unroll
+  for (int l = 0; l < NV2; ++l) q[l] = qi[l * g.N + p];
+  const double h0 = glob(g.h[0])[gi], hw0 = glob(g.hw[0])[gi], h1 = glob(g.h[1])[gj], hw1 = glob(g.hw[1])[gj];
+  __syncthreads();
+  if (!mine) return;
+  // D+ lambda along x and y (T1) and the dissipation (w), from the same staged values
+  double T1[2][NV2], w[NV2], l0[NV2], b2[NV2];
+  const double* lc = sq + (ty + HY) * EX + tx + HX;   // the point in the staged tile
+  const double sx = diss_scale(g, -g.diss_amount, fabs(h1), hw0);
+  const double sy = diss_scale(g, -g.diss_amount, fabs(h0), hw1);
+  if (!t.bx && !t.by) {
+#pragma unroll
+    for (int l = 0; l < NV2; ++l) {
+      double xp[4], xm[4], yp[4], ym[4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        xp[k] = lc[l * EY * EX + k + 1];
+        xm[k] = lc[l * EY * EX - (k + 1)];
+        yp[k] = lc[(l * EY + k + 1) * EX];
+        ym[k] = lc[(l * EY - (k + 1)) * EX];
+      }
+      __builtin_amdgcn_sched_barrier(0);   // one batch of LDS reads, one wait
+      T1[0][l] = skew_sum(xp, xm, d1);
+      T1[1][l] = skew_sum(yp, ym, d1);
+      w[l] = sx * sym9(v[l], xp, xm, ds) + sy * sym9(v[l], yp, ym, ds);
+    }
+  } else {
+    const EdgePlace ex = edge_place(g.dir[0], gi), ey = edge_place(g.dir[1], gj);
+    // the 16 (12) staged values at the end of the line
+    const int ox = ex.right ? t.sx - 1 : 0, oy = ey.right ? t.sy - 1 : 0;
+    const double* bx = sq + (ty + HY) * EX + HX + ox;
+    const double* by = sq + (HY + oy) * EX + tx + HX;
+    const int rx = ex.right ? 15 : 0, ry = ey.right ? 15 : 0;
+    const int qx = ex.right ? 11 : 0, qy = ey.right ? 11 : 0;
+    const bool cx = t.bx && ex.m < 12, cy = t.by && ey.m < 12;
+    double dv[NV2];
+    if (cx)
+      closure_row<16>(tab + 16 * ex.m + (ex.right ? 192 : 0),
+                      [&](int j, int k) { return bx[j * EY * EX + k - rx]; }, T1[0]);
+    if (t.bx && ex.m < 8) {
+      if (g.dissipation)
+        closure_row<12>(tab + 384 + 12 * ex.m + (ex.right ? 96 : 0),
+                        [&](int j, int k) { return bx[j * EY * EX + k - qx] - v[j]; }, dv);
+    } else {
+#pragma unroll
+      for (int l = 0; l < NV2; ++l) {
+        const double* x = lc + l * EY * EX;
+        const double xp[4] = {x[1], x[2], x[3], x[4]}, xm[4] = {x[-1], x[-2], x[-3], x[-4]};
+        if (!cx) T1[0][l] = skew_sum(xp, xm, d1);
+        dv[l] = sym9(v[l], xp, xm, ds);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+#pragma unroll
+    for (int l = 0; l < NV2; ++l) w[l] = sx * dv[l];
+    if (cy)
+      closure_row<16>(tab + 16 * ey.m + (ey.right ? 192 : 0),
+                      [&](int j, int k) { return by[(j * EY + k - ry) * EX]; }, T1[1]);
+    if (t.by && ey.m < 8) {
+      if (g.dissipation)
+        closure_row<12>(tab + 384 + 12 * ey.m + (ey.right ? 96 : 0),
+                        [&](int j, int k) { return by[(j * EY + k - qy) * EX] - v[j]; }, dv);
+    } else {
+#pragma unroll
+      for (int l = 0; l < NV2; ++l) {
+        const double* c = lc + l * EY * EX;
+        const double yp[4] = {c[EX], c[2 * EX], c[3 * EX], c[4 * EX]};
+        const double ym[4] = {c[-EX], c[-2 * EX], c[-3 * EX], c[-4 * EX]};
+        if (!cy) T1[1][l] = skew_sum(yp, ym, d1);
+        dv[l] = sym9(v[l], yp, ym, ds);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+#pragma unroll
+    for (int l = 0; l < NV2; ++l) w[l] = w[l] + sy * dv[l];
+  }
+  // here, not before: the closure rows need the registers
+  const bool sponge = (pmask & P->sponge_mask) != 0;            // uniform per block
+  const double damp = sponge ? glob(P->damp)[p] : 0.0;
+#pragma unroll
+  for (int l = 0; l < NV2; ++l) {
+    const long o = inst * NVN + l * g.N + p;
+    l0[l] = a.stage == 3 || a.stage == 2 ? glob(a.l0)[o] : 0.0;
+    b2[l] = a.stage <= 3 ? glob(a.b2)[o] : 0.0;
+  }
+  const Prim<2> s = prim<2>(q, g.gamma);
+  double r[NV2];
+  const double mx[2] = {h1, h0};   // metric<2>(g, 0, .), metric<2>(g, 1, .)
+  adj_jacobian_rows(mx, s, g.gamma, T1, r);
+  const double jac = 1.0 / (h0 * h1);   // jacobian<2>
+#pragma unroll
+  for (int l = 0; l < NV2; ++l) r[l] = (g.dissipation ? r[l] + w[l] : r[l]) * jac;
+  // far fields, then sponges, then the other patches, each in the order of the patches
+  for (unsigned m = pmask & P->far_mask; m; m &= m - 1) {
+    const int ip = __ffs(m) - 1;
+    ConstPatch& pt = P->p[ip];
+    if (!in_patch(pt, gi, gj)) continue;
+    const double sj = pt.sigma_inv * jac;
+    double f[NV2];
+    if (ip == far.ip[0] || ip == far.ip[1]) {
+      far_formed(far, ip, ff, gi, gj, f);
+    } else {
+      const int kp = (gi - pt.lo[0]) + pt.ls[0] * (gj - pt.lo[1]);
+      const global_ptr<const double> A = glob(pt.aplus) + (long)kp * 16;
+#pragma unroll
+      for (int i = 0; i < NV2; ++i) {
+        f[i] = 0.0;
+#pragma unroll
+        for (int c = 0; c < NV2; ++c) f[i] += A[i * 4 + c] * v[c];
+      }
+    }
+#pragma unroll
+    for (int l = 0; l < NV2; ++l) r[l] = r[l] + sj * f[l];
+  }
+  if (sponge) {
+#pragma unroll
+    for (int l = 0; l < NV2; ++l) r[l] = r[l] + damp * v[l];
+  }
+  unsigned rest = pmask & ~(P->sponge_mask | P->far_mask);
+  while (rest) {
+    const int ip = __ffs(rest) - 1;
+    rest &= rest - 1;
+    ConstPatch& pt = P->p[ip];
+    if (!in_patch(pt, gi, gj)) continue;
+    const int kp = (gi - pt.lo[0]) + pt.ls[0] * (gj - pt.lo[1]);
+    switch (pt.type) {
+      case MGD_PATCH_COST_TARGET: {
+        // acoustic-noise adjoint forcing from the forward state at this point
+        // (src/AcousticNoiseImpl.f90:208-280), scaled by the stage factor
+        if (a.zero_forcing) break;
+        const double F = -2.0 * glob(pt.strength)[kp] * 1.0 * (g.gamma - 1.0) * (s.p - glob(pt.aplus)[kp]);
+        const double ke = s.u[0] * s.u[0] + s.u[1] * s.u[1];
+        r[0] = r[0] + a.forcing_factor * (0.5 * ke * F);
+        r[1] = r[1] + a.forcing_factor * (-s.u[0] * F);
+        r[2] = r[2] + a.forcing_factor * (-s.u[1] * F);
+        r[3] = r[3] + a.forcing_factor * F;
+        break;
+      }
+      case MGD_PATCH_ACTUATOR: {
+        // ThermalActuator gradient and sensitivity on the pre-update adjoint state
+        if (a.grad) glob(a.grad)[inst * a.grad_stride + kp] = v[3] * (glob(pt.strength)[kp] * 1.0);
+        if (a.spartial) {
+          const double F = v[3] * glob(pt.strength)[kp] * 1.0;
+          const double gn = (glob(g.hw[1])[gj] * (glob(g.hw[0])[gi] * 1.0)) * (h0 * h1);   // gnorm<2>
+          glob(a.spartial)[(inst * a.nslots + a.slot) * a.npts + kp] = 1.0 * gn * (F * F);
+        }
+        break;
+      }
+      case MGD_PATCH_KOLMOGOROV:
+        r[0] = r[0] - v[1] * glob(pt.strength)[kp];
+        break;
+      default:
+        break;
+    }
+  }
+  // RK4 adjoint stage update (substepAdjointRK4, src/RK4IntegratorImpl.f90:215-261)
+  const double dt = a.dt;
+#pragma unroll
+  for (int l = 0; l < NV2; ++l) {
+    const long o = inst * NVN + l * g.N + p;
+    const double rl = r[l];
+    double ln;
+    if (a.stage == 4) {
+      glob(a.b2)[o] = v[l] - div6(dt * rl);
+      ln = v[l] - dt * rl / 2.0;
+    } else if (a.stage == 3) {
+      glob(a.b2)[o] = b2[l] - div3(dt * rl);
+      ln = l0[l] - dt * rl / 2.0;
+    } else if (a.stage == 2) {
+      glob(a.b2)[o] = b2[l] - div3(dt * rl);
+      ln = l0[l] - dt * rl;
+    } else {
+      ln = b2[l] - div6(dt * rl);
+    }
+    glob(a.lout)[o] = ln;
+    if (a.rhs_out) glob(a.rhs_out)[o] = rl;
+  }
+}
+
+template <class S>
+__global__ void __launch_bounds__(S::NT, S::waves(S::kFwdLds)) k_fwd_stage2d(Geo g, const Patches* __restrict__ P,
+                                                       Tiling T, FwdStage a) {
+  __shared__ double lds[S::kFwdLds];
+  fwd_stage_body<S>(g, P, T, a, blockIdx.x, blockIdx.y, lds);
+}
+
+template <class S>
+__global__ void __launch_bounds__(S::NT, S::waves(S::kAdjLds)) k_adj_stage2d(Geo g, const Patches* __restrict__ P,
+                                                       Tiling T, AdjStage a) {
+  __shared__ double lds[S::kAdjLds];
+  adj_stage_body<S>(g, P, T, a, blockIdx.x, blockIdx.y, lds);
+}
+
+// One adjoint stage and one forward stage of the same region in one launch: blocks
+// [0, nblk) run the adjoint stage's tiles, blocks [nblk, 2 nblk) the forward stage's (the
+// window recompute beside the adjoint of the next window: independent states, so the
+// same values as two launches).  nblk is a multiple of 8, so a block's XCD -- its index
+// mod 8 -- is the one its tile is dealt to either way.
+template <class S>
+__global__ void __launch_bounds__(S::NT, S::waves(S::kDualLds)) k_dual_stage2d(Geo g, const Patches* __restrict__ P,
+                                                        Tiling T, AdjStage a, FwdStage f) {
+  __shared__ double lds[S::kDualLds];
+  if ((int)blockIdx.x < T.nblk) adj_stage_body<S>(g, P, T, a, blockIdx.x, blockIdx.y, lds);
+  else fwd_stage_body<S>(g, P, T, f, (int)blockIdx.x - T.nblk, blockIdx.y, lds);
 }
 
 // Block sum: wave-level shuffles, then one LDS exchange of the per-wave sums.
@@ -540,495 +944,6 @@ __device__ __forceinline__ double block_sum(double v, double* red) {
   return s;
 }
 
-// x[c0 + j] of a register array with the wave-uniform group offset c0 (a multiple of
-// NC), formed by selects on constant indices (a run-time register index would move the
-// array to scratch memory).
-template <int NC>
-__device__ __forceinline__ double comp(const double* x, int c0, int j) {
-  double v = x[j];
-#pragma unroll
-  for (int k = 1; k * NC + j < NV2; ++k)
-    if (c0 == k * NC) v = x[k * NC + j];
-  return v;
-}
-
-// Rows C0 .. C0 + NC - 1 of sum_d A_d^T-side products of the adjoint rhs:
-// r[j] = sum_d sum_c A_d[C0 + j][c] T1[d][c] (computeRhsAdjoint's Jacobian part for 2-D
-// Euler), with the row offset a compile-time constant so only those rows are formed.
-template <int C0, int NC>
-__device__ __forceinline__ void adj_jacobian_rows(const double* mx, const Prim<2>& s, double gamma,
-                                                  const double (*T1)[NV2], double* r) {
-#pragma unroll
-  for (int j = 0; j < NC; ++j) r[j] = 0.0;
-#pragma unroll
-  for (int d = 0; d < 2; ++d) {
-    double m[2], A[16];
-    m[0] = d == 0 ? mx[0] : 0.0;
-    m[1] = d == 1 ? mx[1] : 0.0;
-    inviscid_jacobian<2>(m, s, gamma, A);
-#pragma unroll
-    for (int j = 0; j < NC; ++j) {
-      double acc = 0.0;
-#pragma unroll
-      for (int c = 0; c < NV2; ++c) acc += A[(C0 + j) * 4 + c] * T1[d][c];
-      r[j] = r[j] + acc;
-    }
-  }
-}
-
-__device__ __forceinline__ bool in_patch(const DPatch& pt, int i, int j) {
-  return i >= pt.lo[0] && i <= pt.hi[0] && j >= pt.lo[1] && j <= pt.hi[1];
-}
-
-// The LDS of a stage body: the staged operand, the flux / scratch space and the tile's
-// grid values.  One allocation per kernel, shared by the forward and adjoint bodies where
-// one kernel runs both (k_dual_stage2d).
-template <class S>
-struct StageLds {
-  double q[S::SQ];
-  double c[S::SSCR];
-  double grid[TileGrid<S>::kSize];
-};
-
-template <class S>
-__device__ __forceinline__ StageLds<S>& stage_lds() {
-  __shared__ StageLds<S> lds;
-  return lds;
-}
-
-// -------------------------------------------------------------------------- forward
-// One forward stage on tile block `blk` of instance `inst` (uniform per work-group).
-template <class S>
-__device__ __forceinline__ void fwd_stage_body(const Geo& g, const Patches* __restrict__ P,
-                                               const Tiling& T, const FwdStage& a, int blk,
-                                               long inst) {
-  constexpr int TX = S::TX, TY = S::TY, EX = S::EX, EY = S::EY, NP = S::NP, NC = S::NC;
-  constexpr int SFX = S::SFX, STX = S::STX;
-  StageLds<S>& lds = stage_lds<S>();
-  double(&sq)[S::SQ] = lds.q;
-  double(&sc)[S::SSCR] = lds.c;
-  double(&sgrid)[TileGrid<S>::kSize] = lds.grid;
-  const int tile = block_tile(T, blk);
-  if (tile < 0) return;   // block beyond the tiles of its XCD (uniform per block)
-  const TileGeo t = tile_geo(T, tile);
-  const long NVN = (long)NV2 * g.N;
-  const double* qi = a.qin + inst * NVN;
-  double* sfx = sc;
-  double* sfy = sc + SFX;
-  const Coefs cf = load_coefs(g, SLOT_FIRST);
-  const double gv = load_tile_grid<S>(g, t);
-  const TileGrid<S> tg{sgrid};
-  const unsigned pmask = T.pmask[tile];
-  // this thread's point and component group
-  const int lane = threadIdx.x % NP, c0 = (threadIdx.x / NP) * NC;
-  int tx, ty;
-  point_of_lane<S>(g, T, tile, lane, &tx, &ty);
-  const bool mine = tx < t.sx && ty < t.sy;
-  const int gi = t.x0 + tx, gj = t.y0 + ty;
-  const long p = gi + (long)g.n[0] * gj;
-  StageRegs<S> sr;
-  stage_load<S>(g, t, qi, sr);
-  // the grid values are needed by the flux metrics; this barrier waits for them only
-  // (the operand loads stay in flight)
-  if (threadIdx.x < TileGrid<S>::kSize) sgrid[threadIdx.x] = gv;
-  __syncthreads();
-  stage_store<S, true>(g, t, sr, tg, sq, sfx, sfy);
-  __syncthreads();
-  const Op& o1 = g.ops[SLOT_FIRST];
-  // the dissipation intermediates are formed from the staged operand together with the
-  // flux derivatives and stored once the flux space they overwrite is free
-  DissSlots<S> dsl;
-  const bool two_level = g.dissipation && !g.composite;
-  if (S::kDissRegs && two_level) diss_compute<S>(g, t, cf, tg, sq, lane, c0, dsl);
-  double r[NC];
-  if (mine) {
-    double dfx[NC], dfy[NC];
-    deriv_lds<12, 8, NC>(o1, cf.d1, g.dir[0], gi, t.ex0, c0,
-                         [&](int l, int e) { return sfx[(l * TY + ty) * EX + e]; }, dfx);
-    deriv_lds<12, 8, NC>(o1, cf.d1, g.dir[1], gj, t.ey0, c0,
-                         [&](int l, int e) { return sfy[(l * EY + e) * TX + tx]; }, dfy);
-#pragma unroll
-    for (int j = 0; j < NC; ++j) r[j] = 0.0 - (dfx[j] + dfy[j]);
-  }
-  // RK operands of this thread's components, fetched after the flux derivatives: every
-  // block issues its operand loads at once at entry, and these (two thirds of the entry
-  // bytes in stages 2 and 3) would lengthen that burst; here they arrive during the
-  // dissipation terms
-  double pq0[NC], pb2[NC];
-  if (mine) {
-#pragma unroll
-    for (int j = 0; j < NC; ++j) {
-      const long o = (c0 + j) * g.N + p;
-      pq0[j] = (a.stage == 2 || a.stage == 3) ? a.q0[inst * NVN + o] : 0.0;
-      pb2[j] = a.stage >= 2 ? a.b2[inst * NVN + o] : 0.0;
-    }
-  }
-  double* stx = sc;
-  double* sty = sc + STX;
-  if (two_level) {
-    __syncthreads();   // fluxes consumed
-    if (S::kDissRegs)
-      diss_store<S>(dsl, c0, stx, sty);
-    else
-      diss_intermediates<S>(g, t, cf, tg, sq, stx, sty, lane, c0);
-    __syncthreads();
-  }
-  double qn[NC];
-  if (mine) {
-    if (g.dissipation) {
-      double w[2][NC];
-      diss_terms<S>(g, t, cf, tg, sq, stx, sty, tx, ty, gi, gj, c0, g.diss_amount, w);
-#pragma unroll
-      for (int d = 0; d < 2; ++d)
-#pragma unroll
-        for (int j = 0; j < NC; ++j) r[j] = r[j] + w[d][j];
-    }
-    const double jac = 1.0 / (tg.h0(tx) * tg.h1(ty));   // jacobian<2>
-    double qp[NV2];
-#pragma unroll
-    for (int l = 0; l < NV2; ++l) qp[l] = sq[(l * EY + ty + HY) * EX + tx + HX];
-#pragma unroll
-    for (int j = 0; j < NC; ++j) r[j] = r[j] * jac;
-    unsigned m = pmask;
-    while (m) {
-      const int ip = __ffs(m) - 1;
-      m &= m - 1;
-      const DPatch& pt = P->p[ip];
-      if (!in_patch(pt, gi, gj)) continue;
-      const int kp = (gi - pt.lo[0]) + pt.ls[0] * (gj - pt.lo[1]);
-      switch (pt.type) {
-        case MGD_PATCH_FAR_FIELD: {
-          const double* A = pt.aplus + (long)kp * 16;
-          const double* qt = pt.aplus + (long)pt.np * 16 + (long)kp * 4;
-          const double sj = pt.sigma_inv * jac;
-#pragma unroll
-          for (int j = 0; j < NC; ++j) {
-            const int i = c0 + j;
-            double v = 0.0;
-#pragma unroll
-            for (int c = 0; c < NV2; ++c) v += A[c * 4 + i] * (qp[c] - qt[c]);
-            r[j] = r[j] - sj * v;
-          }
-          break;
-        }
-        case MGD_PATCH_SPONGE: {
-          const double sp = pt.strength[kp];
-          const double* qt = pt.aplus + (long)kp * 4;
-#pragma unroll
-          for (int j = 0; j < NC; ++j) r[j] = r[j] - sp * (comp<NC>(qp, c0, j) - qt[c0 + j]);
-          break;
-        }
-        case MGD_PATCH_ACTUATOR:
-#pragma unroll
-          for (int j = 0; j < NC; ++j)
-            if (c0 + j == 3 && a.control)
-              r[j] = r[j] + pt.strength[kp] * a.control[inst * a.control_stride + kp];
-          break;
-        case MGD_PATCH_KOLMOGOROV:
-#pragma unroll
-          for (int j = 0; j < NC; ++j)
-            if (c0 + j == 1) r[j] = r[j] + qp[0] * pt.strength[kp];
-          break;
-        default:
-          break;
-      }
-    }
-#pragma unroll
-    for (int j = 0; j < NC; ++j) {
-      if (c0 + j != 3) continue;
-      for (int s = 0; s < a.nsrc; ++s) {
-        const double dx0 = tg.x0(tx) - a.src[s].loc[0];
-        const double dy0 = tg.x1(ty) - a.src[s].loc[1];
-        double rr2 = 0.0;
-        rr2 += dx0 * dx0;
-        rr2 += dy0 * dy0;
-        r[j] = r[j] + a.src_amp[inst * a.src_inst_stride + s] * exp(-a.src[s].gfac * rr2);
-      }
-    }
-    // RK4 stage update (substepForwardRK4, src/RK4IntegratorImpl.f90:115-156).  The
-    // stage outputs are written with non-temporal stores: they stream to HBM during the
-    // launch instead of waiting in L2 for the write-back at its end
-    const double dt = a.dt;
-    double* b2 = a.b2 + inst * NVN;
-#pragma unroll
-    for (int j = 0; j < NC; ++j) {
-      const int l = c0 + j;
-      const long o = l * g.N + p;
-      const double rl = r[j];
-      if (a.stage == 1) {
-        const double ql = comp<NC>(qp, c0, j);
-        __builtin_nontemporal_store(ql + div6(dt * rl), &b2[o]);
-        qn[j] = ql + dt * rl / 2.0;
-      } else if (a.stage == 2) {
-        __builtin_nontemporal_store(pb2[j] + div3(dt * rl), &b2[o]);
-        qn[j] = pq0[j] + dt * rl / 2.0;
-      } else if (a.stage == 3) {
-        __builtin_nontemporal_store(pb2[j] + div3(dt * rl), &b2[o]);
-        qn[j] = pq0[j] + dt * rl;
-      } else {
-        qn[j] = pb2[j] + div6(dt * rl);
-      }
-      __builtin_nontemporal_store(qn[j], &a.qout[inst * NVN + o]);
-      if (a.rhs_out) a.rhs_out[inst * NVN + o] = rl;
-    }
-  }
-  // functional term of the new stage state at cost-target points (needs all components:
-  // with CS > 1 they are exchanged through the operand space)
-  if (a.jpartial && a.ip_cost >= 0 && ((pmask >> a.ip_cost) & 1u)) {   // uniform per block
-    double qa[NV2];
-    if (S::CS == 1) {
-#pragma unroll
-      for (int j = 0; j < NC; ++j) qa[j] = qn[j];
-    } else {
-      __syncthreads();   // every read of the staged operand is done
-      if (mine) {
-#pragma unroll
-        for (int j = 0; j < NC; ++j) sq[(c0 + j) * NP + lane] = qn[j];
-      }
-      __syncthreads();
-#pragma unroll
-      for (int l = 0; l < NV2; ++l) qa[l] = sq[l * NP + lane];
-    }
-    const DPatch& pt = P->p[a.ip_cost];
-    if (mine && c0 == 0 && in_patch(pt, gi, gj)) {
-      const int kp = (gi - pt.lo[0]) + pt.ls[0] * (gj - pt.lo[1]);
-      const Prim<2> s = prim<2>(qa, g.gamma);
-      const double F = s.p - pt.aplus[kp];
-      const double gn = (tg.hw1(ty) * (tg.hw0(tx) * 1.0)) * (tg.h0(tx) * tg.h1(ty));   // gnorm<2>
-      a.jpartial[(inst * a.nslots + a.slot) * a.npts + kp] = 1.0 * gn * (F * F * pt.strength[kp]);
-    }
-  }
-}
-
-// -------------------------------------------------------------------------- adjoint
-// One adjoint stage on tile block `blk` of instance `inst` (uniform per work-group).
-template <class S>
-__device__ __forceinline__ void adj_stage_body(const Geo& g, const Patches* __restrict__ P,
-                                               const Tiling& T, const AdjStage& a, int blk,
-                                               long inst) {
-  constexpr int TX = S::TX, EX = S::EX, EY = S::EY, NP = S::NP, NC = S::NC;
-  constexpr int STX = S::STX;
-  StageLds<S>& lds = stage_lds<S>();
-  double(&sq)[S::SQ] = lds.q;
-  double(&sc)[S::SSCR] = lds.c;
-  double(&sgrid)[TileGrid<S>::kSize] = lds.grid;
-  const int tile = block_tile(T, blk);
-  if (tile < 0) return;   // block beyond the tiles of its XCD (uniform per block)
-  const TileGeo t = tile_geo(T, tile);
-  const long NVN = (long)NV2 * g.N;
-  const double* li = a.lam + inst * NVN;
-  const double* qi = a.q + inst * NVN;
-  const Coefs cf = load_coefs(g, SLOT_ADJ);
-  const double gv = load_tile_grid<S>(g, t);
-  const TileGrid<S> tg{sgrid};
-  const unsigned pmask = T.pmask[tile];
-  const int lane = threadIdx.x % NP, c0 = (threadIdx.x / NP) * NC;
-  // row-major points (the 8 x 8 wave blocks of point_of_lane do not pay here: the
-  // adjoint closure is 12 deep and splits the second block column)
-  const int tx = lane % TX, ty = lane / TX;
-  const bool mine = tx < t.sx && ty < t.sy;
-  const int gi = t.x0 + tx, gj = t.y0 + ty;
-  const long p = gi + (long)g.n[0] * gj;
-  // forward stage state at this thread's point, fetched before the stencil work
-  double pq[NV2];
-  if (mine) {
-#pragma unroll
-    for (int l = 0; l < NV2; ++l) pq[l] = qi[l * g.N + p];
-  }
-  {
-    StageRegs<S> sr;
-    stage_load<S>(g, t, li, sr);
-    if (threadIdx.x < TileGrid<S>::kSize) sgrid[threadIdx.x] = gv;
-    stage_store<S, false>(g, t, sr, tg, sq, nullptr, nullptr);
-  }
-  double* stx = sc;
-  double* sty = sc + STX;
-  __syncthreads();
-  // the dissipation intermediates (into the scratch space) and D+ lambda in one phase
-  const bool two_level = g.dissipation && !g.composite;
-  if (two_level) diss_intermediates<S>(g, t, cf, tg, sq, stx, sty, lane, c0);
-  const Op& oa = g.ops[SLOT_ADJ];
-  double T1[2][NV2];   // D+ lambda along x and y, all components (own ones first)
-  double w[2][NC];     // dissipation terms of this thread's components
-  if (mine) {
-    double u[2][NC];
-    deriv_lds<16, 12, NC>(oa, cf.d1, g.dir[0], gi, t.ex0, c0,
-                          [&](int l, int e) { return sq[(l * EY + ty + HY) * EX + e]; }, u[0]);
-    deriv_lds<16, 12, NC>(oa, cf.d1, g.dir[1], gj, t.ey0, c0,
-                          [&](int l, int e) { return sq[(l * EY + e) * EX + tx + HX]; }, u[1]);
-#pragma unroll
-    for (int d = 0; d < 2; ++d)
-#pragma unroll
-      for (int j = 0; j < NC; ++j) T1[d][j] = u[d][j];
-  }
-  if (two_level) __syncthreads();   // intermediates complete
-  // with component groups the dissipation terms are formed before the exchange
-  if (S::CS > 1 && mine && g.dissipation)
-    diss_terms<S>(g, t, cf, tg, sq, stx, sty, tx, ty, gi, gj, c0, -g.diss_amount, w);
-  if (S::CS > 1) {
-    // every component of D+ lambda is needed by the Jacobian products: exchange them
-    // through the scratch space (the dissipation intermediates are no longer read)
-    __syncthreads();
-    if (mine) {
-#pragma unroll
-      for (int d = 0; d < 2; ++d)
-#pragma unroll
-        for (int j = 0; j < NC; ++j) sc[(d * NV2 + c0 + j) * NP + lane] = T1[d][j];
-    }
-    __syncthreads();
-    if (mine) {
-#pragma unroll
-      for (int d = 0; d < 2; ++d)
-#pragma unroll
-        for (int l = 0; l < NV2; ++l) T1[d][l] = sc[(d * NV2 + l) * NP + lane];
-    }
-  }
-  if (!mine) return;
-  const Prim<2> s = prim<2>(pq, g.gamma);
-  double r[NC];
-  const double mx[2] = {tg.h1(ty), tg.h0(tx)};   // metric<2>(g, 0, .), metric<2>(g, 1, .)
-  if (c0 == 0)
-    adj_jacobian_rows<0, NC>(mx, s, g.gamma, T1, r);
-  else
-    adj_jacobian_rows<(S::CS > 1 ? NC : 0), NC>(mx, s, g.gamma, T1, r);
-  // RK operands, fetched here so that they are not live through the derivative work
-  double pl0[NC], pb2[NC];
-#pragma unroll
-  for (int j = 0; j < NC; ++j) {
-    const long o = (c0 + j) * g.N + p;
-    pl0[j] = (a.stage == 3 || a.stage == 2) ? a.l0[inst * NVN + o] : 0.0;
-    pb2[j] = a.stage <= 3 ? a.b2[inst * NVN + o] : 0.0;
-  }
-  if (g.dissipation) {
-    if (S::CS == 1)
-      diss_terms<S>(g, t, cf, tg, sq, stx, sty, tx, ty, gi, gj, c0, -g.diss_amount, w);
-#pragma unroll
-    for (int d = 0; d < 2; ++d)
-#pragma unroll
-      for (int j = 0; j < NC; ++j) r[j] = r[j] + w[d][j];
-  }
-  const double jac = 1.0 / (tg.h0(tx) * tg.h1(ty));   // jacobian<2>
-#pragma unroll
-  for (int j = 0; j < NC; ++j) r[j] = r[j] * jac;
-  double lp[NV2];
-#pragma unroll
-  for (int l = 0; l < NV2; ++l) lp[l] = sq[(l * EY + ty + HY) * EX + tx + HX];
-  unsigned m = pmask;
-  while (m) {
-    const int ip = __ffs(m) - 1;
-    m &= m - 1;
-    const DPatch& pt = P->p[ip];
-    if (!in_patch(pt, gi, gj)) continue;
-    const int kp = (gi - pt.lo[0]) + pt.ls[0] * (gj - pt.lo[1]);
-    switch (pt.type) {
-      case MGD_PATCH_FAR_FIELD: {
-        const double* A = pt.aplus + (long)kp * 16;
-        const double sj = pt.sigma_inv * jac;
-#pragma unroll
-        for (int j = 0; j < NC; ++j) {
-          const int i = c0 + j;
-          double acc = 0.0;
-#pragma unroll
-          for (int c = 0; c < NV2; ++c) acc += A[i * 4 + c] * lp[c];
-          r[j] = r[j] + sj * acc;
-        }
-        break;
-      }
-      case MGD_PATCH_SPONGE: {
-        const double sp = pt.strength[kp];
-#pragma unroll
-        for (int j = 0; j < NC; ++j) r[j] = r[j] + sp * comp<NC>(lp, c0, j);
-        break;
-      }
-      case MGD_PATCH_COST_TARGET: {
-        // acoustic-noise adjoint forcing from the forward state at this point
-        // (src/AcousticNoiseImpl.f90:208-280), scaled by the stage factor
-        double af[NV2] = {0.0, 0.0, 0.0, 0.0};
-        if (!a.zero_forcing) {
-          const double F = -2.0 * pt.strength[kp] * 1.0 * (g.gamma - 1.0) * (s.p - pt.aplus[kp]);
-          af[3] = F;
-          af[1] = -s.u[0] * F;
-          af[2] = -s.u[1] * F;
-          double ke = 0.0;
-          ke += s.u[0] * s.u[0];
-          ke += s.u[1] * s.u[1];
-          af[0] = 0.5 * ke * F;
-        }
-#pragma unroll
-        for (int j = 0; j < NC; ++j) r[j] = r[j] + a.forcing_factor * comp<NC>(af, c0, j);
-        break;
-      }
-      case MGD_PATCH_ACTUATOR: {
-        // ThermalActuator gradient and sensitivity on the pre-update adjoint state,
-        // written by the group that owns the energy component
-        if (c0 + NC - 1 == 3) {
-          if (a.grad) a.grad[inst * a.grad_stride + kp] = lp[3] * (pt.strength[kp] * 1.0);
-          if (a.spartial) {
-            const double F = lp[3] * pt.strength[kp] * 1.0;
-            const double gn = (tg.hw1(ty) * (tg.hw0(tx) * 1.0)) * (tg.h0(tx) * tg.h1(ty));   // gnorm<2>
-            a.spartial[(inst * a.nslots + a.slot) * a.npts + kp] = 1.0 * gn * (F * F);
-          }
-        }
-        break;
-      }
-      case MGD_PATCH_KOLMOGOROV:
-#pragma unroll
-        for (int j = 0; j < NC; ++j)
-          if (c0 + j == 0) r[j] = r[j] - lp[1] * pt.strength[kp];
-        break;
-    }
-  }
-  // RK4 adjoint stage update (substepAdjointRK4, src/RK4IntegratorImpl.f90:215-261),
-  // non-temporal stores as in the forward stage
-  const double dt = a.dt;
-  double* b2 = a.b2 + inst * NVN;
-#pragma unroll
-  for (int j = 0; j < NC; ++j) {
-    const long o = (c0 + j) * g.N + p;
-    const double rl = r[j];
-    double ln;
-    if (a.stage == 4) {
-      const double ll = comp<NC>(lp, c0, j);
-      __builtin_nontemporal_store(ll - div6(dt * rl), &b2[o]);
-      ln = ll - dt * rl / 2.0;
-    } else if (a.stage == 3) {
-      __builtin_nontemporal_store(pb2[j] - div3(dt * rl), &b2[o]);
-      ln = pl0[j] - dt * rl / 2.0;
-    } else if (a.stage == 2) {
-      __builtin_nontemporal_store(pb2[j] - div3(dt * rl), &b2[o]);
-      ln = pl0[j] - dt * rl;
-    } else {
-      ln = pb2[j] - div6(dt * rl);
-    }
-    __builtin_nontemporal_store(ln, &a.lout[inst * NVN + o]);
-    if (a.rhs_out) a.rhs_out[inst * NVN + o] = rl;
-  }
-}
-
-template <class S>
-__global__ void __launch_bounds__(S::NT, S::kWavesPerEU) k_fwd_stage2d(Geo g, const Patches* __restrict__ P,
-                                                       Tiling T, FwdStage a) {
-  fwd_stage_body<S>(g, P, T, a, blockIdx.x, blockIdx.y);
-}
-
-template <class S>
-__global__ void __launch_bounds__(S::NT, S::kWavesPerEU) k_adj_stage2d(Geo g, const Patches* __restrict__ P,
-                                                       Tiling T, AdjStage a) {
-  adj_stage_body<S>(g, P, T, a, blockIdx.x, blockIdx.y);
-}
-
-// One adjoint stage and one forward stage of the same region in one launch: blocks
-// [0, nblk) run the adjoint stage's tiles, blocks [nblk, 2 nblk) the forward stage's (the
-// window recompute beside the adjoint of the next window: independent states, so the
-// same values as two launches).  nblk is a multiple of 8, so a block's XCD -- its index
-// mod 8 -- is the one its tile is dealt to either way.
-template <class S>
-__global__ void __launch_bounds__(S::NT, S::kWavesPerEU) k_dual_stage2d(Geo g, const Patches* __restrict__ P,
-                                                        Tiling T, AdjStage a, FwdStage f) {
-  if ((int)blockIdx.x < T.nblk) adj_stage_body<S>(g, P, T, a, blockIdx.x, blockIdx.y);
-  else fwd_stage_body<S>(g, P, T, f, (int)blockIdx.x - T.nblk, blockIdx.y);
-}
-
 // Several regions in one launch: launch block k belongs to the member m with
 // mem[m].block0 <= k < mem[m + 1].block0 (members in block order), which sees it as tile
 // block (k - block0) mod nblk of instance (k - block0) / nblk.  args[m]: the stage of m.
@@ -1042,44 +957,26 @@ __device__ __forceinline__ int group_member(const GroupMember* mem, int nmem, in
   return m;
 }
 
-// Copies one trivially copyable descriptor from device memory into LDS, word by word
-// across the work-group (the caller synchronises).
-template <class T>
-__device__ __forceinline__ void copy_to_lds(const T* src, T* dst) {
-  static_assert(sizeof(T) % 4 == 0, "descriptor of whole words");
-  const int* s = reinterpret_cast<const int*>(src);
-  int* d = reinterpret_cast<int*>(dst);
-  for (int i = threadIdx.x; i < (int)(sizeof(T) / 4); i += blockDim.x) d[i] = s[i];
-}
-
-// The member's descriptors are staged in LDS: the body reads them many times, and LDS
-// cannot alias the global stores of the stage, so no read is repeated after a store.
 template <class S>
-__global__ void __launch_bounds__(S::NT, S::kWavesPerEU)
+__global__ void __launch_bounds__(S::NT, S::waves(S::kFwdLds))
     k_fwd_stage2d_group(const GroupMember* __restrict__ mem, int nmem, const FwdStage* __restrict__ args) {
-  __shared__ GroupMember sm;
-  __shared__ FwdStage sa;
+  __shared__ double lds[S::kFwdLds];
   int blk;
   long inst;
   const int m = group_member(mem, nmem, &blk, &inst);
-  copy_to_lds(&mem[m], &sm);
-  copy_to_lds(&args[m], &sa);
-  __syncthreads();
-  fwd_stage_body<S>(sm.g, sm.P, sm.T, sa, blk, inst);
+  const GroupMember& gm = mem[m];
+  fwd_stage_body<S>(gm.g, gm.P, gm.T, args[m], blk, inst, lds);
 }
 
 template <class S>
-__global__ void __launch_bounds__(S::NT, S::kWavesPerEU)
+__global__ void __launch_bounds__(S::NT, 3)   // the descriptors in scalar registers leave fewer for addresses
     k_adj_stage2d_group(const GroupMember* __restrict__ mem, int nmem, const AdjStage* __restrict__ args) {
-  __shared__ GroupMember sm;
-  __shared__ AdjStage sa;
+  __shared__ double lds[S::kAdjLds];
   int blk;
   long inst;
   const int m = group_member(mem, nmem, &blk, &inst);
-  copy_to_lds(&mem[m], &sm);
-  copy_to_lds(&args[m], &sa);
-  __syncthreads();
-  adj_stage_body<S>(sm.g, sm.P, sm.T, sa, blk, inst);
+  const GroupMember& gm = mem[m];
+  adj_stage_body<S>(gm.g, gm.P, gm.T, args[m], blk, inst, lds);
 }
 
 // Stage sums of the per-point quadrature terms of one chunk of stages: one block of
@@ -1131,11 +1028,11 @@ using S32x16 = Shape<32, 16>;
 using S16x32 = Shape<16, 32>;
 using S16x16 = Shape<16, 16>;
 using S24x16 = Shape<24, 16>;
-using S16x16c2 = Shape<16, 16, 2>;
-using S16x12c2 = Shape<16, 12, 2>;
+using S16x24 = Shape<16, 24>;
+using S16x12 = Shape<16, 12>;
 
 static const int kShapeDims[kNumTileShapes][2] = {{32, 16}, {16, 32}, {16, 16}, {24, 16},
-                                                  {16, 16}, {16, 12}};
+                                                  {16, 24}, {16, 12}};
 
 int fused2d_shape_dims(int shape, int* tx, int* ty) {
   if (shape < 0 || shape >= kNumTileShapes) return MGD_ERR_ARG;
@@ -1246,8 +1143,8 @@ void launch_dual_stage2d(const Geo& g, const Patches* P, const Tiling& T, const 
     case 1: dual_launch<S16x32>(g, P, T, a, f, st); break;
     case 2: dual_launch<S16x16>(g, P, T, a, f, st); break;
     case 3: dual_launch<S24x16>(g, P, T, a, f, st); break;
-    case 4: dual_launch<S16x16c2>(g, P, T, a, f, st); break;
-    default: dual_launch<S16x12c2>(g, P, T, a, f, st); break;
+    case 4: dual_launch<S16x24>(g, P, T, a, f, st); break;
+    default: dual_launch<S16x12>(g, P, T, a, f, st); break;
   }
 }
 
@@ -1258,8 +1155,8 @@ void launch_fwd_stage2d(const Geo& g, const Patches* P, const Tiling& T, const F
     case 1: fwd_launch<S16x32>(g, P, T, a, st); break;
     case 2: fwd_launch<S16x16>(g, P, T, a, st); break;
     case 3: fwd_launch<S24x16>(g, P, T, a, st); break;
-    case 4: fwd_launch<S16x16c2>(g, P, T, a, st); break;
-    default: fwd_launch<S16x12c2>(g, P, T, a, st); break;
+    case 4: fwd_launch<S16x24>(g, P, T, a, st); break;
+    default: fwd_launch<S16x12>(g, P, T, a, st); break;
   }
 }
 
@@ -1270,8 +1167,8 @@ void launch_adj_stage2d(const Geo& g, const Patches* P, const Tiling& T, const A
     case 1: adj_launch<S16x32>(g, P, T, a, st); break;
     case 2: adj_launch<S16x16>(g, P, T, a, st); break;
     case 3: adj_launch<S24x16>(g, P, T, a, st); break;
-    case 4: adj_launch<S16x16c2>(g, P, T, a, st); break;
-    default: adj_launch<S16x12c2>(g, P, T, a, st); break;
+    case 4: adj_launch<S16x24>(g, P, T, a, st); break;
+    default: adj_launch<S16x12>(g, P, T, a, st); break;
   }
 }
 

@@ -35,12 +35,19 @@ struct Op {
   int nnorm;
 };
 
+// Interior row of the 4th difference D4 of the two-level dissipation and of its transpose
+// (c_0, c_1 = c_-1, c_2 = c_-2)
+constexpr double kD4[3] = {6.0, -4.0, 1.0};
+
 enum OpKind { OP_FIRST = 0, OP_SECOND = 1, OP_DISS = 2, OP_DISS_T = 3, OP_COMPOSITE = 4 };
+// SLOT_DISS2: the whole dissipation along a line as one operator, D4^T D4 with its closure
+// rows, or the composite operator (fused 2-D kernels)
 enum OpSlot { SLOT_FIRST = 0, SLOT_ADJ = 1, SLOT_DISS = 2, SLOT_DISS_T = 3, SLOT_SECOND = 4,
-              kNumSlots = 5 };
+              SLOT_DISS2 = 5, kNumSlots = 6 };
 
 int op_setup(Op* op, int scheme, int kind);     // sbp.cpp
 void op_adjoint(const Op& op, Op* adj);         // sbp.cpp
+void op_product(const Op& second, const Op& first, Op* out);   // sbp.cpp: second * first
 // Host 1-D application along a contiguous line (grid set-up only).
 void op_apply_line(const Op& op, int len, int periodicity, const double* in, double* out);
 
@@ -89,6 +96,14 @@ struct DPatch {
 struct Patches {
   int count;
   DPatch p[kMaxPatches];
+  // what the fused 2-D kernels read of patches and sources in other layouts: bits of the
+  // far-field and sponge patches; per grid point the sponge strengths' sum and the target
+  // state (null without a sponge); per source the factors of its Gaussian along x and y
+  unsigned far_mask, sponge_mask;
+  const double* damp;
+  const double* qtarget;
+  const double* srcx;
+  const double* srcy;
 };
 
 struct Source {

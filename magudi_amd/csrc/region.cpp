@@ -89,6 +89,7 @@ struct mgd_region {
   bool finalized = false;
   mgd::Patches hpatches;
   mgd::DevBuf d_patches, d_sources;
+  mgd::DevBuf d_damp, d_qtarget, d_srcx, d_srcy;   // fused 2-D tables (Patches)
   int ip_cost = -1, ip_act = -1, has_farfield = 0;
   mgd::FinishInfo fin;                   // the forward finishing pass (set at finalize)
   // HBM-resident state
@@ -1946,6 +1947,43 @@ int group_adjoint_pass(mgd_group* G, const double* dts, int nsteps, int K) {
   return MGD_OK;
 }
 
+// The layouts of sponges, far fields and sources that the fused 2-D kernels read (Patches).
+int fused_tables(mgd_region* r) {
+  Patches& H = r->hpatches;
+  std::vector<double> damp;
+  for (int ip = 0; ip < H.count; ++ip) {
+    const DPatch& D = H.p[ip];
+    if (D.type == MGD_PATCH_FAR_FIELD) H.far_mask |= 1u << ip;
+    if (D.type != MGD_PATCH_SPONGE) continue;
+    H.sponge_mask |= 1u << ip;
+    damp.resize((size_t)r->N, 0.0);
+    const HostPatch& P = *r->patches[ip];
+    for (int k = 0; k < P.np; ++k) damp[patch_point(r, P, k)] += P.strength[k];
+  }
+  if (!damp.empty()) {
+    if (upload(r->d_damp, damp) || upload(r->d_qtarget, r->target)) return MGD_ERR_HIP;
+    H.damp = r->d_damp.p;
+    H.qtarget = r->d_qtarget.p;
+  }
+  const size_t ns = r->sources.size();
+  std::vector<double> ax(ns * r->desc.n[0]), ay(ns * r->desc.n[1]);
+  for (size_t s = 0; s < ns; ++s) {
+    const Source& S = r->sources[s];
+    for (int i = 0; i < r->desc.n[0]; ++i) {
+      const double d = r->line[0][i] - S.loc[0];
+      ax[s * r->desc.n[0] + i] = std::exp(-S.gfac * (d * d));
+    }
+    for (int j = 0; j < r->desc.n[1]; ++j) {
+      const double d = r->line[1][j] - S.loc[1];
+      ay[s * r->desc.n[1] + j] = std::exp(-S.gfac * (d * d));
+    }
+  }
+  if (ns && (upload(r->d_srcx, ax) || upload(r->d_srcy, ay))) return MGD_ERR_HIP;
+  H.srcx = r->d_srcx.p;
+  H.srcy = r->d_srcy.p;
+  return MGD_OK;
+}
+
 // normalizeKolmogorovForcing (src/RegionImpl.f90:910-999, called at :1477): the forces of
 // all Kolmogorov patches summed per grid point, and the number of patches covering each
 // point, are integrated with the norm over the union of those patches
@@ -2083,6 +2121,8 @@ int mgd_region_create(const mgd_region_desc* d, const double* coords, mgd_region
   r->ops[SLOT_DISS] = diss;
   r->ops[SLOT_DISS_T] = dissT;
   r->ops[SLOT_SECOND] = second;   // grid%secondDerivative (src/GridImpl.f90:30-31, 557-567)
+  if (d->composite_dissipation) r->ops[SLOT_DISS2] = diss;
+  else op_product(dissT, diss, &r->ops[SLOT_DISS2]);
   // Grid%update for a rectilinear grid: per-direction coordinate derivative and norm weight
   for (int d0 = 0; d0 < 3; ++d0) {
     const int len = r->desc.n[d0];
@@ -2376,6 +2416,8 @@ int mgd_region_finalize(mgd_region* r) {
     if (whole) r->fin.kolmogorov = D.strength;
     else r->fin.simple = 0;
   }
+  if (r->nd == 2 && !r->desc.viscous)
+    if (int rc = fused_tables(r)) return rc;
   if (r->d_patches.alloc(sizeof(Patches) / sizeof(double) + 1)) return MGD_ERR_HIP;
   MGD_HIP(hipMemcpy(r->d_patches.p, &r->hpatches, sizeof(Patches), hipMemcpyHostToDevice));
   if (r->d_sources.alloc((sizeof(Source) * std::max<size_t>(1, r->sources.size())) / sizeof(double) + 1))
