@@ -18,8 +18,8 @@
 // The functional / sensitivity quadrature terms are written per patch point and stage
 // and reduced by a fixed-order tree, so J and the sensitivity are deterministic and
 // independent of the tile shape and of scheduling.
-#include "device.h"
 #include "fused2d.h"
+#include "rows.h"
 
 namespace mgd {
 
@@ -57,21 +57,6 @@ struct Shape {
   // the tile splits into blocks of 8 x 8 points, one wave each (thread_point)
   static constexpr bool kQuads = TX % 8 == 0 && TY % 8 == 0;
 };
-
-// A pointer that comes out of a descriptor in memory (group kernels) is generic to the
-// compiler: flat accesses, which count as LDS and as global ones at once.  This says that it
-// points to global memory.
-template <class T>
-using global_ptr = __attribute__((address_space(1))) T*;
-template <class T>
-__device__ __forceinline__ global_ptr<T> glob(T* p) {
-  return (global_ptr<T>)p;
-}
-
-// The patch tables: no kernel writes them, so they are read through scalar loads, also behind
-// a barrier or a store.
-using ConstPatches = const __attribute__((address_space(4))) Patches;
-using ConstPatch = const __attribute__((address_space(4))) DPatch;
 
 struct TileGeo {
   int x0, y0, sx, sy;   // origin and size of the tile
@@ -158,96 +143,12 @@ __device__ __forceinline__ HaloSlot halo_slot(const Geo& g, const TileGeo& t, in
   return h;
 }
 
-// The dense closure rows (BD x BW) of operator `slot` into LDS, one value per thread and
-// turn: the left end's, then the right end's (row m: the m-th point from that end).
-template <class S, int BD, int BW>
-__device__ __forceinline__ void stage_rows(const Geo& g, int slot, double* tab) {
-  const Op& op = g.ops[slot];
-  for (int e = threadIdx.x; e < 2 * BD * BW; e += S::NT) {
-    const int m = e / BW % BD, c = e % BW;
-    tab[e] = e < BD * BW ? op.b1[m][c] : op.b2[m][c];
-  }
-}
-
-// A closure row on the BW operands f(j, k) of the components j, in the order of the grid
-// index; four columns of LDS reads at a time (more would spill registers).
-template <int BW, class F>
-__device__ __forceinline__ void closure_row(const double* row, F&& f, double* out) {
-#pragma unroll
-  for (int j = 0; j < NV2; ++j) out[j] = 0.0;
-#pragma unroll
-  for (int k = 0; k < BW; ++k) {
-    const double b = row[k];
-#pragma unroll
-    for (int j = 0; j < NV2; ++j) out[j] += b * f(j, k);
-    if (k % 4 == 3) __builtin_amdgcn_sched_barrier(0);
-  }
-}
-
-// Place of index i on a non-periodic direction: m the distance from the nearer end, right
-// which end that is; m is large on a periodic direction.
-struct EdgePlace {
-  int m;
-  bool right;
-};
-__device__ __forceinline__ EdgePlace edge_place(const Dir& dd, int i) {
-  const int r = dd.len - 1 - i;
-  return {dd.periodic ? 1 << 30 : min(i, r), r < i};
-}
-
-__device__ __forceinline__ double skew_sum(const double* p, const double* m, const double* c) {
-  double s = c[1] * (p[0] - m[0]);
-#pragma unroll
-  for (int k = 2; k <= 4; ++k) s += c[k] * (p[k - 1] - m[k - 1]);
-  return s;
-}
-
-// Interior row of D4 (and of D4^T) on the window w[0..4].  The products with 1 and -4 are
-// exact, so the fused form rounds as the plain sum does.
-__device__ __forceinline__ double d4_row(const double* w) {
-  return __fma_rn(kD4[1], w[3] + w[1], w[4] + w[0]) + kD4[0] * w[2];
-}
-
 // Row of the 9-point symmetric operator c_0..c_4 about x, whose coefficients sum to zero:
 // sum_k c_k (x_k - x).
 __device__ __forceinline__ double sym9(double x, const double* p, const double* m, const double* c) {
   double s = c[1] * ((p[0] - x) + (m[0] - x));
 #pragma unroll
   for (int k = 2; k <= 4; ++k) s = __fma_rn(c[k], (p[k - 1] - x) + (m[k - 1] - x), s);
-  return s;
-}
-
-// D4^T (-arc D4 x) of the two-level dissipation at one point from the nine operands about it
-// (the metric is constant along a line of a rectilinear grid): the five intermediates that
-// the point's row needs are formed again by each thread, 35 operations instead of a pass of
-// the intermediates through LDS with two more barriers.
-__device__ __forceinline__ double two_level(const double* w, double marc) {
-  double z[5];
-#pragma unroll
-  for (int k = 0; k < 5; ++k) z[k] = marc * d4_row(w + k);
-  return d4_row(z);
-}
-
-// The same in a tile at a non-periodic end: w holds the nine operands of the window that
-// starts at index clamp(i - 4, 0, len - 9).  The first two rows of D4 repeat the stencil of
-// the third one, summed in the order of the index; D4^T has 5 closure rows of 7 columns.
-__device__ __forceinline__ double two_level_edge(const double* w, double marc, EdgePlace e,
-                                                 const double* rows) {
-  if (e.m >= 5) return two_level(w, marc);
-  double z[5], first = 0.0;
-#pragma unroll
-  for (int k = 0; k < 5; ++k) z[k] = marc * d4_row(w + k);
-#pragma unroll
-  for (int k = 0; k < 5; ++k) first += kD4[k < 2 ? 2 - k : k - 2] * (e.right ? w[k + 4] : w[k]);
-  first = marc * first;
-  const double* b = rows + (e.right ? 35 : 0) + 7 * e.m;
-  double s = 0.0;
-#pragma unroll
-  for (int c = 0; c < 7; ++c) {
-    const double l = c < 2 ? first : z[c < 2 ? 0 : c - 2];
-    const double r = c < 5 ? z[c < 5 ? c : 0] : first;
-    s += b[c] * (e.right ? r : l);
-  }
   return s;
 }
 
@@ -396,10 +297,10 @@ __device__ __forceinline__ void fwd_stage_body(const Geo& g, const Patches* patc
   for (int k = 1; k <= 4; ++k) d1[k] = g.ops[SLOT_FIRST].c[kMaxHW + k];
   const FarAhead far = far_ahead<S, false>(g, P, t, pmask & P->far_mask, qi, ff);
   if (t.bx || t.by) {
-    stage_rows<S, 8, 12>(g, SLOT_FIRST, tab);
+    stage_rows<S::NT, 8, 12>(g, SLOT_FIRST, tab);
     if (g.dissipation) {
-      if (g.composite) stage_rows<S, 8, 12>(g, SLOT_DISS, tab + 192);
-      else stage_rows<S, 5, 7>(g, SLOT_DISS_T, tab + 192);
+      if (g.composite) stage_rows<S::NT, 8, 12>(g, SLOT_DISS, tab + 192);
+      else stage_rows<S::NT, 5, 7>(g, SLOT_DISS_T, tab + 192);
     }
   }
   // stage the operand and the fluxes
@@ -490,7 +391,7 @@ __device__ __forceinline__ void fwd_stage_body(const Geo& g, const Patches* patc
     double dx[NV2], dy[NV2];
     if (t.bx && ex.m < 8) {
       const double* b = sfx + ty * EX + HX + (ex.right ? t.sx - 12 : 0);
-      closure_row<12>(tab + 12 * ex.m + (ex.right ? 96 : 0),
+      closure_row<NV2, 12>(tab + 12 * ex.m + (ex.right ? 96 : 0),
                       [&](int j, int k) { return b[j * TY * EX + k]; }, dx);
     } else {
 #pragma unroll
@@ -502,7 +403,7 @@ __device__ __forceinline__ void fwd_stage_body(const Geo& g, const Patches* patc
     }
     if (t.by && ey.m < 8) {
       const double* b = sfy + (HY + (ey.right ? t.sy - 12 : 0)) * TX + tx;
-      closure_row<12>(tab + 12 * ey.m + (ey.right ? 96 : 0),
+      closure_row<NV2, 12>(tab + 12 * ey.m + (ey.right ? 96 : 0),
                       [&](int j, int k) { return b[(j * EY + k) * TX]; }, dy);
     } else {
 #pragma unroll
@@ -527,7 +428,7 @@ __device__ __forceinline__ void fwd_stage_body(const Geo& g, const Patches* patc
         if (e.m < 8) {
           const double* b = d == 0 ? sq + (ty + HY) * EX + HX + (e.right ? t.sx - 12 : 0)
                                    : sq + (HY + (e.right ? t.sy - 12 : 0)) * EX + tx + HX;
-          closure_row<12>(tab + 192 + 12 * e.m + (e.right ? 96 : 0),
+          closure_row<NV2, 12>(tab + 192 + 12 * e.m + (e.right ? 96 : 0),
                           [&](int j, int k) { return b[j * EY * EX + k * step]; }, dv);
         } else {
 #pragma unroll
@@ -709,8 +610,8 @@ __device__ __forceinline__ void adj_stage_body(const Geo& g, const Patches* patc
   }
   const FarAhead far = far_ahead<S, true>(g, P, t, pmask & P->far_mask, li, ff);
   if (t.bx || t.by) {
-    stage_rows<S, 12, 16>(g, SLOT_ADJ, tab);
-    if (g.dissipation) stage_rows<S, 8, 12>(g, SLOT_DISS2, tab + 384);
+    stage_rows<S::NT, 12, 16>(g, SLOT_ADJ, tab);
+    if (g.dissipation) stage_rows<S::NT, 8, 12>(g, SLOT_DISS2, tab + 384);
   }
   if (mine) {
 #pragma unroll
@@ -761,11 +662,11 @@ __device__ __forceinline__ void adj_stage_body(const Geo& g, const Patches* patc
     const bool cx = t.bx && ex.m < 12, cy = t.by && ey.m < 12;
     double dv[NV2];
     if (cx)
-      closure_row<16>(tab + 16 * ex.m + (ex.right ? 192 : 0),
+      closure_row<NV2, 16>(tab + 16 * ex.m + (ex.right ? 192 : 0),
                       [&](int j, int k) { return bx[j * EY * EX + k - rx]; }, T1[0]);
     if (t.bx && ex.m < 8) {
       if (g.dissipation)
-        closure_row<12>(tab + 384 + 12 * ex.m + (ex.right ? 96 : 0),
+        closure_row<NV2, 12>(tab + 384 + 12 * ex.m + (ex.right ? 96 : 0),
                         [&](int j, int k) { return bx[j * EY * EX + k - qx] - v[j]; }, dv);
     } else {
 #pragma unroll
@@ -780,11 +681,11 @@ __device__ __forceinline__ void adj_stage_body(const Geo& g, const Patches* patc
 #pragma unroll
     for (int l = 0; l < NV2; ++l) w[l] = sx * dv[l];
     if (cy)
-      closure_row<16>(tab + 16 * ey.m + (ey.right ? 192 : 0),
+      closure_row<NV2, 16>(tab + 16 * ey.m + (ey.right ? 192 : 0),
                       [&](int j, int k) { return by[(j * EY + k - ry) * EX]; }, T1[1]);
     if (t.by && ey.m < 8) {
       if (g.dissipation)
-        closure_row<12>(tab + 384 + 12 * ey.m + (ey.right ? 96 : 0),
+        closure_row<NV2, 12>(tab + 384 + 12 * ey.m + (ey.right ? 96 : 0),
                         [&](int j, int k) { return by[(j * EY + k - qy) * EX] - v[j]; }, dv);
     } else {
 #pragma unroll

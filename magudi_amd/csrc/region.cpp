@@ -15,6 +15,7 @@
 #include <vector>
 
 #include "fused2d.h"
+#include "line1d.h"
 #include "kernels.h"
 #include "mgd_internal.h"
 
@@ -658,6 +659,16 @@ bool fused_ok(const mgd_region* r) {
          !overlap;
 }
 
+// The 1-D kernels that run whole time steps (line1d.hip) cover what the fused 2-D kernels
+// cover; a run with solution limits looks at every stage input and takes the generic kernels.
+bool line_ok(const mgd_region* r) {
+  return r->nd == 1 && !r->force_plain && !r->desc.viscous && !r->lim_on && !has_walls(r) &&
+         r->desc.periodicity[0] != MGD_PERIODIC_OVERLAP;
+}
+
+// Whether a run's J and sensitivity are reduced from per-point terms (prepare_quadrature).
+bool point_terms(const mgd_region* r) { return fused_ok(r) || line_ok(r); }
+
 int upload_ints(DevBuf& b, const void* data, size_t bytes) {
   if (b.alloc(bytes / sizeof(double) + 1)) return MGD_ERR_HIP;
   MGD_HIP(hipMemcpy(b.p, data, bytes, hipMemcpyHostToDevice));
@@ -789,6 +800,61 @@ void fused_forward_step(mgd_region* r, double* q0, double* x, double* y, double*
     FwdStage a = fwd_args(r, in, q0, b2, o, i, dt, 4 * s + i - 1, nst, with_j);
     launch_fwd_stage2d(r->geo, dpatches(r), r->tiling, a, st);
     if (with_j) reduce_chunk(r, r->jpart, n_cost(r), nst, 4 * s + i - 1, false);
+  }
+}
+
+// Forward time steps s0 .. s0 + ns - 1 of a 1-D run from the state at `in`, or, with three
+// stages, the inner stages of step s0 alone.  keep(s, i, &a, &b): where the output of stage i
+// of step s goes (a, and for stage 4 also b; null: nowhere).  A launch that leaves no step's
+// state anywhere passes it on through `out` on the last launch and s1, s2 in turn before it
+// (s1 must not be `in`; s2 may be).
+template <class Keep>
+void line_forward(mgd_region* r, const double* in, double* out, double* s1, double* s2, int s0,
+                  int ns, double dt, int nst, bool with_j, Keep&& keep, int stages = 4) {
+  const int na = n_act(r), nsrc = (int)r->sources.size(), nc = n_cost(r);
+  const int most = line_steps(r->geo);
+  for (int s = s0; s < s0 + ns;) {
+    int m = std::min(most, s0 + ns - s);
+    if (with_j) m = std::min(m, r->chunk / 4 - s % (r->chunk / 4));   // one chunk per launch
+    LineForward a;
+    std::memset(&a, 0, sizeof a);
+    a.in = in;
+    a.nstages = stages < 4 ? stages : 4 * m;
+    a.dt = dt;
+    a.na = na;
+    if (r->control.p && na > 0) {
+      a.control = r->control.p + 4L * s * na;
+      a.control_stride = r->ctrl_stride;
+    }
+    a.src = reinterpret_cast<const Source*>(r->d_sources.p);
+    a.nsrc = nsrc;
+    a.src_amp = r->src_amp.p + 4L * s * std::max(nsrc, 1);
+    a.src_inst_stride = r->src_inst_stride;
+    a.ip_cost = r->ip_cost;
+    a.ip_act = r->ip_act;
+    if (with_j && nc > 0) {
+      a.jpartial = r->jpart.p;
+      a.npts = nc;
+      a.nslots = r->chunk;
+      a.slot = 4 * s % r->chunk;
+    }
+    for (int j = 0; j < a.nstages; ++j) {
+      double* b = nullptr;
+      keep(s + j / 4, j % 4 + 1, &a.keep[j], &b);
+      if (j % 4 == 3) a.keep2[j / 4] = b;
+    }
+    const bool last = s + m == s0 + ns;
+    double* next = a.keep[a.nstages - 1];
+    if (last) {
+      a.out = out;
+    } else if (!next) {
+      next = in == s1 ? s2 : s1;
+      a.out = next;
+    }
+    launch_line_forward(r->geo, dpatches(r), a, r->stream);
+    if (with_j) reduce_chunk(r, r->jpart, nc, nst, 4 * (s + m) - 1, false);
+    in = next;
+    s += m;
   }
 }
 
@@ -1326,6 +1392,13 @@ void recompute_step(mgd_region* r, int t, double dt) {
     r->rec_step = t;
     return;
   }
+  if (line_ok(r)) {
+    line_forward(
+        r, r->sstore.p + (long)t * M, nullptr, nullptr, nullptr, t, 1, dt, 4 * r->ck.nsteps, false,
+        [&](int, int i, double** a, double**) { *a = r->window.p + (long)(i - 1) * M; }, 3);
+    r->rec_step = t;
+    return;
+  }
   if (march_stages(r)) {
     // from the stored state straight into the three slots of `window`
     const double* start = r->sstore.p + (long)t * M;
@@ -1359,7 +1432,41 @@ const double* step_stage_state(mgd_region* r, int t, int stage, double dt, bool 
   return r->window.p + (long)(stage - 2) * M;
 }
 
+// The forward pass of a 1-D run: what plain_forward_pass stores, by the kernels that run whole
+// steps.
+int line_forward_pass(mgd_region* r, double dt, int nsteps, int K) {
+  const int nst = 4 * nsteps;
+  const long M = (long)r->ninst * M_of(r);
+  if (r->step_mode) {
+    r->rec_step = -1;
+    launch_copy(M, r->q.p, r->sstore.p, r->stream);
+    line_forward(r, r->sstore.p, nullptr, nullptr, nullptr, 0, nsteps, dt, nst, true,
+                 [&](int s, int i, double** a, double**) {
+                   if (i == 4) *a = s + 1 < nsteps ? r->sstore.p + (long)(s + 1) * M : r->q.p;
+                   else if (s >= r->scache_first)
+                     *a = r->scache.p + ((long)(s - r->scache_first) * 3 + i - 1) * M;
+                 });
+  } else {
+    launch_copy(M, r->q.p, r->snaps.p, r->stream);
+    if (double* cw = cached_window(r, 0)) launch_copy(M, r->q.p, cw, r->stream);
+    line_forward(r, r->snaps.p, r->q.p, r->b1.p, r->b2.p, 0, nsteps, dt, nst, true,
+                 [&](int s, int i, double** a, double** b) {
+                   const int lt = s - s % K, idx = 4 * (s - lt) + i;
+                   if (idx < 4 * K) {
+                     if (double* cw = cached_window(r, lt)) *a = cw + (long)idx * M;
+                   } else {                  // the first state of the next window
+                     *b = r->snaps.p + (long)((s + 1) / K) * M;
+                     if (s + 1 < nsteps) *a = cached_window(r, s + 1);
+                   }
+                 });
+  }
+  if (n_cost(r) > 0)
+    launch_stage_accumulate(r->ssum.p, nst, r->wts.p, r->acc_J.p, r->ninst, 0, r->stream);
+  return MGD_OK;
+}
+
 int plain_forward_pass(mgd_region* r, double dt, int nsteps, int K) {
+  if (line_ok(r)) return line_forward_pass(r, dt, nsteps, K);
   const int nc = n_cost(r);
   const long M = (long)r->ninst * M_of(r);
   if (r->step_mode && march_stages(r)) {
@@ -1454,6 +1561,93 @@ void plain_adjoint_stage(mgd_region* r, double dt, int nsteps, int t, int i, con
     launch_rk_adjoint(M, i, dt, r->lam.p, r->b1a.p, r->b2a.p, r->rhs.p, r->stream);
 }
 
+// Adjoint time steps t1, t1 - 1, .. t0 of a 1-D run from the adjoint state at `lam`, which comes
+// back in the buffer returned (r->lam when t0 is 0).  q(t, i): the forward state of stage i of
+// step t.
+template <class State>
+const double* line_adjoint(mgd_region* r, const double* lam, int t1, int t0, double dt, int nst,
+                           bool want_grad, State&& q) {
+  const int na = n_act(r);
+  const long M = (long)r->ninst * M_of(r);
+  const int most = line_steps(r->geo);
+  while (t1 >= t0) {
+    const int m = std::min({most, t1 - t0 + 1, t1 % (r->chunk / 4) + 1});   // one chunk per launch
+    const int sidx = 4 * t1 + 3;
+    LineAdjoint a;
+    std::memset(&a, 0, sizeof a);
+    double* const out = t1 + 1 == m && lam != r->lam.p ? r->lam.p
+                        : lam == r->b1a.p              ? r->b2a.p
+                                                       : r->b1a.p;
+    a.in = lam;
+    a.out = out;
+    a.nstages = 4 * m;
+    a.t1 = t1;
+    a.dt = dt;
+    for (int j = 0; j < a.nstages; ++j) a.q[j] = q(t1 - j / 4, 4 - j % 4);
+    a.na = na;
+    a.ip_act = r->ip_act;
+    a.ip_cost = r->ip_cost;
+    if (na > 0) {
+      if (want_grad) {
+        a.grad = r->grad.p + (long)sidx * na;
+        a.grad_stride = (long)nst * na;
+      }
+      a.spartial = r->spart.p;
+      a.npts = na;
+      a.nslots = r->chunk;
+      a.slot = sidx % r->chunk;
+    }
+    launch_line_adjoint(r->geo, dpatches(r), a, r->stream);
+    t1 -= m;
+    reduce_chunk(r, r->spart, na, nst, 4 * (t1 + 1), true);
+    lam = out;
+  }
+  if (t0 == 0 && lam != r->lam.p) {
+    launch_copy(M, lam, r->lam.p, r->stream);
+    lam = r->lam.p;
+  }
+  return lam;
+}
+
+// The adjoint pass of a 1-D run after its terminal condition, over the states that
+// line_forward_pass stored; the windows and steps that it did not keep are computed again.
+int line_adjoint_pass(mgd_region* r, double dt, int nsteps, int K, bool want_grad) {
+  const int nst = 4 * nsteps;
+  const long M = (long)r->ninst * M_of(r);
+  const double* lam = r->lam.p;
+  if (r->step_mode) {
+    if (nsteps > r->scache_first)
+      lam = line_adjoint(r, lam, nsteps - 1, r->scache_first, dt, nst, want_grad,
+                         [&](int t, int i) { return step_stage_state(r, t, i, dt, false); });
+    for (int t = r->scache_first - 1; t >= 0; --t) {
+      recompute_step(r, t, dt);
+      lam = line_adjoint(r, lam, t, t, dt, nst, want_grad,
+                         [&](int s, int i) { return step_stage_state(r, s, i, dt, false); });
+    }
+    r->rec_step = -1;
+  } else {
+    for (int lt = (nsteps - 1) / K * K; lt >= 0; lt -= K) {
+      const int end = std::min(nsteps, lt + K);
+      const double* W = cached_window(r, lt);
+      if (!W) {
+        const double* snap = r->snaps.p + (long)(lt / K) * M;
+        launch_copy(M, snap, r->window.p, r->stream);
+        line_forward(r, snap, nullptr, nullptr, nullptr, lt, end - lt, dt, nst, false,
+                     [&](int s, int i, double** a, double**) {
+                       const int idx = 4 * (s - lt) + i;
+                       if (idx < 4 * K) *a = r->window.p + (long)idx * M;
+                     });
+        W = r->window.p;
+      }
+      lam = line_adjoint(r, lam, end - 1, lt, dt, nst, want_grad,
+                         [&](int t, int i) { return W + (4L * (t - lt) + i - 1) * M; });
+    }
+  }
+  if (n_act(r) > 0)
+    launch_stage_accumulate(r->ssum.p, nst, r->wts.p, r->acc_S.p, r->ninst, 1, r->stream);
+  return MGD_OK;
+}
+
 int plain_adjoint_pass(mgd_region* r, double dt, int nsteps, int K, bool terminal, bool want_grad) {
   const int nc = n_cost(r);
   const long M = (long)r->ninst * M_of(r);
@@ -1463,6 +1657,7 @@ int plain_adjoint_pass(mgd_region* r, double dt, int nsteps, int K, bool termina
     launch_adj_forcing(r->geo, dpatch(r, r->ip_cost), nc, r->qT.p, r->aforce.p, 0, r->stream);
     launch_adj_terminal(r->geo, dpatch(r, r->ip_cost), nc, r->aforce.p, -dt / 6.0, r->lam.p, r->stream);
   }
+  if (line_ok(r)) return nsteps > 0 ? line_adjoint_pass(r, dt, nsteps, K, want_grad) : MGD_OK;
   if (r->step_mode) {
     // every step's inner stage states are recomputed in this pass (a captured pass replays
     // the recompute too), the held ones read from the step cache
@@ -1587,7 +1782,7 @@ int prepare_forward_ck(mgd_region* r, double t0, double dt, int nsteps, int K, c
       if (int rc = plan_plain_storage(r, nsteps, K, M)) return rc;
     }
   }
-  if (fused_ok(r)) {
+  if (point_terms(r)) {
     if (int rc = prepare_quadrature(r, nst, dt)) return rc;
   }
   return MGD_OK;
@@ -1617,8 +1812,10 @@ int prepare_adjoint_ck(mgd_region* r, bool inputs_fresh = false) {
     if (int rc = upload_run_inputs(r)) return rc;
   }
   if (na > 0 && r->grad.alloc((size_t)r->ninst * nst * na)) return MGD_ERR_HIP;
-  if (fused_ok(r)) {
+  if (point_terms(r)) {
     if (int rc = prepare_quadrature(r, nst, r->ck.dt)) return rc;
+  }
+  if (fused_ok(r)) {
     if (r->ly.alloc(M) || r->l0.alloc(M) ||
         r->window2.alloc((size_t)(r->step_mode ? 3 : 4 * r->ck.K) * M) || r->b2r.alloc(M) ||
         r->qsr.alloc(M))
@@ -1649,6 +1846,16 @@ int enqueue_forward_run(mgd_region* r, double dt, int nsteps) {
     if (n_cost(r) > 0)
       launch_stage_accumulate(r->ssum.p, nst, r->wts.p, r->acc_J.p, r->ninst, 0, r->stream);
     r->checking = false;
+    return MGD_OK;
+  }
+  if (line_ok(r)) {
+    r->checking = false;
+    const long M = (long)r->ninst * M_of(r);
+    launch_copy(M, r->q.p, r->b1.p, r->stream);
+    line_forward(r, r->b1.p, r->q.p, r->b2.p, r->b1.p, 0, nsteps, dt, nst, true,
+                 [](int, int, double**, double**) {});
+    if (n_cost(r) > 0 && nsteps > 0)
+      launch_stage_accumulate(r->ssum.p, nst, r->wts.p, r->acc_J.p, r->ninst, 0, r->stream);
     return MGD_OK;
   }
   for (int s = 0; s < nsteps; ++s)
@@ -1686,7 +1893,7 @@ int limits_outcome(mgd_region* r, double* J, double* sensitivity) {
 // (control, source amplitudes, states) live in those buffers and are re-uploaded before
 // each replay.  Captured work holds kernels, copies, fills and event waits only.
 std::vector<uintptr_t> graph_key(mgd_region* r, int kind, std::initializer_list<uintptr_t> extra) {
-  std::vector<uintptr_t> k = {(uintptr_t)kind, (uintptr_t)r->tiling.shape, (uintptr_t)fused_ok(r),
+  std::vector<uintptr_t> k = {(uintptr_t)kind, (uintptr_t)r->tiling.shape, (uintptr_t)fused_ok(r), (uintptr_t)line_ok(r),
                               (uintptr_t)r->ctrl_stride, (uintptr_t)r->src_inst_stride,
                               (uintptr_t)r->chunk, (uintptr_t)r->ck.nsteps, (uintptr_t)r->ck.K,
                               (uintptr_t)r->resident, (uintptr_t)r->dual};
@@ -2782,7 +2989,7 @@ int mgd_run_forward(mgd_region* r, double t0, double dt, int nsteps, const doubl
   std::vector<double> amp;
   run_source_table(r, t0, dt, std::max(nsteps, 1), amp);
   if (upload(r->src_amp, amp)) return MGD_ERR_HIP;
-  if (fused_ok(r))
+  if (point_terms(r))
     if (int rc = prepare_quadrature(r, std::max(nst, 1), dt)) return rc;
   uint64_t dtb;
   std::memcpy(&dtb, &dt, sizeof dtb);
