@@ -302,8 +302,8 @@ int mgd_last_timings(mgd_region* r, double* out, int* launches);
 /* Region options.  MGD_OPT_FORCE_PLAIN = 1 runs the generic per-operator kernels even
  * where the fused 2-D stage kernels apply (comparison and testing).
  * MGD_OPT_TILE_SHAPE selects the tile of the fused 2-D kernels: -1 (default) autotune at
- * the first run, 0: 32 x 16, 1: 16 x 32, 2: 16 x 16, 3: 24 x 16, 4: 16 x 24, 5: 16 x 12
- * points.  No result depends on the tile shape.
+ * the first run, 0: 32 x 16, 1: 16 x 32, 2: 16 x 16, 3: 24 x 16, 5: 16 x 12 points with one
+ * thread per point, 4: 16 x 16 points with two.  No result depends on the tile shape.
  * MGD_OPT_RESIDENT_STATES (fused 2-D path): 1 keeps every RK stage state of a
  * checkpointed forward run in device memory ((4 nsteps + 1) states, e.g. 19.8 GB for
  * 401^2 x 960 steps) so that the adjoint pass recomputes nothing; 0: the step store

@@ -7,21 +7,39 @@
 namespace mgd {
 
 // Tile shapes of the fused kernels (points along x, y): 0: 32 x 16, 1: 16 x 32,
-// 2: 16 x 16, 3: 24 x 16, 4: 16 x 24, 5: 16 x 12; one thread per point.
+// 2: 16 x 16, 3: 24 x 16, one thread per point; 4: 16 x 16, two threads per point (one for
+// each direction); 5: 16 x 12, one.
 constexpr int kNumTileShapes = 6;
 constexpr int kNumXcd = 8;   // XCDs of an MI355X; work-groups are dealt to them round-robin
+
+// The far-field points of one patch in one tile, for the terms formed ahead: w x h points from
+// (i0, j0), their A+ blocks and target states (rows of the patch ls points apart); ip -1: none.
+struct TileFar {
+  int ip, i0, j0, w, h, ls;
+  double sigma_inv;
+  const double* aplus;
+  const double* target;
+};
+
+// What a tile holds: the patches that intersect it, and two of its far fields.
+struct TileInfo {
+  unsigned pmask, pad;
+  TileFar far[2];
+};
 
 // Tile partition of a 2-D grid (device view): nbx x nby tiles of at most TX x TY points
 // from a balanced partition of each direction whose larger tiles sit at both ends --
 // along x, tile b holds qx points, plus one when b < lx or b >= nbx - rx, and starts at
-// b qx + min(b, lx) + max(0, b - (nbx - rx)) (likewise along y) -- and pmask: patches
-// per tile (tile index bx + nbx * by).  Launch block k works on tile
+// b qx + min(b, lx) + max(0, b - (nbx - rx)) (likewise along y) -- and info: the tiles'
+// contents (tile index bx + nbx * by).  Launch block k works on tile
 // (k % kNumXcd) band + k / kNumXcd, or on none when that is beyond the last tile.
 struct Tiling {
   int shape;
   int nbx, nby, nblk, band;
   int qx, lx, rx, qy, ly, ry;
-  const unsigned* pmask;
+  unsigned inv_nbx;              // floor((2^32 - 1) / nbx)
+  const TileInfo* info;
+  StageTables tables;
 };
 
 struct HostTiling {
@@ -29,7 +47,7 @@ struct HostTiling {
   int nbx = 0, nby = 0, nblk = 0, band = 0;
   int qx = 0, lx = 0, rx = 0, qy = 0, ly = 0, ry = 0;
   std::vector<int> org, size;          // tile origins / sizes: x tiles, then y tiles
-  std::vector<unsigned> pmask;
+  std::vector<TileInfo> info;
   std::vector<int> tile_of_block;      // launch block -> tile, or -1
 };
 

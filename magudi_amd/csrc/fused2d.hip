@@ -29,25 +29,28 @@ constexpr int kMinEdgeTile = 12;    // closure depth of the adjoint 4-8 operator
 constexpr int kRedThreads = 256;    // block size of the reduction kernels
 constexpr int kFarPoints = 32;      // far-field points of one patch that a tile forms ahead
 
-// Tile shape: TX x TY points, one thread per point.  A thread beyond a partial tile loads and
-// stages clamped points and stores nothing.  LDS (doubles): the staged operand q[4][EY][EX];
-// forward, the contravariant fluxes of the tile rows (x) and columns (y); the boundary closure
-// rows of an edge tile; the far-field terms.
-template <int TX_, int TY_>
+// Tile shape: TX x TY points.  D = 1: one thread per point.  D = 2: two, one group of threads
+// for each direction -- half the chain of a thread, for launches that leave the chip idle: the
+// first group stages the points and does the x lines and the end of the stage, the second the
+// halo and the y lines, whose sums it hands over through LDS.  A thread beyond a partial tile
+// loads and stages clamped points and stores nothing.  LDS (doubles): the staged operand
+// q[4][EY][EX]; forward, the contravariant fluxes of the tile rows (x) and columns (y); the
+// boundary closure rows of an edge tile; the far-field terms; the sums handed over.
+template <int TX_, int TY_, int D_>
 struct Shape {
-  static constexpr int TX = TX_, TY = TY_, NT = TX * TY;
-  static_assert(NT % 64 == 0, "whole waves");
+  static constexpr int TX = TX_, TY = TY_, D = D_, NP = TX * TY, NT = NP * D;
+  static_assert(NP % 64 == 0, "whole waves");
   static constexpr int EX = TX + 2 * HX, EY = TY + 2 * HY;
   // halo points (the corners are never read): x-halo columns, then y-halo rows
   static constexpr int kHalo = 2 * HX * TY + 2 * HY * TX;
-  static constexpr int kHaloIters = (kHalo + NT - 1) / NT;
+  static constexpr int kHaloIters = (kHalo + NP - 1) / NP;
   static constexpr int SQ = NV2 * EY * EX, SFX = NV2 * TY * EX, SFY = NV2 * EY * TX;
-  static constexpr int kFar = 2 * 4 * kFarPoints;
+  static constexpr int kFar = 2 * 4 * kFarPoints, kSums = D == 2 ? 2 * NV2 * NP : 0;
   // closure rows of both ends: first derivative 8 x 12 and composite 8 x 12 (or dissipation
   // transpose 5 x 7); adjoint derivative 12 x 16 and dissipation 8 x 12
   static constexpr int kTabF = 2 * 96 + 2 * 96, kTabA = 2 * 192 + 2 * 96;
-  static constexpr int kFwdLds = SQ + SFX + SFY + kTabF + kFar;
-  static constexpr int kAdjLds = SQ + kTabA + kFar;
+  static constexpr int kFwdLds = SQ + SFX + SFY + kTabF + kFar + kSums;
+  static constexpr int kAdjLds = SQ + kTabA + kFar + kSums;
   static constexpr int kDualLds = kFwdLds > kAdjLds ? kFwdLds : kAdjLds;
   // waves per SIMD that the LDS use allows (160 KiB per CU), the register budget: at most 4
   static constexpr int waves(int lds) {
@@ -56,6 +59,8 @@ struct Shape {
   }
   // the tile splits into blocks of 8 x 8 points, one wave each (thread_point)
   static constexpr bool kQuads = TX % 8 == 0 && TY % 8 == 0;
+  // components whose LDS reads go out together, as the register budget allows
+  static constexpr int kBatchF = waves(kFwdLds) <= 3 ? 2 : 1, kBatchA = D;
 };
 
 struct TileGeo {
@@ -71,7 +76,10 @@ __device__ __forceinline__ int block_tile(const Tiling& T, int b) {
 }
 
 __device__ __forceinline__ TileGeo tile_geo(const Geo& g, const Tiling& T, int tile) {
-  const int bx = tile % T.nbx, by = tile / T.nbx;
+  // by = tile / nbx: the product is that or one less
+  int by = (int)__umulhi((unsigned)tile, T.inv_nbx);
+  if (tile - by * T.nbx >= T.nbx) ++by;
+  const int bx = tile - by * T.nbx;
   TileGeo t;
   t.x0 = bx * T.qx + min(bx, T.lx) + max(0, bx - (T.nbx - T.rx));
   t.sx = T.qx + (bx < T.lx || bx >= T.nbx - T.rx ? 1 : 0);
@@ -89,7 +97,7 @@ __device__ __forceinline__ TileGeo tile_geo(const Geo& g, const Tiling& T, int t
 // start from its left.  False: the thread has no point of its own.
 template <class S>
 __device__ __forceinline__ bool thread_point(const TileGeo& t, int* tx, int* ty) {
-  const int e = threadIdx.x;
+  const int e = threadIdx.x % S::NP;
   if (S::kQuads && t.bx) {
     const int l = e & 63, w = e >> 6;
     constexpr int QX = S::TX / 8;
@@ -117,7 +125,7 @@ struct HaloSlot {
 };
 template <class S>
 __device__ __forceinline__ HaloSlot halo_slot(const Geo& g, const TileGeo& t, int it) {
-  const int e = threadIdx.x + it * S::NT;
+  const int e = threadIdx.x % S::NP + it * S::NP;
   HaloSlot h;
   bool in;
   if (e < 2 * HX * S::TY) {
@@ -150,6 +158,132 @@ __device__ __forceinline__ double sym9(double x, const double* p, const double* 
 #pragma unroll
   for (int k = 2; k <= 4; ++k) s = __fma_rn(c[k], (p[k - 1] - x) + (m[k - 1] - x), s);
   return s;
+}
+
+// The staged line through a point: c the point (components CS apart, neighbours STEP), pos its
+// place in the tile of `size` points along the line, edge whether the tile is at an end of the
+// line, e the point's place there.
+struct StagedLine {
+  const double* c;
+  int pos, size;
+  bool edge;
+  EdgePlace e;
+};
+
+// Skew derivative with closure rows BD x BW (tab) and interior coefficients cf on the line.
+template <int STEP, int CS, int NB>
+__device__ __forceinline__ void line_derivative(const StagedLine& t, const double* tab,
+                                                const double* cf, double* out) {
+  if (t.edge && t.e.m < 8) {
+    const double* b = t.c + ((t.e.right ? t.size - 12 : 0) - t.pos) * STEP;
+    closure_row<NV2, 12>(tab + 12 * t.e.m + (t.e.right ? 96 : 0),
+                         [&](int l, int k) { return b[l * CS + k * STEP]; }, out);
+    return;
+  }
+#pragma unroll
+  for (int l0 = 0; l0 < NV2; l0 += NB) {
+    double p[NB][4], m[NB][4];
+#pragma unroll
+    for (int l = 0; l < NB; ++l)
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        p[l][k] = t.c[(l0 + l) * CS + (k + 1) * STEP];
+        m[l][k] = t.c[(l0 + l) * CS - (k + 1) * STEP];
+      }
+    __builtin_amdgcn_sched_barrier(0);   // one batch of LDS reads, one wait
+#pragma unroll
+    for (int l = 0; l < NB; ++l) out[l0 + l] = skew_sum(p[l], m[l], cf);
+  }
+}
+
+// H^-1 times the dissipation of the operand on the line (-arc: marc).
+template <int STEP, int CS, int NB>
+__device__ __forceinline__ void line_dissipation(const Geo& g, const StagedLine& t, double marc,
+                                                 double hw, const double* tab, double* out) {
+  if (g.composite) {
+    if (t.e.m < 8) {
+      const double* b = t.c + ((t.e.right ? t.size - 12 : 0) - t.pos) * STEP;
+      closure_row<NV2, 12>(tab + 12 * t.e.m + (t.e.right ? 96 : 0),
+                           [&](int l, int k) { return b[l * CS + k * STEP]; }, out);
+      return;
+    }
+#pragma unroll
+    for (int l = 0; l < NV2; ++l) {
+      const double* x = t.c + l * CS;
+      double s = 0.0;
+#pragma unroll
+      for (int k = 1; k <= 4; ++k)
+        s += g.ops[SLOT_DISS].c[kMaxHW + k] * (x[k * STEP] + x[-k * STEP]);
+      out[l] = s + g.ops[SLOT_DISS].c[kMaxHW] * x[0];
+    }
+    return;
+  }
+  // the window of nine operands, moved inside the domain at its ends
+  const int m = t.e.m;
+  const int move = t.edge && m < 4 ? (t.e.right ? m - 4 : 4 - m) : 0;
+  const double* b = t.c + (move - 4) * STEP;
+  // a point's closure weights: held, or read again for each component where registers are short
+  double cw[7];
+  if (NB > 1 && t.edge) closure_weights(tab, t.e, cw);
+  const double* rows = tab + (t.e.right ? 35 : 0) + 7 * min(t.e.m, 4);
+#pragma unroll
+  for (int l0 = 0; l0 < NV2; l0 += NB) {
+    double w[NB][9];
+#pragma unroll
+    for (int l = 0; l < NB; ++l)
+#pragma unroll
+      for (int k = 0; k < 9; ++k) w[l][k] = b[(l0 + l) * CS + k * STEP];
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int l = 0; l < NB; ++l) {
+      if (!t.edge) {
+        out[l0 + l] = two_level(w[l], marc);
+      } else {
+        const double v = two_level_edge(w[l], marc, t.e, NB > 1 ? cw : rows);
+        out[l0 + l] = hw != 1.0 ? v / hw : v;   // 1 away from the first / last boundary rows
+      }
+    }
+  }
+}
+
+// D+ of the staged adjoint state (T) and the sum of its 9-point dissipation (w) on the line; v:
+// the state at the point.
+template <int STEP, int CS, int NB>
+__device__ __forceinline__ void line_adjoint(const Geo& g, const StagedLine& t, const double* v,
+                                             const double* tab, const double* cf, const double* ds,
+                                             double* T, double* w) {
+  const bool closure = t.edge && t.e.m < 12;
+  // the last (first) of the 16 and 12 staged values that the closure rows of an end reach
+  const double* b = t.c + ((t.e.right ? t.size - 1 : 0) - t.pos) * STEP;
+  if (closure) {
+    const double* b16 = b - (t.e.right ? 15 * STEP : 0);
+    closure_row<NV2, 16>(tab + 16 * t.e.m + (t.e.right ? 192 : 0),
+                         [&](int l, int k) { return b16[l * CS + k * STEP]; }, T);
+  }
+  if (t.edge && t.e.m < 8) {
+    if (!g.dissipation) return;
+    const double* b12 = b - (t.e.right ? 11 * STEP : 0);
+    closure_row<NV2, 12>(tab + 384 + 12 * t.e.m + (t.e.right ? 96 : 0),
+                         [&](int l, int k) { return b12[l * CS + k * STEP] - v[l]; }, w);
+    return;
+  }
+#pragma unroll
+  for (int l0 = 0; l0 < NV2; l0 += NB) {
+    double p[NB][4], m[NB][4];
+#pragma unroll
+    for (int l = 0; l < NB; ++l)
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        p[l][k] = t.c[(l0 + l) * CS + (k + 1) * STEP];
+        m[l][k] = t.c[(l0 + l) * CS - (k + 1) * STEP];
+      }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int l = 0; l < NB; ++l) {
+      if (!closure) T[l0 + l] = skew_sum(p[l], m[l], cf);
+      w[l0 + l] = sym9(v[l0 + l], p[l], m[l], ds);
+    }
+  }
 }
 
 // Scale of the one-level (9-point) dissipation sum of the adjoint stage along a direction:
@@ -188,92 +322,88 @@ __device__ __forceinline__ bool in_patch(ConstPatch& pt, int i, int j) {
 }
 
 // The far-field terms of a tile formed ahead of the stencil work, while its operand loads are
-// in flight: of the first two far-field patches in the tile with at most kFarPoints of its
-// points, thread 4 k + i forms component i of point k -- sum_c A+[c][i] (q_c - qt_c)
-// forward, sum_c A+[i][c] lambda_c adjoint -- into LDS, where the point's thread finds it
-// (a chain of loads per patch at the end of the kernel otherwise, on the slowest tiles).
-struct FarAhead {
-  int ip[2];       // patch, or -1
-  int i0[2], j0[2], w[2];
-};
+// in flight (a chain of loads per patch at the end of the kernel otherwise, on the slowest
+// tiles): of two far fields with at most kFarPoints points in the tile, thread 4 k + i of their
+// half of the threads forms component i of point k -- sum_c A+[c][i] (q_c - qt_c) forward,
+// sum_c A+[i][c] lambda_c adjoint -- into LDS, where the point's thread finds it.
+using ConstTileInfo = const __attribute__((address_space(4))) TileInfo;
 template <class S, bool ADJ>
-__device__ __forceinline__ FarAhead far_ahead(const Geo& g, ConstPatches* P,
-                                              const TileGeo& t, unsigned m, global_ptr<const double> x,
-                                              double* ff) {
-  FarAhead f;
+__device__ __forceinline__ void far_ahead(const Geo& g, ConstTileInfo* I,
+                                          global_ptr<const double> x, double* ff) {
 #pragma unroll
   for (int s = 0; s < 2; ++s) {
-    f.ip[s] = -1;
-    f.i0[s] = f.j0[s] = f.w[s] = 0;
-    if (!m) continue;
-    const int ip = __ffs(m) - 1;
-    m &= m - 1;
-    ConstPatch& pt = P->p[ip];
-    const int i0 = max(pt.lo[0], t.x0), i1 = min(pt.hi[0], t.x0 + t.sx - 1);
-    const int j0 = max(pt.lo[1], t.y0), j1 = min(pt.hi[1], t.y0 + t.sy - 1);
-    const int w = i1 - i0 + 1, n = w * (j1 - j0 + 1);
-    if (n <= 0 || n > kFarPoints) continue;
-    f.ip[s] = ip;
-    f.i0[s] = i0;
-    f.j0[s] = j0;
-    f.w[s] = w;
-    for (int e = threadIdx.x; e < 4 * n; e += S::NT) {
-      const int k = e >> 2, i = e & 3;
-      const int gi = i0 + k % w, gj = j0 + k / w;
-      const long p = gi + (long)g.n[0] * gj;
-      const int kp = (gi - pt.lo[0]) + pt.ls[0] * (gj - pt.lo[1]);
-      const global_ptr<const double> A = glob(pt.aplus) + (long)kp * 16;
-      double v = 0.0;
-      if (ADJ) {
+    if (I->far[s].ip < 0) continue;
+    const int w = I->far[s].w, h = I->far[s].h, e = (int)threadIdx.x - (S::NT >= 8 * kFarPoints ? 4 * kFarPoints * s : 0);
+    if (e < 0 || e >= 4 * w * h) continue;
+    const int k = e >> 2, i = e & 3;
+    const int dx = w == 1 ? 0 : h == 1 ? k : k % w, dy = w == 1 ? k : h == 1 ? 0 : k / w;
+    const long p = (I->far[s].i0 + dx) + (long)g.n[0] * (I->far[s].j0 + dy);
+    const long kp = dx + (long)I->far[s].ls * dy;
+    const global_ptr<const double> A = glob(I->far[s].aplus) + kp * 16;
+    double v = 0.0;
+    if (ADJ) {
 #pragma unroll
-        for (int c = 0; c < NV2; ++c) v += A[i * 4 + c] * x[c * g.N + p];
-      } else {
-        const global_ptr<const double> qt = glob(pt.aplus) + (long)pt.np * 16 + (long)kp * 4;
+      for (int c = 0; c < NV2; ++c) v += A[i * 4 + c] * x[c * g.N + p];
+    } else {
+      const global_ptr<const double> qt = glob(I->far[s].target) + kp * 4;
 #pragma unroll
-        for (int c = 0; c < NV2; ++c) v += A[c * 4 + i] * (x[c * g.N + p] - qt[c]);
-      }
-      ff[s * 4 * kFarPoints + e] = v;
+      for (int c = 0; c < NV2; ++c) v += A[c * 4 + i] * (x[c * g.N + p] - qt[c]);
     }
+    ff[s * 4 * kFarPoints + e] = v;
   }
-  return f;
 }
 
-// The terms of patch ip (one of those formed ahead) at grid point (gi, gj).
-__device__ __forceinline__ void far_formed(const FarAhead& f, int ip, const double* ff, int gi,
-                                           int gj, double* out) {
-  const int s = ip == f.ip[0] ? 0 : 1;
-  const double* x = ff + s * 4 * kFarPoints + 4 * ((gi - f.i0[s]) + f.w[s] * (gj - f.j0[s]));
+// Far field ip of the tile at grid point (gi, gj): its term f and strength where the point is
+// in the patch and the term was formed ahead (1), 0 where the point is not, -1 if not formed.
+__device__ __forceinline__ int far_formed(ConstTileInfo* I, int ip, const double* ff, int gi, int gj,
+                                          double* f, double* sigma_inv) {
+  const int s = ip == I->far[0].ip ? 0 : ip == I->far[1].ip ? 1 : -1;
+  if (s < 0) return -1;
+  const int kx = gi - I->far[s].i0, ky = gj - I->far[s].j0, w = I->far[s].w;
+  if ((unsigned)kx >= (unsigned)w || (unsigned)ky >= (unsigned)I->far[s].h) return 0;
+  const double* x = ff + s * 4 * kFarPoints + 4 * (kx + w * ky);
 #pragma unroll
-  for (int l = 0; l < NV2; ++l) out[l] = x[l];
+  for (int l = 0; l < NV2; ++l) f[l] = x[l];
+  *sigma_inv = I->far[s].sigma_inv;
+  return 1;
 }
 
 // -------------------------------------------------------------------------- forward
 // What bounds the stage: on small grids (a few blocks per CU) the chain load - LDS - stencils -
-// store of one block, so there is one barrier, and every operand is asked for before it; on
-// batches the 160 bytes per point and stage (0.09 ms for 20 instances of 401 x 401 at the rate
+// store of one block, most of all of a corner tile's (101^2, cycles: 1800 to the first load, 3000
+// to the barrier, 7300 of stencils against 4400 in an interior tile, 2900 to the end); so there
+// is one barrier, every operand is asked for before it, and what a tile holds of patches comes
+// with one record.  On batches the 160 bytes per point and stage (0.09 ms for 20 instances of 401 x 401 at the rate
 // of a copy) beside 0.07 ms of FP64 issue and 0.06 ms of LDS reads, which overlap in part.
 // Plain stores: the rows of a tile end inside cache lines that the neighbour completes, and
 // non-temporal stores sent them to memory in pieces (8 x 273^2: 39.3 against 36.9 us).
 // Against the stage with the dissipation's intermediates in LDS (three barriers, every patch
-// read at the end): 401^2 15.2 -> 13.3 us, 201^2 10.8 -> 10.1, 20 x 401^2 191 -> 173.
+// read at the end): 401^2 15.2 -> 12.6 us, 201^2 10.8 -> 8.7, 20 x 401^2 191 -> 162.  One / two
+// threads per point: 101^2 9.0 / 8.5 us, 257^2 10.0 / 9.9, 401^2 12.6 / 15.4.
 // One forward stage on tile block `blk` of instance `inst` (uniform per work-group).
 template <class S>
 __device__ __forceinline__ void fwd_stage_body(const Geo& g, const Patches* patches,
                                                const Tiling& T, const FwdStage& a, int blk,
                                                long inst, double* lds) {
   constexpr int TX = S::TX, TY = S::TY, EX = S::EX, EY = S::EY, HS = S::kHaloIters;
+  constexpr int NB = S::kBatchF;
+  // D = 2: the group of threads, uniform per wave
+  const int grp = S::D == 2 ? __builtin_amdgcn_readfirstlane(threadIdx.x / S::NP) : 0;
+  const bool lead = grp == 0, halo = S::D == 1 || grp == 1;
   double* sq = lds;
   double* sfx = sq + S::SQ;
   double* sfy = sfx + S::SFX;
   double* tab = sfy + S::SFY;
   double* ff = tab + S::kTabF;
+  double* sums = ff + S::kFar + threadIdx.x % S::NP;
   const int tile = block_tile(T, blk);
   ConstPatches* P = (ConstPatches*)patches;
   if (tile < 0) return;   // block beyond the tiles of its XCD (uniform per block)
   const TileGeo t = tile_geo(g, T, tile);
   const long NVN = (long)NV2 * g.N;
   const global_ptr<const double> qi = glob(a.qin) + inst * NVN;
-  const unsigned pmask = glob(T.pmask)[tile];
+  ConstTileInfo* I = (ConstTileInfo*)T.info + tile;
+  const unsigned pmask = I->pmask;
   int tx, ty;
   const bool mine = thread_point<S>(t, &tx, &ty);
   const int gi = t.x0 + (mine ? tx : 0), gj = t.y0 + (mine ? ty : 0);
@@ -283,19 +413,22 @@ __device__ __forceinline__ void fwd_stage_body(const Geo& g, const Patches* patc
   double v[NV2], hv[HS][NV2], hm[HS];
 #pragma unroll
   for (int l = 0; l < NV2; ++l) v[l] = qi[l * g.N + p];
+  if (halo) {
 #pragma unroll
-  for (int it = 0; it < HS; ++it) {
-    const HaloSlot h = halo_slot<S>(g, t, it);
-    const long pp = h.gi + (long)g.n[0] * h.gj;
+    for (int it = 0; it < HS; ++it) {
+      const HaloSlot h = halo_slot<S>(g, t, it);
+      const long pp = h.gi + (long)g.n[0] * h.gj;
 #pragma unroll
-    for (int l = 0; l < NV2; ++l) hv[it][l] = qi[l * g.N + pp];
-    hm[it] = h.kind == 2 ? glob(g.h[0])[h.gi] : glob(g.h[1])[h.gj];   // metric<2> of the halo's direction
+      for (int l = 0; l < NV2; ++l) hv[it][l] = qi[l * g.N + pp];
+      // metric<2> of the halo's direction
+      hm[it] = h.kind == 2 ? glob(g.h[0])[h.gi] : glob(g.h[1])[h.gj];
+    }
   }
   const double h0 = glob(g.h[0])[gi], hw0 = glob(g.hw[0])[gi], h1 = glob(g.h[1])[gj], hw1 = glob(g.hw[1])[gj];
   double d1[5];                     // interior coefficients
 #pragma unroll
   for (int k = 1; k <= 4; ++k) d1[k] = g.ops[SLOT_FIRST].c[kMaxHW + k];
-  const FarAhead far = far_ahead<S, false>(g, P, t, pmask & P->far_mask, qi, ff);
+  far_ahead<S, false>(g, I, qi, ff);
   if (t.bx || t.by) {
     stage_rows<S::NT, 8, 12>(g, SLOT_FIRST, tab);
     if (g.dissipation) {
@@ -304,7 +437,7 @@ __device__ __forceinline__ void fwd_stage_body(const Geo& g, const Patches* patc
     }
   }
   // stage the operand and the fluxes
-  if (mine) {
+  if (mine && lead) {
     const Prim<2> s = prim<2>(v, g.gamma);
     double f0[NV2], f1[NV2];
     inviscid_flux<2>(v, s, 0, f0);
@@ -316,169 +449,108 @@ __device__ __forceinline__ void fwd_stage_body(const Geo& g, const Patches* patc
       sfy[(l * EY + ty + HY) * TX + tx] = h0 * f1[l];
     }
   }
+  if (halo) {
 #pragma unroll
-  for (int it = 0; it < HS; ++it) {
-    const HaloSlot h = halo_slot<S>(g, t, it);
-    if (h.kind == 0) continue;
-    const Prim<2> s = prim<2>(hv[it], g.gamma);
-    double f[NV2];
-    if (h.kind == 1) {
-      inviscid_flux<2>(hv[it], s, 0, f);
+    for (int it = 0; it < HS; ++it) {
+      const HaloSlot h = halo_slot<S>(g, t, it);
+      if (h.kind == 0) continue;
+      const Prim<2> s = prim<2>(hv[it], g.gamma);
+      double f[NV2];
+      if (h.kind == 1) {
+        inviscid_flux<2>(hv[it], s, 0, f);
 #pragma unroll
-      for (int l = 0; l < NV2; ++l) sfx[(l * TY + h.ey - HY) * EX + h.ex] = hm[it] * f[l];
-    } else {
-      inviscid_flux<2>(hv[it], s, 1, f);
+        for (int l = 0; l < NV2; ++l) sfx[(l * TY + h.ey - HY) * EX + h.ex] = hm[it] * f[l];
+      } else {
+        inviscid_flux<2>(hv[it], s, 1, f);
 #pragma unroll
-      for (int l = 0; l < NV2; ++l) sfy[(l * EY + h.ey) * TX + h.ex - HX] = hm[it] * f[l];
+        for (int l = 0; l < NV2; ++l) sfy[(l * EY + h.ey) * TX + h.ex - HX] = hm[it] * f[l];
+      }
+#pragma unroll
+      for (int l = 0; l < NV2; ++l) sq[(l * EY + h.ey) * EX + h.ex] = hv[it][l];
     }
-#pragma unroll
-    for (int l = 0; l < NV2; ++l) sq[(l * EY + h.ey) * EX + h.ex] = hv[it][l];
   }
   // RK operands, sponge, source and cost-target values, fetched while the stencils run
-  const bool sponge = (pmask & P->sponge_mask) != 0;            // uniform per block
+  const bool sponge = (pmask & T.tables.sponge_mask) != 0;            // uniform per block
   const bool cost = a.jpartial && a.ip_cost >= 0 && ((pmask >> a.ip_cost) & 1u);
   double q0[NV2], b2[NV2], qt[NV2], damp = 0.0, sx0 = 0.0, sy0 = 0.0, pb = 0.0, mo = 0.0;
-#pragma unroll
-  for (int l = 0; l < NV2; ++l) {
-    const long o = inst * NVN + l * g.N + p;
-    q0[l] = a.stage == 2 || a.stage == 3 ? glob(a.q0)[o] : 0.0;
-    b2[l] = a.stage >= 2 ? glob(a.b2)[o] : 0.0;
-    qt[l] = 0.0;
-  }
-  if (sponge) {
-    damp = glob(P->damp)[p];
-#pragma unroll
-    for (int l = 0; l < NV2; ++l) qt[l] = glob(P->qtarget)[l * g.N + p];
-  }
-  if (a.nsrc > 0) {
-    sx0 = glob(P->srcx)[gi];
-    sy0 = glob(P->srcy)[gj];
-  }
   bool jin = false;
   int kj = 0;
-  if (cost) {
-    ConstPatch& pt = P->p[a.ip_cost];
-    jin = mine && in_patch(pt, gi, gj);
-    kj = jin ? (gi - pt.lo[0]) + pt.ls[0] * (gj - pt.lo[1]) : 0;
-    pb = glob(pt.aplus)[kj];
-    mo = glob(pt.strength)[kj];
-  }
-  __syncthreads();
-  // r = 0 - (D_x F_x + D_y F_y) and the dissipation in x and y
-  double r[NV2];
-  const double ax = -fabs(h1), ay = -fabs(h0);          // -arc length along x, y
-  const double* fx = sfx + ty * EX + tx + HX;           // the point in the staged arrays
-  const double* fy = sfy + (ty + HY) * TX + tx;
-  const double* qc = sq + (ty + HY) * EX + tx + HX;
-  if (!mine) {
-    // nothing: no point of its own
-  } else if (!t.bx && !t.by) {
+#pragma unroll
+  for (int l = 0; l < NV2; ++l) q0[l] = b2[l] = qt[l] = 0.0;
+  if (lead) {
 #pragma unroll
     for (int l = 0; l < NV2; ++l) {
-      double xp[4], xm[4], yp[4], ym[4];
+      const long o = inst * NVN + l * g.N + p;
+      if (a.stage == 2 || a.stage == 3) q0[l] = glob(a.q0)[o];
+      if (a.stage >= 2) b2[l] = glob(a.b2)[o];
+    }
+    if (sponge) {
+      damp = glob(T.tables.damp)[p];
 #pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        xp[k] = fx[l * TY * EX + k + 1];
-        xm[k] = fx[l * TY * EX - (k + 1)];
-        yp[k] = fy[(l * EY + k + 1) * TX];
-        ym[k] = fy[(l * EY - (k + 1)) * TX];
-      }
-      __builtin_amdgcn_sched_barrier(0);   // one batch of LDS reads, one wait
-      r[l] = 0.0 - (skew_sum(xp, xm, d1) + skew_sum(yp, ym, d1));
+      for (int l = 0; l < NV2; ++l) qt[l] = glob(T.tables.qtarget)[l * g.N + p];
+    }
+    if (a.nsrc > 0) {
+      sx0 = glob(T.tables.srcx)[gi];
+      sy0 = glob(T.tables.srcy)[gj];
+    }
+    if (cost) {
+      ConstPatch& pt = P->p[a.ip_cost];
+      jin = mine && in_patch(pt, gi, gj);
+      kj = jin ? (gi - pt.lo[0]) + pt.ls[0] * (gj - pt.lo[1]) : 0;
+      pb = glob(pt.aplus)[kj];
+      mo = glob(pt.strength)[kj];
+    }
+  }
+  __syncthreads();
+  // r = 0 - (D_x F_x + D_y F_y), then the dissipation in x and in y
+  double r[NV2];
+  const EdgePlace ex = edge_place(g.dir[0], gi), ey = edge_place(g.dir[1], gj);
+  const double ax = -fabs(h1), ay = -fabs(h0);          // -arc length along x, y
+  const StagedLine fx = {sfx + ty * EX + tx + HX, tx, t.sx, t.bx, ex};
+  const StagedLine fy = {sfy + (ty + HY) * TX + tx, ty, t.sy, t.by, ey};
+  const StagedLine qx = {sq + (ty + HY) * EX + tx + HX, tx, t.sx, t.bx, ex};
+  const StagedLine qy = {qx.c, ty, t.sy, t.by, ey};
+  if (S::D == 1) {
+    if (!mine) return;
+    double d[NV2];
+    line_derivative<1, TY * EX, NB>(fx, tab, d1, r);
+    line_derivative<TX, EY * TX, NB>(fy, tab, d1, d);
+#pragma unroll
+    for (int l = 0; l < NV2; ++l) r[l] = 0.0 - (r[l] + d[l]);
+    if (g.dissipation) {
+      line_dissipation<1, EY * EX, NB>(g, qx, ax, hw0, tab + 192, d);
+#pragma unroll
+      for (int l = 0; l < NV2; ++l) r[l] = r[l] + g.diss_amount * d[l];
+      line_dissipation<EX, EY * EX, NB>(g, qy, ay, hw1, tab + 192, d);
+#pragma unroll
+      for (int l = 0; l < NV2; ++l) r[l] = r[l] + g.diss_amount * d[l];
     }
   } else {
-    const EdgePlace ex = edge_place(g.dir[0], gi), ey = edge_place(g.dir[1], gj);
-    double dx[NV2], dy[NV2];
-    if (t.bx && ex.m < 8) {
-      const double* b = sfx + ty * EX + HX + (ex.right ? t.sx - 12 : 0);
-      closure_row<NV2, 12>(tab + 12 * ex.m + (ex.right ? 96 : 0),
-                      [&](int j, int k) { return b[j * TY * EX + k]; }, dx);
-    } else {
+    double d[NV2], e[NV2];
+    if (mine && !lead) {
+      line_derivative<TX, EY * TX, NB>(fy, tab, d1, d);
+      if (g.dissipation) line_dissipation<EX, EY * EX, NB>(g, qy, ay, hw1, tab + 192, e);
 #pragma unroll
       for (int l = 0; l < NV2; ++l) {
-        const double* x = fx + l * TY * EX;
-        const double xp[4] = {x[1], x[2], x[3], x[4]}, xm[4] = {x[-1], x[-2], x[-3], x[-4]};
-        dx[l] = skew_sum(xp, xm, d1);
+        sums[l * S::NP] = d[l];
+        if (g.dissipation) sums[(NV2 + l) * S::NP] = e[l];
       }
     }
-    if (t.by && ey.m < 8) {
-      const double* b = sfy + (HY + (ey.right ? t.sy - 12 : 0)) * TX + tx;
-      closure_row<NV2, 12>(tab + 12 * ey.m + (ey.right ? 96 : 0),
-                      [&](int j, int k) { return b[(j * EY + k) * TX]; }, dy);
-    } else {
-#pragma unroll
-      for (int l = 0; l < NV2; ++l) {
-        const double* c = fy + l * EY * TX;
-        const double yp[4] = {c[TX], c[2 * TX], c[3 * TX], c[4 * TX]};
-        const double ym[4] = {c[-TX], c[-2 * TX], c[-3 * TX], c[-4 * TX]};
-        dy[l] = skew_sum(yp, ym, d1);
-      }
+    if (mine && lead) {
+      line_derivative<1, TY * EX, NB>(fx, tab, d1, d);
+      if (g.dissipation) line_dissipation<1, EY * EX, NB>(g, qx, ax, hw0, tab + 192, e);
     }
+    __syncthreads();
+    if (!mine || !lead) return;
 #pragma unroll
-    for (int l = 0; l < NV2; ++l) r[l] = 0.0 - (dx[l] + dy[l]);
-  }
-  if (g.dissipation && mine) {
-    if (g.composite) {
-      const EdgePlace ex = edge_place(g.dir[0], gi), ey = edge_place(g.dir[1], gj);
-#pragma unroll 1
-      for (int d = 0; d < 2; ++d) {
-        const EdgePlace e = d == 0 ? ex : ey;
-        const int step = d == 0 ? 1 : EX;
-        double dv[NV2];
-        if (e.m < 8) {
-          const double* b = d == 0 ? sq + (ty + HY) * EX + HX + (e.right ? t.sx - 12 : 0)
-                                   : sq + (HY + (e.right ? t.sy - 12 : 0)) * EX + tx + HX;
-          closure_row<NV2, 12>(tab + 192 + 12 * e.m + (e.right ? 96 : 0),
-                          [&](int j, int k) { return b[j * EY * EX + k * step]; }, dv);
-        } else {
-#pragma unroll
-          for (int l = 0; l < NV2; ++l) {
-            const double* x = qc + l * EY * EX;
-            double s = 0.0;
-#pragma unroll
-            for (int k = 1; k <= 4; ++k)
-              s += g.ops[SLOT_DISS].c[kMaxHW + k] * (x[k * step] + x[-k * step]);
-            dv[l] = s + g.ops[SLOT_DISS].c[kMaxHW] * x[0];
-          }
-        }
-#pragma unroll
-        for (int l = 0; l < NV2; ++l) r[l] = r[l] + g.diss_amount * dv[l];
-      }
-    } else if (!t.bx && !t.by) {
-#pragma unroll
-      for (int l = 0; l < NV2; ++l) {
-        double w[9];
-#pragma unroll
-        for (int k = 0; k < 9; ++k) w[k] = k == 4 ? v[l] : qc[l * EY * EX + k - 4];
-        __builtin_amdgcn_sched_barrier(0);
-        r[l] = r[l] + g.diss_amount * two_level(w, ax);
-#pragma unroll
-        for (int k = 0; k < 9; ++k) w[k] = k == 4 ? v[l] : qc[(l * EY + k - 4) * EX];
-        __builtin_amdgcn_sched_barrier(0);
-        r[l] = r[l] + g.diss_amount * two_level(w, ay);
-      }
-    } else {
-      const EdgePlace ex = edge_place(g.dir[0], gi), ey = edge_place(g.dir[1], gj);
-      // the windows of nine operands, moved inside the domain at its ends
-      const double* bx = qc - 4 + (ex.m < 4 ? (ex.right ? ex.m - 4 : 4 - ex.m) : 0);
-      const double* by = qc + (-4 + (ey.m < 4 ? (ey.right ? ey.m - 4 : 4 - ey.m) : 0)) * EX;
-#pragma unroll
-      for (int l = 0; l < NV2; ++l) {
-        double w[9];
-#pragma unroll
-        for (int k = 0; k < 9; ++k) w[k] = bx[l * EY * EX + k];
-        double dv = two_level_edge(w, ax, ex, tab + 192);
-        if (hw0 != 1.0) dv = dv / hw0;   // 1 away from the first / last boundary rows
-        r[l] = r[l] + g.diss_amount * dv;
-#pragma unroll
-        for (int k = 0; k < 9; ++k) w[k] = by[(l * EY + k) * EX];
-        dv = two_level_edge(w, ay, ey, tab + 192);
-        if (hw1 != 1.0) dv = dv / hw1;
-        r[l] = r[l] + g.diss_amount * dv;
+    for (int l = 0; l < NV2; ++l) {
+      r[l] = 0.0 - (d[l] + sums[l * S::NP]);
+      if (g.dissipation) {
+        r[l] = r[l] + g.diss_amount * e[l];
+        r[l] = r[l] + g.diss_amount * sums[(NV2 + l) * S::NP];
       }
     }
   }
-  if (!mine) return;
   // point terms, RK4 stage update (substepForwardRK4, src/RK4IntegratorImpl.f90:115-156) and
   // the functional term of the new stage state
   const double dt = a.dt;
@@ -486,15 +558,15 @@ __device__ __forceinline__ void fwd_stage_body(const Geo& g, const Patches* patc
 #pragma unroll
   for (int l = 0; l < NV2; ++l) r[l] = r[l] * jac;
   // far fields, then sponges, then the other patches, each in the order of the patches
-  for (unsigned m = pmask & P->far_mask; m; m &= m - 1) {
+  for (unsigned m = pmask & T.tables.far_mask; m; m &= m - 1) {
     const int ip = __ffs(m) - 1;
-    ConstPatch& pt = P->p[ip];
-    if (!in_patch(pt, gi, gj)) continue;
-    const double sj = pt.sigma_inv * jac;
-    double f[NV2];
-    if (ip == far.ip[0] || ip == far.ip[1]) {
-      far_formed(far, ip, ff, gi, gj, f);
-    } else {
+    double f[NV2], sigma_inv;
+    const int formed = far_formed(I, ip, ff, gi, gj, f, &sigma_inv);
+    if (formed == 0) continue;
+    if (formed < 0) {
+      ConstPatch& pt = P->p[ip];
+      if (!in_patch(pt, gi, gj)) continue;
+      sigma_inv = pt.sigma_inv;
       const int kp = (gi - pt.lo[0]) + pt.ls[0] * (gj - pt.lo[1]);
       const global_ptr<const double> A = glob(pt.aplus) + (long)kp * 16;
       const global_ptr<const double> qf = glob(pt.aplus) + (long)pt.np * 16 + (long)kp * 4;
@@ -505,6 +577,7 @@ __device__ __forceinline__ void fwd_stage_body(const Geo& g, const Patches* patc
         for (int c = 0; c < NV2; ++c) f[i] += A[c * 4 + i] * (v[c] - qf[c]);
       }
     }
+    const double sj = sigma_inv * jac;
 #pragma unroll
     for (int l = 0; l < NV2; ++l) r[l] = r[l] - sj * f[l];
   }
@@ -512,7 +585,7 @@ __device__ __forceinline__ void fwd_stage_body(const Geo& g, const Patches* patc
 #pragma unroll
     for (int l = 0; l < NV2; ++l) r[l] = r[l] - damp * (v[l] - qt[l]);
   }
-  unsigned rest = pmask & ~(P->sponge_mask | P->far_mask);
+  unsigned rest = pmask & ~(T.tables.sponge_mask | T.tables.far_mask);
   if (a.ip_cost >= 0) rest &= ~(1u << a.ip_cost);
   while (rest) {
     const int ip = __ffs(rest) - 1;
@@ -535,7 +608,7 @@ __device__ __forceinline__ void fwd_stage_body(const Geo& g, const Patches* patc
   if (a.nsrc > 0) r[3] = r[3] + glob(a.src_amp)[inst * a.src_inst_stride] * (sx0 * sy0);
   for (int s = 1; s < a.nsrc; ++s)
     r[3] = r[3] + glob(a.src_amp)[inst * a.src_inst_stride + s] *
-                      (glob(P->srcx)[(long)s * g.n[0] + gi] * glob(P->srcy)[(long)s * g.n[1] + gj]);
+                      (glob(T.tables.srcx)[(long)s * g.n[0] + gi] * glob(T.tables.srcy)[(long)s * g.n[1] + gj]);
   double qn[NV2];
 #pragma unroll
   for (int l = 0; l < NV2; ++l) {
@@ -570,16 +643,19 @@ __device__ __forceinline__ void fwd_stage_body(const Geo& g, const Patches* patc
 // D+ reads anyway, and the Jacobian products go through the enthalpy.  The RK operands are
 // loaded behind the stencils: held across them, they cost 100 bytes of scratch per thread and
 // 0.1 ms (20 x 401^2: 252 against 162 us; with the edge tiles' closures kept from spilling the
-// last 20 bytes, 141).  Before: 401^2 15.1 -> 12.1 us, 201^2 10.8 -> 9.4, 20 x 401^2 170 -> 142.
+// last 20 bytes, 141).  Before: 401^2 15.1 -> 11.0 us, 201^2 10.8 -> 7.7, 20 x 401^2 170 -> 139.
 // One adjoint stage on tile block `blk` of instance `inst` (uniform per work-group).
 template <class S>
 __device__ __forceinline__ void adj_stage_body(const Geo& g, const Patches* patches,
                                                const Tiling& T, const AdjStage& a, int blk,
                                                long inst, double* lds) {
-  constexpr int EX = S::EX, EY = S::EY, HS = S::kHaloIters;
+  constexpr int EX = S::EX, EY = S::EY, HS = S::kHaloIters, NB = S::kBatchA;
+  const int grp = S::D == 2 ? __builtin_amdgcn_readfirstlane(threadIdx.x / S::NP) : 0;
+  const bool lead = grp == 0, halo = S::D == 1 || grp == 1;
   double* sq = lds;
   double* tab = sq + S::SQ;
   double* ff = tab + S::kTabA;
+  double* sums = ff + S::kFar + threadIdx.x % S::NP;
   const int tile = block_tile(T, blk);
   ConstPatches* P = (ConstPatches*)patches;
   if (tile < 0) return;   // block beyond the tiles of its XCD (uniform per block)
@@ -587,7 +663,8 @@ __device__ __forceinline__ void adj_stage_body(const Geo& g, const Patches* patc
   const long NVN = (long)NV2 * g.N;
   const global_ptr<const double> li = glob(a.lam) + inst * NVN;
   const global_ptr<const double> qi = glob(a.q) + inst * NVN;
-  const unsigned pmask = glob(T.pmask)[tile];
+  ConstTileInfo* I = (ConstTileInfo*)T.info + tile;
+  const unsigned pmask = I->pmask;
   int tx, ty;
   const bool mine = thread_point<S>(t, &tx, &ty);
   const int gi = t.x0 + (mine ? tx : 0), gj = t.y0 + (mine ? ty : 0);
@@ -595,12 +672,14 @@ __device__ __forceinline__ void adj_stage_body(const Geo& g, const Patches* patc
   double v[NV2], hv[HS][NV2], q[NV2];
 #pragma unroll
   for (int l = 0; l < NV2; ++l) v[l] = li[l * g.N + p];
+  if (halo) {
 #pragma unroll
-  for (int it = 0; it < HS; ++it) {
-    const HaloSlot h = halo_slot<S>(g, t, it);
-    const long pp = h.gi + (long)g.n[0] * h.gj;
+    for (int it = 0; it < HS; ++it) {
+      const HaloSlot h = halo_slot<S>(g, t, it);
+      const long pp = h.gi + (long)g.n[0] * h.gj;
 #pragma unroll
-    for (int l = 0; l < NV2; ++l) hv[it][l] = li[l * g.N + pp];
+      for (int l = 0; l < NV2; ++l) hv[it][l] = li[l * g.N + pp];
+    }
   }
   double d1[5], ds[5];              // interior coefficients
 #pragma unroll
@@ -608,102 +687,67 @@ __device__ __forceinline__ void adj_stage_body(const Geo& g, const Patches* patc
     d1[k] = g.ops[SLOT_ADJ].c[kMaxHW + k];
     ds[k] = g.ops[SLOT_DISS2].c[kMaxHW + k];
   }
-  const FarAhead far = far_ahead<S, true>(g, P, t, pmask & P->far_mask, li, ff);
+  far_ahead<S, true>(g, I, li, ff);
   if (t.bx || t.by) {
     stage_rows<S::NT, 12, 16>(g, SLOT_ADJ, tab);
     if (g.dissipation) stage_rows<S::NT, 8, 12>(g, SLOT_DISS2, tab + 384);
   }
-  if (mine) {
+  if (mine && lead) {
 #pragma unroll
     for (int l = 0; l < NV2; ++l) sq[(l * EY + ty + HY) * EX + tx + HX] = v[l];
   }
+  if (halo) {
 #pragma unroll
-  for (int it = 0; it < HS; ++it) {
-    const HaloSlot h = halo_slot<S>(g, t, it);
-    if (h.kind == 0) continue;
+    for (int it = 0; it < HS; ++it) {
+      const HaloSlot h = halo_slot<S>(g, t, it);
+      if (h.kind == 0) continue;
 #pragma unroll
-    for (int l = 0; l < NV2; ++l) sq[(l * EY + h.ey) * EX + h.ex] = hv[it][l];
+      for (int l = 0; l < NV2; ++l) sq[(l * EY + h.ey) * EX + h.ex] = hv[it][l];
+    }
   }
   // the forward stage state at the point and the grid values, fetched while the stencils run
+  if (lead) {
 #pragma unroll
-  for (int l = 0; l < NV2; ++l) q[l] = qi[l * g.N + p];
+    for (int l = 0; l < NV2; ++l) q[l] = qi[l * g.N + p];
+  }
   const double h0 = glob(g.h[0])[gi], hw0 = glob(g.hw[0])[gi], h1 = glob(g.h[1])[gj], hw1 = glob(g.hw[1])[gj];
   __syncthreads();
-  if (!mine) return;
   // D+ lambda along x and y (T1) and the dissipation (w), from the same staged values
-  double T1[2][NV2], w[NV2], l0[NV2], b2[NV2];
-  const double* lc = sq + (ty + HY) * EX + tx + HX;   // the point in the staged tile
+  double T1[2][NV2], w[NV2], l0[NV2], b2[NV2], d[NV2];
   const double sx = diss_scale(g, -g.diss_amount, fabs(h1), hw0);
   const double sy = diss_scale(g, -g.diss_amount, fabs(h0), hw1);
-  if (!t.bx && !t.by) {
+  const double* lc = sq + (ty + HY) * EX + tx + HX;
+  const StagedLine lx = {lc, tx, t.sx, t.bx, edge_place(g.dir[0], gi)};
+  const StagedLine ly = {lc, ty, t.sy, t.by, edge_place(g.dir[1], gj)};
+  if (S::D == 1) {
+    if (!mine) return;
+    line_adjoint<1, EY * EX, NB>(g, lx, v, tab, d1, ds, T1[0], d);
+#pragma unroll
+    for (int l = 0; l < NV2; ++l) w[l] = sx * d[l];
+    line_adjoint<EX, EY * EX, NB>(g, ly, v, tab, d1, ds, T1[1], d);
+#pragma unroll
+    for (int l = 0; l < NV2; ++l) w[l] = w[l] + sy * d[l];
+  } else {
+    if (mine && !lead) {
+      line_adjoint<EX, EY * EX, NB>(g, ly, v, tab, d1, ds, T1[1], d);
+#pragma unroll
+      for (int l = 0; l < NV2; ++l) {
+        sums[l * S::NP] = T1[1][l];
+        if (g.dissipation) sums[(NV2 + l) * S::NP] = sy * d[l];
+      }
+    }
+    if (mine && lead) line_adjoint<1, EY * EX, NB>(g, lx, v, tab, d1, ds, T1[0], d);
+    __syncthreads();
+    if (!mine || !lead) return;
 #pragma unroll
     for (int l = 0; l < NV2; ++l) {
-      double xp[4], xm[4], yp[4], ym[4];
-#pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        xp[k] = lc[l * EY * EX + k + 1];
-        xm[k] = lc[l * EY * EX - (k + 1)];
-        yp[k] = lc[(l * EY + k + 1) * EX];
-        ym[k] = lc[(l * EY - (k + 1)) * EX];
-      }
-      __builtin_amdgcn_sched_barrier(0);   // one batch of LDS reads, one wait
-      T1[0][l] = skew_sum(xp, xm, d1);
-      T1[1][l] = skew_sum(yp, ym, d1);
-      w[l] = sx * sym9(v[l], xp, xm, ds) + sy * sym9(v[l], yp, ym, ds);
+      T1[1][l] = sums[l * S::NP];
+      if (g.dissipation) w[l] = sx * d[l] + sums[(NV2 + l) * S::NP];
     }
-  } else {
-    const EdgePlace ex = edge_place(g.dir[0], gi), ey = edge_place(g.dir[1], gj);
-    // the 16 (12) staged values at the end of the line
-    const int ox = ex.right ? t.sx - 1 : 0, oy = ey.right ? t.sy - 1 : 0;
-    const double* bx = sq + (ty + HY) * EX + HX + ox;
-    const double* by = sq + (HY + oy) * EX + tx + HX;
-    const int rx = ex.right ? 15 : 0, ry = ey.right ? 15 : 0;
-    const int qx = ex.right ? 11 : 0, qy = ey.right ? 11 : 0;
-    const bool cx = t.bx && ex.m < 12, cy = t.by && ey.m < 12;
-    double dv[NV2];
-    if (cx)
-      closure_row<NV2, 16>(tab + 16 * ex.m + (ex.right ? 192 : 0),
-                      [&](int j, int k) { return bx[j * EY * EX + k - rx]; }, T1[0]);
-    if (t.bx && ex.m < 8) {
-      if (g.dissipation)
-        closure_row<NV2, 12>(tab + 384 + 12 * ex.m + (ex.right ? 96 : 0),
-                        [&](int j, int k) { return bx[j * EY * EX + k - qx] - v[j]; }, dv);
-    } else {
-#pragma unroll
-      for (int l = 0; l < NV2; ++l) {
-        const double* x = lc + l * EY * EX;
-        const double xp[4] = {x[1], x[2], x[3], x[4]}, xm[4] = {x[-1], x[-2], x[-3], x[-4]};
-        if (!cx) T1[0][l] = skew_sum(xp, xm, d1);
-        dv[l] = sym9(v[l], xp, xm, ds);
-        __builtin_amdgcn_sched_barrier(0);
-      }
-    }
-#pragma unroll
-    for (int l = 0; l < NV2; ++l) w[l] = sx * dv[l];
-    if (cy)
-      closure_row<NV2, 16>(tab + 16 * ey.m + (ey.right ? 192 : 0),
-                      [&](int j, int k) { return by[(j * EY + k - ry) * EX]; }, T1[1]);
-    if (t.by && ey.m < 8) {
-      if (g.dissipation)
-        closure_row<NV2, 12>(tab + 384 + 12 * ey.m + (ey.right ? 96 : 0),
-                        [&](int j, int k) { return by[(j * EY + k - qy) * EX] - v[j]; }, dv);
-    } else {
-#pragma unroll
-      for (int l = 0; l < NV2; ++l) {
-        const double* c = lc + l * EY * EX;
-        const double yp[4] = {c[EX], c[2 * EX], c[3 * EX], c[4 * EX]};
-        const double ym[4] = {c[-EX], c[-2 * EX], c[-3 * EX], c[-4 * EX]};
-        if (!cy) T1[1][l] = skew_sum(yp, ym, d1);
-        dv[l] = sym9(v[l], yp, ym, ds);
-        __builtin_amdgcn_sched_barrier(0);
-      }
-    }
-#pragma unroll
-    for (int l = 0; l < NV2; ++l) w[l] = w[l] + sy * dv[l];
   }
   // here, not before: the closure rows need the registers
-  const bool sponge = (pmask & P->sponge_mask) != 0;            // uniform per block
-  const double damp = sponge ? glob(P->damp)[p] : 0.0;
+  const bool sponge = (pmask & T.tables.sponge_mask) != 0;            // uniform per block
+  const double damp = sponge ? glob(T.tables.damp)[p] : 0.0;
 #pragma unroll
   for (int l = 0; l < NV2; ++l) {
     const long o = inst * NVN + l * g.N + p;
@@ -718,15 +762,15 @@ __device__ __forceinline__ void adj_stage_body(const Geo& g, const Patches* patc
 #pragma unroll
   for (int l = 0; l < NV2; ++l) r[l] = (g.dissipation ? r[l] + w[l] : r[l]) * jac;
   // far fields, then sponges, then the other patches, each in the order of the patches
-  for (unsigned m = pmask & P->far_mask; m; m &= m - 1) {
+  for (unsigned m = pmask & T.tables.far_mask; m; m &= m - 1) {
     const int ip = __ffs(m) - 1;
-    ConstPatch& pt = P->p[ip];
-    if (!in_patch(pt, gi, gj)) continue;
-    const double sj = pt.sigma_inv * jac;
-    double f[NV2];
-    if (ip == far.ip[0] || ip == far.ip[1]) {
-      far_formed(far, ip, ff, gi, gj, f);
-    } else {
+    double f[NV2], sigma_inv;
+    const int formed = far_formed(I, ip, ff, gi, gj, f, &sigma_inv);
+    if (formed == 0) continue;
+    if (formed < 0) {
+      ConstPatch& pt = P->p[ip];
+      if (!in_patch(pt, gi, gj)) continue;
+      sigma_inv = pt.sigma_inv;
       const int kp = (gi - pt.lo[0]) + pt.ls[0] * (gj - pt.lo[1]);
       const global_ptr<const double> A = glob(pt.aplus) + (long)kp * 16;
 #pragma unroll
@@ -736,6 +780,7 @@ __device__ __forceinline__ void adj_stage_body(const Geo& g, const Patches* patc
         for (int c = 0; c < NV2; ++c) f[i] += A[i * 4 + c] * v[c];
       }
     }
+    const double sj = sigma_inv * jac;
 #pragma unroll
     for (int l = 0; l < NV2; ++l) r[l] = r[l] + sj * f[l];
   }
@@ -743,7 +788,7 @@ __device__ __forceinline__ void adj_stage_body(const Geo& g, const Patches* patc
 #pragma unroll
     for (int l = 0; l < NV2; ++l) r[l] = r[l] + damp * v[l];
   }
-  unsigned rest = pmask & ~(P->sponge_mask | P->far_mask);
+  unsigned rest = pmask & ~(T.tables.sponge_mask | T.tables.far_mask);
   while (rest) {
     const int ip = __ffs(rest) - 1;
     rest &= rest - 1;
@@ -925,15 +970,15 @@ __global__ void __launch_bounds__(kRedThreads) k_stage_accumulate(
 }
 
 // ------------------------------------------------------------------------ host side
-using S32x16 = Shape<32, 16>;
-using S16x32 = Shape<16, 32>;
-using S16x16 = Shape<16, 16>;
-using S24x16 = Shape<24, 16>;
-using S16x24 = Shape<16, 24>;
-using S16x12 = Shape<16, 12>;
+using S32x16 = Shape<32, 16, 1>;
+using S16x32 = Shape<16, 32, 1>;
+using S16x16 = Shape<16, 16, 1>;
+using S24x16 = Shape<24, 16, 1>;
+using S16x16d2 = Shape<16, 16, 2>;
+using S16x12 = Shape<16, 12, 1>;
 
 static const int kShapeDims[kNumTileShapes][2] = {{32, 16}, {16, 32}, {16, 16}, {24, 16},
-                                                  {16, 24}, {16, 12}};
+                                                  {16, 16}, {16, 12}};
 
 int fused2d_shape_dims(int shape, int* tx, int* ty) {
   if (shape < 0 || shape >= kNumTileShapes) return MGD_ERR_ARG;
@@ -977,18 +1022,27 @@ int fused2d_make_tiling(const Geo& g, const Patches& hp, int shape, HostTiling* 
     const int last = d == 0 ? out->nbx - 1 : out->nbx + out->nby - 1;
     if (out->size[first] < kMinEdgeTile || out->size[last] < kMinEdgeTile) return MGD_ERR_UNSUPPORTED;
   }
-  out->pmask.assign((size_t)out->nbx * out->nby, 0u);
+  TileInfo none{};
+  none.far[0].ip = none.far[1].ip = -1;
+  out->info.assign((size_t)out->nbx * out->nby, none);
   for (int by = 0; by < out->nby; ++by)
     for (int bx = 0; bx < out->nbx; ++bx) {
       const int xa = out->org[bx], xb = xa + out->size[bx] - 1;
       const int ya = out->org[out->nbx + by], yb = ya + out->size[out->nbx + by] - 1;
-      unsigned m = 0;
+      TileInfo& info = out->info[(size_t)by * out->nbx + bx];
+      int nfar = 0;
       for (int ip = 0; ip < hp.count; ++ip) {
         const DPatch& pt = hp.p[ip];
         if (xb < pt.lo[0] || xa > pt.hi[0] || yb < pt.lo[1] || ya > pt.hi[1]) continue;
-        m |= 1u << ip;
+        info.pmask |= 1u << ip;
+        if (pt.type != MGD_PATCH_FAR_FIELD || nfar == 2) continue;
+        const int i0 = std::max(pt.lo[0], xa), j0 = std::max(pt.lo[1], ya);
+        const int w = std::min(pt.hi[0], xb) - i0 + 1, h = std::min(pt.hi[1], yb) - j0 + 1;
+        if (w * h > kFarPoints) continue;
+        const long k = (i0 - pt.lo[0]) + (long)pt.ls[0] * (j0 - pt.lo[1]);
+        info.far[nfar++] = {ip, i0, j0, w, h, pt.ls[0], pt.sigma_inv, pt.aplus + 16 * k,
+                            pt.aplus + 16L * pt.np + 4 * k};
       }
-      out->pmask[(size_t)by * out->nbx + bx] = m;
     }
   // XCD-aware block -> tile map.  Work-groups are dealt to the XCDs round-robin by
   // linear block index, and each XCD has its own L2: XCD x receives blocks x, x + 8, ...
@@ -1044,7 +1098,7 @@ void launch_dual_stage2d(const Geo& g, const Patches* P, const Tiling& T, const 
     case 1: dual_launch<S16x32>(g, P, T, a, f, st); break;
     case 2: dual_launch<S16x16>(g, P, T, a, f, st); break;
     case 3: dual_launch<S24x16>(g, P, T, a, f, st); break;
-    case 4: dual_launch<S16x24>(g, P, T, a, f, st); break;
+    case 4: dual_launch<S16x16d2>(g, P, T, a, f, st); break;
     default: dual_launch<S16x12>(g, P, T, a, f, st); break;
   }
 }
@@ -1056,7 +1110,7 @@ void launch_fwd_stage2d(const Geo& g, const Patches* P, const Tiling& T, const F
     case 1: fwd_launch<S16x32>(g, P, T, a, st); break;
     case 2: fwd_launch<S16x16>(g, P, T, a, st); break;
     case 3: fwd_launch<S24x16>(g, P, T, a, st); break;
-    case 4: fwd_launch<S16x24>(g, P, T, a, st); break;
+    case 4: fwd_launch<S16x16d2>(g, P, T, a, st); break;
     default: fwd_launch<S16x12>(g, P, T, a, st); break;
   }
 }
@@ -1068,7 +1122,7 @@ void launch_adj_stage2d(const Geo& g, const Patches* P, const Tiling& T, const A
     case 1: adj_launch<S16x32>(g, P, T, a, st); break;
     case 2: adj_launch<S16x16>(g, P, T, a, st); break;
     case 3: adj_launch<S24x16>(g, P, T, a, st); break;
-    case 4: adj_launch<S16x24>(g, P, T, a, st); break;
+    case 4: adj_launch<S16x16d2>(g, P, T, a, st); break;
     default: adj_launch<S16x12>(g, P, T, a, st); break;
   }
 }

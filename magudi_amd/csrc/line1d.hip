@@ -131,12 +131,14 @@ __device__ __forceinline__ void line_dissipation(const Geo& g, const double (*s)
   }
   const int m = t.edge.m;
   const int col = t.e + 4 - 4 + (m < 4 ? (t.edge.right ? m - 4 : 4 - m) : 0);
+  double b[7];
+  closure_weights(tab, t.edge, b);
 #pragma unroll
   for (int l = 0; l < kLN; ++l) {
     double w[9];
 #pragma unroll
     for (int k = 0; k < 9; ++k) w[k] = s[l][col + k];
-    double v = two_level_edge(w, -1.0, t.edge, tab);    // the metric of a line is 1
+    double v = two_level_edge(w, -1.0, t.edge, b);    // the metric of a line is 1
     if (hw != 1.0) v = v / hw;       // 1 away from the first / last boundary rows
     r[l] = r[l] + amount * v;
   }

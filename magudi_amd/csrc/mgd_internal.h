@@ -96,9 +96,12 @@ struct DPatch {
 struct Patches {
   int count;
   DPatch p[kMaxPatches];
-  // what the fused 2-D kernels read of patches and sources in other layouts: bits of the
-  // far-field and sponge patches; per grid point the sponge strengths' sum and the target
-  // state (null without a sponge); per source the factors of its Gaussian along x and y
+};
+
+// What the fused 2-D kernels read of patches and sources in other layouts: bits of the
+// far-field and sponge patches; per grid point the sponge strengths' sum and the target state
+// (null without a sponge); per source the factors of its Gaussian along x and y.
+struct StageTables {
   unsigned far_mask, sponge_mask;
   const double* damp;
   const double* qtarget;

@@ -90,7 +90,8 @@ struct mgd_region {
   bool finalized = false;
   mgd::Patches hpatches;
   mgd::DevBuf d_patches, d_sources;
-  mgd::DevBuf d_damp, d_qtarget, d_srcx, d_srcy;   // fused 2-D tables (Patches)
+  mgd::DevBuf d_damp, d_qtarget, d_srcx, d_srcy;   // fused 2-D tables
+  mgd::StageTables tables{};
   int ip_cost = -1, ip_act = -1, has_farfield = 0;
   mgd::FinishInfo fin;                   // the forward finishing pass (set at finalize)
   // HBM-resident state
@@ -105,12 +106,12 @@ struct mgd_region {
   double wts_dt = 0.0;
   mgd::HostTiling htile;
   mgd::Tiling tiling{};
-  mgd::DevBuf d_tile_mask;
+  mgd::DevBuf d_tile_info;
   // the 16 x 16 tiling of group launches, held beside the region's own (built at the first
   // group run; the two are swapped for each group run)
   mgd::HostTiling g_htile;
   mgd::Tiling g_tiling{};
-  mgd::DevBuf g_tile_mask;
+  mgd::DevBuf g_tile_info;
   bool g_built = false, g_swapped = false;
   bool tiling_ok = false;
   int tile_shape = -1;                   // MGD_OPT_TILE_SHAPE: -1 autotune, else fixed
@@ -681,7 +682,7 @@ int upload_ints(DevBuf& b, const void* data, size_t bytes) {
 int make_tiling(mgd_region* r, int shape, HostTiling& Hout, Tiling& T, DevBuf& mask) {
   HostTiling H;
   if (fused2d_make_tiling(r->geo, r->hpatches, shape, &H) != MGD_OK) return MGD_ERR_UNSUPPORTED;
-  if (upload_ints(mask, H.pmask.data(), H.pmask.size() * sizeof(unsigned))) return MGD_ERR_HIP;
+  if (upload_ints(mask, H.info.data(), H.info.size() * sizeof(TileInfo))) return MGD_ERR_HIP;
   Hout = H;
   T.shape = H.shape;
   T.nbx = H.nbx;
@@ -694,20 +695,22 @@ int make_tiling(mgd_region* r, int shape, HostTiling& Hout, Tiling& T, DevBuf& m
   T.qy = H.qy;
   T.ly = H.ly;
   T.ry = H.ry;
-  T.pmask = reinterpret_cast<const unsigned*>(mask.p);
+  T.inv_nbx = 0xffffffffu / (unsigned)H.nbx;
+  T.info = reinterpret_cast<const TileInfo*>(mask.p);
+  T.tables = r->tables;
   return MGD_OK;
 }
 
 int install_tiling(mgd_region* r, int shape) {
-  return make_tiling(r, shape, r->htile, r->tiling, r->d_tile_mask);
+  return make_tiling(r, shape, r->htile, r->tiling, r->d_tile_info);
 }
 
 // Exchanges the region's tiling with the group tiling held beside it.
 void swap_tilings(mgd_region* r) {
   std::swap(r->htile, r->g_htile);
   std::swap(r->tiling, r->g_tiling);
-  std::swap(r->d_tile_mask.p, r->g_tile_mask.p);
-  std::swap(r->d_tile_mask.n, r->g_tile_mask.n);
+  std::swap(r->d_tile_info.p, r->g_tile_info.p);
+  std::swap(r->d_tile_info.n, r->g_tile_info.n);
   r->g_swapped = !r->g_swapped;
 }
 
@@ -1901,7 +1904,7 @@ std::vector<uintptr_t> graph_key(mgd_region* r, int kind, std::initializer_list<
                           &r->G, &r->T1, &r->S, &r->qs, &r->aforce, &r->control, &r->grad,
                           &r->acc_J, &r->acc_S, &r->partial, &r->src_amp, &r->snaps, &r->window,
                           &r->qy, &r->ly, &r->l0, &r->jpart, &r->spart, &r->ssum, &r->wts,
-                          &r->window2, &r->b2r, &r->qsr, &r->qT, &r->d_tile_mask, &r->wall};
+                          &r->window2, &r->b2r, &r->qsr, &r->qT, &r->d_tile_info, &r->wall};
   for (const DevBuf* b : bufs) k.push_back((uintptr_t)b->p);
   k.push_back((uintptr_t)r->q_alt.p);
   k.push_back((uintptr_t)r->qs_alt.p);
@@ -2154,23 +2157,25 @@ int group_adjoint_pass(mgd_group* G, const double* dts, int nsteps, int K) {
   return MGD_OK;
 }
 
-// The layouts of sponges, far fields and sources that the fused 2-D kernels read (Patches).
+// The layouts of sponges, far fields and sources that the fused 2-D kernels read (StageTables).
 int fused_tables(mgd_region* r) {
-  Patches& H = r->hpatches;
+  const Patches& H = r->hpatches;
+  StageTables& T = r->tables;
+  T = StageTables{};
   std::vector<double> damp;
   for (int ip = 0; ip < H.count; ++ip) {
     const DPatch& D = H.p[ip];
-    if (D.type == MGD_PATCH_FAR_FIELD) H.far_mask |= 1u << ip;
+    if (D.type == MGD_PATCH_FAR_FIELD) T.far_mask |= 1u << ip;
     if (D.type != MGD_PATCH_SPONGE) continue;
-    H.sponge_mask |= 1u << ip;
+    T.sponge_mask |= 1u << ip;
     damp.resize((size_t)r->N, 0.0);
     const HostPatch& P = *r->patches[ip];
     for (int k = 0; k < P.np; ++k) damp[patch_point(r, P, k)] += P.strength[k];
   }
   if (!damp.empty()) {
     if (upload(r->d_damp, damp) || upload(r->d_qtarget, r->target)) return MGD_ERR_HIP;
-    H.damp = r->d_damp.p;
-    H.qtarget = r->d_qtarget.p;
+    T.damp = r->d_damp.p;
+    T.qtarget = r->d_qtarget.p;
   }
   const size_t ns = r->sources.size();
   std::vector<double> ax(ns * r->desc.n[0]), ay(ns * r->desc.n[1]);
@@ -2186,8 +2191,8 @@ int fused_tables(mgd_region* r) {
     }
   }
   if (ns && (upload(r->d_srcx, ax) || upload(r->d_srcy, ay))) return MGD_ERR_HIP;
-  H.srcx = r->d_srcx.p;
-  H.srcy = r->d_srcy.p;
+  T.srcx = r->d_srcx.p;
+  T.srcy = r->d_srcy.p;
   return MGD_OK;
 }
 
@@ -3533,7 +3538,7 @@ int mgd_group_run_adjoint(mgd_group* G, double t0, const double* dt, int nsteps,
       if (int rc = prepare_adjoint_ck(r, true)) return rc;
       if (r->tiling.shape != kGroupShape) {
         // the group tiling, built once per region, in place of the region's own
-        if (!r->g_built && make_tiling(r, kGroupShape, r->g_htile, r->g_tiling, r->g_tile_mask) != MGD_OK) {
+        if (!r->g_built && make_tiling(r, kGroupShape, r->g_htile, r->g_tiling, r->g_tile_info) != MGD_OK) {
           set_error("a group member does not fit the 16 x 16 tiles of a group launch");
           return MGD_ERR_UNSUPPORTED;
         }

@@ -81,27 +81,40 @@ __device__ __forceinline__ double two_level(const double* w, double marc) {
   return d4_row(z);
 }
 
-// The same in a tile at a non-periodic end: w holds the nine operands of the window that
-// starts at index clamp(i - 4, 0, len - 9).  The first two rows of D4 repeat the stencil of
-// the third one, summed in the order of the index; D4^T has 5 closure rows of 7 columns.
+// The same on a line with ends: w holds the nine operands of the window that starts at index
+// clamp(i - 4, 0, len - 9), b the weights of the point's closure row.  The first two
+// rows of D4 repeat the stencil of the third one, summed in the order of the index; D4^T has 5
+// closure rows of 7 columns.
 __device__ __forceinline__ double two_level_edge(const double* w, double marc, EdgePlace e,
-                                                 const double* rows) {
-  if (e.m >= 5) return two_level(w, marc);
-  double z[5], first = 0.0;
+                                                 const double* b) {
+  double z[5];
 #pragma unroll
   for (int k = 0; k < 5; ++k) z[k] = marc * d4_row(w + k);
+  if (e.m >= 5) return d4_row(z);
+  const int o = e.right ? 4 : 0;
+  double first = 0.0, s = 0.0;
 #pragma unroll
-  for (int k = 0; k < 5; ++k) first += kD4[k < 2 ? 2 - k : k - 2] * (e.right ? w[k + 4] : w[k]);
+  for (int k = 0; k < 5; ++k) first += kD4[k < 2 ? 2 - k : k - 2] * (o ? w[k + 4] : w[k]);
   first = marc * first;
-  const double* b = rows + (e.right ? 35 : 0) + 7 * e.m;
-  double s = 0.0;
+  if (!e.right) {
+    s += b[0] * first;
+    s += b[1] * first;
 #pragma unroll
-  for (int c = 0; c < 7; ++c) {
-    const double l = c < 2 ? first : z[c < 2 ? 0 : c - 2];
-    const double r = c < 5 ? z[c < 5 ? c : 0] : first;
-    s += b[c] * (e.right ? r : l);
+    for (int k = 0; k < 5; ++k) s += b[k + 2] * z[k];
+  } else {
+#pragma unroll
+    for (int k = 0; k < 5; ++k) s += b[k] * z[k];
+    s += b[5] * first;
+    s += b[6] * first;
   }
   return s;
+}
+
+// The weights of the closure row of D4^T at a point (of some row where it has none).
+__device__ __forceinline__ void closure_weights(const double* rows, EdgePlace e, double* b) {
+  const double* r = rows + (e.right ? 35 : 0) + 7 * min(e.m, 4);
+#pragma unroll
+  for (int c = 0; c < 7; ++c) b[c] = r[c];
 }
 
 }  // namespace mgd
