@@ -1,0 +1,120 @@
+// hostcopy.cpp -- large copies between device memory and a caller's pageable array.
+//
+// The runtime's own pageable device-to-host copy moves the data with one thread, which also
+// takes the page faults of a fresh destination: 10 GB/s.  Here chunks of 2 MiB (the huge page
+// that backs large arrays, so no two threads fault on one) arrive in pinned slots and several
+// threads copy them out: 671 MB 65 -> 18 ms, 40 MB 4.2 -> 1.4 ms, 8.4 MB 1.1 -> 0.7 ms, 5.1 MB
+// 0.8 -> 0.65 ms.  Below kLeast the threads cost more than they save (2.4 MB 0.56 -> 0.63 ms).
+// The slots are as many as a copy needs, sixteen at most: pinning them takes 0.1 ms per MB
+// once.  Host-to-device copies have no faults to share and stay as they are.
+#include "hostcopy.h"
+
+#include <algorithm>
+#include <atomic>
+#include <cstdint>
+#include <cstring>
+#include <system_error>
+#include <thread>
+#include <vector>
+
+namespace mgd {
+
+namespace {
+constexpr size_t kLeast = size_t(4) << 20;
+constexpr unsigned kMostThreads = 8;
+}  // namespace
+
+HostCopy::~HostCopy() {
+  for (hipEvent_t e : ev_)
+    if (e) (void)hipEventDestroy(e);
+  if (buf_) (void)hipHostFree(buf_);
+}
+
+bool HostCopy::prepare(int slots) {
+  if (slots_ >= slots) return true;
+  if (failed_) return false;
+  if (buf_) (void)hipHostFree(buf_);
+  buf_ = nullptr;
+  slots_ = 0;
+  void* p = nullptr;
+  bool ok = hipHostMalloc(&p, kChunk * slots, hipHostMallocDefault) == hipSuccess;
+  for (hipEvent_t& e : ev_) ok = ok && (e || hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess);
+  if (!ok) {
+    (void)hipGetLastError();     // no pinned memory left: plain copies from here on
+    if (p) (void)hipHostFree(p);
+    failed_ = true;
+    return false;
+  }
+  buf_ = static_cast<char*>(p);
+  slots_ = slots;
+  return true;
+}
+
+hipError_t HostCopy::to_host(void* host, const void* dev, size_t bytes, hipStream_t st) {
+  // chunk c covers [edge(c), edge(c + 1)): the first one ends at a chunk boundary of the address
+  const size_t first = kChunk - reinterpret_cast<uintptr_t>(host) % kChunk;
+  const long n = bytes > first ? 1 + (long)((bytes - first + kChunk - 1) / kChunk) : 1;
+  auto edge = [&](long c) { return c == 0 ? size_t(0) : std::min(bytes, first + (size_t)(c - 1) * kChunk); };
+  const unsigned cpus = std::thread::hardware_concurrency();
+  const unsigned want = (unsigned)std::min<long>(n, std::min(kMostThreads, cpus / 2));
+  const int slots = (int)std::min<long>(n, kMostSlots);
+  if (bytes < kLeast || want < 2 || !prepare(slots)) {
+    const hipError_t e = hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, st);
+    return e != hipSuccess ? e : hipStreamSynchronize(st);
+  }
+  char* const dst = static_cast<char*>(host);
+  const char* const src = static_cast<const char*>(dev);
+  std::atomic<long> arrived{0};            // chunks in their slots
+  std::atomic<bool> stop{false};
+  std::atomic<unsigned> threads{0};        // set once all have started
+  std::vector<std::atomic<long>> copied(kMostThreads);   // chunks that each thread has finished
+  for (auto& c : copied) c.store(0);
+  auto work = [&](unsigned t) {
+    unsigned T;
+    while ((T = threads.load(std::memory_order_acquire)) == 0) std::this_thread::yield();
+    for (long c = t; c < n; c += T) {
+      while (arrived.load(std::memory_order_acquire) <= c) {
+        if (stop.load(std::memory_order_relaxed)) return;
+        std::this_thread::yield();
+      }
+      std::memcpy(dst + edge(c), buf_ + (c % slots) * kChunk, edge(c + 1) - edge(c));
+      copied[t].fetch_add(1, std::memory_order_release);
+    }
+  };
+  std::vector<std::thread> pool;
+  pool.reserve(want);
+  try {
+    for (unsigned t = 0; t < want; ++t) pool.emplace_back(work, t);
+  } catch (const std::system_error&) {     // as many as there are
+  }
+  const unsigned T = (unsigned)pool.size();
+  if (T == 0) {
+    const hipError_t e = hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, st);
+    return e != hipSuccess ? e : hipStreamSynchronize(st);
+  }
+  threads.store(T, std::memory_order_release);
+  hipError_t err = hipSuccess;
+  auto fetch = [&](long c) {               // chunk c into its slot
+    err = hipMemcpyAsync(buf_ + (c % slots) * kChunk, src + edge(c), edge(c + 1) - edge(c),
+                         hipMemcpyDeviceToHost, st);
+    if (err == hipSuccess) err = hipEventRecord(ev_[c % slots], st);
+  };
+  for (long c = 0; c < slots && err == hipSuccess; ++c) fetch(c);
+  for (long c = 0; c < n && err == hipSuccess; ++c) {
+    err = hipEventSynchronize(ev_[c % slots]);
+    if (err != hipSuccess) break;
+    arrived.store(c + 1, std::memory_order_release);
+    // the slot of a chunk half a ring back is free once its thread has copied it out
+    const long b = c - slots / 2;
+    if (b >= 0 && b + slots < n) {
+      while (copied[b % T].load(std::memory_order_acquire) <= b / T) std::this_thread::yield();
+      fetch(b + slots);
+    }
+  }
+  if (err != hipSuccess) stop.store(true);
+  for (std::thread& t : pool) t.join();
+  if (err != hipSuccess) (void)hipStreamSynchronize(st);   // no copy into the slots is left behind
+  return err;
+}
+
+}  // namespace mgd

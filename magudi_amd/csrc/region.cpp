@@ -15,6 +15,7 @@
 #include <vector>
 
 #include "fused2d.h"
+#include "hostcopy.h"
 #include "line1d.h"
 #include "kernels.h"
 #include "mgd_internal.h"
@@ -92,6 +93,7 @@ struct mgd_region {
   mgd::DevBuf d_patches, d_sources;
   mgd::DevBuf d_damp, d_qtarget, d_srcx, d_srcy;   // fused 2-D tables
   mgd::StageTables tables{};
+  mgd::HostCopy hostcopy;                // staging of large state copies
   int ip_cost = -1, ip_act = -1, has_farfield = 0;
   mgd::FinishInfo fin;                   // the forward finishing pass (set at finalize)
   // HBM-resident state
@@ -2816,8 +2818,7 @@ int mgd_state_get(mgd_region* r, int which, int inst, double* host) {
   DevBuf* b = state_buf(r, which, false);
   if (!b) { set_error("unknown or empty state array"); return MGD_ERR_ARG; }
   const size_t M = (size_t)M_of(r);
-  MGD_HIP(hipMemcpyAsync(host, b->p + inst * M, M * sizeof(double), hipMemcpyDeviceToHost, r->stream));
-  MGD_HIP(hipStreamSynchronize(r->stream));
+  MGD_HIP(r->hostcopy.to_host(host, b->p + inst * M, M * sizeof(double), r->stream));
   return MGD_OK;
 }
 
