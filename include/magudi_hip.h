@@ -331,7 +331,9 @@ int mgd_last_timings(mgd_region* r, double* out, int* launches);
  * n >= 0: at most n save_interval steps), the three inner stage states of its last steps;
  * the adjoint pass recomputes the inner stage states of the other steps from the stored
  * state, three RK stages per step instead of 4 save_interval - 1 per window from a
- * snapshot, with no window buffer.  -1 (default): where nsteps + 3 states (fused path:
+ * snapshot, with no window buffer.  Where the held steps are not limited, half of the memory
+ * left then keeps what the forward stages form of viscous 3-D states for the adjoint stages
+ * at the same states (the stress and heat flux).  -1 (default): where nsteps + 3 states (fused path:
  * nsteps + 6, two recompute buffers) fit in the memory left free less the reserve and MGD_OPT_WINDOW_CACHE is at its default; 0: off
  * (snapshots and windows); 1: on where the states of every step can be allocated.
  * Identical results. */
