@@ -893,13 +893,21 @@ __device__ __forceinline__ double block_sum(double v, double* red) {
 // Several regions in one launch: launch block k belongs to the member m with
 // mem[m].block0 <= k < mem[m + 1].block0 (members in block order), which sees it as tile
 // block (k - block0) mod nblk of instance (k - block0) / nblk.  args[m]: the stage of m.
+// Each lane looks at one member (a walk through the members is a chain of loads).
+static_assert(kMaxGroup <= 64, "a lane for each member");
 __device__ __forceinline__ int group_member(const GroupMember* mem, int nmem, int* blk,
                                             long* inst) {
-  int m = 0;
-  while (m + 1 < nmem && (int)blockIdx.x >= mem[m + 1].block0) ++m;
-  const int lb = (int)blockIdx.x - mem[m].block0;
-  *blk = lb % mem[m].T.nblk;
-  *inst = lb / mem[m].T.nblk;
+  const int lane = threadIdx.x & 63;
+  const bool before = lane < nmem && mem[min(lane, nmem - 1)].block0 <= (int)blockIdx.x;
+  const int m = __builtin_amdgcn_readfirstlane(__popcll(__ballot(before)) - 1);
+  int lb = (int)blockIdx.x - mem[m].block0;
+  const int nblk = mem[m].T.nblk;
+  *inst = 0;
+  if (lb >= nblk) {
+    *inst = lb / nblk;
+    lb %= nblk;
+  }
+  *blk = lb;
   return m;
 }
 

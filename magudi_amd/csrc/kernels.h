@@ -72,6 +72,14 @@ void launch_rk_forward(long M, int stage, double dt, double* q, double* b1, doub
                        const double* rhs, double* qcopy, hipStream_t st);
 void launch_rk_adjoint(long M, int stage, double dt, double* lam, double* b1, double* b2,
                        const double* rhs, hipStream_t st);
+// One copy of a group run.
+struct GroupCopy {
+  const double* src;
+  double* dst;
+  long n;
+};
+// n copies in one launch; `most`: the longest.
+void launch_copy_group(const GroupCopy* items, int n, long most, hipStream_t st);
 void launch_copy(long M, const double* a, double* b, hipStream_t st);
 void launch_fill(long M, double v, double* b, hipStream_t st);
 int reduce_blocks(int np);

@@ -1154,6 +1154,11 @@ __global__ void __launch_bounds__(kBlock) k_copy(long M, const double* __restric
   if (i < M) b[i] = a[i];
 }
 
+__global__ void __launch_bounds__(kBlock) k_copy_group(const GroupCopy* __restrict__ items) {
+  const GroupCopy c = items[blockIdx.y];
+  for (long i = gidx(); i < c.n; i += (long)gridDim.x * kBlock) c.dst[i] = c.src[i];
+}
+
 __global__ void __launch_bounds__(kBlock) k_fill(long M, double v, double* __restrict__ b) {
   const long i = gidx();
   if (i < M) b[i] = v;
@@ -2500,6 +2505,11 @@ void launch_rk_adjoint(long M, int stage, double dt, double* lam, double* b1, do
                        const double* rhs, hipStream_t st) {
   k_rk_adjoint<<<(unsigned)((M + kBlock - 1) / kBlock), kBlock, 0, st>>>(M, stage, dt, lam, b1, b2,
                                                                          rhs);
+}
+
+void launch_copy_group(const GroupCopy* items, int n, long most, hipStream_t st) {
+  const long blocks = (most + kBlock - 1) / kBlock;
+  k_copy_group<<<dim3((unsigned)(blocks < 256 ? blocks : 256), n), kBlock, 0, st>>>(items);
 }
 
 void launch_copy(long M, const double* a, double* b, hipStream_t st) {

@@ -209,6 +209,8 @@ using namespace mgd;
 // (mgd_group_*): the stage arguments of every member and stage are built on the host
 // once per run and read by the kernels from device tables.
 struct mgd_group {
+  long maxcopy = 0;                      // points of the largest member (group copies)
+  mgd::DevBuf dcopy;
   std::vector<mgd_region*> m;
   hipStream_t st = nullptr, st_rec = nullptr;
   hipEvent_t ev_fwd = nullptr, ev_ready[2] = {nullptr, nullptr}, ev_free[2] = {nullptr, nullptr};
@@ -2088,7 +2090,24 @@ int group_tables(mgd_group* G, double dt0, const double* dts, int nsteps, int K,
     }
   }
   G->nblocks = block0;
+  // the copies of all members, one table entry per set (GroupCopySet) and member
+  const int nsnap = nsteps / K + 1, nw = (nsteps + K - 1) / K;
+  std::vector<GroupCopy> copies((size_t)(2 + nsnap + nw) * n);
+  G->maxcopy = 0;
+  for (int k = 0; k < n; ++k) {
+    mgd_region* r = G->m[k];
+    const long M = (long)r->ninst * M_of(r);
+    auto set = [&](int i, const double* src, double* dst) { copies[(size_t)i * n + k] = {src, dst, M}; };
+    G->maxcopy = std::max(G->maxcopy, M);
+    set(0, r->q.p, r->qT.p);
+    set(1, r->resident ? r->wall.p + 4L * nsteps * M : r->q.p, r->q.p);
+    for (int j = 0; j < nsnap; ++j)
+      set(2 + j, r->q.p, r->resident ? r->wall.p : r->snaps.p + (long)j * M);
+    for (int w = 0; w < nw; ++w)
+      set(2 + nsnap + w, r->snaps.p + (long)w * M, w % 2 ? r->window2.p : r->window.p);
+  }
   if (upload_ints(G->dmem, mem.data(), mem.size() * sizeof(GroupMember)) ||
+      upload_ints(G->dcopy, copies.data(), copies.size() * sizeof(GroupCopy)) ||
       upload_ints(G->dfwd, fwd.data(), fwd.size() * sizeof(FwdStage)) ||
       upload_ints(G->drec, rec.data(), rec.size() * sizeof(FwdStage)) ||
       upload_ints(G->dadj, adj.data(), adj.size() * sizeof(AdjStage)))
@@ -2103,13 +2122,20 @@ const FwdStage* stage_table(const DevBuf& b, int sidx, int n) {
 // fused_forward_pass + the enqueue_forward_ck bookkeeping of every member, one launch
 // per stage for all members, on the group stream (every member's stream is the group's
 // for the duration of the run).
+// Copies of all members in one launch: the final states (0), the resident final states into q
+// (1), q into snapshot j (2 + j; j = 0 also the resident start), snapshot w into its window
+// (after the snapshots).  A launch for each member costs as much as a stage of all of them.
+void group_copy(mgd_group* G, int set, hipStream_t st) {
+  const int n = (int)G->m.size();
+  launch_copy_group(reinterpret_cast<const GroupCopy*>(G->dcopy.p) + (size_t)set * n, n, G->maxcopy, st);
+}
+
 int group_forward_pass(mgd_group* G, int nsteps, int K) {
   const int n = (int)G->m.size(), nst = 4 * nsteps;
   const GroupMember* mem = reinterpret_cast<const GroupMember*>(G->dmem.p);
-  for (mgd_region* r : G->m) {
-    launch_fill(r->ninst, 0.0, r->acc_J.p, G->st);
-    launch_copy((long)r->ninst * M_of(r), r->q.p, r->resident ? r->wall.p : r->snaps.p, G->st);
-  }
+  for (mgd_region* r : G->m) launch_fill(r->ninst, 0.0, r->acc_J.p, G->st);
+  const bool resident = G->m[0]->resident;   // the same for every member
+  group_copy(G, 2, G->st);
   for (int s = 0; s < nsteps; ++s) {
     for (int i = 1; i <= 4; ++i) {
       const int sidx = 4 * s + i - 1;
@@ -2118,20 +2144,13 @@ int group_forward_pass(mgd_group* G, int nsteps, int K) {
         return rc;
       for (mgd_region* r : G->m) reduce_chunk(r, r->jpart, n_cost(r), nst, sidx, false);
     }
-    if ((s + 1) % K == 0)
-      for (mgd_region* r : G->m) {
-        if (r->resident) continue;
-        const long M = (long)r->ninst * M_of(r);
-        launch_copy(M, r->q.p, r->snaps.p + (long)((s + 1) / K) * M, G->st);
-      }
+    if ((s + 1) % K == 0 && !resident) group_copy(G, 2 + (s + 1) / K, G->st);
   }
-  for (mgd_region* r : G->m) {
-    const long M = (long)r->ninst * M_of(r);
-    if (r->resident) launch_copy(M, r->wall.p + 4L * nsteps * M, r->q.p, G->st);   // final state
+  if (resident) group_copy(G, 1, G->st);     // final state
+  for (mgd_region* r : G->m)
     if (n_cost(r) > 0)
       launch_stage_accumulate(r->ssum.p, nst, r->wts.p, r->acc_J.p, r->ninst, 0, G->st);
-    launch_copy((long)r->ninst * M_of(r), r->q.p, r->qT.p, G->st);
-  }
+  group_copy(G, 0, G->st);
   return MGD_OK;
 }
 
@@ -2142,17 +2161,14 @@ int group_adjoint_pass(mgd_group* G, const double* dts, int nsteps, int K) {
   const int n = (int)G->m.size(), nst = 4 * nsteps;
   const GroupMember* mem = reinterpret_cast<const GroupMember*>(G->dmem.p);
   const bool resident = G->m[0]->resident;   // the same for every member
-  const int nw = resident ? 1 : (nsteps + K - 1) / K;
+  const int nw = resident ? 1 : (nsteps + K - 1) / K, nsnap = nsteps / K + 1;
   if (resident) K = nsteps;                  // one window: the resident states
   for (mgd_region* r : G->m) launch_fill(r->ninst, 0.0, r->acc_S.p, G->st);
   MGD_HIP(hipEventRecord(G->ev_fwd, G->st));
   MGD_HIP(hipStreamWaitEvent(G->st_rec, G->ev_fwd, 0));
   auto recompute = [&](int w) -> int {
     const int t0w = w * K, t1w = std::min(nsteps, t0w + K);
-    for (mgd_region* r : G->m) {
-      const long M = (long)r->ninst * M_of(r);
-      launch_copy(M, r->snaps.p + (long)w * M, (w % 2 ? r->window2.p : r->window.p), G->st_rec);
-    }
+    group_copy(G, nsnap + 2 + w, G->st_rec);
     for (int t = t0w; t < t1w; ++t)
       for (int i = 1; i <= 4; ++i)
         if (int rc = launch_fwd_stage2d_group(kGroupShape, mem, n, G->nblocks,
