@@ -492,7 +492,7 @@ def monopole_legs(a, extras):
            "checkpoint_plan": plan,
            "value": value, "unit": "grid-pt-steps/s", "ms_per_run": t_step * 1e3,
            "path": "fused 2-D stage kernels",
-           "tile_shape": ["32x16", "16x32", "16x16", "24x16", "16x16/2", "16x12/2"][R.tile_shape]
+           "tile_shape": ["32x16", "16x32", "16x16", "24x16", "16x16/2", "16x12"][R.tile_shape]
            if R.tile_shape >= 0 else "generic",
            "kernels": {k: {"avg_launch_us": round(ms * 1e3, 3), "bytes_per_launch": b,
                            "achieved_GBs": round(b / (ms * 1e-3) / 1e9, 1),
