@@ -320,7 +320,7 @@ int mgd_last_timings(mgd_region* r, double* out, int* launches);
  * n > 0: at most n.
  * MGD_OPT_Z_CHUNK: planes per work unit of the 3-D z marches (periodic 3-D regions): 0
  * (default) autotune at the first run -- one forward RK4 step and one adjoint rhs timed
- * for each of 32, 64 and 128, and for 8 and 16 on grids that these leave too few units --,
+ * for each of 32, 64 and 128, and for smaller ones on grids that these leave too few units --,
  * or 32, 64 or 128 fixed.  MGD_OPT_MARCH_TILE: the width of
  * their tiles, 16 (16 x 16 points, 256 threads) or 32 (32 x 16, 512 threads; x sizes that
  * are multiples of 32), 0 (default) autotuned with the z chunk; the forward march and the
