@@ -1978,6 +1978,14 @@ std::vector<uintptr_t> graph_key(mgd_region* r, int kind, std::initializer_list<
   return k;
 }
 
+// Drops the captured runs; the next ones are captured anew.
+void drop_graphs(mgd_region* r) {
+  for (GraphSlot& gs : r->graphs) {
+    if (gs.exec) (void)hipGraphExecDestroy(gs.exec);
+    gs.exec = nullptr;
+  }
+}
+
 template <class F>
 int run_device_work(mgd_region* r, bool use_graph, int slot, const std::vector<uintptr_t>& key,
                     F&& enqueue) {
@@ -2472,8 +2480,7 @@ int mgd_region_create(const mgd_region_desc* d, const double* coords, mgd_region
 int mgd_region_destroy(mgd_region* r) {
   if (!r) return MGD_OK;
   if (r->stream) (void)hipStreamSynchronize(r->stream);
-  for (GraphSlot& gs : r->graphs)
-    if (gs.exec) (void)hipGraphExecDestroy(gs.exec);
+  drop_graphs(r);
   if (r->ev0) (void)hipEventDestroy(r->ev0);
   if (r->ev1) (void)hipEventDestroy(r->ev1);
   for (hipEvent_t e : r->tev) (void)hipEventDestroy(e);
@@ -2555,6 +2562,11 @@ int mgd_region_finalize(mgd_region* r) {
   const int nd = r->nd, nv = r->nv;
   const long N = r->N;
   const double g = r->desc.gamma;
+  // A region finalized before, with patches, sources or fields set since: captured runs and the
+  // group tiling hold copies of the masks and addresses that are set anew here (StageTables,
+  // TileInfo, launch arguments), so both are made again at their next use.
+  drop_graphs(r);
+  r->g_built = false;
   std::memset(&r->hpatches, 0, sizeof r->hpatches);
   r->hpatches.count = (int)r->patches.size();
   for (size_t ip = 0; ip < r->patches.size(); ++ip) {
