@@ -1314,26 +1314,25 @@ int plan_window_cache(mgd_region* r, int nsteps, int K, long M) {
   return MGD_OK;
 }
 
-// Step mode on the 3-D marches: the stress slots that a forward stage forms of its input are
-// those that the adjoint stage at the same state needs.  The forward pass keeps them for as
-// many of the last held steps as half of the `rest` of the budget takes (none where the caller
-// limits the held steps), which saves the adjoint pass its stress kernel: 468 of 2160 us per
-// stage on 256^3, 47 of 226 on 100^3, 20 of 79 on 64^3.
-void plan_stress_cache(mgd_region* r, int nsteps, size_t rest) {
-  int n = 0;
-  if (r->sreuse && r->opt_cache < 0)
-    n = (int)std::min<size_t>((size_t)r->nscache, rest / 2 / (4 * r->G.bytes()));
-  const size_t step = 4 * r->G.n;
-  // what an earlier run held stays unless the plan is well above it, as for the states
-  const int have = step > 0 && r->gcache.n % step == 0 ? (int)(r->gcache.n / step) : 0;
-  if (n > 0 && have > 0 && have <= r->nscache && n <= have + std::max(2, have / 16)) n = have;
-  if (r->gcache.n != step * n) r->gcache.release();
-  if (n > 0 && r->gcache.alloc(step * n) != MGD_OK) {
-    (void)hipGetLastError();
-    n = 0;
+// Entries that a cache of `unit`-double entries should have, of which `buf` holds some: `plan`,
+// or what it holds when that is near it (the free memory moves a little between runs, and a
+// captured run is good only for the buffers it was captured with).  At most a sixteenth (or two)
+// below the plan; above it, at most 2 GiB of the reserve of storage_budget.
+int cache_entries(const DevBuf& buf, size_t unit, int plan, int most) {
+  const int have = unit > 0 && buf.n % unit == 0 ? (int)(buf.n / unit) : 0;
+  const int above = unit > 0 ? (int)std::min<size_t>(((size_t)2 << 30) / (unit * sizeof(double)), 1 << 20) : 0;
+  if (plan <= 0 || have <= 0 || have > most) return plan;
+  return plan <= have + std::max(2, have / 16) && have <= plan + above ? have : plan;
+}
+
+// Allocates `want` entries of `unit` doubles, or half as many for as long as they do not fit.
+int alloc_entries(DevBuf& buf, size_t unit, int want) {
+  if (buf.n != unit * want) buf.release();
+  while (want > 0 && buf.alloc(unit * want) != MGD_OK) {
+    (void)hipGetLastError();               // fewer than planned: the rest are computed again
+    want /= 2;
   }
-  r->ngcache = n;
-  r->gcache_first = nsteps - n;
+  return want;
 }
 
 // The kept stress slots of the state of stage i (1 .. 4) of step t, or null.
@@ -1351,15 +1350,24 @@ double* kept_stress(mgd_region* r, int t, int i) {
 // (MGD_OPT_WINDOW_CACHE n >= 0: at most n save_interval steps); the adjoint pass recomputes
 // three stages per step not held, against 4 save_interval - 1 per window in window mode.
 // The recompute buffer holds three states; the fused path has two (the recompute of one
-// step shares its launches with the adjoint stages of the next).  Window mode (always for
-// the fused members of a group launch): snapshots every K steps, a window buffer and, on
-// the generic kernels, whole cached windows.
+// step shares its launches with the adjoint stages of the next).
+// On the viscous 3-D marches step mode also keeps stress slots: those of the recomputed stages
+// (sreuse) and, as half of what is then left of the budget takes (none where the caller limits
+// the held steps), those that the forward stages of the last held steps formed of their inputs,
+// which the adjoint stages at the same states need: they save the adjoint pass its stress
+// kernel, 468 of 2160 us per stage on 256^3, 47 of 226 on 100^3, 20 of 79 on 64^3.
+// The whole plan is made first, and what it does not keep of an earlier run's storage is given
+// back before anything is allocated: the budget counts all of that as free.
+// Window mode (always for the fused members of a group launch): snapshots every K steps, a
+// window buffer and, on the generic kernels, whole cached windows.
 int plan_plain_storage(mgd_region* r, int nsteps, int K, long M) {
   const size_t S = (size_t)M * sizeof(double);
   const bool fused = fused_ok(r);
   const size_t nrec = fused ? 6 : 3;   // states of the recompute buffers
   r->rec_step = -1;
   r->step_mode = false;
+  r->sreuse = false;
+  r->nscache = r->ngcache = 0;
   const bool allowed = !(fused && r->group_run);
   bool step = r->opt_step == 1 && allowed;
   size_t budget = 0;
@@ -1367,61 +1375,54 @@ int plan_plain_storage(mgd_region* r, int nsteps, int K, long M) {
     budget = storage_budget(r);
     if (r->opt_step < 0) step = r->opt_cache < 0 && (size_t)(nsteps + nrec) * S <= budget;
   }
-  size_t fixed = (size_t)(nsteps + nrec) * S;
   if (step) {
+    size_t fixed = (size_t)(nsteps + nrec) * S;
+    const size_t GB = r->G.bytes();
+    bool reuse = !fused && stress_reuse_path(r->geo, r->fin, (int)r->sources.size()) && GB > 0 &&
+                 fixed + 3 * GB <= budget;
+    if (reuse) fixed += 3 * GB;
+    size_t rest = budget > fixed ? budget - fixed : 0;
+    const int most = r->opt_cache < 0 ? nsteps : (int)std::min((long)nsteps, (long)r->opt_cache * K);
+    int nsc = (int)std::min<size_t>((size_t)most, rest / (3 * S));
+    nsc = cache_entries(r->scache, (size_t)3 * M, nsc, most);
+    rest = rest > 3 * S * nsc ? rest - 3 * S * nsc : 0;
+    int ngc = 0;
+    if (reuse && r->opt_cache < 0) {
+      ngc = (int)std::min<size_t>((size_t)nsc, rest / 2 / (4 * GB));
+      ngc = cache_entries(r->gcache, 4 * r->G.n, ngc, nsc);
+    }
     for (int k = 0; k < mgd_region::kMaxCache; ++k) r->wcache[k].release();
     r->ncache = 0;
     r->snaps.release();
     if (r->window.n != (size_t)3 * M) r->window.release();
     if (fused && r->window2.n != (size_t)3 * M) r->window2.release();
     if (r->sstore.n != (size_t)nsteps * M) r->sstore.release();
-    if (r->window.alloc((size_t)3 * M) || (fused && r->window2.alloc((size_t)3 * M)) ||
-        r->sstore.alloc((size_t)nsteps * M)) {
-      // taken meanwhile (regions of a group plan one after another): window mode
-      (void)hipGetLastError();
-      step = false;
+    if (!reuse) r->sbuf.release();
+    if (r->scache.n != (size_t)3 * M * nsc) r->scache.release();
+    if (r->gcache.n != 4 * r->G.n * ngc) r->gcache.release();
+    if (r->window.alloc((size_t)3 * M) == MGD_OK &&
+        (!fused || r->window2.alloc((size_t)3 * M) == MGD_OK) &&
+        r->sstore.alloc((size_t)nsteps * M) == MGD_OK) {
+      if (reuse && r->sbuf.alloc(3 * r->G.n) != MGD_OK) {
+        (void)hipGetLastError();
+        reuse = false;
+        ngc = 0;
+      }
+      r->sreuse = reuse;
+      r->nscache = alloc_entries(r->scache, (size_t)3 * M, nsc);
+      r->ngcache = alloc_entries(r->gcache, 4 * r->G.n, std::min(ngc, r->nscache));
+      r->scache_first = nsteps - r->nscache;
+      r->gcache_first = nsteps - r->ngcache;
+      r->step_mode = true;
+      return MGD_OK;
     }
-  }
-  r->sreuse = false;
-  if (step && !fused && stress_reuse_path(r->geo, r->fin, (int)r->sources.size()) && r->G.n > 0 &&
-      fixed + 3 * r->G.bytes() <= budget) {
-    if (r->sbuf.alloc(3 * r->G.n) == MGD_OK) {
-      r->sreuse = true;
-      fixed += 3 * r->G.bytes();
-    } else {
-      (void)hipGetLastError();
-    }
-  }
-  if (!r->sreuse) r->sbuf.release();
-  if (step) {
-    const size_t rest = budget > fixed ? budget - fixed : 0;
-    int nsc = (int)std::min<size_t>((size_t)nsteps, rest / (3 * S));
-    if (r->opt_cache >= 0) nsc = std::min(nsc, r->opt_cache * K);
-    // a cache held from an earlier run stays unless the plan is well above it (the free
-    // memory moves a little between runs; reallocating ~100 GB each run would cost more
-    // than the few steps it adds)
-    const size_t step3 = (size_t)3 * M;
-    const int have = r->scache.n % step3 == 0 ? (int)(r->scache.n / step3) : -1;
-    if (have > 0 && have <= nsteps && (r->opt_cache < 0 || have <= r->opt_cache * K) &&
-        nsc <= have + std::max(2, have / 16))
-      nsc = have;
-    if (r->scache.n != (size_t)3 * nsc * M) r->scache.release();
-    while (nsc > 0 && r->scache.alloc((size_t)3 * nsc * M) != MGD_OK) {
-      (void)hipGetLastError();             // fewer steps than planned: the rest recompute
-      nsc /= 2;
-    }
-    r->nscache = nsc;
-    r->scache_first = nsteps - nsc;
-    r->step_mode = true;
-    plan_stress_cache(r, nsteps, budget > fixed + 3 * S * nsc ? budget - fixed - 3 * S * nsc : 0);
-    return MGD_OK;
+    // taken meanwhile (regions of a group plan one after another): window mode
+    (void)hipGetLastError();
   }
   r->sstore.release();
   r->scache.release();
   r->sbuf.release();
   r->gcache.release();
-  r->ngcache = 0;
-  r->nscache = 0;
   const int nsnap = nsteps / K + 1;
   if (r->snaps.alloc((size_t)nsnap * M) || r->window.alloc((size_t)4 * K * M)) return MGD_ERR_HIP;
   return plan_window_cache(r, nsteps, K, M);
