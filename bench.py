@@ -662,7 +662,7 @@ def main():
     for _ in range(max(1, a.warmup)):
         K.one()
     t_step, J, t_fwd, launches, with_copy, march_ms = K.timed(a.steps)
-    march_shape = K.R.march_shape
+    march_shape = K.R.march_units
     plan = K.R.checkpoint_plan
     value = K.pts / t_step
     print(f"headline: {t_step:.3f} s per pass ({value:.4g} grid-pt-steps/s)", file=sys.stderr,

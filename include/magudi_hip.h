@@ -321,10 +321,10 @@ int mgd_last_timings(mgd_region* r, double* out, int* launches);
  * MGD_OPT_Z_CHUNK: planes per work unit of the 3-D z marches (periodic 3-D regions): 0
  * (default) autotune at the first run -- one forward RK4 step and one adjoint rhs timed
  * for each of 32, 64 and 128, and for smaller ones on grids that these leave too few units --,
- * or 32, 64 or 128 fixed.  MGD_OPT_MARCH_TILE: the width of
- * their tiles, 16 (16 x 16 points, 256 threads) or 32 (32 x 16, 512 threads; x sizes that
- * are multiples of 32), 0 (default) autotuned with the z chunk; the forward march and the
- * adjoint marches are tuned apart.  No result depends on either.
+ * or fixed: 1 .. 1024.  MGD_OPT_MARCH_TILE: the width of
+ * their tiles, 16 (16 x 16 points, 256 threads) or 32 (32 x 16, 512 threads), 0 (default)
+ * autotuned with the z chunk; the forward march and the adjoint marches are tuned apart.
+ * No result depends on either.
  * MGD_OPT_STEP_STORE (generic-kernel path; fused 2-D path where the stage states are not
  * resident, except for the members of a group launch): the checkpointed forward pass keeps the state
  * at the start of every step (nsteps states) and, in the memory left (MGD_OPT_WINDOW_CACHE
@@ -358,8 +358,10 @@ int mgd_region_get_checkpoint_plan(mgd_region* r, int* plan);
 /* Tile shape the fused 2-D kernels use now (-1: the region runs the generic kernels). */
 int mgd_region_get_tile_shape(mgd_region* r, int* shape);
 /* Work-unit shape the 3-D marches use now (MGD_OPT_MARCH_TILE, MGD_OPT_Z_CHUNK; after the
- * autotuner, if it ran): shape[0..1] tile width and z chunk of the forward march (chunks
- * below 32 are reported as 32), shape[2..3] those of the adjoint marches. */
+ * autotuner, if it ran): shape[0..1] tile width and z chunk of the forward march,
+ * shape[2..3] those of the adjoint marches. */
+int mgd_region_get_march_units(mgd_region* r, int* shape);
+/* The same with chunks below 32 planes given as 32, for callers that know no smaller ones. */
 int mgd_region_get_march_shape(mgd_region* r, int* shape);
 
 /* Times one kernel on the region stream with HIP events after one warm-up repetition.

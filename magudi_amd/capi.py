@@ -89,6 +89,7 @@ def lib():
         "mgd_sync": [vp],
         "mgd_region_set_option": [vp, C.c_int, C.c_int],
         "mgd_region_get_tile_shape": [vp, C.POINTER(C.c_int)],
+        "mgd_region_get_march_units": [vp, C.POINTER(C.c_int)],
         "mgd_region_get_march_shape": [vp, C.POINTER(C.c_int)],
         "mgd_region_get_checkpoint_plan": [vp, C.POINTER(C.c_int)],
         "mgd_time_kernel": [vp, C.c_int, C.c_int, dp, dp],

@@ -122,7 +122,7 @@ struct mgd_region {
   // (k_dual_stage2d) or launches them one after the other (the autotuner's choice; with a
   // fixed tile shape: shared for one instance, where single launches leave the GPU half idle)
   bool dual = true;
-  int opt_zchunk = 0;                    // MGD_OPT_Z_CHUNK: 0 autotune, else 32, 64 or 128
+  int opt_zchunk = 0;                    // MGD_OPT_Z_CHUNK: 0 autotune, else the planes
   int opt_mtile = 0;                     // MGD_OPT_MARCH_TILE: 0 autotune, else 16 or 32
   bool zc_tuned = false;
   int force_plain = 0;
@@ -945,7 +945,7 @@ int tune_tiling(mgd_region* r) {
   return install_tiling(r, best);
 }
 
-// The shape of the 3-D marches' work units -- the z chunk (8 to 128 planes) and the tile
+// The shape of the 3-D marches' work units -- the z chunk (2 to 128 planes) and the tile
 // width (16 or 32 points, 16 rows) -- unless fixed by option: one forward RK4 step
 // (stress pass and march per stage, out of place) and one adjoint rhs (stress pass and
 // the two marches, where they serve the region) timed with HIP events for each shape, in
@@ -991,16 +991,16 @@ int tune_march(mgd_region* r) {
     const long columns = units(nz), room = mt == 32 ? 256 : 512;
     const int fill = columns <= room ? (int)((nz + room / columns - 1) / (room / columns)) : 0;
     std::vector<int> chunks = {4, 8, 16, 32, 64, 128};
-    if (fill >= 2 && fill < 32 && fill != 4 && fill != 8 && fill != 16) chunks.push_back(fill);
+    if (r->opt_zchunk != 0) chunks = {r->opt_zchunk};
+    else if (fill >= 2 && fill < 32 && fill != 4 && fill != 8 && fill != 16) chunks.push_back(fill);
     for (int zc : chunks) {
       const bool want = zc == fill ? units(32) < 512
                         : zc == 4  ? units(8) < 256
                         : zc < 32  ? units(32) < 512
                                    : zc == 32 || units(zc) >= 128;
-      if (r->opt_zchunk == 0 ? want : zc == r->opt_zchunk) shapes.emplace_back(mt, zc);
+      if (r->opt_zchunk != 0 || want) shapes.emplace_back(mt, zc);
     }
   }
-  if (shapes.empty()) shapes.emplace_back(16, 64);
   // the forward step and the adjoint rhs are timed apart and each keeps its own shape
   hipEvent_t evm = nullptr;
   MGD_HIP(hipEventCreate(&evm));
@@ -2790,12 +2790,18 @@ int mgd_region_set_time_offsets(mgd_region* r, const double* offsets) {
   return MGD_OK;
 }
 
-int mgd_region_get_march_shape(mgd_region* r, int* shape) {
+int mgd_region_get_march_units(mgd_region* r, int* shape) {
   if (!r || !shape) { set_error("null argument"); return MGD_ERR_ARG; }
   shape[0] = r->geo.mtile;
-  shape[1] = std::max(r->geo.zchunk, 32);   // reported as 32 below it
+  shape[1] = r->geo.zchunk;
   shape[2] = r->geo.mtile_adj;
-  shape[3] = std::max(r->geo.zchunk_adj, 32);
+  shape[3] = r->geo.zchunk_adj;
+  return MGD_OK;
+}
+
+int mgd_region_get_march_shape(mgd_region* r, int* shape) {
+  if (int rc = mgd_region_get_march_units(r, shape)) return rc;
+  for (int k : {1, 3}) shape[k] = std::max(shape[k], 32);
   return MGD_OK;
 }
 
@@ -2844,8 +2850,8 @@ int mgd_region_set_option(mgd_region* r, int option, int value) {
       r->opt_step = value;
       return MGD_OK;
     case MGD_OPT_Z_CHUNK:
-      if (value != 0 && value != 32 && value != 64 && value != 128) {
-        set_error("z chunk: 0 (autotune), 32, 64 or 128");
+      if (value < 0 || value > 1024) {
+        set_error("z chunk: 0 (autotune) or 1 .. 1024");
         return MGD_ERR_ARG;
       }
       r->opt_zchunk = value;
@@ -2855,10 +2861,6 @@ int mgd_region_set_option(mgd_region* r, int option, int value) {
     case MGD_OPT_MARCH_TILE:
       if (value != 0 && value != 16 && value != 32) {
         set_error("march tile: 0 (autotune), 16 or 32");
-        return MGD_ERR_ARG;
-      }
-      if (value == 32 && r->nd == 3 && r->geo.n[0] % 32 != 0) {
-        set_error("march tile 32 needs an x size that is a multiple of 32");
         return MGD_ERR_ARG;
       }
       r->opt_mtile = value;

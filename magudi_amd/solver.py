@@ -280,8 +280,8 @@ class Region:
         check(capi.lib().mgd_region_set_option(self.handle, capi.OPT_STEP_STORE, int(mode)))
 
     def set_z_chunk(self, zc: int):
-        """MGD_OPT_Z_CHUNK: 0 autotunes the 3-D marches' z chunk at the first run, or 32,
-        64, 128 fixes it."""
+        """MGD_OPT_Z_CHUNK: 0 autotunes the 3-D marches' z chunk at the first run, 1 .. 1024
+        fixes it."""
         check(capi.lib().mgd_region_set_option(self.handle, capi.OPT_Z_CHUNK, int(zc)))
 
     def set_march_tile(self, width: int):
@@ -290,9 +290,16 @@ class Region:
         check(capi.lib().mgd_region_set_option(self.handle, capi.OPT_MARCH_TILE, int(width)))
 
     @property
-    def march_shape(self):
+    def march_units(self):
         """((tile width, z chunk) of the forward march, (tile width, z chunk) of the adjoint
         marches) in use (after the autotuner, if it ran)."""
+        out = (C.c_int * 4)()
+        check(capi.lib().mgd_region_get_march_units(self.handle, out))
+        return (out[0], out[1]), (out[2], out[3])
+
+    @property
+    def march_shape(self):
+        """``march_units`` with z chunks below 32 given as 32."""
         out = (C.c_int * 4)()
         check(capi.lib().mgd_region_get_march_shape(self.handle, out))
         return (out[0], out[1]), (out[2], out[3])
@@ -312,12 +319,12 @@ class Region:
     @property
     def march_tile(self) -> int:
         """The forward march's tile width in use."""
-        return self.march_shape[0][0]
+        return self.march_units[0][0]
 
     @property
     def z_chunk(self) -> int:
         """The forward march's z chunk in use."""
-        return self.march_shape[0][1]
+        return self.march_units[0][1]
 
     def kernel_timer(self, on: bool, which: int = None):
         """Starts (on) or stops per-launch HIP-event timing of the z-march forward kernel
