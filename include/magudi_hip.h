@@ -319,7 +319,7 @@ int mgd_last_timings(mgd_region* r, double* out, int* launches);
  * preparation less a reserve of max(8 GiB, 1/32 of the device), at most 8; 0: none;
  * n > 0: at most n.
  * MGD_OPT_Z_CHUNK: planes per work unit of the 3-D z marches (periodic 3-D regions): 0
- * (default) autotune at the first run -- one forward RK4 step and one adjoint rhs timed
+ * (default) autotune at the first run -- one forward RK4 step and one adjoint RK stage timed
  * for each of 32, 64 and 128, and for smaller ones on grids that these leave too few units --,
  * or fixed: 1 .. 1024.  MGD_OPT_MARCH_TILE: the width of
  * their tiles, 16 (16 x 16 points, 256 threads) or 32 (32 x 16, 512 threads), 0 (default)

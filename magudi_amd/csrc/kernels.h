@@ -57,10 +57,6 @@ bool launch_rhs_adjoint(const Geo& g, const Patches* P, const double* q, const d
 // heat-flux kernel (9 slots of the 12-slot gradient buffer S); the march itself, which
 // writes rhs, or with rk (rk->yout set, not q) applies the RK4 stage out of place.
 bool fwd3d_march_path(const Geo& g, const FinishInfo& fin, int nsrc);
-// Rows of a march tile, and the work units of a march with tiles of mtile x kMarchRows points
-// and zc planes per unit (per instance).
-constexpr int kMarchRows = 16;
-int march_units(const Geo& g, int mtile, int zc);
 // Whether the forward and the adjoint rhs both run on the 3-D marches, each from the stress
 // / heat-flux slots of its state that launch_stress3d writes into G: then slots the forward
 // stage computed serve the adjoint stage about the same state.

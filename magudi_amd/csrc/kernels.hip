@@ -9,6 +9,7 @@
 
 #include "device.h"
 #include "kernels.h"
+#include "march_shapes.h"
 
 namespace mgd {
 
@@ -2299,13 +2300,9 @@ static void with_stage(const Geo& g, int stage, F&& f) {
     default: go(std::integral_constant<int, 4>{}); break;
   }
 }
-int march_units(const Geo& g, int mtile, int zc) {
-  return ((g.n[0] + mtile - 1) / mtile) * ((g.n[1] + kMarchRows - 1) / kMarchRows) *
-         ((g.n[2] + zc - 1) / zc);
-}
 // grid of a march: its work units padded to a multiple of 8
 static dim3 units_grid(const Geo& g, int mtile, int zc) {
-  return dim3(8 * ((march_units(g, mtile, zc) + 7) / 8), 1, g.ninst);
+  return dim3(8 * ((march_units(g.n, mtile, zc) + 7) / 8), 1, g.ninst);
 }
 // The gradient / stress pass runs on 16 x 16 tiles, two work-groups a CU (256^3: 464 us, 480
 // on 32 x 16 with one; 64^3: 54 and 80), over chunks of at most 64 planes (500 us at 128).

@@ -1,0 +1,77 @@
+// march_shapes.h -- the work-unit shapes of the 3-D marches that the autotuner tries, and how it
+// picks one from their timings (host code without HIP).
+#pragma once
+#include <algorithm>
+#include <vector>
+
+namespace mgd {
+
+// Rows of a march tile.
+constexpr int kMarchRows = 16;
+
+// Work units of a march over an nx x ny x nz grid: tiles of mtile x kMarchRows points, zc planes
+// per unit.
+inline int march_units(const int* n, int mtile, int zc) {
+  return ((n[0] + mtile - 1) / mtile) * ((n[1] + kMarchRows - 1) / kMarchRows) *
+         ((n[2] + zc - 1) / zc);
+}
+
+struct MarchShape {
+  int tile, chunk;
+};
+
+// Tile widths of 16 and 32 points, unless one is fixed (opt_tile), with a fixed chunk
+// (opt_chunk) as it is; else with every chunk of 32, 64 and 128 planes but those that leave most
+// of the GPU idle (fewer units than half its 256 CUs, unless a chunk of 32 is no better off), and
+// shorter ones only where 32 planes do not fill it: their units spend most of their planes on the
+// z windows' lead-in.  Among those the one whose units just fill the GPU in one go (two
+// work-groups of a 16-wide tile per CU, one of a 32-wide): forward and adjoint run of 64^3 8.1 ms
+// at 8 planes, 5.8 at 4, 5.7 at 2; of 100^3 16.6 at 8, 14.5 at 10.
+inline std::vector<MarchShape> march_shapes(const int* n, int instances, int opt_tile,
+                                            int opt_chunk) {
+  std::vector<MarchShape> shapes;
+  for (int tile : {16, 32}) {
+    if (opt_tile != 0 && tile != opt_tile) continue;
+    if (opt_chunk != 0) {
+      shapes.push_back({tile, opt_chunk});
+      continue;
+    }
+    const auto units = [&](int zc) { return (long)instances * march_units(n, tile, zc); };
+    if (units(32) < 512) {
+      const long columns = units(n[2]), room = tile == 32 ? 256 : 512;
+      const int fill = columns <= room ? (int)((n[2] + room / columns - 1) / (room / columns)) : 0;
+      if (units(8) < 256) shapes.push_back({tile, 4});
+      shapes.push_back({tile, 8});
+      shapes.push_back({tile, 16});
+      if (fill >= 2 && fill < 32 && fill != 8 && fill != 16 && !(fill == 4 && units(8) < 256))
+        shapes.push_back({tile, fill});
+    }
+    for (int chunk : {32, 64, 128})
+      if (chunk == 32 || units(chunk) >= 128) shapes.push_back({tile, chunk});
+  }
+  return shapes;
+}
+
+// The shapes of the least forward and the least adjoint time among n: sample(k, &f, &a) times
+// shape k once and says whether it could.  Two rounds over every shape, since one sample in
+// some is off by 10 % and more, then a third among those within a twentieth of the best (the
+// samples of later rounds repeat within 1 %); the least sample of each counts.
+template <class F>
+bool pick_march_shapes(int n, F&& sample, int* forward, int* adjoint) {
+  std::vector<float> f(n), a(n);
+  for (int round = 0; round < 3; ++round) {
+    const float fm = *std::min_element(f.begin(), f.end()), am = *std::min_element(a.begin(), a.end());
+    for (int k = 0; k < n; ++k) {
+      if (round == 2 && f[k] > 1.05f * fm && a[k] > 1.05f * am) continue;
+      float fk = 0.f, ak = 0.f;
+      if (!sample(k, &fk, &ak)) return false;
+      f[k] = round == 0 ? fk : std::min(f[k], fk);
+      a[k] = round == 0 ? ak : std::min(a[k], ak);
+    }
+  }
+  *forward = (int)(std::min_element(f.begin(), f.end()) - f.begin());
+  *adjoint = (int)(std::min_element(a.begin(), a.end()) - a.begin());
+  return true;
+}
+
+}  // namespace mgd

@@ -18,6 +18,7 @@
 #include "hostcopy.h"
 #include "line1d.h"
 #include "kernels.h"
+#include "march_shapes.h"
 #include "mgd_internal.h"
 
 namespace mgd {
@@ -947,19 +948,17 @@ int tune_tiling(mgd_region* r) {
 
 // The shape of the 3-D marches' work units -- the z chunk (2 to 128 planes) and the tile
 // width (16 or 32 points, 16 rows) -- unless fixed by option: one forward RK4 step
-// (stress pass and march per stage, out of place) and one adjoint rhs (stress pass and
-// the two marches, where they serve the region) timed with HIP events for each shape, in
-// two interleaved rounds (the second among the shapes within a tenth of the fastest), the
-// fastest round of each compared; the forward march (with
-// the stress pass) and the adjoint marches each keep their own.  No value depends on the
-// shape.
+// (stress pass and march per stage, out of place) and one adjoint RK stage (stress pass and
+// the two marches, where they serve the region) timed with HIP events for each shape of
+// march_shapes; the forward march (with the stress pass) and the adjoint marches each keep
+// their own.  No value depends on the shape.
 int tune_march(mgd_region* r) {
   r->zc_tuned = true;
   const long M = (long)r->ninst * M_of(r);
   if (int rc = ensure_adjoint(r)) return rc;
   if (r->qs.alloc(M) || r->qy.alloc(M) || r->qs_alt2.alloc(M)) return MGD_ERR_HIP;
   const double dt = 1e-3;
-  // the state copies, one forward RK4 step, then (after event `mid`, if given) one adjoint rhs
+  // the state copies, one forward RK4 step, then (after event `mid`, if given) one adjoint stage
   auto round_trip = [&](hipEvent_t mid = nullptr) {
     launch_copy(M, r->q.p, r->qs.p, r->stream);
     launch_copy(M, r->q.p, r->b2.p, r->stream);
@@ -974,75 +973,35 @@ int tune_march(mgd_region* r) {
       launch_fwd3d_march(r->geo, rk.y, r->G.p, r->fin.kolmogorov, r->rhs.p, &rk, r->stream);
     }
     if (mid) (void)hipEventRecord(mid, r->stream);
+    const RkStage rk{3, dt, r->lam.p, r->qy.p, r->qs_alt2.p, nullptr};
     launch_rhs_adjoint(r->geo, dpatches(r), r->qs.p, r->lam.p, r->rhs.p, r->w.p, r->G.p, r->t.p,
-                       r->T1.p, r->S.p, nullptr, 0, 1.0, r->fin, r->stream);
+                       r->T1.p, r->S.p, nullptr, 0, 1.0, r->fin, r->stream, &rk);
   };
-  std::vector<std::pair<int, int>> shapes;   // (tile width, z chunk)
-  for (int mt : {16, 32}) {
-    if (r->opt_mtile != 0 && mt != r->opt_mtile) continue;
-    // a fixed chunk as it is; else every chunk but those that leave most of the GPU idle
-    // (fewer units than half its 256 CUs, unless the next smaller chunk is no better off),
-    // the chunks below 32 only where one of 32 does not fill it: their units spend most of
-    // their planes on the z windows' lead-in.  Among those the one whose units just fill the
-    // GPU in one go (two work-groups of a 16-wide tile per CU, one of a 32-wide): forward and
-    // adjoint run of 64^3 8.1 ms at 8 planes, 5.8 at 4, 5.7 at 2; of 100^3 16.6 at 8, 14.5 at 10
-    const auto units = [&](int z) { return (long)r->ninst * march_units(r->geo, mt, z); };
-    const int nz = r->geo.n[2];
-    const long columns = units(nz), room = mt == 32 ? 256 : 512;
-    const int fill = columns <= room ? (int)((nz + room / columns - 1) / (room / columns)) : 0;
-    std::vector<int> chunks = {4, 8, 16, 32, 64, 128};
-    if (r->opt_zchunk != 0) chunks = {r->opt_zchunk};
-    else if (fill >= 2 && fill < 32 && fill != 4 && fill != 8 && fill != 16) chunks.push_back(fill);
-    for (int zc : chunks) {
-      const bool want = zc == fill ? units(32) < 512
-                        : zc == 4  ? units(8) < 256
-                        : zc < 32  ? units(32) < 512
-                                   : zc == 32 || units(zc) >= 128;
-      if (r->opt_zchunk != 0 || want) shapes.emplace_back(mt, zc);
-    }
-  }
-  // the forward step and the adjoint rhs are timed apart and each keeps its own shape
+  const std::vector<MarchShape> shapes =
+      march_shapes(r->geo.n, r->ninst, r->opt_mtile, r->opt_zchunk);
+  const auto use = [&](int kf, int ka) {
+    r->geo.mtile = shapes[kf].tile;
+    r->geo.zchunk = shapes[kf].chunk;
+    r->geo.mtile_adj = shapes[ka].tile;
+    r->geo.zchunk_adj = shapes[ka].chunk;
+  };
   hipEvent_t evm = nullptr;
   MGD_HIP(hipEventCreate(&evm));
-  std::vector<float> best_f(shapes.size(), 0.f), best_a(shapes.size(), 0.f);
-  int rc = MGD_OK;
-  for (int round = 0; round < 2 && rc == MGD_OK; ++round) {
-    float lead_f = 0.f, lead_a = 0.f;
-    for (size_t k = 0; k < shapes.size(); ++k) {
-      lead_f = k == 0 ? best_f[k] : std::min(lead_f, best_f[k]);
-      lead_a = k == 0 ? best_a[k] : std::min(lead_a, best_a[k]);
-    }
-    for (size_t k = 0; k < shapes.size(); ++k) {
-      // the second round is among the shapes that came near the first one's fastest
-      if (round > 0 && best_f[k] > 1.1f * lead_f && best_a[k] > 1.1f * lead_a) continue;
-      r->geo.mtile = r->geo.mtile_adj = shapes[k].first;
-      r->geo.zchunk = r->geo.zchunk_adj = shapes[k].second;
-      if (round == 0) round_trip();   // warm-up
-      float ms_f = 0.f, ms_a = 0.f;
-      if (hipEventRecord(r->ev0, r->stream) != hipSuccess) { rc = MGD_ERR_HIP; break; }
-      round_trip(evm);
-      if (hipEventRecord(r->ev1, r->stream) != hipSuccess || hipGetLastError() != hipSuccess ||
-          hipEventSynchronize(r->ev1) != hipSuccess ||
-          hipEventElapsedTime(&ms_f, r->ev0, evm) != hipSuccess ||
-          hipEventElapsedTime(&ms_a, evm, r->ev1) != hipSuccess) {
-        rc = MGD_ERR_HIP;
-        break;
-      }
-      if (round == 0 || ms_f < best_f[k]) best_f[k] = ms_f;
-      if (round == 0 || ms_a < best_a[k]) best_a[k] = ms_a;
-    }
-  }
+  use(0, 0);
+  round_trip();   // warm-up
+  int kf = 0, ka = 0;
+  const bool ok = pick_march_shapes((int)shapes.size(), [&](int k, float* ms_f, float* ms_a) {
+    use(k, k);
+    if (hipEventRecord(r->ev0, r->stream) != hipSuccess) return false;
+    round_trip(evm);
+    return hipEventRecord(r->ev1, r->stream) == hipSuccess && hipGetLastError() == hipSuccess &&
+           hipEventSynchronize(r->ev1) == hipSuccess &&
+           hipEventElapsedTime(ms_f, r->ev0, evm) == hipSuccess &&
+           hipEventElapsedTime(ms_a, evm, r->ev1) == hipSuccess;
+  }, &kf, &ka);
   (void)hipEventDestroy(evm);
-  if (rc != MGD_OK) { set_error("HIP error in the march autotuner"); return rc; }
-  size_t kf = 0, ka = 0;
-  for (size_t k = 1; k < shapes.size(); ++k) {
-    if (best_f[k] < best_f[kf]) kf = k;
-    if (best_a[k] < best_a[ka]) ka = k;
-  }
-  r->geo.mtile = shapes[kf].first;
-  r->geo.zchunk = shapes[kf].second;
-  r->geo.mtile_adj = shapes[ka].first;
-  r->geo.zchunk_adj = shapes[ka].second;
+  use(kf, ka);
+  if (!ok) { set_error("HIP error in the march autotuner"); return MGD_ERR_HIP; }
   return MGD_OK;
 }
 
