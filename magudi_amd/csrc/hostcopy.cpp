@@ -11,8 +11,10 @@
 
 #include <algorithm>
 #include <atomic>
+#include <condition_variable>
 #include <cstdint>
 #include <cstring>
+#include <mutex>
 #include <system_error>
 #include <thread>
 #include <vector>
@@ -66,12 +68,18 @@ hipError_t HostCopy::to_host(void* host, const void* dev, size_t bytes, hipStrea
   const char* const src = static_cast<const char*>(dev);
   std::atomic<long> arrived{0};            // chunks in their slots
   std::atomic<bool> stop{false};
-  std::atomic<unsigned> threads{0};        // set once all have started
+  std::mutex mu;                           // the threads sleep until the first chunk is there: it
+  std::condition_variable cv;              // comes after all other work on the stream
+  unsigned threads = 0;                    // set then, and once all have started
   std::vector<std::atomic<long>> copied(kMostThreads);   // chunks that each thread has finished
   for (auto& c : copied) c.store(0);
   auto work = [&](unsigned t) {
     unsigned T;
-    while ((T = threads.load(std::memory_order_acquire)) == 0) std::this_thread::yield();
+    {
+      std::unique_lock<std::mutex> lock(mu);
+      cv.wait(lock, [&] { return threads != 0; });
+      T = threads;
+    }
     for (long c = t; c < n; c += T) {
       while (arrived.load(std::memory_order_acquire) <= c) {
         if (stop.load(std::memory_order_relaxed)) return;
@@ -92,7 +100,13 @@ hipError_t HostCopy::to_host(void* host, const void* dev, size_t bytes, hipStrea
     const hipError_t e = hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, st);
     return e != hipSuccess ? e : hipStreamSynchronize(st);
   }
-  threads.store(T, std::memory_order_release);
+  auto wake = [&] {
+    {
+      std::lock_guard<std::mutex> lock(mu);
+      threads = T;
+    }
+    cv.notify_all();
+  };
   hipError_t err = hipSuccess;
   auto fetch = [&](long c) {               // chunk c into its slot
     err = hipMemcpyAsync(buf_ + (c % slots) * kChunk, src + edge(c), edge(c + 1) - edge(c),
@@ -104,6 +118,7 @@ hipError_t HostCopy::to_host(void* host, const void* dev, size_t bytes, hipStrea
     err = hipEventSynchronize(ev_[c % slots]);
     if (err != hipSuccess) break;
     arrived.store(c + 1, std::memory_order_release);
+    if (c == 0) wake();
     // the slot of a chunk half a ring back is free once its thread has copied it out
     const long b = c - slots / 2;
     if (b >= 0 && b + slots < n) {
@@ -111,7 +126,10 @@ hipError_t HostCopy::to_host(void* host, const void* dev, size_t bytes, hipStrea
       fetch(b + slots);
     }
   }
-  if (err != hipSuccess) stop.store(true);
+  if (err != hipSuccess) {
+    stop.store(true);
+    wake();
+  }
   for (std::thread& t : pool) t.join();
   if (err != hipSuccess) (void)hipStreamSynchronize(st);   // no copy into the slots is left behind
   return err;

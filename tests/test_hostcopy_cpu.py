@@ -1,0 +1,133 @@
+"""The copies of large states to the host (hostcopy.cpp) without a GPU: compiled here with the
+host compiler against a stand-in for the few runtime calls it makes, whose events complete after a
+set time."""
+import os
+import shutil
+import subprocess
+
+import pytest
+
+CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "magudi_amd", "csrc")
+
+RUNTIME = r"""
+#pragma once
+#include <chrono>
+#include <cstdlib>
+#include <cstring>
+#include <thread>
+enum hipError_t { hipSuccess = 0, hipErrorInvalidValue = 1, hipErrorInvalidResource = 400 };
+enum { hipMemcpyDeviceToHost = 2, hipEventDisableTiming = 2, hipHostMallocDefault = 0 };
+struct Stream { int device; };
+struct Event { int device; int waits_ms; };
+typedef Stream* hipStream_t;
+typedef Event* hipEvent_t;
+inline int g_wait_ms = 0, g_copies = 0, g_fail_copy = -1, g_events = 0, g_pinned = 0;
+inline hipError_t hipGetLastError() { return hipSuccess; }
+inline hipError_t hipHostMalloc(void** p, size_t n, unsigned = 0) { *p = std::malloc(n); ++g_pinned; return hipSuccess; }
+inline hipError_t hipHostFree(void* p) { std::free(p); --g_pinned; return hipSuccess; }
+inline hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) {
+  *e = static_cast<Event*>(std::malloc(sizeof(Event)));
+  **e = {0, 0};
+  ++g_events;
+  return hipSuccess;
+}
+inline hipError_t hipEventDestroy(hipEvent_t e) { std::free(e); --g_events; return hipSuccess; }
+inline hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, int, hipStream_t) {
+  if (g_copies++ == g_fail_copy) return hipErrorInvalidValue;
+  std::memcpy(d, s, n);
+  return hipSuccess;
+}
+inline hipError_t hipEventRecord(hipEvent_t e, hipStream_t st) {
+  if (e->device != st->device) return hipErrorInvalidResource;
+  e->waits_ms = g_wait_ms;     // the first event after other work on the stream
+  g_wait_ms = 0;
+  return hipSuccess;
+}
+inline hipError_t hipEventSynchronize(hipEvent_t e) {
+  if (e->waits_ms) std::this_thread::sleep_for(std::chrono::milliseconds(e->waits_ms));
+  e->waits_ms = 0;
+  return hipSuccess;
+}
+inline hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
+"""
+
+MAIN = r"""
+#include <cstdio>
+#include <ctime>
+#include <vector>
+#include "hostcopy.h"
+static double cpu() {
+  timespec t;
+  clock_gettime(CLOCK_PROCESS_CPUTIME_ID, &t);
+  return t.tv_sec + 1e-9 * t.tv_nsec;
+}
+int main(int argc, char** argv) {
+  const size_t n = (size_t)atol(argv[2]), off = (size_t)atol(argv[3]);
+  std::vector<unsigned char> src(n), room(n + off + 64, 0xcc);
+  for (size_t i = 0; i < n; ++i) src[i] = (unsigned char)(i * 2654435761u >> 13);
+  Stream st{0};
+  mgd::HostCopy hc;
+  const auto good = [&] {
+    for (size_t i = 0; i < off; ++i) if (room[i] != 0xcc) return 0;
+    for (size_t i = 0; i < 64; ++i) if (room[off + n + i] != 0xcc) return 0;
+    return std::memcmp(room.data() + off, src.data(), n) == 0 ? 1 : 0;
+  };
+  if (!std::strcmp(argv[1], "copy")) {
+    g_fail_copy = atoi(argv[4]);
+    const int rc = hc.to_host(room.data() + off, src.data(), n, &st);
+    std::printf("%d %d %d\n", rc, rc == 0 ? good() : 0, g_copies);
+    g_fail_copy = -1;
+    const int rc2 = hc.to_host(room.data() + off, src.data(), n, &st);
+    std::printf("%d %d\n", rc2, good());
+  } else if (!std::strcmp(argv[1], "wait")) {
+    (void)hc.to_host(room.data() + off, src.data(), n, &st);
+    g_wait_ms = 400;
+    const double t0 = cpu();
+    const int rc = hc.to_host(room.data() + off, src.data(), n, &st);
+    std::printf("%d %d %.6f\n", rc, good(), cpu() - t0);
+  }
+  return 0;
+}
+"""
+
+
+@pytest.fixture(scope="module")
+def tool(tmp_path_factory):
+    cxx = shutil.which("g++")
+    if not cxx:
+        pytest.skip("no host compiler")
+    if len(os.sched_getaffinity(0)) < 4:
+        pytest.skip("copies take several threads on 4 CPUs or more")
+    d = tmp_path_factory.mktemp("hostcopy")
+    (d / "hip").mkdir()
+    (d / "hip" / "hip_runtime.h").write_text(RUNTIME)
+    (d / "main.cpp").write_text(MAIN)
+    exe = str(d / "t")
+    subprocess.check_call([cxx, "-std=c++17", "-O1", "-Wall", "-I", str(d), "-I", CSRC, "-o", exe,
+                           str(d / "main.cpp"), os.path.join(CSRC, "hostcopy.cpp"), "-pthread"])
+
+    def run(*args):
+        out = subprocess.run([exe, *map(str, args)], capture_output=True, text=True, timeout=60)
+        assert out.returncode == 0, (args, out.returncode, out.stderr)
+        return [line.split() for line in out.stdout.splitlines()]
+    return run
+
+
+MIB = 1 << 20
+
+
+@pytest.mark.parametrize("n,off", [(4 * MIB - 1, 0), (4 * MIB, 8), (5 * MIB + 13, 4096), (33 * MIB, 24),
+                                   (71 * MIB + 5, 3)])
+def test_copies(tool, n, off):
+    for fail in (-1, 0, 1, 2):
+        first, second = tool("copy", n, off, fail)
+        failed = 0 <= fail < int(first[2])
+        assert (int(first[0]) != 0) == failed and int(first[1]) == (0 if failed else 1), fail
+        assert second == ["0", "1"], fail
+
+
+def test_threads_sleep_while_the_stream_is_busy(tool):
+    """A copy behind 0.4 s of other work on its stream: the process spends next to no CPU time."""
+    (rc, good, cpu), = tool("wait", 12 * MIB, 0)
+    assert rc == "0" and good == "1"
+    assert float(cpu) < 0.1, cpu
