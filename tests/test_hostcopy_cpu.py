@@ -11,6 +11,7 @@ CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))),
 
 RUNTIME = r"""
 #pragma once
+#include <atomic>
 #include <chrono>
 #include <cstdlib>
 #include <cstring>
@@ -21,7 +22,10 @@ struct Stream { int device; };
 struct Event { int device; int waits_ms; };
 typedef Stream* hipStream_t;
 typedef Event* hipEvent_t;
-inline int g_wait_ms = 0, g_copies = 0, g_fail_copy = -1, g_events = 0, g_pinned = 0;
+inline volatile int g_wait_ms = 0;      // of the next event; below 0: until g_release
+inline volatile bool g_release = false;
+inline std::atomic<int> g_copies{0};
+inline int g_fail_copy = -1, g_events = 0, g_pinned = 0;
 inline hipError_t hipGetLastError() { return hipSuccess; }
 inline hipError_t hipHostMalloc(void** p, size_t n, unsigned = 0) { *p = std::malloc(n); ++g_pinned; return hipSuccess; }
 inline hipError_t hipHostFree(void* p) { std::free(p); --g_pinned; return hipSuccess; }
@@ -44,7 +48,8 @@ inline hipError_t hipEventRecord(hipEvent_t e, hipStream_t st) {
   return hipSuccess;
 }
 inline hipError_t hipEventSynchronize(hipEvent_t e) {
-  if (e->waits_ms) std::this_thread::sleep_for(std::chrono::milliseconds(e->waits_ms));
+  while (e->waits_ms < 0 && !g_release) std::this_thread::sleep_for(std::chrono::milliseconds(1));
+  if (e->waits_ms > 0) std::this_thread::sleep_for(std::chrono::milliseconds(e->waits_ms));
   e->waits_ms = 0;
   return hipSuccess;
 }
@@ -52,6 +57,7 @@ inline hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
 """
 
 MAIN = r"""
+#include <algorithm>
 #include <cstdio>
 #include <ctime>
 #include <vector>
@@ -63,8 +69,8 @@ static double cpu() {
 }
 int main(int argc, char** argv) {
   const size_t n = (size_t)atol(argv[2]), off = (size_t)atol(argv[3]);
-  std::vector<unsigned char> src(n), room(n + off + 64, 0xcc);
-  for (size_t i = 0; i < n; ++i) src[i] = (unsigned char)(i * 2654435761u >> 13);
+  std::vector<unsigned char> src(std::max(n, size_t(40) << 20)), room(n + off + 64, 0xcc);
+  for (size_t i = 0; i < src.size(); ++i) src[i] = (unsigned char)(i * 2654435761u >> 13);
   Stream st{0};
   mgd::HostCopy hc;
   const auto good = [&] {
@@ -75,7 +81,7 @@ int main(int argc, char** argv) {
   if (!std::strcmp(argv[1], "copy")) {
     g_fail_copy = atoi(argv[4]);
     const int rc = hc.to_host(room.data() + off, src.data(), n, &st);
-    std::printf("%d %d %d\n", rc, rc == 0 ? good() : 0, g_copies);
+    std::printf("%d %d %d\n", rc, rc == 0 ? good() : 0, g_copies.load());
     g_fail_copy = -1;
     const int rc2 = hc.to_host(room.data() + off, src.data(), n, &st);
     std::printf("%d %d\n", rc2, good());
@@ -85,6 +91,28 @@ int main(int argc, char** argv) {
     const double t0 = cpu();
     const int rc = hc.to_host(room.data() + off, src.data(), n, &st);
     std::printf("%d %d %.6f\n", rc, good(), cpu() - t0);
+  } else if (!std::strcmp(argv[1], "beside")) {
+    // `others` copies that wait for their streams, then one more: the runtime copies it makes
+    const int others = atoi(argv[4]);
+    const size_t no = (size_t)atol(argv[5]);
+    std::vector<std::thread> busy;
+    for (int k = 0; k < others; ++k) {
+      g_wait_ms = -1;
+      busy.emplace_back([&] {
+        std::vector<unsigned char> room2(no);
+        mgd::HostCopy hc2;
+        Stream st2{0};
+        (void)hc2.to_host(room2.data(), src.data(), no, &st2);   // 33 MiB: 16 slots and more
+      });
+      while (g_copies < 16 * (k + 1)) std::this_thread::yield();   // it has filled its ring
+    }
+    std::this_thread::sleep_for(std::chrono::milliseconds(20));
+    const int before = g_copies;
+    const int rc = hc.to_host(room.data() + off, src.data(), n, &st);
+    const int made = g_copies - before;
+    g_release = true;
+    for (std::thread& t : busy) t.join();
+    std::printf("%d %d %d\n", rc, good(), made);
   }
   return 0;
 }
@@ -131,3 +159,12 @@ def test_threads_sleep_while_the_stream_is_busy(tool):
     (rc, good, cpu), = tool("wait", 12 * MIB, 0)
     assert rc == "0" and good == "1"
     assert float(cpu) < 0.1, cpu
+
+
+@pytest.mark.parametrize("n,others,threads", [(5 * MIB, 0, True), (5 * MIB, 1, False), (40 * MIB, 1, True),
+                                              (40 * MIB, 4, True)])
+def test_copies_beside_others(tool, n, others, threads):
+    """A small copy beside another one is one plain copy, a large one is not."""
+    (rc, good, made), = tool("beside", n, 0, others, 33 * MIB)
+    assert rc == "0" and good == "1"
+    assert (int(made) > 1) == threads
