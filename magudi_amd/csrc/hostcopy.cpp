@@ -35,6 +35,17 @@ struct Copying {
   const int others = g_copies.fetch_add(1);
   ~Copying() { g_copies.fetch_sub(1); }
 };
+
+// Whether the runtime knows the destination (pinned, managed or device memory): a copy there is
+// one transfer at the link's rate, without faults (671 MB 11.8 ms, 16.6 through the ring).
+bool registered(const void* p) {
+  hipPointerAttribute_t a;
+  if (hipPointerGetAttributes(&a, p) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  return a.type != hipMemoryTypeUnregistered;
+}
 }  // namespace
 
 HostCopy::~HostCopy() {
@@ -73,7 +84,7 @@ hipError_t HostCopy::to_host(void* host, const void* dev, size_t bytes, hipStrea
   const int slots = (int)std::min<long>(n, kMostSlots);
   const Copying now;
   const bool beside = now.others == 0 || bytes >= kLeastBeside;
-  if (bytes < kLeast || want < 2 || !beside || !prepare(slots)) {
+  if (bytes < kLeast || want < 2 || !beside || registered(host) || !prepare(slots)) {
     const hipError_t e = hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, st);
     return e != hipSuccess ? e : hipStreamSynchronize(st);
   }

@@ -26,6 +26,13 @@ inline volatile int g_wait_ms = 0;      // of the next event; below 0: until g_r
 inline volatile bool g_release = false;
 inline std::atomic<int> g_copies{0};
 inline int g_fail_copy = -1, g_events = 0, g_pinned = 0;
+enum hipMemoryType { hipMemoryTypeUnregistered = 0, hipMemoryTypeHost = 1 };
+struct hipPointerAttribute_t { hipMemoryType type; };
+inline const void* g_registered = nullptr;
+inline hipError_t hipPointerGetAttributes(hipPointerAttribute_t* a, const void* p) {
+  a->type = p == g_registered ? hipMemoryTypeHost : hipMemoryTypeUnregistered;
+  return p == g_registered ? hipSuccess : hipErrorInvalidValue;
+}
 inline hipError_t hipGetLastError() { return hipSuccess; }
 inline hipError_t hipHostMalloc(void** p, size_t n, unsigned = 0) { *p = std::malloc(n); ++g_pinned; return hipSuccess; }
 inline hipError_t hipHostFree(void* p) { std::free(p); --g_pinned; return hipSuccess; }
@@ -91,6 +98,10 @@ int main(int argc, char** argv) {
     const double t0 = cpu();
     const int rc = hc.to_host(room.data() + off, src.data(), n, &st);
     std::printf("%d %d %.6f\n", rc, good(), cpu() - t0);
+  } else if (!std::strcmp(argv[1], "registered")) {
+    g_registered = room.data() + off;
+    const int rc = hc.to_host(room.data() + off, src.data(), n, &st);
+    std::printf("%d %d %d\n", rc, good(), g_copies.load());
   } else if (!std::strcmp(argv[1], "beside")) {
     // `others` copies that wait for their streams, then one more: the runtime copies it makes
     const int others = atoi(argv[4]);
@@ -168,3 +179,8 @@ def test_copies_beside_others(tool, n, others, threads):
     (rc, good, made), = tool("beside", n, 0, others, 33 * MIB)
     assert rc == "0" and good == "1"
     assert (int(made) > 1) == threads
+
+
+@pytest.mark.parametrize("n", [5 * MIB, 40 * MIB])
+def test_registered_memory_is_copied_to_directly(tool, n):
+    assert tool("registered", n, 8) == [["0", "1", "1"]]
