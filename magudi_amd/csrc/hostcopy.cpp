@@ -15,9 +15,7 @@
 #include <cstdint>
 #include <cstring>
 #include <mutex>
-#include <system_error>
 #include <thread>
-#include <vector>
 
 namespace mgd {
 
@@ -95,7 +93,7 @@ hipError_t HostCopy::to_host(void* host, const void* dev, size_t bytes, hipStrea
   std::mutex mu;                           // the threads sleep until the first chunk is there: it
   std::condition_variable cv;              // comes after all other work on the stream
   unsigned threads = 0;                    // set then, and once all have started
-  std::vector<std::atomic<long>> copied(kMostThreads);   // chunks that each thread has finished
+  std::atomic<long> copied[kMostThreads];  // chunks that each thread has finished
   for (auto& c : copied) c.store(0);
   auto work = [&](unsigned t) {
     unsigned T;
@@ -113,13 +111,12 @@ hipError_t HostCopy::to_host(void* host, const void* dev, size_t bytes, hipStrea
       copied[t].fetch_add(1, std::memory_order_release);
     }
   };
-  std::vector<std::thread> pool;
-  pool.reserve(want);
+  std::thread pool[kMostThreads];
+  unsigned T = 0;
   try {
-    for (unsigned t = 0; t < want; ++t) pool.emplace_back(work, t);
-  } catch (const std::system_error&) {     // as many as there are
+    for (; T < want; ++T) pool[T] = std::thread(work, T);
+  } catch (...) {                          // no thread or no memory: as many as there are
   }
-  const unsigned T = (unsigned)pool.size();
   if (T == 0) {
     const hipError_t e = hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, st);
     return e != hipSuccess ? e : hipStreamSynchronize(st);
@@ -154,7 +151,7 @@ hipError_t HostCopy::to_host(void* host, const void* dev, size_t bytes, hipStrea
     stop.store(true);
     wake();
   }
-  for (std::thread& t : pool) t.join();
+  for (unsigned t = 0; t < T; ++t) pool[t].join();
   if (err != hipSuccess) (void)hipStreamSynchronize(st);   // no copy into the slots is left behind
   return err;
 }

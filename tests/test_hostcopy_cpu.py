@@ -67,6 +67,7 @@ MAIN = r"""
 #include <algorithm>
 #include <cstdio>
 #include <ctime>
+#include <new>
 #include <vector>
 #include "hostcopy.h"
 static double cpu() {
@@ -74,6 +75,16 @@ static double cpu() {
   clock_gettime(CLOCK_PROCESS_CPUTIME_ID, &t);
   return t.tv_sec + 1e-9 * t.tv_nsec;
 }
+// this thread's allocations fail from the g_left-th on (a thread start makes one)
+static std::atomic<long> g_left{-1};
+static thread_local bool g_watched = false;
+void* operator new(std::size_t n) {
+  if (g_watched && g_left >= 0 && g_left-- <= 0) throw std::bad_alloc();
+  if (void* p = std::malloc(n ? n : 1)) return p;
+  throw std::bad_alloc();
+}
+void operator delete(void* p) noexcept { std::free(p); }
+void operator delete(void* p, std::size_t) noexcept { std::free(p); }
 int main(int argc, char** argv) {
   const size_t n = (size_t)atol(argv[2]), off = (size_t)atol(argv[3]);
   std::vector<unsigned char> src(std::max(n, size_t(40) << 20)), room(n + off + 64, 0xcc);
@@ -98,6 +109,16 @@ int main(int argc, char** argv) {
     const double t0 = cpu();
     const int rc = hc.to_host(room.data() + off, src.data(), n, &st);
     std::printf("%d %d %.6f\n", rc, good(), cpu() - t0);
+  } else if (!std::strcmp(argv[1], "memory")) {
+    g_watched = true;
+    g_left = atoi(argv[4]);
+    int rc = -1;
+    try {
+      rc = hc.to_host(room.data() + off, src.data(), n, &st);
+    } catch (...) {                        // nothing may pass the C entry points
+    }
+    g_left = -1;
+    std::printf("%d %d\n", rc, good());
   } else if (!std::strcmp(argv[1], "registered")) {
     g_registered = room.data() + off;
     const int rc = hc.to_host(room.data() + off, src.data(), n, &st);
@@ -184,3 +205,10 @@ def test_copies_beside_others(tool, n, others, threads):
 @pytest.mark.parametrize("n", [5 * MIB, 40 * MIB])
 def test_registered_memory_is_copied_to_directly(tool, n):
     assert tool("registered", n, 8) == [["0", "1", "1"]]
+
+
+@pytest.mark.parametrize("left", range(9))
+def test_without_memory_for_threads(tool, left):
+    """Memory runs out at the first, second, .. allocation of a copy: fewer threads or a plain copy,
+    the same bytes, no exception."""
+    assert tool("memory", 20 * MIB, 16, left) == [["0", "1"]]
