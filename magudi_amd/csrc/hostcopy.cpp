@@ -52,9 +52,23 @@ HostCopy::~HostCopy() {
   if (buf_) (void)hipHostFree(buf_);
 }
 
-bool HostCopy::prepare(int slots) {
+bool HostCopy::prepare(int slots, hipStream_t st) {
   if (slots_ >= slots) return true;
   if (failed_) return false;
+  // events are recorded on the stream's device, which need not be the caller's current one
+  int current = 0;
+  hipDevice_t device = 0;
+  if (hipGetDevice(&current) != hipSuccess || hipStreamGetDevice(st, &device) != hipSuccess ||
+      (current != device && hipSetDevice(device) != hipSuccess)) {
+    (void)hipGetLastError();
+    return false;
+  }
+  const bool ok = make(slots);
+  if (current != device) (void)hipSetDevice(current);
+  return ok;
+}
+
+bool HostCopy::make(int slots) {
   if (buf_) (void)hipHostFree(buf_);
   buf_ = nullptr;
   slots_ = 0;
@@ -82,7 +96,7 @@ hipError_t HostCopy::to_host(void* host, const void* dev, size_t bytes, hipStrea
   const int slots = (int)std::min<long>(n, kMostSlots);
   const Copying now;
   const bool beside = now.others == 0 || bytes >= kLeastBeside;
-  if (bytes < kLeast || want < 2 || !beside || registered(host) || !prepare(slots)) {
+  if (bytes < kLeast || want < 2 || !beside || registered(host) || !prepare(slots, st)) {
     const hipError_t e = hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, st);
     return e != hipSuccess ? e : hipStreamSynchronize(st);
   }

@@ -20,7 +20,8 @@ class HostCopy {
  private:
   static constexpr size_t kChunk = size_t(2) << 20;
   static constexpr int kMostSlots = 16;
-  bool prepare(int slots);
+  bool prepare(int slots, hipStream_t st);
+  bool make(int slots);
   char* buf_ = nullptr;
   int slots_ = 0;
   hipEvent_t ev_[kMostSlots] = {};

@@ -33,12 +33,17 @@ inline hipError_t hipPointerGetAttributes(hipPointerAttribute_t* a, const void* 
   a->type = p == g_registered ? hipMemoryTypeHost : hipMemoryTypeUnregistered;
   return p == g_registered ? hipSuccess : hipErrorInvalidValue;
 }
+typedef int hipDevice_t;
+inline int g_device = 0;
+inline hipError_t hipGetDevice(int* d) { *d = g_device; return hipSuccess; }
+inline hipError_t hipSetDevice(int d) { g_device = d; return hipSuccess; }
+inline hipError_t hipStreamGetDevice(hipStream_t st, hipDevice_t* d) { *d = st->device; return hipSuccess; }
 inline hipError_t hipGetLastError() { return hipSuccess; }
 inline hipError_t hipHostMalloc(void** p, size_t n, unsigned = 0) { *p = std::malloc(n); ++g_pinned; return hipSuccess; }
 inline hipError_t hipHostFree(void* p) { std::free(p); --g_pinned; return hipSuccess; }
 inline hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) {
   *e = static_cast<Event*>(std::malloc(sizeof(Event)));
-  **e = {0, 0};
+  **e = {g_device, 0};
   ++g_events;
   return hipSuccess;
 }
@@ -119,6 +124,10 @@ int main(int argc, char** argv) {
     }
     g_left = -1;
     std::printf("%d %d\n", rc, good());
+  } else if (!std::strcmp(argv[1], "device")) {
+    g_device = 1;
+    const int rc = hc.to_host(room.data() + off, src.data(), n, &st);
+    std::printf("%d %d %d\n", rc, good(), g_device);
   } else if (!std::strcmp(argv[1], "registered")) {
     g_registered = room.data() + off;
     const int rc = hc.to_host(room.data() + off, src.data(), n, &st);
@@ -212,3 +221,8 @@ def test_without_memory_for_threads(tool, left):
     """Memory runs out at the first, second, .. allocation of a copy: fewer threads or a plain copy,
     the same bytes, no exception."""
     assert tool("memory", 20 * MIB, 16, left) == [["0", "1"]]
+
+
+def test_another_current_device(tool):
+    """The region is on device 0, the caller's current device is 1, and stays so."""
+    assert tool("device", 12 * MIB, 0) == [["0", "1", "1"]]
