@@ -1274,14 +1274,15 @@ int plan_window_cache(mgd_region* r, int nsteps, int K, long M) {
 }
 
 // Entries that a cache of `unit`-double entries should have, of which `buf` holds some: `plan`,
-// or what it holds when that is near it (the free memory moves a little between runs, and a
-// captured run is good only for the buffers it was captured with).  At most a sixteenth (or two)
-// below the plan; above it, at most 2 GiB of the reserve of storage_budget.
-int cache_entries(const DevBuf& buf, size_t unit, int plan, int most) {
+// or what it holds where that serves (at most `most` entries), is no more than a sixteenth (or
+// two) below the plan, and fits in `room` bytes.  The free memory moves a little between runs,
+// so 2 GiB of the reserve of storage_budget count as room; what other regions took since does
+// not make a cache that still fits smaller, else two regions running in turn would allocate
+// theirs again in every run.
+int cache_entries(const DevBuf& buf, size_t unit, int plan, int most, size_t room) {
   const int have = unit > 0 && buf.n % unit == 0 ? (int)(buf.n / unit) : 0;
-  const int above = unit > 0 ? (int)std::min<size_t>(((size_t)2 << 30) / (unit * sizeof(double)), 1 << 20) : 0;
-  if (plan <= 0 || have <= 0 || have > most) return plan;
-  return plan <= have + std::max(2, have / 16) && have <= plan + above ? have : plan;
+  const bool fits = have > 0 && have <= most && buf.bytes() <= room + ((size_t)2 << 30);
+  return fits && plan > 0 && plan <= have + std::max(2, have / 16) ? have : plan;
 }
 
 // Allocates `want` entries of `unit` doubles, or half as many for as long as they do not fit.
@@ -1343,12 +1344,12 @@ int plan_plain_storage(mgd_region* r, int nsteps, int K, long M) {
     size_t rest = budget > fixed ? budget - fixed : 0;
     const int most = r->opt_cache < 0 ? nsteps : (int)std::min((long)nsteps, (long)r->opt_cache * K);
     int nsc = (int)std::min<size_t>((size_t)most, rest / (3 * S));
-    nsc = cache_entries(r->scache, (size_t)3 * M, nsc, most);
+    nsc = cache_entries(r->scache, (size_t)3 * M, nsc, most, rest);
     rest = rest > 3 * S * nsc ? rest - 3 * S * nsc : 0;
     int ngc = 0;
     if (reuse && r->opt_cache < 0) {
       ngc = (int)std::min<size_t>((size_t)nsc, rest / 2 / (4 * GB));
-      ngc = cache_entries(r->gcache, 4 * r->G.n, ngc, nsc);
+      ngc = cache_entries(r->gcache, 4 * r->G.n, ngc, nsc, rest);
     }
     for (int k = 0; k < mgd_region::kMaxCache; ++k) r->wcache[k].release();
     r->ncache = 0;

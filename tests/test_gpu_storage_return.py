@@ -14,6 +14,29 @@ BUDGET = 40 << 30
 STEPS = (24, 110, 24, 300, 110)      # all held, all held, all held, some held, all held
 
 
+def _region(c):
+    from magudi_amd.solver import Region
+    R = Region(c)
+    R.set_march_tile(16)
+    R.set_z_chunk(32)
+    return R
+
+
+def _fill(c, regions):
+    """A tensor that leaves BUDGET to plan with beside `regions` regions and the reserve."""
+    import torch
+    gc.collect()
+    torch.cuda.empty_cache()
+    free, total = torch.cuda.mem_get_info()
+    state = 40 * c.npoints
+    own = 40 * state                           # a region's other arrays, generously
+    reserve = max(8 << 30, total // 32)
+    hold = free - reserve - regions * own - BUDGET
+    if hold < 0:
+        pytest.skip("needs 60 GB of device memory")
+    return torch.empty(hold, dtype=torch.uint8, device="cuda")
+
+
 def _run(R, c, nsteps, q0):
     from magudi_amd.solver import Solver
     R.states[0].conservedVariables = q0
@@ -27,32 +50,15 @@ def _run(R, c, nsteps, q0):
 def test_plans_of_one_region_equal_a_fresh_regions():
     import torch
     from magudi_amd import cases
-    from magudi_amd.solver import Region
-
-    def region():
-        R = Region(c)
-        R.set_march_tile(16)
-        R.set_z_chunk(32)
-        return R
-
     c = cases.kolmogorov3d(n=128, nsteps=24)
     q0 = c.initial_state()
-    gc.collect()
-    torch.cuda.empty_cache()
-    free, total = torch.cuda.mem_get_info()
-    state = 40 * c.npoints
-    own = 40 * state                           # the region's other arrays, generously
-    reserve = max(8 << 30, total // 32)
-    hold = free - reserve - own - BUDGET
-    if hold < 0:
-        pytest.skip("needs 60 GB of device memory")
-    filler = torch.empty(hold, dtype=torch.uint8, device="cuda")
+    filler = _fill(c, 1)
     try:
-        R = region()
+        R = _region(c)
         once = [_run(R, c, n, q0) for n in STEPS]
         R.close()
         for n, (plan, J, lam) in zip(STEPS, once):
-            F = region()
+            F = _region(c)
             fresh = _run(F, c, n, q0)
             F.close()
             print(f"storage: {n} steps, plan {plan}, fresh {fresh[0]}", flush=True)
@@ -61,13 +67,39 @@ def test_plans_of_one_region_equal_a_fresh_regions():
             assert abs(plan["held"] - fresh[0]["held"]) <= (0 if n < 300 else 2)
             assert plan["held"] == n if n < 300 else 0 < plan["held"] < n
             assert J == fresh[1] and np.array_equal(lam, fresh[2])
-        F = region()
+        F = _region(c)
         F.set_step_store(1)
         F.set_window_cache(0)                  # no step held, no slots kept
         bare = _run(F, c, STEPS[0], q0)
         F.close()
         assert bare[0]["held"] == 0
         assert bare[1] == once[0][1] and np.array_equal(bare[2], once[0][2])
+    finally:
+        del filler
+        torch.cuda.empty_cache()
+
+
+def test_two_regions_in_turn_keep_their_storage():
+    """Each region's run leaves the other's storage as it is: after the first run of each, runs in
+    turn allocate nothing."""
+    import torch
+    from magudi_amd import cases
+    c = cases.kolmogorov3d(n=128, nsteps=24)
+    q0 = c.initial_state()
+    filler = _fill(c, 2)
+    try:
+        A, B = _region(c), _region(c)
+        first = [_run(R, c, 24, q0) for R in (A, B)]
+        free = []
+        for turn in range(3):
+            for R in (A, B):
+                plan, J, lam = _run(R, c, 24, q0)
+                assert plan["held"] == 24 and J == first[0][1] and np.array_equal(lam, first[0][2])
+                free.append(torch.cuda.mem_get_info()[0])
+        print(f"storage in turn: free {free}", flush=True)
+        assert len(set(free)) == 1
+        A.close()
+        B.close()
     finally:
         del filler
         torch.cuda.empty_cache()
