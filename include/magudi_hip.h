@@ -336,7 +336,10 @@ int mgd_last_timings(mgd_region* r, double* out, int* launches);
  * at the same states (the stress and heat flux).  -1 (default): where nsteps + 3 states (fused path:
  * nsteps + 6, two recompute buffers) fit in the memory left free less the reserve and MGD_OPT_WINDOW_CACHE is at its default; 0: off
  * (snapshots and windows); 1: on where the states of every step can be allocated.
- * Identical results. */
+ * Identical results.
+ * MGD_OPT_WIDE_OFFSETS: 1 lets the 3-D forward march and the gradient pass address with 64-bit
+ * offsets, as they do by themselves (0, default) on grids of 2^29 - 1024 points and more
+ * (comparison and testing); the adjoint marches serve smaller grids only.  Identical results. */
 #define MGD_OPT_FORCE_PLAIN 1
 #define MGD_OPT_TILE_SHAPE 2
 #define MGD_OPT_RESIDENT_STATES 3
@@ -344,6 +347,7 @@ int mgd_last_timings(mgd_region* r, double* out, int* launches);
 #define MGD_OPT_Z_CHUNK 5
 #define MGD_OPT_MARCH_TILE 6
 #define MGD_OPT_STEP_STORE 7
+#define MGD_OPT_WIDE_OFFSETS 8
 int mgd_region_set_option(mgd_region* r, int option, int value);
 
 /* Storage plan of the last checkpointed forward run: plan[0] = 1 step store, plan[1] steps

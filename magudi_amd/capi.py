@@ -21,7 +21,7 @@ CONSERVED, ADJOINT_VARS, RHS, INITIAL_STATE, FINAL_STATE, SCRATCH = 0, 1, 2, 4, 
 FIELD_TARGET_STATE, FIELD_CONTROL_MOLLIFIER, FIELD_TARGET_MOLLIFIER = 0, 1, 2
 OP_FIRST, OP_ADJOINT_FIRST, OP_DISS, OP_DISS_T, OP_SECOND = 0, 1, 2, 3, 4
 OPT_FORCE_PLAIN, OPT_TILE_SHAPE, OPT_RESIDENT_STATES, OPT_WINDOW_CACHE, OPT_Z_CHUNK = 1, 2, 3, 4, 5
-OPT_MARCH_TILE, OPT_STEP_STORE = 6, 7
+OPT_MARCH_TILE, OPT_STEP_STORE, OPT_WIDE_OFFSETS = 6, 7, 8
 TERMINAL_KINETIC_ENERGY = 0
 KERNEL_FWD_STAGE, KERNEL_ADJ_STAGE, KERNEL_COPY, KERNEL_RHS_FORWARD, KERNEL_RHS_ADJOINT = 0, 1, 2, 3, 4
 KERNEL_FWD_MARCH3D = 5

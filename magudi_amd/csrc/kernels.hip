@@ -143,19 +143,22 @@ __device__ __forceinline__ MarchThread march_thread(const Geo& g, const MarchUni
   return m;
 }
 
-// Element access at a 32-bit byte offset from a wave-uniform base pointer: the address
+// Element access at a byte offset from a wave-uniform base pointer.  O = unsigned: the address
 // form of a global load / store with a scalar base and a 32-bit vector offset, so a
 // thread keeps one 32-bit offset per point instead of a 64-bit address per component.
 // Callers keep byte offsets below 2^32 - 4096 (fewer than 2^29 - 1024 points per component
-// array, so that the offsets of spare threads lie past its end).
-__device__ __forceinline__ double ld8(const double* base, unsigned off) {
+// array, so that the offsets of spare threads lie past its end).  O = unsigned long: component
+// arrays of any size (Geo::wide).
+template <class O>
+__device__ __forceinline__ double ld8(const double* base, O off) {
   return *reinterpret_cast<const double*>(reinterpret_cast<const char*>(base) + off);
 }
-__device__ __forceinline__ void st8(double* base, unsigned off, double v) {
+template <class O>
+__device__ __forceinline__ void st8(double* base, O off, double v) {
   *reinterpret_cast<double*>(reinterpret_cast<char*>(base) + off) = v;
 }
-template <bool STREAM>
-__device__ __forceinline__ double ld8_own(const double* base, unsigned off) {
+template <bool STREAM, class O>
+__device__ __forceinline__ double ld8_own(const double* base, O off) {
   return ld_own<STREAM>(reinterpret_cast<const double*>(reinterpret_cast<const char*>(base) + off));
 }
 // Store at byte offset `off` of an array of `bytes` bytes through a buffer descriptor, whose
@@ -165,6 +168,14 @@ __device__ __forceinline__ void st8_own(double* base, unsigned bytes, unsigned o
   typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
   const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(base, 0, bytes, 0x00027000);
   __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, v), r, off, 0, STREAM ? 2 : 0);
+}
+// At a 64-bit offset: all bits set for the threads whose store is dropped.
+template <bool STREAM>
+__device__ __forceinline__ void st8_own(double* base, unsigned long, unsigned long off, double v) {
+  if (off == ~0ul) return;
+  double* p = reinterpret_cast<double*>(reinterpret_cast<char*>(base) + off);
+  if (STREAM) __builtin_nontemporal_store(v, p);
+  else *p = v;
 }
 
 // The eight neighbours of a staged value along x (stride 1) and y (stride sy) that the
@@ -217,7 +228,7 @@ __device__ __forceinline__ double ld_const(const double* p, int i) {
 // (visc_point's operations, so the same values); 72 instead of 96 bytes per point.
 // POWER: the viscosity follows a power law of the temperature (pow per point); without
 // it the transport coefficients are constants and the kernel needs far fewer registers.
-template <int BX, int BY, bool STRESS = false, bool POWER = true>
+template <int BX, int BY, bool STRESS, bool POWER, class O>
 __global__ void __launch_bounds__(BX * BY, STRESS ? 2 : 4) k_grad3d_periodic(Geo g, int zc,
                                                               const double* __restrict__ q,
                                                               double* __restrict__ G) {
@@ -235,11 +246,11 @@ __global__ void __launch_bounds__(BX * BY, STRESS ? 2 : 4) k_grad3d_periodic(Geo
   // place of the halo point in the one haloed tile
   const int hx = m.hmask == 2 ? m.hx + 4 : m.hx, hy = m.hmask == 1 ? m.hy + 4 : m.hy;
   const Dir dz = g.dir[2];
-  const unsigned n0 = (unsigned)g.n[0], plane8 = 8u * n0 * (unsigned)g.n[1];
-  const unsigned col8 = 8u * ((unsigned)m.i + n0 * (unsigned)m.j);
-  const unsigned hcol8 = 8u * ((unsigned)m.hi + n0 * (unsigned)m.hj);
+  const O n0 = (O)g.n[0], plane8 = 8 * n0 * (O)g.n[1];
+  const O col8 = 8 * ((O)m.i + n0 * (O)m.j);
+  const O hcol8 = 8 * ((O)m.hi + n0 * (O)m.hj);
   const double h0 = g.h[0][m.i], h1 = g.h[1][m.j], h01 = h0 * h1;
-  auto load_v = [&](unsigned off, double* v) {
+  auto load_v = [&](O off, double* v) {
 #pragma unroll
     for (int l = 0; l < 5; ++l) v[l] = ld8(qi + l * g.N, off);
   };
@@ -248,11 +259,11 @@ __global__ void __launch_bounds__(BX * BY, STRESS ? 2 : 4) k_grad3d_periodic(Geo
     w[0] = s.u[0]; w[1] = s.u[1]; w[2] = s.u[2]; w[3] = s.T;
   };
   // halo planes beyond the chunk are not used: the last one is loaded again
-  auto halo_plane = [&](int z) { return hcol8 + plane8 * (unsigned)min(z, u.z1 - 1); };
+  auto halo_plane = [&](int z) { return hcol8 + plane8 * (O)min(z, u.z1 - 1); };
   double Q[9][NW], v[5], hv[5];
 #pragma unroll
   for (int k = 0; k < 8; ++k) {
-    load_v(col8 + plane8 * (unsigned)wrap(u.z0 - 4 + k, dz), v);
+    load_v(col8 + plane8 * (O)wrap(u.z0 - 4 + k, dz), v);
     to_w(v, Q[k]);
   }
 #pragma unroll
@@ -265,7 +276,7 @@ __global__ void __launch_bounds__(BX * BY, STRESS ? 2 : 4) k_grad3d_periodic(Geo
       for (int c = 0; c < NW; ++c) hring[k][c][ht] = hw[c];
     }
   }
-  load_v(col8 + plane8 * (unsigned)wrap(u.z0 + 4, dz), v);   // the lead plane z0 + 4
+  load_v(col8 + plane8 * (O)wrap(u.z0 + 4, dz), v);   // the lead plane z0 + 4
   load_v(halo_plane(u.z0 + 4), hv);
   const Op& op = g.ops[SLOT_FIRST];
   const double c1 = op.c[kMaxHW + 1], c2 = op.c[kMaxHW + 2], c3 = op.c[kMaxHW + 3], c4 = op.c[kMaxHW + 4];
@@ -275,7 +286,7 @@ __global__ void __launch_bounds__(BX * BY, STRESS ? 2 : 4) k_grad3d_periodic(Geo
     double hw[NW];
     to_w(hv, hw);
     // the next lead plane's points: the loads stay in flight through this plane's work
-    load_v(col8 + plane8 * (unsigned)wrap(min(zo + 5, u.z1 + 3), dz), v);
+    load_v(col8 + plane8 * (O)wrap(min(zo + 5, u.z1 + 3), dz), v);
     load_v(halo_plane(zo + 5), hv);
 #pragma unroll
     for (int c = 0; c < NW; ++c) sw[buf][c][ty + 4][tx + 4] = Q[4][c];
@@ -288,7 +299,7 @@ __global__ void __launch_bounds__(BX * BY, STRESS ? 2 : 4) k_grad3d_periodic(Geo
       }
     }
     __syncthreads();
-    const unsigned p8 = col8 + plane8 * (unsigned)zo;
+    const O p8 = col8 + plane8 * (O)zo;
     const double h2 = ld_const(g.h[2], zo);
     const double jac = 1.0 / (h01 * h2);                                  // jacobian<3>
     const double jm[3] = {jac * (h1 * h2), jac * (h0 * h2), jac * h01};   // times metric<3>
@@ -1634,7 +1645,7 @@ __global__ void __launch_bounds__(kBlock) k_deriv_line(Geo g, int d, int slot,
 // only the RK operands of its output plane that its update reads (early, so that their
 // latency overlaps the divergence).
 // STREAM (march_streams): RK operands and outputs non-temporal.
-template <int BX, int BY, int STAGE, bool STREAM>
+template <int BX, int BY, int STAGE, bool STREAM, class O>
 __global__ void __launch_bounds__(BX * BY, 512 / (BX * BY)) k_fwd3d_march(Geo g, int zc, const double* __restrict__ q,
                                                           const double* __restrict__ S,
                                                           const double* __restrict__ kstr,
@@ -1657,11 +1668,13 @@ __global__ void __launch_bounds__(BX * BY, 512 / (BX * BY)) k_fwd3d_march(Geo g,
   const MarchThread m = march_thread<BX, BY>(g, u);
   const int t = threadIdx.x, tx = m.tx, ty = m.ty, hmask = m.hmask;
   const Dir dz = g.dir[2];
-  const unsigned n0 = (unsigned)g.n[0], plane8 = 8u * n0 * (unsigned)g.n[1];
-  const unsigned bytes = 8u * (unsigned)g.N;
-  const unsigned col8 = 8u * ((unsigned)m.i + n0 * (unsigned)m.j);
-  const unsigned hcol8 = 8u * ((unsigned)m.hi + n0 * (unsigned)m.hj);
-  const double kk = kstr ? kstr[n0 * (unsigned)m.j] : 0.0;
+  const O n0 = (O)g.n[0], plane8 = 8 * n0 * (O)g.n[1];
+  const O bytes = 8 * (O)g.N;
+  const O col8 = 8 * ((O)m.i + n0 * (O)m.j);
+  const O hcol8 = 8 * ((O)m.hi + n0 * (O)m.hj);
+  // the offset of a store that is dropped has these bits set
+  const O spare = sizeof(O) == 8 ? (m.spare ? ~(O)0 : (O)0) : (O)m.spare;
+  const double kk = kstr ? kstr[n0 * (O)m.j] : 0.0;
   // the grid values of the metrics: metric<3> of d = 0, 1, 2 is h1 h2, h0 h2, h0 h1
   const double h0 = g.h[0][m.i], h1 = g.h[1][m.j], h01 = h0 * h1;
   const double hh = hmask == 2 ? g.h[0][m.hi] : g.h[1][m.hj];   // of the halo point's direction
@@ -1672,7 +1685,7 @@ __global__ void __launch_bounds__(BX * BY, 512 / (BX * BY)) k_fwd3d_march(Geo g,
     double v[NV];
     double sv[9];
   };
-  auto load_pt = [&](unsigned off, auto xy, Pt& P) {
+  auto load_pt = [&](O off, auto xy, Pt& P) {
 #pragma unroll
     for (int l = 0; l < NV; ++l) P.v[l] = ld8(qi + l * g.N, off);
     if (g.viscous) {
@@ -1694,7 +1707,7 @@ __global__ void __launch_bounds__(BX * BY, 512 / (BX * BY)) k_fwd3d_march(Geo g,
     hs[2] = Si + (y ? 4 : 2) * g.N;
     hs[3] = Si + (y ? 7 : 6) * g.N;
   }
-  auto load_halo = [&](unsigned off, HaloPt& P) {
+  auto load_halo = [&](O off, HaloPt& P) {
 #pragma unroll
     for (int l = 0; l < NV; ++l) P.v[l] = ld8(qi + l * g.N, off);
     if (g.viscous) {
@@ -1734,18 +1747,18 @@ __global__ void __launch_bounds__(BX * BY, 512 / (BX * BY)) k_fwd3d_march(Geo g,
   // the four planes before the chunk enter the window (slots 4 .. 7) with their z fluxes
 #pragma unroll
   for (int k = 0; k < 4; ++k) {
-    load_pt(col8 + plane8 * (unsigned)wrap(z0 - 4 + k, dz), no, ct);
+    load_pt(col8 + plane8 * (O)wrap(z0 - 4 + k, dz), no, ct);
     flux_z(ct, prim<3>(ct.v, g.gamma), W[k + 4]);
   }
-  load_pt(col8 + plane8 * (unsigned)z0, yes, ct);
-  load_halo(hcol8 + plane8 * (unsigned)z0, ch);
+  load_pt(col8 + plane8 * (O)z0, yes, ct);
+  load_halo(hcol8 + plane8 * (O)z0, ch);
   // One lead plane zl: XY: inside the chunk, its x / y fluxes are formed; OUT: the plane
   // zl - 4 is finished.  Compile-time cases, so that the loads of each are unconditional
   // and their waits exact; a plane inside the chunk loads the next one with its halo, also
   // where that lies just beyond the chunk.
   auto plane = [&](int zl, auto XY, auto OUT) {
-    const unsigned p8 = col8 + plane8 * (unsigned)(zl - 4);   // output plane (OUT only)
-    const unsigned w8 = p8 | m.spare;
+    const O p8 = col8 + plane8 * (O)(zl - 4);   // output plane (OUT only)
+    const O w8 = p8 | spare;
     const double h2 = ld_const(g.h[2], wrap(zl, dz));
     double f[2][NV], fh[NV];
     {
@@ -1777,7 +1790,7 @@ __global__ void __launch_bounds__(BX * BY, 512 / (BX * BY)) k_fwd3d_march(Geo g,
       }
     }
     // this plane's operands are spent: load the next plane's now
-    const unsigned n8 = plane8 * (unsigned)wrap(min(zl + 1, z1 + 3), dz);
+    const O n8 = plane8 * (O)wrap(min(zl + 1, z1 + 3), dz);
     load_pt(col8 + n8, XY, ct);
     if constexpr (XY) load_halo(hcol8 + n8, ch);
     if constexpr (OUT) {
@@ -2251,10 +2264,9 @@ static dim3 grid_pts(const Geo& g) {
 
 // Where the one-pass gradient kernel and the marches apply: 3-D, periodic in every direction,
 // any size (their tiles may be partial; regions hold at least 9 points along a periodic
-// direction), and component arrays that 32-bit byte offsets reach.
+// direction).
 static bool grad3d_applies(const Geo& g) {
-  return g.nd == 3 && g.nv == 5 && g.dir[0].periodic && g.dir[1].periodic && g.dir[2].periodic &&
-         g.N < (1L << 29) - 1024;
+  return g.nd == 3 && g.nv == 5 && g.dir[0].periodic && g.dir[1].periodic && g.dir[2].periodic;
 }
 
 // x / y flux divergence kernel of 3-D grids periodic in x and y with sizes that are
@@ -2285,6 +2297,12 @@ static void with_march(const Geo& g, bool adj, F&& f) {
 // found there again (forward stages 256^3: 935 us, 887 streamed; 160^3: 256 and 247), not
 // where they do, and the next kernel reads them from it (100^3: 112 us, 136 streamed).
 static bool march_streams(const Geo& g) { return g.N * g.ninst > 1500000; }
+// f is called with a value of the offset type that reaches the grid's component arrays
+template <class F>
+static void with_offsets(const Geo& g, F&& f) {
+  if (g.wide) f(0ul);
+  else f(0u);
+}
 // f is called with the RK stage (0: none) and march_streams as compile-time values
 template <class F>
 static void with_stage(const Geo& g, int stage, F&& f) {
@@ -2314,7 +2332,10 @@ template <int ND>
 static void launch_gradients(const Geo& g, const double* q, double* w, double* G, const dim3& grid,
                              hipStream_t st) {
   if (ND == 3 && grad3d_applies(g)) {
-    k_grad3d_periodic<kG3X, kG3Y><<<grad3d_grid(g), kG3X * kG3Y, 0, st>>>(g, grad3d_chunk(g), q, G);
+    with_offsets(g, [&](auto o) {
+      k_grad3d_periodic<kG3X, kG3Y, false, true, decltype(o)>
+          <<<grad3d_grid(g), kG3X * kG3Y, 0, st>>>(g, grad3d_chunk(g), q, G);
+    });
     return;
   }
   k_prim<ND><<<grid, kBlock, 0, st>>>(g, q, w);
@@ -2330,12 +2351,12 @@ bool fwd3d_march_path(const Geo& g, const FinishInfo& fin, int nsrc) {
   return fin.simple && !g.dissipation && nsrc == 0 && grad3d_applies(g);
 }
 
-// The two-march adjoint path: viscous, periodic in every direction with the march tile
-// sizes, no dissipation, no far field and at most one whole-domain Kolmogorov forcing (the
+// The two-march adjoint path: viscous, periodic in every direction, component arrays that 32-bit
+// offsets reach (a viscous adjoint run with longer ones does not fit the GPU), no dissipation, no far field and at most one whole-domain Kolmogorov forcing (the
 // chain rule and the forcing then sit in the finishing march).
 static bool adj3d_march_path(const Geo& g, const FinishInfo& fin) {
   return g.viscous && !g.dissipation && !fin.has_farfield && fin.simple &&
-         grad3d_applies(g);
+         grad3d_applies(g) && !g.wide;
 }
 
 bool stress_reuse_path(const Geo& g, const FinishInfo& fin, int nsrc) {
@@ -2345,10 +2366,13 @@ bool stress_reuse_path(const Geo& g, const FinishInfo& fin, int nsrc) {
 void launch_stress3d(const Geo& g, const double* q, double* S, hipStream_t st) {
   const dim3 gg = grad3d_grid(g);
   const int zc = grad3d_chunk(g);
-  if (g.power_law > 0.0)
-    k_grad3d_periodic<kG3X, kG3Y, true, true><<<gg, kG3X * kG3Y, 0, st>>>(g, zc, q, S);
-  else
-    k_grad3d_periodic<kG3X, kG3Y, true, false><<<gg, kG3X * kG3Y, 0, st>>>(g, zc, q, S);
+  with_offsets(g, [&](auto o) {
+    using O = decltype(o);
+    if (g.power_law > 0.0)
+      k_grad3d_periodic<kG3X, kG3Y, true, true, O><<<gg, kG3X * kG3Y, 0, st>>>(g, zc, q, S);
+    else
+      k_grad3d_periodic<kG3X, kG3Y, true, false, O><<<gg, kG3X * kG3Y, 0, st>>>(g, zc, q, S);
+  });
 }
 
 void launch_fwd3d_march(const Geo& g, const double* q, const double* S, const double* kstr,
@@ -2359,9 +2383,14 @@ void launch_fwd3d_march(const Geo& g, const double* q, const double* S, const do
   with_march(g, false, [&](auto X) {
     constexpr int BX = decltype(X)::value, BY = kMarchRows;
     with_stage(g, rk ? rk->stage : 0, [&](auto ST, auto NT) {
-      k_fwd3d_march<BX, BY, decltype(ST)::value, decltype(NT)::value><<<gm, BX * BY, 0, st>>>(
-          g, zc, q, S, kstr, rhs, rk ? rk->dt : 0.0, rk ? rk->yout : nullptr, rk ? rk->b1 : nullptr,
-          rk ? rk->b2 : nullptr, rk ? rk->copy : nullptr);
+      const auto go = [&](auto nt, auto o) {
+        k_fwd3d_march<BX, BY, decltype(ST)::value, decltype(nt)::value, decltype(o)>
+            <<<gm, BX * BY, 0, st>>>(g, zc, q, S, kstr, rhs, rk ? rk->dt : 0.0,
+                                     rk ? rk->yout : nullptr, rk ? rk->b1 : nullptr,
+                                     rk ? rk->b2 : nullptr, rk ? rk->copy : nullptr);
+      };
+      if (g.wide) go(std::true_type{}, 0ul);   // far above the size from which it streams
+      else go(NT, 0u);
     });
   });
   if (rk && rk->ev_end) (void)hipEventRecord(rk->ev_end, st);

@@ -75,6 +75,7 @@ struct Geo {
                             // stress pass
   int mtile;                // x extent of the forward march tiles (16 or 32; 16 rows)
   int zchunk_adj, mtile_adj;  // the same for the adjoint marches
+  int wide;                 // component arrays that 32-bit byte offsets do not reach
 };
 
 // Device patch descriptor.

@@ -474,6 +474,10 @@ int ensure_adjoint(mgd_region* r) {
   return MGD_OK;
 }
 
+// Whether the 3-D marches need 64-bit byte offsets into a component array of n points: the 32-bit
+// ones keep 4 KiB beyond the end for the stores that they drop.
+int wide_grid(long n) { return n >= (1L << 29) - 1024; }
+
 int n_act(const mgd_region* r) { return r->ip_act < 0 ? 0 : r->patches[r->ip_act]->np; }
 int n_cost(const mgd_region* r) { return r->ip_cost < 0 ? 0 : r->patches[r->ip_cost]->np; }
 const DPatch* dpatch(const mgd_region* r, int ip) {
@@ -1910,7 +1914,7 @@ int limits_outcome(mgd_region* r, double* J, double* sensitivity) {
 // (control, source amplitudes, states) live in those buffers and are re-uploaded before
 // each replay.  Captured work holds kernels, copies, fills and event waits only.
 std::vector<uintptr_t> graph_key(mgd_region* r, int kind, std::initializer_list<uintptr_t> extra) {
-  std::vector<uintptr_t> k = {(uintptr_t)kind, (uintptr_t)r->tiling.shape, (uintptr_t)fused_ok(r), (uintptr_t)line_ok(r),
+  std::vector<uintptr_t> k = {(uintptr_t)kind, (uintptr_t)r->geo.wide, (uintptr_t)r->tiling.shape, (uintptr_t)fused_ok(r), (uintptr_t)line_ok(r),
                               (uintptr_t)r->ctrl_stride, (uintptr_t)r->src_inst_stride,
                               (uintptr_t)r->chunk, (uintptr_t)r->ck.nsteps, (uintptr_t)r->ck.K,
                               (uintptr_t)r->resident, (uintptr_t)r->dual};
@@ -2426,6 +2430,7 @@ int mgd_region_create(const mgd_region_desc* d, const double* coords, mgd_region
   g.composite = d->composite_dissipation;
   g.zchunk = g.zchunk_adj = 64;
   g.mtile = g.mtile_adj = 16;
+  g.wide = wide_grid(N);
   if (int rc = scratch_setup(&r->device)) return rc;
   MGD_HIP(hipStreamCreate(&r->stream));
   MGD_HIP(hipEventCreate(&r->ev0));
@@ -2826,6 +2831,11 @@ int mgd_region_set_option(mgd_region* r, int option, int value) {
       r->opt_mtile = value;
       r->geo.mtile = r->geo.mtile_adj = value == 0 ? 16 : value;
       r->zc_tuned = value != 0 && r->opt_zchunk != 0;
+      return MGD_OK;
+    case MGD_OPT_WIDE_OFFSETS:
+      if (value != 0 && value != 1) { set_error("wide offsets: 0 (by size) or 1"); return MGD_ERR_ARG; }
+      r->geo.wide = value || wide_grid(r->N);
+      r->zc_tuned = r->opt_zchunk != 0 && r->opt_mtile != 0;
       return MGD_OK;
     case MGD_OPT_TILE_SHAPE: {
       if (value < -1 || value >= kNumTileShapes) { set_error("tile shape must be -1 .. 5"); return MGD_ERR_ARG; }
