@@ -1240,13 +1240,16 @@ double* cached_window(mgd_region* r, int lt) {
 // Device memory a new storage plan of a checkpointed run may take: what is free plus the
 // storage held for earlier runs, less a reserve of max(8 GiB, 1/32 of the device) for
 // what the runtime and other allocations of the process take later.
-size_t storage_budget(mgd_region* r) {
+// `slack`: how far into the reserve storage held from an earlier run may stay.
+size_t storage_budget(mgd_region* r, size_t* slack = nullptr) {
   size_t fr = 0, tot = 0;
+  if (slack) *slack = 0;
   if (hipMemGetInfo(&fr, &tot) != hipSuccess) return 0;
   size_t held = r->window.bytes() + r->window2.bytes() + r->snaps.bytes() + r->sstore.bytes() +
                 r->scache.bytes() + r->sbuf.bytes() + r->gcache.bytes() + r->wall.bytes();
   for (int k = 0; k < mgd_region::kMaxCache; ++k) held += r->wcache[k].bytes();
   const size_t reserve = std::max((size_t)8 << 30, tot / 32);
+  if (slack) *slack = reserve / 2;
   return fr + held > reserve ? fr + held - reserve : 0;
 }
 
@@ -1279,13 +1282,12 @@ int plan_window_cache(mgd_region* r, int nsteps, int K, long M) {
 
 // Entries that a cache of `unit`-double entries should have, of which `buf` holds some: `plan`,
 // or what it holds where that serves (at most `most` entries), is no more than a sixteenth (or
-// two) below the plan, and fits in `room` bytes.  The free memory moves a little between runs,
-// so 2 GiB of the reserve of storage_budget count as room; what other regions took since does
-// not make a cache that still fits smaller, else two regions running in turn would allocate
-// theirs again in every run.
+// two) below the plan, and fits in `room` bytes.  Allocating a cache again costs more than the
+// run (172 GB: 5 s), so what this region allocated after its first plan, or other regions since,
+// does not make one that still fits smaller.
 int cache_entries(const DevBuf& buf, size_t unit, int plan, int most, size_t room) {
   const int have = unit > 0 && buf.n % unit == 0 ? (int)(buf.n / unit) : 0;
-  const bool fits = have > 0 && have <= most && buf.bytes() <= room + ((size_t)2 << 30);
+  const bool fits = have > 0 && have <= most && buf.bytes() <= room;
   return fits && plan > 0 && plan <= have + std::max(2, have / 16) ? have : plan;
 }
 
@@ -1334,26 +1336,28 @@ int plan_plain_storage(mgd_region* r, int nsteps, int K, long M) {
   r->nscache = r->ngcache = 0;
   const bool allowed = !(fused && r->group_run);
   bool step = r->opt_step == 1 && allowed;
-  size_t budget = 0;
+  size_t budget = 0, slack = 0;
   if (r->opt_step != 0 && allowed) {
-    budget = storage_budget(r);
-    if (r->opt_step < 0) step = r->opt_cache < 0 && (size_t)(nsteps + nrec) * S <= budget;
+    budget = storage_budget(r, &slack);
+    // the store of an earlier run of this length stays as far as the slack reaches
+    const size_t room = r->sstore.n == (size_t)nsteps * M ? budget + slack : budget;
+    if (r->opt_step < 0) step = r->opt_cache < 0 && (size_t)(nsteps + nrec) * S <= room;
   }
   if (step) {
     size_t fixed = (size_t)(nsteps + nrec) * S;
     const size_t GB = r->G.bytes();
+    const auto left = [](size_t total, size_t taken) { return total > taken ? total - taken : 0; };
     bool reuse = !fused && stress_reuse_path(r->geo, r->fin, (int)r->sources.size()) && GB > 0 &&
-                 fixed + 3 * GB <= budget;
+                 fixed + 3 * GB <= (r->sbuf.n == 3 * r->G.n ? budget + slack : budget);
     if (reuse) fixed += 3 * GB;
-    size_t rest = budget > fixed ? budget - fixed : 0;
     const int most = r->opt_cache < 0 ? nsteps : (int)std::min((long)nsteps, (long)r->opt_cache * K);
-    int nsc = (int)std::min<size_t>((size_t)most, rest / (3 * S));
-    nsc = cache_entries(r->scache, (size_t)3 * M, nsc, most, rest);
-    rest = rest > 3 * S * nsc ? rest - 3 * S * nsc : 0;
+    int nsc = (int)std::min<size_t>((size_t)most, left(budget, fixed) / (3 * S));
+    nsc = cache_entries(r->scache, (size_t)3 * M, nsc, most, left(budget + slack, fixed));
+    fixed += 3 * S * nsc;
     int ngc = 0;
     if (reuse && r->opt_cache < 0) {
-      ngc = (int)std::min<size_t>((size_t)nsc, rest / 2 / (4 * GB));
-      ngc = cache_entries(r->gcache, 4 * r->G.n, ngc, nsc, rest);
+      ngc = (int)std::min<size_t>((size_t)nsc, left(budget, fixed) / 2 / (4 * GB));
+      ngc = cache_entries(r->gcache, 4 * r->G.n, ngc, nsc, left(budget + slack, fixed));
     }
     for (int k = 0; k < mgd_region::kMaxCache; ++k) r->wcache[k].release();
     r->ncache = 0;

@@ -103,3 +103,29 @@ def test_two_regions_in_turn_keep_their_storage():
     finally:
         del filler
         torch.cuda.empty_cache()
+
+
+def test_other_allocations_leave_the_storage_as_it_is():
+    """3 GB that the process takes after a region's first run, far less than the reserve is for:
+    the next runs keep that run's storage and allocate nothing."""
+    import torch
+    from magudi_amd import cases
+    c = cases.kolmogorov3d(n=128, nsteps=300)
+    q0 = c.initial_state()
+    filler = _fill(c, 1)
+    later = None
+    try:
+        R = _region(c)
+        first = _run(R, c, 300, q0)
+        assert 0 < first[0]["held"] < 300
+        later = torch.empty(3 << 30, dtype=torch.uint8, device="cuda")
+        free = torch.cuda.mem_get_info()[0]
+        for _ in range(2):
+            plan, J, lam = _run(R, c, 300, q0)
+            print(f"storage beside 3 GB more: {plan} after {first[0]}", flush=True)
+            assert plan == first[0] and torch.cuda.mem_get_info()[0] == free
+            assert J == first[1] and np.array_equal(lam, first[2])
+        R.close()
+    finally:
+        del filler, later
+        torch.cuda.empty_cache()
