@@ -21,12 +21,12 @@ struct MarchShape {
 };
 
 // Tile widths of 16 and 32 points, unless one is fixed (opt_tile), with a fixed chunk
-// (opt_chunk) as it is; else with every chunk of 32, 64 and 128 planes but those that leave most
-// of the GPU idle (fewer units than half its 256 CUs, unless a chunk of 32 is no better off), and
-// shorter ones only where 32 planes do not fill it: their units spend most of their planes on the
-// z windows' lead-in.  Among those the one whose units just fill the GPU in one go (two
-// work-groups of a 16-wide tile per CU, one of a 32-wide): forward and adjoint run of 64^3 8.1 ms
-// at 8 planes, 5.8 at 4, 5.7 at 2; of 100^3 16.6 at 8, 14.5 at 10.
+// (opt_chunk) as it is; else with chunks of 32, 64 and 128 planes, and shorter ones only where 32
+// planes do not fill the GPU: their units spend most of their planes on the z windows' lead-in.
+// Among those the one whose units just fill the GPU in one go (two work-groups of a 16-wide tile
+// per CU, one of a 32-wide): forward and adjoint run of 64^3 8.1 ms at 8 planes, 5.8 at 4, 5.7 at
+// 2; of 100^3 16.6 at 8, 14.5 at 10.  Chunks that leave half of the 256 CUs without a unit are not
+// tried (64^3, forward step: 0.15 ms at 4 planes, 0.34 at 16, 0.62 at 32), but for the shortest.
 inline std::vector<MarchShape> march_shapes(const int* n, int instances, int opt_tile,
                                             int opt_chunk) {
   std::vector<MarchShape> shapes;
@@ -37,17 +37,18 @@ inline std::vector<MarchShape> march_shapes(const int* n, int instances, int opt
       continue;
     }
     const auto units = [&](int zc) { return (long)instances * march_units(n, tile, zc); };
+    std::vector<int> chunks = {32, 64, 128};
     if (units(32) < 512) {
       const long columns = units(n[2]), room = tile == 32 ? 256 : 512;
       const int fill = columns <= room ? (int)((n[2] + room / columns - 1) / (room / columns)) : 0;
-      if (units(8) < 256) shapes.push_back({tile, 4});
-      shapes.push_back({tile, 8});
-      shapes.push_back({tile, 16});
-      if (fill >= 2 && fill < 32 && fill != 8 && fill != 16 && !(fill == 4 && units(8) < 256))
-        shapes.push_back({tile, fill});
+      chunks.push_back(8);
+      chunks.push_back(16);
+      if (units(8) < 256 || fill == 4) chunks.push_back(4);
+      if (fill >= 2 && fill < 32 && fill != 4 && fill != 8 && fill != 16) chunks.push_back(fill);
     }
-    for (int chunk : {32, 64, 128})
-      if (chunk == 32 || units(chunk) >= 128) shapes.push_back({tile, chunk});
+    const int least = *std::min_element(chunks.begin(), chunks.end());
+    for (int chunk : chunks)
+      if (chunk == least || units(chunk) >= 128) shapes.push_back({tile, chunk});
   }
   return shapes;
 }
