@@ -955,18 +955,21 @@ int tune_tiling(mgd_region* r) {
 // (stress pass and march per stage, out of place) and one adjoint RK stage (stress pass and
 // the two marches, where they serve the region) timed with HIP events for each shape of
 // march_shapes; the forward march (with the stress pass) and the adjoint marches each keep
-// their own.  No value depends on the shape.
+// their own.  No value depends on the shape.  The conserved and adjoint states are not touched.
 int tune_march(mgd_region* r) {
   r->zc_tuned = true;
   const long M = (long)r->ninst * M_of(r);
   if (int rc = ensure_adjoint(r)) return rc;
   if (r->qs.alloc(M) || r->qy.alloc(M) || r->qs_alt2.alloc(M)) return MGD_ERR_HIP;
   const double dt = 1e-3;
+  // an adjoint state to march back: the block that only the per-operator kernels use
+  double* const lam =
+      stress_reuse_path(r->geo, r->fin, (int)r->sources.size()) ? r->S.p : r->qy.p;
   // the state copies, one forward RK4 step, then (after event `mid`, if given) one adjoint stage
   auto round_trip = [&](hipEvent_t mid = nullptr) {
     launch_copy(M, r->q.p, r->qs.p, r->stream);
     launch_copy(M, r->q.p, r->b2.p, r->stream);
-    launch_copy(M, r->q.p, r->lam.p, r->stream);
+    launch_copy(M, r->q.p, lam, r->stream);
     // the stages as the runs issue them: qs -> qy -> qs_alt2 -> qy -> qs, stages 2 and 3
     // reading the state at the start of the step from qs
     double* const in[4] = {r->qs.p, r->qy.p, r->qs_alt2.p, r->qy.p};
@@ -977,8 +980,8 @@ int tune_march(mgd_region* r) {
       launch_fwd3d_march(r->geo, rk.y, r->G.p, r->fin.kolmogorov, r->rhs.p, &rk, r->stream);
     }
     if (mid) (void)hipEventRecord(mid, r->stream);
-    const RkStage rk{3, dt, r->lam.p, r->qy.p, r->qs_alt2.p, nullptr};
-    launch_rhs_adjoint(r->geo, dpatches(r), r->qs.p, r->lam.p, r->rhs.p, r->w.p, r->G.p, r->t.p,
+    const RkStage rk{3, dt, lam, r->qy.p, r->qs_alt2.p, nullptr};
+    launch_rhs_adjoint(r->geo, dpatches(r), r->qs.p, lam, r->rhs.p, r->w.p, r->G.p, r->t.p,
                        r->T1.p, r->S.p, nullptr, 0, 1.0, r->fin, r->stream, &rk);
   };
   const std::vector<MarchShape> shapes =

@@ -97,3 +97,33 @@ def test_rhs_on_overlap_grids(overlap, kind):
                 ref = out
             else:
                 assert np.array_equal(out, ref), (mode, units)
+
+
+@pytest.mark.parametrize("shape", [(33, 20, 35), (32, 16, 40)])
+@pytest.mark.parametrize("kind", ["viscous", "inviscid", "sponge"])
+def test_autotuner_leaves_the_adjoint_state(shape, kind):
+    """An adjoint state put before a region's first call, which is when the tuner runs, is the one
+    that this call marches back, or leaves as it is."""
+    from magudi_amd.solver import Region, RK4Integrator, Solver
+    c = inviscid_box(shape) if kind == "inviscid" else periodic_box(shape, dissipation=False)
+    if kind == "sponge":
+        c = _plain(c)
+    q = perturbed(c, 67)
+    lam = np.random.default_rng(68).standard_normal((c.nv, c.npoints))
+    out = []
+    for fixed in (True, False):
+        R = Region(c)
+        if fixed:
+            R.set_march_tile(16)
+            R.set_z_chunk(32)
+        R.states[0].conservedVariables = q
+        R.states[0].adjointVariables = lam
+        R.updateAdjointForcing(no_adjoint_forcing=True)
+        RK4Integrator().substepAdjoint(R, 0.0, c.dt, 1, 4)
+        out.append(R.states[0].adjointVariables)
+    assert np.array_equal(out[0], out[1]) and not np.array_equal(out[0], lam)
+    R = Region(c)
+    R.states[0].conservedVariables = q
+    R.states[0].adjointVariables = lam
+    Solver(R, dt=c.dt, nsteps=1, save_interval=1).runForward()
+    assert np.array_equal(R.states[0].adjointVariables, lam)
