@@ -3,8 +3,9 @@
 // The runtime's own pageable device-to-host copy moves the data with one thread, which also
 // takes the page faults of a fresh destination: 10 GB/s.  Here chunks of 2 MiB (the huge page
 // that backs large arrays, so no two threads fault on one) arrive in pinned slots and several
-// threads copy them out: 671 MB 65 -> 18 ms, 40 MB 4.2 -> 1.4 ms, 8.4 MB 1.1 -> 0.7 ms, 5.1 MB
-// 0.8 -> 0.65 ms.  Below kLeast the threads cost more than they save (2.4 MB 0.56 -> 0.63 ms).
+// threads copy them out, into a fresh array: 671 MB 64 -> 16.8 ms, 41 MB 4.0 -> 1.3 ms, 8.4 MB
+// 0.48 -> 0.32 ms, 5.2 MB 0.29 -> 0.22 ms.  Below kLeast the threads cost more than they save
+// (2.4 MB, with the array's allocation, 0.56 -> 0.63 ms).
 // The slots are as many as a copy needs, sixteen at most: pinning them takes 0.1 ms per MB
 // once.  Host-to-device copies have no faults to share and stay as they are.
 #include "hostcopy.h"

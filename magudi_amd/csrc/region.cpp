@@ -1324,7 +1324,7 @@ double* kept_stress(mgd_region* r, int t, int i) {
 // (sreuse) and, as half of what is then left of the budget takes (none where the caller limits
 // the held steps), those that the forward stages of the last held steps formed of their inputs,
 // which the adjoint stages at the same states need: they save the adjoint pass its stress
-// kernel, 468 of 2160 us per stage on 256^3, 47 of 226 on 100^3, 20 of 79 on 64^3.
+// kernel, 453 of 2424 us per stage on 256^3, 38 of 197 on 100^3, 15 of 56 on 64^3.
 // The whole plan is made first, and what it does not keep of an earlier run's storage is given
 // back before anything is allocated: the budget counts all of that as free.
 // Window mode (always for the fused members of a group launch): snapshots every K steps, a
