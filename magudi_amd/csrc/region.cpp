@@ -1291,7 +1291,7 @@ int plan_window_cache(mgd_region* r, int nsteps, int K, long M) {
 int cache_entries(const DevBuf& buf, size_t unit, int plan, int most, size_t room) {
   const int have = unit > 0 && buf.n % unit == 0 ? (int)(buf.n / unit) : 0;
   const bool fits = have > 0 && have <= most && buf.bytes() <= room;
-  return fits && plan > 0 && plan <= have + std::max(2, have / 16) ? have : plan;
+  return fits && plan <= have + std::max(2, have / 16) ? have : plan;
 }
 
 // Allocates `want` entries of `unit` doubles, or half as many for as long as they do not fit.
